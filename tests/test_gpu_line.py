@@ -1,0 +1,104 @@
+"""The Kelsall registry kernels on the ray's line (``forward_line``).
+
+Against the oracle and against the kind switch (variant 0) where the line kernels can go
+wrong: rays through the Sun and at the poles, pointings normal to the observer's
+direction, observers off the plane and outside cut-off spheres, exponents at the ends
+of the range the kernels accept (and just outside, where the general kernel runs), ray
+counts around the block and lane edges. Tolerance: the framework's parity bound, 1e-10
+relative per value; the node radius (5e-15) enters the values at most to its 20th power
+and, through exp(-zeta^6), with the exponent (below 746) times six, so 5e-15 x 4476 =
+2e-11 bounds what two evaluations may differ by.
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import zodi_oracle
+from oracle.zodi_oracle import OracleModel
+from zodipy_amd import Model, healpix
+from zodipy_amd import units as u
+from zodipy_amd._lib import Launch
+from zodipy_amd.runtime import OUT_COMPS
+
+pytestmark = pytest.mark.gpu
+
+RTOL = 1e-10
+
+
+def pointings(obs):
+    """Map pixels plus the directions at which the geometry degenerates."""
+    o = np.asarray(obs) / np.linalg.norm(obs)
+    normal = np.array([-o[1], o[0], 0.0]) / np.hypot(o[0], o[1])
+    special = [[0, 0, 1], [0, 0, -1], [1, 0, 0], [0, 1, 0], [0, -1, 0], -o, o, normal,
+               [np.sin(1e-9), 0, np.cos(1e-9)], [-np.cos(1e-7), np.sin(1e-7), 0]]
+    return np.concatenate([healpix.pix2vec(4), np.array(special, dtype=float).T], axis=1)
+
+
+def same(got, want):
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    ok = ~np.isnan(want)
+    zero = ok & (want == 0)
+    assert np.all(got[zero] == 0)
+    ok &= ~zero
+    rel = np.abs(got[ok] - want[ok]) / np.abs(want[ok])
+    assert rel.max(initial=0.0) <= RTOL, rel.max()
+
+
+def both(model, v, obs):
+    dm = model.device_model
+    a = dm.forward(v, obs, obs, out_mode=OUT_COMPS).cpu().numpy()
+    b = dm.forward(v, obs, obs, out_mode=OUT_COMPS, launch=Launch(variant=0)).cpu().numpy()
+    return a, b
+
+
+@pytest.mark.parametrize("x", [25 * u.micron, 1.25 * u.micron])
+@pytest.mark.parametrize("obs", [(1.0, 0.0, 0.0), (0.0, 0.9, 0.0), (0.7, -0.6, 0.3),
+                                 (0.0, 0.0, 1.1), (1.25, 0.1, 0.0), (3.0, 2.0, 0.1)])
+def test_degenerate_directions_against_oracle(gpu, monkeypatch, x, obs):
+    # within 1e-7 of the directions to and from the Sun the arc cosine of a rounded cosine
+    # holds only half the digits; the oracle takes the same angle from its tangent
+    def angle(R_los, R_helio, X_los, X_helio):
+        cross = np.cross(X_los, X_helio, axis=0)
+        return np.arctan2(np.sqrt((cross**2).sum(axis=0)), -(X_los * X_helio).sum(axis=0))
+
+    monkeypatch.setattr(zodi_oracle, "get_scattering_angle", angle)
+    obs = np.array(obs)
+    v = pointings(obs if obs[0] or obs[1] else obs + [1e-3, 0, 0])
+    got = Model(x).device_model.forward(v, obs, obs, out_mode=OUT_COMPS).cpu().numpy()
+    same(got, OracleModel(x).evaluate_vectors(v, obs, obs))
+
+
+# delta and alpha up to 2 and gamma in [1/2, 6] run on the line, the rest in general.
+@pytest.mark.parametrize("change", [{"delta": 2.0}, {"delta": 2.01}, {"delta": 0.0},
+                                    {"delta": -0.3}, {"alpha": 2.0}, {"alpha": 2.2},
+                                    {"alpha": 0.0}, {"gamma": 0.5}, {"gamma": 0.49},
+                                    {"gamma": 6.0}, {"gamma": 1.0}, {"beta": 60.0},
+                                    {"mu": 1e-3}, {"mu": 2.0}])
+def test_exponents_against_general_kernel(gpu, change):
+    model = Model(25 * u.micron)
+    p = model.get_parameters()
+    for k, v in change.items():
+        if k in p:
+            p[k] = v
+        else:
+            p["comps"]["cloud"][k] = v
+    model.update_parameters(p)
+    obs = np.array([0.98, 0.17, 0.004])
+    got, want = both(model, pointings(obs), obs)
+    same(got, want)
+
+
+@pytest.mark.parametrize("n", [1, 31, 32, 33, 63, 65, 255, 257, 1023])
+@pytest.mark.parametrize("lanes", [0, 1, 2, 4, 8])
+def test_ragged_counts(gpu, n, lanes):
+    obs = np.array([0.99, 0.1, 0.0])
+    model = Model(12 * u.micron)
+    v = healpix.pix2vec(16)[:, ::3][:, :n]
+    got = model.device_model.forward(v, obs, obs, out_mode=OUT_COMPS,
+                                     launch=Launch(variant=1, lanes_per_ray=lanes)).cpu().numpy()
+    want = model.device_model.forward(torch.as_tensor(healpix.pix2vec(16)[:, ::3].copy()), obs,
+                                      obs, out_mode=OUT_COMPS).cpu().numpy()[:, :n]
+    assert np.array_equal(got, want)

@@ -26,6 +26,7 @@ HEADERS = [
     CSRC / "zodi_common.hpp",
     CSRC / "zodi_device.hpp",
     CSRC / "zodi_grad.hpp",
+    CSRC / "zodi_line.hpp",
     CSRC / "zodi_math.hpp",
     CSRC / "zodi_trig.hpp",
     CSRC / "zodi_trig_coeffs.inc",

@@ -4,10 +4,12 @@
 #include <hip/hip_runtime.h>
 
 #include <initializer_list>
+#include <tuple>
 #include <utility>
 
 #include "zodi_device.hpp"
 #include "zodi_hip.h"
+#include "zodi_line.hpp"
 
 namespace zodi {
 
@@ -80,24 +82,14 @@ struct Ray {
   RayGeom G;
   uint32_t bits;
   int64_t r;
+  int64_t s;  // its observer's row
   bool active;
 };
 
-template <int RAYS>
-__device__ __forceinline__ Ray load_ray(const FwdArgs& a, int64_t tile, int local) {
-  Ray y;
-  const int64_t n = a.n_rays;
-  y.r = tile * RAYS + local;
-  y.active = y.r < n;
+// The values of ray y.r (past the last ray, of the last one) and its observer.
+__device__ __forceinline__ void read_ray(const FwdArgs& a, Ray& y) {
+  const int64_t n = a.n_rays, s = y.s;
   const int64_t rr = y.active ? y.r : n - 1;
-  int64_t s;
-  if (a.obs_mode == ZODI_OBS_PER_RAY) {
-    s = rr;
-  } else {
-    const int64_t s0 = find_segment(a.seg, a.n_seg, tile * RAYS);
-    s = walk_segment(a.seg, a.n_seg, s0, rr);
-  }
-  y.bits = a.beyond[a.obs_mode == ZODI_OBS_PER_RAY ? 0 : s];
   const double* __restrict__ U = a.u;
   y.ux = U[rr];
   y.uy = U[n + rr];
@@ -109,6 +101,23 @@ __device__ __forceinline__ Ray load_ray(const FwdArgs& a, int64_t tile, int loca
   y.ex = a.earth[s];
   y.ey = a.earth[os + s];
   y.G = ray_geometry(y.ux, y.uy, y.uz, y.ox, y.oy, y.oz);
+}
+
+template <int RAYS>
+__device__ __forceinline__ Ray load_ray(const FwdArgs& a, int64_t tile, int local) {
+  Ray y;
+  const int64_t n = a.n_rays;
+  y.r = tile * RAYS + local;
+  y.active = y.r < n;
+  const int64_t rr = y.active ? y.r : n - 1;
+  if (a.obs_mode == ZODI_OBS_PER_RAY) {
+    y.s = rr;
+  } else {
+    const int64_t s0 = find_segment(a.seg, a.n_seg, tile * RAYS);
+    y.s = walk_segment(a.seg, a.n_seg, s0, rr);
+  }
+  y.bits = a.beyond[a.obs_mode == ZODI_OBS_PER_RAY ? 0 : y.s];
+  read_ray(a, y);
   return y;
 }
 
@@ -567,5 +576,113 @@ __device__ __forceinline__ Ctx make_ctx(ModelPtr M, const double* sTab, int sub)
   return cx;
 }
 
+
+
+// ---------------------------------------------------------- line kernels (Kelsall)
+template <int KIND, int CUT>
+__device__ __forceinline__ double line_density(ParamPtr P, const LineComp<KIND>& c,
+                                               const LineCtx& cx, const Line& l,
+                                               const LineNode& nd, double& cut) {
+  if constexpr (KIND == ZODI_CLOUD) return line_cloud(P, c, cx, nd);
+  if constexpr (KIND == ZODI_BAND) return line_band<CUT>(P, c, cx, nd, cut);
+  if constexpr (KIND == ZODI_RING) return line_ring(P, c, cx, nd);
+  if constexpr (KIND == ZODI_FEATURE) return line_feature(P, c, cx, l, nd);
+}
+
+// One group of a Kelsall registry layout for one ray: group_pass on the ray's line.
+// PROPS: only its kShareCut bits are read (every band is centred with p = 4, every other
+// component but the cloud centred; the host checks, props_match and line_match).
+template <int L, uint32_t PROPS, bool NOSCAT, int... Ks, int... J>
+__device__ __forceinline__ void line_group(Grp<Ks...>, std::integer_sequence<int, J...>,
+                                           const LineCtx& cx, const FwdArgs& a, const Ray& y,
+                                           const Line& l, int g, int first, double& total) {
+  constexpr int C = sizeof...(Ks);
+  constexpr int kinds[C] = {Ks...};
+  const ModelPtr M = cx.M;
+  double h, mid;
+  group_range(M, g, y, h, mid);
+  const double th = l.n * h, tm = fma(l.n, mid, l.t0);  // t = th x + tm
+  const std::tuple<LineComp<Ks>...> lc{LineComp<Ks>(M->comp[first + J], l, y.ex, y.ey)...};
+  bool scatter = false;
+  if constexpr (!NOSCAT) {
+    ((scatter = scatter || (M->comp_flags[first + J] & ZODI_CF_SCATTER)), ...);
+  }
+  LinePhase lp = {0.0, 0.0};
+  if (scatter) lp = line_phase(l);
+  double acc[C] = {};
+  for (int k0 = 0; k0 < cx.K; k0 += L) {
+    // with L lanes a ray, lane `sub` takes node k0 + sub (past the last node it repeats
+    // that one, and its term is not added)
+    const int k = L == 1 ? k0 : (k0 + cx.sub < cx.K ? k0 + cx.sub : cx.K - 1);
+    const ModelPtr Mk = opaque(M);
+    const double wk = Mk->gl_w[k];
+    LineNode nd;
+    nd.t = fma(th, Mk->gl_x[k], tm);
+    nd.R2 = fma(nd.t, nd.t, l.d2);
+    norm_and_inverse_node(nd.R2, nd.R, nd.inv_R);
+    Node tn;  // what node_term reads
+    tn.inv_R = nd.inv_R;
+    tn.B = planck_shifted(pow_table(cx.tab->temperature, cx.pt, nd.R2) - cx.uo1, cx.tab->planck);
+    tn.phi = 0.0;
+    if constexpr (!NOSCAT) {
+      if (scatter) tn.phi = line_phase_function(lp, l, cx.ec, nd.t, Mk->shared);
+    }
+    const double wB = wk * tn.B;
+    double cut = 0.0;  // a band's cut-off, for the bands that share it (in order)
+    NodeTerm t[C];
+    ((t[J] = node_term<ZODI_INTEGRAND_KELSALL, NOSCAT>(
+          Mk->comp[first + J], Mk->comp_flags[first + J], tn, wk, wB,
+          line_density<kinds[J], cut_mode<PROPS, J, Ks...>()>(Mk->comp[first + J],
+                                                              std::get<J>(lc), cx, l, nd, cut),
+          Mk->shared[ZODI_S_SOLAR])),
+     ...);
+    if constexpr (L == 1) {
+      ((acc[J] = node_add(acc[J], t[J])), ...);
+    } else {
+      add_in_node_order<L>(acc, t, cx.K - k0);
+    }
+  }
+  const bool write = y.active && cx.sub == 0;
+  (
+      [&] {
+        const double e = finish<ZODI_INTEGRAND_KELSALL, NOSCAT>(
+            M->comp[first + J], M->comp_flags[first + J], acc[J], h, 0.0);
+        if (a.out_mode == ZODI_OUT_COMPS) {
+          if (write) a.out[(int64_t)(first + J) * a.n_rays + y.r] = e;
+        } else {
+          total = __dadd_rn(total, e);
+        }
+      }(),
+      ...);
+}
+
+template <int L, uint32_t PROPS, bool NOSCAT, int INTEGRAND, class... Gs, int... G>
+__device__ __forceinline__ void run_line_groups(Layout<INTEGRAND, Gs...>,
+                                                std::integer_sequence<int, G...>,
+                                                const LineCtx& cx, const FwdArgs& a, Ray& y,
+                                                double& total) {
+  (
+      [&] {
+        // The first group's node loop needs the registers: what the later groups take
+        // from the ray is read and formed again (L2 holds it) instead of living across it.
+        if constexpr (G == 1) {
+          FwdArgs again = a;
+          asm volatile("" : "+s"(again.u), "+s"(again.obs), "+s"(again.earth));
+          read_ray(again, y);
+        }
+        const Line l = make_line(y.ux, y.uy, y.uz, y.ox, y.oy, y.oz);
+        line_group<L, props_shift(PROPS, group_first<Gs...>(G)), NOSCAT>(
+            Gs{}, std::make_integer_sequence<int, Gs::size>{}, cx, a, y, l, G,
+            group_first<Gs...>(G), total);
+      }(),
+      ...);
+}
+
+template <int L, uint32_t PROPS, bool NOSCAT, int INTEGRAND, class... Gs>
+__device__ __forceinline__ void run_line(Layout<INTEGRAND, Gs...> lay, const LineCtx& cx,
+                                         const FwdArgs& a, Ray& y, double& total) {
+  run_line_groups<L, PROPS, NOSCAT>(lay, std::make_integer_sequence<int, sizeof...(Gs)>{}, cx, a,
+                                    y, total);
+}
 
 }  // namespace zodi

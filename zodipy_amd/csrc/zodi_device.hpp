@@ -103,30 +103,45 @@ struct RayGeom {
   double r_obs;
 };
 
-// Not inlined: the trigonometric routines' literal coefficients then live only
-// inside this once-per-ray call instead of in vector registers across the
-// kernels' node loops (where they were spilled to scratch); the call costs a
-// few instructions per ray.
-__device__ __attribute__((noinline)) RayGeom ray_geometry(double ux, double uy, double uz,
-                                                          double ox, double oy, double oz) {
-  const double lon = atan2(uy, ux);
-  const double lat = asin(uz);
-  const double cos_lat = cos(lat);
+// The trigonometric form, for the pointings the algebraic one leaves to it. Not inlined:
+// the routines' literal coefficients then live only inside this rare call.
+__device__ __attribute__((noinline)) double ray_linear_trig(double ux, double uy, double uz,
+                                                            double ox, double oy) {
+  const double cos_lat = cos(asin(uz));
   double sl, cl;
-  sincos(lon, &sl, &cl);
+  sincos(atan2(uy, ux), &sl, &cl);
+  return 2.0 * (ox * cos_lat * cl + oy * cos_lat * sl);
+}
+
+// cos(lat) = sqrt(1 - uz^2) (the FMA rounds 1 - uz^2 once), cos(lon) and sin(lon) as
+// (ux, uy) over their length: the same b to rounding without the four trigonometric
+// routines. Left to them are the pointings at which the reference's values come
+// from the rounding of pi: the poles, a pointing normal to the observer's direction
+// (cos(pi/2) = 6e-17 there, so b is not the exact 0 that gives NaN), and |uz| > 1 or a
+// non-finite pointing (NaN).
+__device__ __forceinline__ RayGeom ray_geometry(double ux, double uy, double uz, double ox,
+                                                double oy, double oz) {
   RayGeom g;
-  g.b = 2.0 * (ox * cos_lat * cl + oy * cos_lat * sl);
-  g.r_obs = sqrt(ox * ox + oy * oy + oz * oz);
+  const double rho2 = fma(ux, ux, uy * uy), c2 = fma(-uz, uz, 1.0);
+  double rho, inv_rho, cos_lat, inv_cos;
+  norm_and_inverse(rho2, rho, inv_rho);
+  norm_and_inverse(c2, cos_lat, inv_cos);
+  g.b = 2.0 * ((cos_lat * inv_rho) * fma(ox, ux, oy * uy));
+  const bool plain = rho2 > 0x1p-900 && rho2 < 0x1p900 && c2 > 0.0;
+  if (!plain || g.b == 0.0) g.b = ray_linear_trig(ux, uy, uz, ox, oy);
+  const double r2 = fma(ox, ox, fma(oy, oy, oz * oz));
+  g.r_obs = sqrt(r2);
   return g;
 }
 
 // Distance from the observer to the heliocentric sphere of radius `cutoff`
 // (zodipy/line_of_sight.py:81-85): c = r_obs^2 - cutoff^2,
-// q = -b/2 (1 + sqrt(b^2 - 4c)/|b|), result max(q, c/q). b == 0 gives NaN.
+// q = -b/2 (1 + sqrt(b^2 - 4c)/|b|) = -(b + sign(b) sqrt(b^2 - 4c))/2, result
+// max(q, c/q). b == 0 gives NaN.
 __device__ __forceinline__ double sphere_distance(const RayGeom& g, double cutoff) {
   const double c = g.r_obs * g.r_obs - cutoff * cutoff;
-  const double q = -0.5 * g.b * (1.0 + sqrt(g.b * g.b - 4.0 * c) / fabs(g.b));
-  return np_maximum(q, c / q);
+  const double q = -0.5 * (g.b + __builtin_copysign(sqrt(g.b * g.b - 4.0 * c), g.b));
+  return g.b == 0.0 ? __builtin_nan("") : np_maximum(q, c / q);
 }
 
 // Linear interpolation in the Planck table with np.interp semantics, on the

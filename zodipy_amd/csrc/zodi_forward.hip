@@ -106,15 +106,11 @@ zodi_status validate_model(const zodi_model* m) {
 
 
 // Minimum waves per SIMD the register allocator must leave room for, per layout
-// (1 = no constraint). Measured on MI355X: DIRBE and Kelsall4 run at 5 (93 and
-// 84 VGPRs in their registry variants, 89 and 79 without scattering code, no
-// spill; DIRBE 2.7 % faster than at 4, and 6 waves with a spill gains nothing,
-// 0.8 % slower without scattering code); RRM at 4 (128 VGPRs with a small
+// (1 = no constraint). Measured on MI355X: RRM at 4 (128 VGPRs with a small
 // spill), 15 % faster than its unconstrained 190 VGPRs / 2 waves and 3.7 %
-// faster than 3 waves without the spill. The kind switch (forward_generic)
-// runs at 3. The split-lane variants (L > 1) run only where the
-// launch is small, so they ask for 2 and keep their registers (DIRBE: 98 VGPRs
-// instead of 96 with a 16-byte spill; 3072 rays at 8 lanes 36.2 -> 34.6 us).
+// faster than 3 waves without the spill; the Kelsall layouts at 5. The kind switch
+// (forward_generic) runs at 3. The split-lane variants (L > 1) run only where the
+// launch is small, so they ask for 2 and keep their registers.
 template <class LAYOUT>
 struct ForwardOccupancy {
   static constexpr int value = 1;
@@ -136,15 +132,10 @@ struct ForwardOccupancy<LayoutKelsall4> {
   static constexpr int value = 5;
 };
 
-// SPEC: every component's frame path and form fixed at compile time to the
-// registry models' (RegistryProps); the host runs it only for blocks that meet
-// its preconditions (props_match). SHARE (with SPEC): the bands that share a
-// radial cut-off reuse it (kShareCut), for blocks whose delta_r values allow it
-// (the registry parameters; a fit that moves them runs SPEC alone). NOSCAT (with
-// SHARE): no component scatters, so no scattering code is compiled in (no flag
-// test per component and node; 1.5-2 % faster on the DIRBE 12 um, planck18 and
-// six-component 857 GHz batches).
-template <class LAYOUT, int BLOCK, int L, bool SPEC, bool SHARE = false, bool NOSCAT = false>
+// SPEC: every component's frame path fixed at compile time to the registry models'
+// (RegistryProps); the host runs it only for blocks that meet its preconditions
+// (props_match).
+template <class LAYOUT, int BLOCK, int L, bool SPEC>
 __global__ __launch_bounds__(BLOCK)
 __attribute__((amdgpu_waves_per_eu(L == 1 ? ForwardOccupancy<LAYOUT>::value : 2))) void
 forward_layout(FwdArgs a) {
@@ -158,11 +149,36 @@ forward_layout(FwdArgs a) {
   for (int64_t tile = blockIdx.x; tile < a.n_tiles; tile += gridDim.x) {
     const Ray y = load_ray<RAYS>(a, tile, local);
     double total = 0.0;
-    constexpr uint32_t kProps =
-        !SPEC ? 0u
-              : (SHARE ? RegistryProps<LAYOUT>::value
-                       : props_without_share(RegistryProps<LAYOUT>::value));
-    run_layout<L, kProps, NOSCAT>(LAYOUT{}, cx, a, y, total);
+    constexpr uint32_t kProps = SPEC ? RegistryProps<LAYOUT>::value : 0u;
+    run_layout<L, kProps, false>(LAYOUT{}, cx, a, y, total);
+    if (a.out_mode == ZODI_OUT_SUM && y.active && cx.sub == 0) a.out[y.r] = total;
+  }
+}
+
+// The Kelsall layouts' registry blocks (props_match without the shared cut-off, and
+// line_match) on the ray's line (zodi_line.hpp): bound by FP64 vector issue, the three node
+// loops of the DIRBE layout take 1346 issue cycles per wave and node where forming every
+// node's position and its powers by exp(p log x) took 1968. Measured: DIRBE 12 um, 50.7 M
+// rays, 34.4 -> 25.2 ms (7.4e10 -> 1.01e11 ray-nodes/s);
+// planck18 857 GHz, 22.5 M rays, 8.29 -> 6.12 ms; DIRBE 1.25 um with scattering, 196 608
+// rays, 0.317 -> 0.26 ms. SHARE: the bands that share a radial cut-off reuse it
+// (kShareCut), for blocks whose delta_r values allow it (the registry parameters; a fit
+// that moves them runs without). NOSCAT (with SHARE): no component scatters, so no
+// scattering code is compiled in.
+template <class LAYOUT, int BLOCK, int L, bool SHARE, bool NOSCAT>
+__global__ __launch_bounds__(BLOCK)
+__attribute__((amdgpu_waves_per_eu(L == 1 ? ForwardOccupancy<LAYOUT>::value : 2))) void
+forward_line(FwdArgs a) {
+  __shared__ LineTables tables;
+  const LineCtx cx = line_ctx(as_const(a.m), tables, threadIdx.x % L);
+  constexpr int RAYS = BLOCK / L;
+  constexpr uint32_t kProps = SHARE ? RegistryProps<LAYOUT>::value
+                                    : props_without_share(RegistryProps<LAYOUT>::value);
+  const int local = threadIdx.x / L;
+  for (int64_t tile = blockIdx.x; tile < a.n_tiles; tile += gridDim.x) {
+    Ray y = load_ray<RAYS>(a, tile, local);
+    double total = 0.0;
+    run_line<L, kProps, NOSCAT>(LAYOUT{}, cx, a, y, total);
     if (a.out_mode == ZODI_OUT_SUM && y.active && cx.sub == 0) a.out[y.r] = total;
   }
 }
@@ -351,36 +367,59 @@ inline bool no_scattering(const zodi_model* m) {
   return true;
 }
 
-template <class LAYOUT, int BLOCK>
-FwdKernel pick_shared_cut(const zodi_model* m) {
-  if (no_scattering(m)) return forward_layout<LAYOUT, BLOCK, 1, true, true, true>;
-  return forward_layout<LAYOUT, BLOCK, 1, true, true>;
+template <class LAYOUT, int BLOCK, int L>
+FwdKernel pick_line_terms(bool share, bool noscat) {
+  if (L > 1 || !share) return forward_line<LAYOUT, BLOCK, L, false, false>;
+  if (noscat) return forward_line<LAYOUT, BLOCK, 1, true, true>;
+  return forward_line<LAYOUT, BLOCK, 1, true, false>;
 }
 
-// The registry variant when the block meets its preconditions (with the shared
-// cut-offs for one lane per ray, the launch the tuner picks for large batches,
-// and without scattering code when no component scatters), else the one that
-// tests each component's flags.
+template <class LAYOUT, int BLOCK>
+FwdKernel pick_line_lanes(int L, bool share, bool noscat) {
+  switch (L) {
+    case 1:
+      return pick_line_terms<LAYOUT, BLOCK, 1>(share, noscat);
+    case 2:
+      return pick_line_terms<LAYOUT, BLOCK, 2>(share, noscat);
+    case 4:
+      return pick_line_terms<LAYOUT, BLOCK, 4>(share, noscat);
+    case 8:
+      return pick_line_terms<LAYOUT, BLOCK, 8>(share, noscat);
+    default:
+      return nullptr;
+  }
+}
+
+template <class LAYOUT>
+FwdKernel pick_line(const zodi_model* m, int block, int L) {
+  const bool share = props_match(m, RegistryProps<LAYOUT>::value), noscat = no_scattering(m);
+  switch (block) {
+    case 64:
+      return pick_line_lanes<LAYOUT, 64>(L, share, noscat);
+    case 128:
+      return pick_line_lanes<LAYOUT, 128>(L, share, noscat);
+    case 256:
+      return pick_line_lanes<LAYOUT, 256>(L, share, noscat);
+    case 512:
+      return pick_line_lanes<LAYOUT, 512>(L, share, noscat);
+    default:
+      return nullptr;
+  }
+}
+
+// The registry kernel when the block meets its preconditions (the Kelsall layouts: on
+// the ray's line, with the shared cut-offs for one lane per ray, the launch the
+// tuner picks for large batches, and without scattering code when no component
+// scatters), else the one that tests each component's flags.
 template <class LAYOUT>
 FwdKernel pick_layout(const zodi_model* m, int block, int L) {
-  constexpr uint32_t kProps = RegistryProps<LAYOUT>::value;
-  if constexpr (kProps != props_without_share(kProps)) {
-    if (L == 1 && props_match(m, kProps)) {
-      switch (block) {
-        case 64:
-          return pick_shared_cut<LAYOUT, 64>(m);
-        case 128:
-          return pick_shared_cut<LAYOUT, 128>(m);
-        case 256:
-          return pick_shared_cut<LAYOUT, 256>(m);
-        case 512:
-          return pick_shared_cut<LAYOUT, 512>(m);
-        default:
-          return nullptr;
-      }
-    }
+  constexpr uint32_t kProps = props_without_share(RegistryProps<LAYOUT>::value);
+  const bool spec = props_match(m, kProps);
+  if constexpr (layout_integrand<LAYOUT>() == ZODI_INTEGRAND_KELSALL) {
+    if (spec && line_match(m)) return pick_line<LAYOUT>(m, block, L);
+  } else {
+    if (spec) return pick_layout_block<LAYOUT, true>(block, L);
   }
-  if (props_match(m, props_without_share(kProps))) return pick_layout_block<LAYOUT, true>(block, L);
   return pick_layout_block<LAYOUT, false>(block, L);
 }
 
