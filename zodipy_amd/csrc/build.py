@@ -20,6 +20,7 @@ ROOT = PKG.parent
 INCLUDE = ROOT / "include"
 LIB = PKG / "libzodi_hip.so"
 SOURCES = [CSRC / "zodi_forward.hip", CSRC / "zodi_adjoint.hip", CSRC / "zodi_adjoint_generic.hip",
+           CSRC / "zodi_line_adjoint_dirbe.hip", CSRC / "zodi_line_adjoint_kelsall4.hip",
            CSRC / "zodi_table_adjoint.hip", CSRC / "zodi_pointing.hip", CSRC / "zodi_spectral.hip"]
 HEADERS = [
     CSRC / "zodi_adjoint.hpp",
@@ -27,6 +28,7 @@ HEADERS = [
     CSRC / "zodi_device.hpp",
     CSRC / "zodi_grad.hpp",
     CSRC / "zodi_line.hpp",
+    CSRC / "zodi_line_adjoint.hpp",
     CSRC / "zodi_math.hpp",
     CSRC / "zodi_trig.hpp",
     CSRC / "zodi_trig_coeffs.inc",

@@ -39,27 +39,24 @@
 
 namespace zodi {
 
-// The registry layouts' adjoint kernel. SPEC: the registry variant
-// (RegistryProps; the host checks props_match). NOSCAT: see adjoint_group. NREG:
-// components of a chunk whose accumulators stay in registers (the rest sum in
-// LDS). SHARE (with SPEC, four-component passes): bands with a shared radial
-// cut-off (kShareCut) reuse it.
-template <class LAYOUT, int CHUNK, int SPLIT, bool JAC, bool SPEC = false, bool NOSCAT = false,
-          int NREG = reg_comps<JAC, CHUNK>(), bool SHARE = false>
+// The layout kernels: RRM, and the Kelsall layouts where a block does not meet what
+// the line kernels assume or the caller chooses the components per pass. SPEC: the
+// registry variant (RegistryProps; the host checks props_match). Jacobian chunks of four
+// keep two components' accumulators in registers, the others in LDS.
+template <class LAYOUT, int CHUNK, int SPLIT, bool JAC, bool SPEC = false>
 __global__ __launch_bounds__(kAdjBlock) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 adjoint_layout(AdjArgs a) {
   constexpr uint32_t PROPS =
-      !SPEC ? 0u
-            : (SHARE ? RegistryProps<LAYOUT>::value
-                     : props_without_share(RegistryProps<LAYOUT>::value));
+      SPEC ? props_without_share(RegistryProps<LAYOUT>::value) : 0u;
+  constexpr int NREG = reg_comps<JAC, CHUNK>();
   // Components of a chunk beyond NREG: LDS accumulators, per wave kLdsSlots rows
   // of 64 lanes.
   constexpr int kLdsSlots = layout_lds_slots<CHUNK, NREG>(LAYOUT{});
   adjoint_body<SPLIT, JAC, kLdsSlots>(
       a, [&](const Ctx& cx, const Ray& y, double gscale, double* row, int lane, int sub,
              double* lane_acc) {
-        run_adjoint<SPLIT, CHUNK, NREG, JAC, PROPS, NOSCAT>(LAYOUT{}, cx, a, y, gscale, row, lane,
-                                                            sub, lane_acc);
+        run_adjoint<SPLIT, CHUNK, NREG, JAC, PROPS, false>(LAYOUT{}, cx, a, y, gscale, row, lane,
+                                                           sub, lane_acc);
       });
 }
 
@@ -201,61 +198,66 @@ static __device__ __align__(256) double scratch[kScratchDoubles];
 namespace {
 
 
-template <class LAYOUT, int CHUNK, bool SPEC, bool NOSCAT>
+template <class LAYOUT, int CHUNK, bool SPEC>
 AdjKernel pick_adj_split(int split, bool jac) {
-  if (jac) return split == 1 ? adjoint_layout<LAYOUT, CHUNK, 1, true, SPEC, NOSCAT> : nullptr;
+  if (jac) return split == 1 ? adjoint_layout<LAYOUT, CHUNK, 1, true, SPEC> : nullptr;
   switch (split) {
     case 1:
-      return adjoint_layout<LAYOUT, CHUNK, 1, false, SPEC, NOSCAT>;
+      return adjoint_layout<LAYOUT, CHUNK, 1, false, SPEC>;
     case 2:
-      return adjoint_layout<LAYOUT, CHUNK, 2, false, SPEC, NOSCAT>;
+      return adjoint_layout<LAYOUT, CHUNK, 2, false, SPEC>;
     case 4:
-      return adjoint_layout<LAYOUT, CHUNK, 4, false, SPEC, NOSCAT>;
+      return adjoint_layout<LAYOUT, CHUNK, 4, false, SPEC>;
     default:
       return nullptr;
   }
 }
 
-// Components of a four-component Jacobian chunk whose accumulators stay in
-// registers in the NOSCAT variants: without the scattering sums a third one fits
-// (250 VGPRs for the DIRBE layout, 237 for Kelsall4, no spill), which halves the
-// LDS adds per node; with all four in registers the kernel spills. With the
-// shared band cut-off as well (SHARE) all four fit (Kelsall4 in 256 VGPRs; DIRBE
-// spills 12, 64 bytes of scratch per lane), and no sum goes through LDS: 2.7 %
-// (DIRBE) and 5 % (Kelsall4) faster than three.
-constexpr int kJacRegCompsNoscat = 3;
-constexpr int kJacRegCompsShare = 4;
+// The components per pass of a caller that leaves them open: four in the Jacobian pass,
+// two in the weighted pass.
+bool default_chunk(int chunk, bool jac) { return chunk == (jac ? 4 : 2); }
 
-// The registry variants (SPEC, and NOSCAT for Kelsall layouts) exist for the
-// default plans: four components per pass in the Jacobian pass, two in the
-// weighted pass; SHARE (with NOSCAT) for the Jacobian pass of the layouts whose
-// registry properties share a band cut-off. `spec` and `share` say whether the
-// block meets the preconditions without and with the sharing.
+// Whether the line kernels take a block: a Kelsall layout with its registry properties
+// and exponents the kernels' exp holds. They run every group in one pass, faster than any
+// choice of components per pass of the layout kernels at every ray count, so that choice
+// does not apply to them.
 template <class LAYOUT>
-AdjKernel pick_adj_chunk(int chunk, int split, bool jac, bool spec, bool share, bool noscat) {
-  constexpr bool kKelsall = layout_integrand<LAYOUT>() == ZODI_INTEGRAND_KELSALL;
-  constexpr uint32_t kProps = RegistryProps<LAYOUT>::value;
-  const bool default_plan = jac ? chunk == 4 : chunk == 2;
-  if (spec && default_plan) {
-    if (jac) {
-      if (split != 1) return nullptr;
-      if constexpr (kKelsall && kProps != props_without_share(kProps)) {
-        if (noscat && share)
-          return adjoint_layout<LAYOUT, 4, 1, true, true, true, kJacRegCompsShare, true>;
-      }
-      if constexpr (kKelsall) {
-        if (noscat) return adjoint_layout<LAYOUT, 4, 1, true, true, true, kJacRegCompsNoscat>;
-      }
-      return adjoint_layout<LAYOUT, 4, 1, true, true, false>;
+bool line_eligible(const zodi_model* m) {
+  return props_match(m, props_without_share(RegistryProps<LAYOUT>::value)) &&
+         line_adjoint_match(m);
+}
+
+bool takes_line(const zodi_model* m) {
+  switch (match_layout(m)) {
+    case kLayoutDirbe:
+      return line_eligible<LayoutDirbe>(m);
+    case kLayoutKelsall4:
+      return line_eligible<LayoutKelsall4>(m);
+    default:
+      return false;
+  }
+}
+
+// Band 3 takes band 1's radial cut-off (both centred, the same delta_r).
+bool shares_cut(const zodi_model* m) {
+  return match_layout(m) == kLayoutDirbe ? props_match(m, RegistryProps<LayoutDirbe>::value)
+                                         : props_match(m, RegistryProps<LayoutKelsall4>::value);
+}
+
+template <class LAYOUT>
+AdjKernel pick_adj_layout(const zodi_model* m, int chunk, int split, bool jac) {
+  // The registry variant exists for the RRM layouts' default plans.
+  if constexpr (layout_integrand<LAYOUT>() == ZODI_INTEGRAND_RRM) {
+    if (default_chunk(chunk, jac) && props_match(m, RegistryProps<LAYOUT>::value)) {
+      if (jac) return split == 1 ? adjoint_layout<LAYOUT, 4, 1, true, true> : nullptr;
+      return pick_adj_split<LAYOUT, 2, true>(split, false);
     }
-    if (kKelsall && noscat) return pick_adj_split<LAYOUT, 2, true, kKelsall>(split, false);
-    return pick_adj_split<LAYOUT, 2, true, false>(split, false);
   }
   switch (chunk) {
     case 1:
-      return pick_adj_split<LAYOUT, 1, false, false>(split, jac);
+      return pick_adj_split<LAYOUT, 1, false>(split, jac);
     case 2:
-      return pick_adj_split<LAYOUT, 2, false, false>(split, jac);
+      return pick_adj_split<LAYOUT, 2, false>(split, jac);
     case 4:  // the Jacobian pass (adjoint_plan maps 4 to 2 elsewhere)
       return jac && split == 1 ? adjoint_layout<LAYOUT, 4, 1, true> : nullptr;
     default:
@@ -263,14 +265,12 @@ AdjKernel pick_adj_chunk(int chunk, int split, bool jac, bool spec, bool share, 
   }
 }
 
-template <class LAYOUT>
-AdjKernel pick_adj_layout(const zodi_model* m, int chunk, int split, bool jac) {
-  constexpr uint32_t kProps = RegistryProps<LAYOUT>::value;
-  return pick_adj_chunk<LAYOUT>(chunk, split, jac, props_match(m, props_without_share(kProps)),
-                                props_match(m, kProps), block_noscat(m));
-}
-
 AdjKernel pick_adjoint(const zodi_model* m, int chunk, int split, bool jac) {
+  if (takes_line(m)) {
+    const int scat = block_noscat(m) ? 0 : ((m->flags & 1) == 0 ? 1 : 2);
+    return match_layout(m) == kLayoutDirbe ? line_adjoint_dirbe(scat, jac)
+                                           : line_adjoint_kelsall4(scat, jac);
+  }
   switch (match_layout(m)) {
     case kLayoutDirbe:
       return pick_adj_layout<LayoutDirbe>(m, chunk, split, jac);
@@ -356,7 +356,8 @@ struct AdjPlan {
 // that does. Each extra lane per ray repeats the per-ray set-up and the wave
 // reductions, which costs more than a partly idle last round. The Jacobian pass
 // (jac) always uses one lane per ray.
-zodi_status adjoint_plan(const zodi_launch* launch, int64_t n_rays, bool jac, AdjPlan& p) {
+zodi_status adjoint_plan(const zodi_model* m, const zodi_launch* launch, int64_t n_rays, bool jac,
+                         AdjPlan& p) {
   p.chunk = jac ? kDefaultJacChunk : kDefaultChunk;
   p.split = 0;
   p.per_cu = kDefaultBlocksPerCu;
@@ -383,7 +384,14 @@ zodi_status adjoint_plan(const zodi_launch* launch, int64_t n_rays, bool jac, Ad
     if (p.split > 1)
       return fail(ZODI_ERR_ARG, "the Jacobian pass uses one lane per ray, got lanes_per_ray %d",
                   p.split);
-    p.split = 1;
+    // Small ray counts leave the line kernels' resident waves idle: up to 8 lanes a ray.
+    if (p.split == 0 && takes_line(m)) {
+      const int64_t slots = (int64_t)p.per_cu * cu_count() * kAdjWaves;
+      p.split = 8;
+      while (p.split > 1 && (n_rays * p.split + kWave - 1) / kWave > slots) p.split /= 2;
+    } else {
+      p.split = 1;
+    }
   }
   const int64_t waves = (int64_t)p.per_cu * cu_count() * kAdjWaves;
   if (p.split == 0) {
@@ -421,7 +429,7 @@ zodi_status table_plan(const zodi_model* m, const zodi_launch* launch, int64_t n
   zodi_launch l = launch != nullptr ? *launch : zodi_launch{0, 0, 0, 0};
   if (l.blocks_per_cu == 0) l.blocks_per_cu = any.waves;
   l.variant = 0;
-  const zodi_status st = adjoint_plan(&l, n_rays, false, p);
+  const zodi_status st = adjoint_plan(m, &l, n_rays, false, p);
   if (st != ZODI_OK) return st;
   k = table_adjoint_kernel(m, p.split, eff).k;
   if (k == nullptr)
@@ -455,9 +463,11 @@ bool jacobian_eligible(const zodi_launch* launch, int np, int64_t n_rays) {
 AdjArgs make_args(const zodi_model* model_dev, const double* u, int64_t n_rays,
                   const int64_t* seg_offsets, int32_t n_seg, const double* obs,
                   const double* earth, int32_t obs_mode, const uint32_t* beyond,
-                  const AdjPlan& plan, int n_params) {
+                  const AdjPlan& plan, const zodi_model* m) {
   AdjArgs a;
   memset(&a, 0, sizeof(a));
+  a.split = plan.split;
+  a.share = shares_cut(m) ? 1 : 0;
   a.f.m = model_dev;
   a.f.u = u;
   a.f.n_rays = n_rays;
@@ -470,7 +480,7 @@ AdjArgs make_args(const zodi_model* model_dev, const double* u, int64_t n_rays,
   a.f.beyond = beyond;
   a.f.out_mode = ZODI_OUT_SUM;
   a.f.n_tiles = plan.n_tiles;
-  a.n_params = n_params;
+  a.n_params = m->n_params;
   return a;
 }
 
@@ -544,7 +554,7 @@ zodi_status adjoint_recompute(const zodi_model* model_host, const zodi_model* mo
     if (st != ZODI_OK) return st;
   }
   AdjArgs a = make_args(model_dev, r.u, r.n_rays, r.seg_offsets, r.n_seg, r.obs, r.earth,
-                        r.obs_mode, r.beyond, plan, np);
+                        r.obs_mode, r.beyond, plan, model_host);
   a.weights = weights;
   a.target = target;
   a.inv_var = inv_var;
@@ -643,11 +653,11 @@ int64_t zodi_adjoint_workspace(const zodi_model* model_host, int64_t n_rays, int
   const int np = model_host->n_params;
   if (mode == ZODI_ADJ_CHI2 && jacobian_eligible(launch, np, n_rays)) {
     AdjPlan p;
-    if (adjoint_plan(launch, n_rays, true, p) != ZODI_OK) return -1;
+    if (adjoint_plan(model_host, launch, n_rays, true, p) != ZODI_OK) return -1;
     return jacobian_bytes(np, n_rays);
   }
   AdjPlan p;
-  if (adjoint_plan(launch, n_rays, false, p) != ZODI_OK) return -1;
+  if (adjoint_plan(model_host, launch, n_rays, false, p) != ZODI_OK) return -1;
   return recompute_bytes(p, np + 1, n_rays);
 }
 
@@ -664,13 +674,13 @@ zodi_status zodi_jacobian(const zodi_model* model_host, const zodi_model* model_
   if (ld_jac < n_rays)
     return fail(ZODI_ERR_ARG, "ld_jac %lld < n_rays %lld", (long long)ld_jac, (long long)n_rays);
   AdjPlan plan;
-  st = adjoint_plan(launch, n_rays, true, plan);
+  st = adjoint_plan(model_host, launch, n_rays, true, plan);
   if (st != ZODI_OK) return st;
   AdjKernel k = pick_checked(model_host, plan, true, st);
   if (k == nullptr) return st;
   if (n_rays == 0) return ZODI_OK;
   AdjArgs a = make_args(model_dev, u, n_rays, seg_offsets, n_seg, obs, earth, obs_mode, beyond,
-                        plan, model_host->n_params);
+                        plan, model_host);
   a.jac = jac;
   a.ld_jac = ld_jac;
   a.model_vals_out = model_out;
@@ -704,7 +714,7 @@ zodi_status zodi_adjoint(const zodi_model* model_host, const zodi_model* model_d
   if (mode == ZODI_ADJ_CHI2 && jacobian_eligible(launch, np, n_rays) &&
       workspace_bytes >= jacobian_bytes(np, n_rays)) {
     AdjPlan plan;
-    st = adjoint_plan(launch, n_rays, true, plan);
+    st = adjoint_plan(model_host, launch, n_rays, true, plan);
     if (st != ZODI_OK) return st;
     AdjKernel k = pick_checked(model_host, plan, true, st);
     if (k == nullptr) return st;
@@ -714,7 +724,7 @@ zodi_status zodi_adjoint(const zodi_model* model_host, const zodi_model* model_d
     double* vals = model_out != nullptr ? model_out : partials + chunks * np1;
     if (n_rays > 0) {
       AdjArgs a = make_args(model_dev, u, n_rays, seg_offsets, n_seg, obs, earth, obs_mode,
-                            beyond, plan, np);
+                            beyond, plan, model_host);
       a.jac = workspace;
       a.ld_jac = n_rays;
       a.model_vals_out = vals;
@@ -738,7 +748,7 @@ zodi_status zodi_adjoint(const zodi_model* model_host, const zodi_model* model_d
   }
 
   AdjPlan plan;
-  st = adjoint_plan(launch, n_rays, false, plan);
+  st = adjoint_plan(model_host, launch, n_rays, false, plan);
   if (st != ZODI_OK) return st;
   AdjKernel k = pick_checked(model_host, plan, false, st);
   if (k == nullptr) return st;
@@ -810,7 +820,7 @@ zodi_status zodi_adjoint_noalloc(const zodi_model* model_host, const zodi_model*
   }
   const int np1 = model_host->n_params + 1;
   AdjPlan plan;
-  st = adjoint_plan(launch, n_rays, false, plan);
+  st = adjoint_plan(model_host, launch, n_rays, false, plan);
   if (st != ZODI_OK) return st;
   AdjKernel k = pick_checked(model_host, plan, false, st);
   if (k == nullptr) return st;

@@ -31,6 +31,8 @@ struct AdjArgs {
   double* model_vals_out;    // Jacobian pass: I [n_rays]
   int32_t n_params;
   int32_t mode;              // ZODI_ADJ_*
+  int32_t split;             // line kernels: lanes per ray (1, 2, 4 or 8)
+  int32_t share;             // line kernels: band 3 takes band 1's radial cut-off
 };
 
 // Sum over the 64 lanes of a wave; a + b == b + a in IEEE arithmetic, so every
@@ -547,6 +549,17 @@ inline bool block_noscat(const zodi_model* m) {
 // the effective spectral parameters).
 using AdjKernel = void (*)(AdjArgs);
 AdjKernel generic_adjoint_kernel(int integrand, int split, bool jac);
+
+// The line kernels of the Kelsall registry layouts (scat: see zodi_line_adjoint.hpp), and
+// whether a block that meets the layout's registry properties may take them.
+AdjKernel line_adjoint_dirbe(int scat, bool jac);
+AdjKernel line_adjoint_kelsall4(int scat, bool jac);
+inline bool line_adjoint_match(const zodi_model* m) {
+  const auto in = [](double v, double most) { return v >= -most && v <= most; };
+  for (int g = 0; g < m->n_groups; ++g)
+    if (!in(m->group_delta[g], 1e3)) return false;
+  return in(m->comp[0][7], 1e3) && in(m->comp[0][8], 1e6) && in(m->comp[0][9], 1e3);
+}
 
 // Resident waves per SIMD the table kernels are compiled for (their register
 // budgets): the registry layouts; the Kelsall ones with the spectral sums of

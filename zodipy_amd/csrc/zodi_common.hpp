@@ -103,20 +103,26 @@ __device__ __forceinline__ void read_ray(const FwdArgs& a, Ray& y) {
   y.G = ray_geometry(y.ux, y.uy, y.uz, y.ox, y.oy, y.oz);
 }
 
-template <int RAYS>
-__device__ __forceinline__ Ray load_ray(const FwdArgs& a, int64_t tile, int local) {
+// The ray `local` places after the tile's first one, and its observer's row.
+__device__ __forceinline__ Ray find_ray(const FwdArgs& a, int64_t first, int local) {
   Ray y;
   const int64_t n = a.n_rays;
-  y.r = tile * RAYS + local;
+  y.r = first + local;
   y.active = y.r < n;
   const int64_t rr = y.active ? y.r : n - 1;
   if (a.obs_mode == ZODI_OBS_PER_RAY) {
     y.s = rr;
   } else {
-    const int64_t s0 = find_segment(a.seg, a.n_seg, tile * RAYS);
+    const int64_t s0 = find_segment(a.seg, a.n_seg, first);
     y.s = walk_segment(a.seg, a.n_seg, s0, rr);
   }
   y.bits = a.beyond[a.obs_mode == ZODI_OBS_PER_RAY ? 0 : y.s];
+  return y;
+}
+
+template <int RAYS>
+__device__ __forceinline__ Ray load_ray(const FwdArgs& a, int64_t tile, int local) {
+  Ray y = find_ray(a, tile * RAYS, local);
   read_ray(a, y);
   return y;
 }

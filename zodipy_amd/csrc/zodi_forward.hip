@@ -394,10 +394,6 @@ template <class LAYOUT>
 FwdKernel pick_line(const zodi_model* m, int block, int L) {
   const bool share = props_match(m, RegistryProps<LAYOUT>::value), noscat = no_scattering(m);
   switch (block) {
-    case 64:
-      return pick_line_lanes<LAYOUT, 64>(L, share, noscat);
-    case 128:
-      return pick_line_lanes<LAYOUT, 128>(L, share, noscat);
     case 256:
       return pick_line_lanes<LAYOUT, 256>(L, share, noscat);
     case 512:
@@ -412,13 +408,23 @@ FwdKernel pick_line(const zodi_model* m, int block, int L) {
 // tuner picks for large batches, and without scattering code when no component
 // scatters), else the one that tests each component's flags.
 template <class LAYOUT>
+bool line_eligible(const zodi_model* m) {
+  return props_match(m, props_without_share(RegistryProps<LAYOUT>::value)) && line_match(m);
+}
+
+bool takes_line(const zodi_model* m, LayoutId id) {
+  if (id == kLayoutDirbe) return line_eligible<LayoutDirbe>(m);
+  if (id == kLayoutKelsall4) return line_eligible<LayoutKelsall4>(m);
+  return false;
+}
+
+template <class LAYOUT>
 FwdKernel pick_layout(const zodi_model* m, int block, int L) {
-  constexpr uint32_t kProps = props_without_share(RegistryProps<LAYOUT>::value);
-  const bool spec = props_match(m, kProps);
   if constexpr (layout_integrand<LAYOUT>() == ZODI_INTEGRAND_KELSALL) {
-    if (spec && line_match(m)) return pick_line<LAYOUT>(m, block, L);
+    if (line_eligible<LAYOUT>(m)) return pick_line<LAYOUT>(m, block, L);
   } else {
-    if (spec) return pick_layout_block<LAYOUT, true>(block, L);
+    if (props_match(m, RegistryProps<LAYOUT>::value))
+      return pick_layout_block<LAYOUT, true>(block, L);
   }
   return pick_layout_block<LAYOUT, false>(block, L);
 }
@@ -486,8 +492,13 @@ int default_lanes(const zodi_model* m, int variant, int64_t n_rays) {
   return 1;
 }
 
-FwdKernel pick_forward(const zodi_model* m, int block, int L, int variant) {
+// The line kernels' tables take 23 KB of LDS a block, so that blocks of 64 and 128
+// threads would leave a CU with 6 and 12 waves: smaller requests run as 256.
+constexpr int kLineMinBlock = 256;
+
+FwdKernel pick_forward(const zodi_model* m, int& block, int L, int variant) {
   const LayoutId id = variant == 0 ? kLayoutGeneric : match_layout(m);
+  if (takes_line(m, id) && (block == 64 || block == 128)) block = kLineMinBlock;
   switch (id) {
     case kLayoutDirbe:
       return pick_layout<LayoutDirbe>(m, block, L);
