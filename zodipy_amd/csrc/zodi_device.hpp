@@ -130,7 +130,9 @@ __device__ __forceinline__ RayGeom ray_geometry(double ux, double uy, double uz,
   const bool plain = rho2 > 0x1p-900 && rho2 < 0x1p900 && c2 > 0.0;
   if (!plain || g.b == 0.0) g.b = ray_linear_trig(ux, uy, uz, ox, oy);
   const double r2 = fma(ox, ox, fma(oy, oy, oz * oz));
-  g.r_obs = sqrt(r2);
+  double inv_r;
+  norm_and_inverse(r2, g.r_obs, inv_r);
+  if (r2 == 0.0) g.r_obs = 0.0;
   return g;
 }
 
@@ -140,8 +142,12 @@ __device__ __forceinline__ RayGeom ray_geometry(double ux, double uy, double uz,
 // max(q, c/q). b == 0 gives NaN.
 __device__ __forceinline__ double sphere_distance(const RayGeom& g, double cutoff) {
   const double c = g.r_obs * g.r_obs - cutoff * cutoff;
-  const double q = -0.5 * (g.b + __builtin_copysign(sqrt(g.b * g.b - 4.0 * c), g.b));
-  return g.b == 0.0 ? __builtin_nan("") : np_maximum(q, c / q);
+  const double d = g.b * g.b - 4.0 * c;
+  double root, inv_root;
+  norm_and_inverse(d, root, inv_root);
+  if (d == 0.0) root = 0.0;
+  const double q = -0.5 * (g.b + __builtin_copysign(root, g.b));
+  return g.b == 0.0 ? __builtin_nan("") : np_maximum(q, zodi_trig::quotient(c, q));
 }
 
 // Linear interpolation in the Planck table with np.interp semantics, on the
