@@ -1,4 +1,4 @@
-"""The Kelsall registry kernels on the ray's line (``forward_line``).
+"""The registry kernels on the ray's line (``forward_line``, ``forward_rrm``).
 
 Against the oracle and against the kind switch (variant 0) where the line kernels can go
 wrong: rays through the Sun and at the poles, pointings normal to the observer's
@@ -71,6 +71,37 @@ def test_degenerate_directions_against_oracle(gpu, monkeypatch, x, obs):
     same(got, OracleModel(x).evaluate_vectors(v, obs, obs))
 
 
+@pytest.mark.parametrize("obs", [(1.0, 0.0, 0.0), (0.7, -0.6, 0.3), (1.25, 0.1, 0.0),
+                                 (3.0, 2.0, 0.1)])
+def test_rrm_against_oracle(gpu, obs):
+    """Rays inside, across and along the planes (Z_0, the bands' latitude limits)."""
+    obs = np.array(obs)
+    x = 25 * u.micron
+    phi = np.linspace(0, 2 * np.pi, 13)
+    low = np.stack([np.cos(phi), np.sin(phi), np.full(13, 0.02)])
+    v = np.concatenate([pointings(obs), low / np.linalg.norm(low, axis=0)], axis=1)
+    model = Model(x, name="rrm-experimental")
+    got = model.device_model.forward(v, obs, obs, out_mode=OUT_COMPS).cpu().numpy()
+    same(got, OracleModel(x, name="rrm-experimental").evaluate_vectors(v, obs, obs))
+
+
+@pytest.mark.parametrize("change", [{"fan": {"Q": 0.0}}, {"fan": {"Z_0": 5.0}},
+                                    {"comet": {"Z_0": 1e-6, "P": 0.0}},
+                                    {"inner_narrow_band": {"gamma": 0.0, "beta_nb": 90.0}},
+                                    {"broad_band": {"sigma_bb": 0.2, "gamma": -2.0}},
+                                    {"fan": {"R_outer": 0.9}}, {"fan": {"x_0": 0.01}}])
+def test_rrm_parameters_against_general_kernel(gpu, change):
+    """The last one, off centre, runs the general layout kernel."""
+    model = Model(25 * u.micron, name="rrm-experimental")
+    p = model.get_parameters()
+    for comp, values in change.items():
+        p["comps"][comp].update(values)
+    model.update_parameters(p)
+    obs = np.array([0.98, 0.17, 0.004])
+    got, want = both(model, pointings(obs), obs)
+    same(got, want)
+
+
 # delta and alpha up to 2 and gamma in [1/2, 6] run on the line, the rest in general.
 @pytest.mark.parametrize("change", [{"delta": 2.0}, {"delta": 2.01}, {"delta": 0.0},
                                     {"delta": -0.3}, {"alpha": 2.0}, {"alpha": 2.2},
@@ -93,9 +124,10 @@ def test_exponents_against_general_kernel(gpu, change):
 
 @pytest.mark.parametrize("n", [1, 31, 32, 33, 63, 65, 255, 257, 1023])
 @pytest.mark.parametrize("lanes", [0, 1, 2, 4, 8])
-def test_ragged_counts(gpu, n, lanes):
+@pytest.mark.parametrize("name", ["dirbe", "rrm-experimental"])
+def test_ragged_counts(gpu, n, lanes, name):
     obs = np.array([0.99, 0.1, 0.0])
-    model = Model(12 * u.micron)
+    model = Model(12 * u.micron, name=name)
     v = healpix.pix2vec(16)[:, ::3][:, :n]
     got = model.device_model.forward(v, obs, obs, out_mode=OUT_COMPS,
                                      launch=Launch(variant=1, lanes_per_ray=lanes)).cpu().numpy()

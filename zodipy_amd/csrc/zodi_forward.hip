@@ -12,7 +12,8 @@
 // Two kernel families:
 //  * forward_layout<Layout, BLOCK, L>: the component kinds of every group are
 //    template parameters, so each slot carries only its own density code
-//    (registry layouts: DIRBE/planck13, planck15/18/odegard, RRM);
+//    (registry layouts: DIRBE/planck13, planck15/18/odegard, RRM), with forward_line and
+//    forward_rrm for blocks that have the registry models' properties;
 //  * forward_generic<BLOCK, L>: any layout the model block can describe; one
 //    density switch per slot, per-slot accumulators in LDS.
 //
@@ -28,6 +29,7 @@
 #include <utility>
 
 #include "zodi_common.hpp"
+#include "zodi_line_rrm.hpp"
 
 namespace zodi {
 
@@ -106,11 +108,10 @@ zodi_status validate_model(const zodi_model* m) {
 
 
 // Minimum waves per SIMD the register allocator must leave room for, per layout
-// (1 = no constraint). Measured on MI355X: RRM at 4 (128 VGPRs with a small
-// spill), 15 % faster than its unconstrained 190 VGPRs / 2 waves and 3.7 %
-// faster than 3 waves without the spill; the Kelsall layouts at 5. The kind switch
-// (forward_generic) runs at 3. The split-lane variants (L > 1) run only where the
-// launch is small, so they ask for 2 and keep their registers.
+// (1 = no constraint): the Kelsall layouts at 5 (96 VGPRs; 0.5-1 % faster than at 4), RRM
+// at 4 (105 VGPRs, no spill; at 5 it is 1 % slower). The kind switch (forward_generic)
+// runs at 3. The split-lane variants (L > 1) run only where the launch is small, so
+// they ask for 2 and keep their registers.
 template <class LAYOUT>
 struct ForwardOccupancy {
   static constexpr int value = 1;
@@ -132,10 +133,9 @@ struct ForwardOccupancy<LayoutKelsall4> {
   static constexpr int value = 5;
 };
 
-// SPEC: every component's frame path fixed at compile time to the registry models'
-// (RegistryProps); the host runs it only for blocks that meet its preconditions
-// (props_match).
-template <class LAYOUT, int BLOCK, int L, bool SPEC>
+// A layout whose components' frames are tested per node: blocks that the line kernels do
+// not take (an offset component, a band with p other than 4).
+template <class LAYOUT, int BLOCK, int L>
 __global__ __launch_bounds__(BLOCK)
 __attribute__((amdgpu_waves_per_eu(L == 1 ? ForwardOccupancy<LAYOUT>::value : 2))) void
 forward_layout(FwdArgs a) {
@@ -149,8 +149,7 @@ forward_layout(FwdArgs a) {
   for (int64_t tile = blockIdx.x; tile < a.n_tiles; tile += gridDim.x) {
     const Ray y = load_ray<RAYS>(a, tile, local);
     double total = 0.0;
-    constexpr uint32_t kProps = SPEC ? RegistryProps<LAYOUT>::value : 0u;
-    run_layout<L, kProps, false>(LAYOUT{}, cx, a, y, total);
+    run_layout<L, 0u, false>(LAYOUT{}, cx, a, y, total);
     if (a.out_mode == ZODI_OUT_SUM && y.active && cx.sub == 0) a.out[y.r] = total;
   }
 }
@@ -179,6 +178,27 @@ forward_line(FwdArgs a) {
     Ray y = load_ray<RAYS>(a, tile, local);
     double total = 0.0;
     run_line<L, kProps, NOSCAT>(LAYOUT{}, cx, a, y, total);
+    if (a.out_mode == ZODI_OUT_SUM && y.active && cx.sub == 0) a.out[y.r] = total;
+  }
+}
+
+// The RRM layouts' registry blocks (every component centred) on the ray's line: 3580 issue
+// cycles per wave and node over the six groups where the arc sines, sines, cosines and
+// powers of every node took 6750 (and less where a wave skips a branch). Measured: RRM 25
+// um, 196 608 rays with the pixel vectors, 0.524 -> 0.329 ms.
+template <class LAYOUT, int BLOCK, int L>
+__global__ __launch_bounds__(BLOCK)
+__attribute__((amdgpu_waves_per_eu(L == 1 ? ForwardOccupancy<LAYOUT>::value : 2))) void
+forward_rrm(FwdArgs a) {
+  __shared__ LineAdjTables tables;
+  LineAdjCtx cx = line_adj_ctx(as_const(a.m), tables);
+  cx.sub = threadIdx.x % L;
+  constexpr int RAYS = BLOCK / L;
+  const int local = threadIdx.x / L;
+  for (int64_t tile = blockIdx.x; tile < a.n_tiles; tile += gridDim.x) {
+    const Ray y = load_ray<RAYS>(a, tile, local);
+    double total = 0.0;
+    run_rrm<L>(LAYOUT{}, cx, a, y, total);
     if (a.out_mode == ZODI_OUT_SUM && y.active && cx.sub == 0) a.out[y.r] = total;
   }
 }
@@ -328,33 +348,61 @@ namespace {
 
 using FwdKernel = void (*)(FwdArgs);
 
-template <class LAYOUT, int BLOCK, bool SPEC>
+template <class LAYOUT, int BLOCK>
 FwdKernel pick_layout_lanes(int L) {
   switch (L) {
     case 1:
-      return forward_layout<LAYOUT, BLOCK, 1, SPEC>;
+      return forward_layout<LAYOUT, BLOCK, 1>;
     case 2:
-      return forward_layout<LAYOUT, BLOCK, 2, SPEC>;
+      return forward_layout<LAYOUT, BLOCK, 2>;
     case 4:
-      return forward_layout<LAYOUT, BLOCK, 4, SPEC>;
+      return forward_layout<LAYOUT, BLOCK, 4>;
     case 8:
-      return forward_layout<LAYOUT, BLOCK, 8, SPEC>;
+      return forward_layout<LAYOUT, BLOCK, 8>;
     default:
       return nullptr;
   }
 }
 
-template <class LAYOUT, bool SPEC>
+template <class LAYOUT>
 FwdKernel pick_layout_block(int block, int L) {
   switch (block) {
     case 64:
-      return pick_layout_lanes<LAYOUT, 64, SPEC>(L);
+      return pick_layout_lanes<LAYOUT, 64>(L);
     case 128:
-      return pick_layout_lanes<LAYOUT, 128, SPEC>(L);
+      return pick_layout_lanes<LAYOUT, 128>(L);
     case 256:
-      return pick_layout_lanes<LAYOUT, 256, SPEC>(L);
+      return pick_layout_lanes<LAYOUT, 256>(L);
     case 512:
-      return pick_layout_lanes<LAYOUT, 512, SPEC>(L);
+      return pick_layout_lanes<LAYOUT, 512>(L);
+    default:
+      return nullptr;
+  }
+}
+
+template <class LAYOUT, int BLOCK>
+FwdKernel pick_rrm_lanes(int L) {
+  switch (L) {
+    case 1:
+      return forward_rrm<LAYOUT, BLOCK, 1>;
+    case 2:
+      return forward_rrm<LAYOUT, BLOCK, 2>;
+    case 4:
+      return forward_rrm<LAYOUT, BLOCK, 4>;
+    case 8:
+      return forward_rrm<LAYOUT, BLOCK, 8>;
+    default:
+      return nullptr;
+  }
+}
+
+template <class LAYOUT>
+FwdKernel pick_rrm(int block, int L) {
+  switch (block) {
+    case 256:
+      return pick_rrm_lanes<LAYOUT, 256>(L);
+    case 512:
+      return pick_rrm_lanes<LAYOUT, 512>(L);
     default:
       return nullptr;
   }
@@ -403,30 +451,42 @@ FwdKernel pick_line(const zodi_model* m, int block, int L) {
   }
 }
 
-// The registry kernel when the block meets its preconditions (the Kelsall layouts: on
-// the ray's line, with the shared cut-offs for one lane per ray, the launch the
-// tuner picks for large batches, and without scattering code when no component
-// scatters), else the one that tests each component's flags.
+// The line kernels when the block has the layout's registry properties (the Kelsall
+// layouts: with the shared cut-offs for one lane per ray, the launch the tuner picks
+// for large batches, and without scattering code when no component scatters), else the
+// one that tests each component's flags.
 template <class LAYOUT>
 bool line_eligible(const zodi_model* m) {
-  return props_match(m, props_without_share(RegistryProps<LAYOUT>::value)) && line_match(m);
+  constexpr bool kKelsall = layout_integrand<LAYOUT>() == ZODI_INTEGRAND_KELSALL;
+  return props_match(m, props_without_share(RegistryProps<LAYOUT>::value)) &&
+         (!kKelsall || line_match(m));
 }
 
 bool takes_line(const zodi_model* m, LayoutId id) {
-  if (id == kLayoutDirbe) return line_eligible<LayoutDirbe>(m);
-  if (id == kLayoutKelsall4) return line_eligible<LayoutKelsall4>(m);
-  return false;
+  switch (id) {
+    case kLayoutDirbe:
+      return line_eligible<LayoutDirbe>(m);
+    case kLayoutKelsall4:
+      return line_eligible<LayoutKelsall4>(m);
+    case kLayoutRRM:
+      return line_eligible<LayoutRRM>(m);
+    case kLayoutRRMSplit:
+      return line_eligible<LayoutRRMSplit>(m);
+    default:
+      return false;
+  }
 }
 
 template <class LAYOUT>
 FwdKernel pick_layout(const zodi_model* m, int block, int L) {
-  if constexpr (layout_integrand<LAYOUT>() == ZODI_INTEGRAND_KELSALL) {
-    if (line_eligible<LAYOUT>(m)) return pick_line<LAYOUT>(m, block, L);
-  } else {
-    if (props_match(m, RegistryProps<LAYOUT>::value))
-      return pick_layout_block<LAYOUT, true>(block, L);
+  if (line_eligible<LAYOUT>(m)) {
+    if constexpr (layout_integrand<LAYOUT>() == ZODI_INTEGRAND_KELSALL) {
+      return pick_line<LAYOUT>(m, block, L);
+    } else {
+      return pick_rrm<LAYOUT>(block, L);
+    }
   }
-  return pick_layout_block<LAYOUT, false>(block, L);
+  return pick_layout_block<LAYOUT>(block, L);
 }
 
 template <int BLOCK>
@@ -492,8 +552,8 @@ int default_lanes(const zodi_model* m, int variant, int64_t n_rays) {
   return 1;
 }
 
-// The line kernels' tables take 23 KB of LDS a block, so that blocks of 64 and 128
-// threads would leave a CU with 6 and 12 waves: smaller requests run as 256.
+// The line kernels' tables take 12 to 23 KB of LDS a block, so that blocks of 64 and 128
+// threads would leave a CU with few waves: smaller requests run as 256.
 constexpr int kLineMinBlock = 256;
 
 FwdKernel pick_forward(const zodi_model* m, int& block, int L, int variant) {
