@@ -21,6 +21,7 @@ INCLUDE = ROOT / "include"
 LIB = PKG / "libzodi_hip.so"
 SOURCES = [CSRC / "zodi_forward.hip", CSRC / "zodi_adjoint.hip", CSRC / "zodi_adjoint_generic.hip",
            CSRC / "zodi_line_adjoint_dirbe.hip", CSRC / "zodi_line_adjoint_kelsall4.hip",
+           CSRC / "zodi_line_adjoint_rrm.hip",
            CSRC / "zodi_table_adjoint.hip", CSRC / "zodi_pointing.hip", CSRC / "zodi_spectral.hip"]
 HEADERS = [
     CSRC / "zodi_adjoint.hpp",

@@ -39,15 +39,12 @@
 
 namespace zodi {
 
-// The layout kernels: RRM, and the Kelsall layouts where a block does not meet what
-// the line kernels assume or the caller chooses the components per pass. SPEC: the
-// registry variant (RegistryProps; the host checks props_match). Jacobian chunks of four
-// keep two components' accumulators in registers, the others in LDS.
-template <class LAYOUT, int CHUNK, int SPLIT, bool JAC, bool SPEC = false>
+// The layout kernels, for blocks that the line kernels do not take (an offset component, a
+// band with p other than 4). Jacobian chunks of four keep two components' accumulators in
+// registers, the others in LDS.
+template <class LAYOUT, int CHUNK, int SPLIT, bool JAC>
 __global__ __launch_bounds__(kAdjBlock) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 adjoint_layout(AdjArgs a) {
-  constexpr uint32_t PROPS =
-      SPEC ? props_without_share(RegistryProps<LAYOUT>::value) : 0u;
   constexpr int NREG = reg_comps<JAC, CHUNK>();
   // Components of a chunk beyond NREG: LDS accumulators, per wave kLdsSlots rows
   // of 64 lanes.
@@ -55,8 +52,8 @@ adjoint_layout(AdjArgs a) {
   adjoint_body<SPLIT, JAC, kLdsSlots>(
       a, [&](const Ctx& cx, const Ray& y, double gscale, double* row, int lane, int sub,
              double* lane_acc) {
-        run_adjoint<SPLIT, CHUNK, NREG, JAC, PROPS, false>(LAYOUT{}, cx, a, y, gscale, row, lane,
-                                                           sub, lane_acc);
+        run_adjoint<SPLIT, CHUNK, NREG, JAC, 0u, false>(LAYOUT{}, cx, a, y, gscale, row, lane,
+                                                        sub, lane_acc);
       });
 }
 
@@ -198,29 +195,25 @@ static __device__ __align__(256) double scratch[kScratchDoubles];
 namespace {
 
 
-template <class LAYOUT, int CHUNK, bool SPEC>
+template <class LAYOUT, int CHUNK>
 AdjKernel pick_adj_split(int split, bool jac) {
-  if (jac) return split == 1 ? adjoint_layout<LAYOUT, CHUNK, 1, true, SPEC> : nullptr;
+  if (jac) return split == 1 ? adjoint_layout<LAYOUT, CHUNK, 1, true> : nullptr;
   switch (split) {
     case 1:
-      return adjoint_layout<LAYOUT, CHUNK, 1, false, SPEC>;
+      return adjoint_layout<LAYOUT, CHUNK, 1, false>;
     case 2:
-      return adjoint_layout<LAYOUT, CHUNK, 2, false, SPEC>;
+      return adjoint_layout<LAYOUT, CHUNK, 2, false>;
     case 4:
-      return adjoint_layout<LAYOUT, CHUNK, 4, false, SPEC>;
+      return adjoint_layout<LAYOUT, CHUNK, 4, false>;
     default:
       return nullptr;
   }
 }
 
-// The components per pass of a caller that leaves them open: four in the Jacobian pass,
-// two in the weighted pass.
-bool default_chunk(int chunk, bool jac) { return chunk == (jac ? 4 : 2); }
-
-// Whether the line kernels take a block: a Kelsall layout with its registry properties
-// and exponents the kernels' exp holds. They run every group in one pass, faster than any
-// choice of components per pass of the layout kernels at every ray count, so that choice
-// does not apply to them.
+// Whether the line kernels take a block: a layout with its registry properties (and, of a
+// Kelsall one, exponents the kernels' exp holds). They run every component of a group in
+// one pass, faster than any choice of components per pass of the layout kernels at every
+// ray count, so that choice does not apply to them.
 template <class LAYOUT>
 bool line_eligible(const zodi_model* m) {
   return props_match(m, props_without_share(RegistryProps<LAYOUT>::value)) &&
@@ -233,6 +226,10 @@ bool takes_line(const zodi_model* m) {
       return line_eligible<LayoutDirbe>(m);
     case kLayoutKelsall4:
       return line_eligible<LayoutKelsall4>(m);
+    case kLayoutRRM:
+      return line_eligible<LayoutRRM>(m);
+    case kLayoutRRMSplit:
+      return line_eligible<LayoutRRMSplit>(m);
     default:
       return false;
   }
@@ -240,24 +237,23 @@ bool takes_line(const zodi_model* m) {
 
 // Band 3 takes band 1's radial cut-off (both centred, the same delta_r).
 bool shares_cut(const zodi_model* m) {
-  return match_layout(m) == kLayoutDirbe ? props_match(m, RegistryProps<LayoutDirbe>::value)
-                                         : props_match(m, RegistryProps<LayoutKelsall4>::value);
+  switch (match_layout(m)) {
+    case kLayoutDirbe:
+      return props_match(m, RegistryProps<LayoutDirbe>::value);
+    case kLayoutKelsall4:
+      return props_match(m, RegistryProps<LayoutKelsall4>::value);
+    default:
+      return false;
+  }
 }
 
 template <class LAYOUT>
-AdjKernel pick_adj_layout(const zodi_model* m, int chunk, int split, bool jac) {
-  // The registry variant exists for the RRM layouts' default plans.
-  if constexpr (layout_integrand<LAYOUT>() == ZODI_INTEGRAND_RRM) {
-    if (default_chunk(chunk, jac) && props_match(m, RegistryProps<LAYOUT>::value)) {
-      if (jac) return split == 1 ? adjoint_layout<LAYOUT, 4, 1, true, true> : nullptr;
-      return pick_adj_split<LAYOUT, 2, true>(split, false);
-    }
-  }
+AdjKernel pick_adj_layout(int chunk, int split, bool jac) {
   switch (chunk) {
     case 1:
-      return pick_adj_split<LAYOUT, 1, false>(split, jac);
+      return pick_adj_split<LAYOUT, 1>(split, jac);
     case 2:
-      return pick_adj_split<LAYOUT, 2, false>(split, jac);
+      return pick_adj_split<LAYOUT, 2>(split, jac);
     case 4:  // the Jacobian pass (adjoint_plan maps 4 to 2 elsewhere)
       return jac && split == 1 ? adjoint_layout<LAYOUT, 4, 1, true> : nullptr;
     default:
@@ -266,20 +262,22 @@ AdjKernel pick_adj_layout(const zodi_model* m, int chunk, int split, bool jac) {
 }
 
 AdjKernel pick_adjoint(const zodi_model* m, int chunk, int split, bool jac) {
+  const LayoutId id = match_layout(m);
   if (takes_line(m)) {
+    if (id == kLayoutRRM || id == kLayoutRRMSplit)
+      return line_adjoint_rrm(id == kLayoutRRMSplit, jac);
     const int scat = block_noscat(m) ? 0 : ((m->flags & 1) == 0 ? 1 : 2);
-    return match_layout(m) == kLayoutDirbe ? line_adjoint_dirbe(scat, jac)
-                                           : line_adjoint_kelsall4(scat, jac);
+    return id == kLayoutDirbe ? line_adjoint_dirbe(scat, jac) : line_adjoint_kelsall4(scat, jac);
   }
-  switch (match_layout(m)) {
+  switch (id) {
     case kLayoutDirbe:
-      return pick_adj_layout<LayoutDirbe>(m, chunk, split, jac);
+      return pick_adj_layout<LayoutDirbe>(chunk, split, jac);
     case kLayoutKelsall4:
-      return pick_adj_layout<LayoutKelsall4>(m, chunk, split, jac);
+      return pick_adj_layout<LayoutKelsall4>(chunk, split, jac);
     case kLayoutRRM:
-      return pick_adj_layout<LayoutRRM>(m, chunk, split, jac);
+      return pick_adj_layout<LayoutRRM>(chunk, split, jac);
     case kLayoutRRMSplit:
-      return pick_adj_layout<LayoutRRMSplit>(m, chunk, split, jac);
+      return pick_adj_layout<LayoutRRMSplit>(chunk, split, jac);
     default:
       return nullptr;
   }
@@ -361,6 +359,7 @@ zodi_status adjoint_plan(const zodi_model* m, const zodi_launch* launch, int64_t
   p.chunk = jac ? kDefaultJacChunk : kDefaultChunk;
   p.split = 0;
   p.per_cu = kDefaultBlocksPerCu;
+  if (m->integrand == ZODI_INTEGRAND_RRM && takes_line(m)) p.per_cu = kRrmAdjWaves;
   if (launch != nullptr) {
     if (launch->block != 0 && launch->block != kAdjBlock)
       return fail(ZODI_ERR_ARG, "adjoint block must be %d, got %d", kAdjBlock, launch->block);

@@ -554,7 +554,17 @@ AdjKernel generic_adjoint_kernel(int integrand, int split, bool jac);
 // whether a block that meets the layout's registry properties may take them.
 AdjKernel line_adjoint_dirbe(int scat, bool jac);
 AdjKernel line_adjoint_kelsall4(int scat, bool jac);
+AdjKernel line_adjoint_rrm(bool split_layout, bool jac);
+
+// Resident blocks per CU (waves per SIMD) that the line adjoint kernels are compiled for.
+// Kelsall at 2: at 3 (168 VGPRs) 42 spilled registers make chi^2 8 % slower on 4.5 M rays.
+// RRM at 4 (128 VGPRs, 33 spilled outside the node loops): the Jacobian of 1 M rays takes
+// 2.46, 2.20 and 2.18 ms at 2, 3 and 4, of 100 000 rays 325, 326 and 294 us.
+constexpr int kLineAdjWaves = 2;
+constexpr int kRrmAdjWaves = 4;
+
 inline bool line_adjoint_match(const zodi_model* m) {
+  if (m->integrand == ZODI_INTEGRAND_RRM) return true;
   const auto in = [](double v, double most) { return v >= -most && v <= most; };
   for (int g = 0; g < m->n_groups; ++g)
     if (!in(m->group_delta[g], 1e3)) return false;

@@ -594,6 +594,7 @@ __device__ __forceinline__ void line_adj_layout(Layout<ZODI_INTEGRAND_KELSALL, G
 // of additions these are. The lanes of a ray are adjacent.
 template <class LAYOUT, int SCAT, bool JAC>
 __device__ __forceinline__ void line_adj_body(const AdjArgs& a) {
+  constexpr int NSH = layout_integrand<LAYOUT>() == ZODI_INTEGRAND_KELSALL ? 6 : 1;
   extern __shared__ double sRows[];  // kAdjWaves rows of n_params + 1 (not used by JAC)
   __shared__ LineAdjTables tables;
   const ModelPtr M = as_const(a.f.m);
@@ -639,14 +640,14 @@ __device__ __forceinline__ void line_adj_body(const AdjArgs& a) {
       if (y.active && cx.sub == 0) {
         a.model_vals_out[y.r] = total;
 #pragma unroll
-        for (int q = 0; q < 6; ++q) a.jac[M->grad_shared[q] * a.ld_jac + y.r] = sh[q];
+        for (int q = 0; q < NSH; ++q) a.jac[M->grad_shared[q] * a.ld_jac + y.r] = sh[q];
       }
     } else {
 #pragma unroll
-      for (int q = 0; q < 6; ++q) sh[q] = wave_sum(sh[q]);
+      for (int q = 0; q < NSH; ++q) sh[q] = wave_sum(sh[q]);
       if (lane == 0) {
 #pragma unroll
-        for (int q = 0; q < 6; ++q) row[M->grad_shared[q]] += sh[q];
+        for (int q = 0; q < NSH; ++q) row[M->grad_shared[q]] += sh[q];
       }
     }
   }
@@ -661,7 +662,8 @@ __device__ __forceinline__ void line_adj_body(const AdjArgs& a) {
 }
 
 template <class LAYOUT, int SCAT, bool JAC>
-__global__ __launch_bounds__(kAdjBlock) __attribute__((amdgpu_waves_per_eu(2, 2))) void
+__global__ __launch_bounds__(kAdjBlock)
+__attribute__((amdgpu_waves_per_eu(kLineAdjWaves, kLineAdjWaves))) void
 line_adjoint(AdjArgs a) {
   line_adj_body<LAYOUT, SCAT, JAC>(a);
 }
