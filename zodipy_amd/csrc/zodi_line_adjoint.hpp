@@ -590,74 +590,89 @@ __device__ __forceinline__ void line_adj_layout(Layout<ZODI_INTEGRAND_KELSALL, G
       total);
 }
 
-// One wave per tile of 64 / split rays; see adjoint_body, whose rows, weights and order
-// of additions these are. The lanes of a ray are adjacent.
-template <class LAYOUT, int SCAT, bool JAC>
-__device__ __forceinline__ void line_adj_body(const AdjArgs& a) {
-  constexpr int NSH = layout_integrand<LAYOUT>() == ZODI_INTEGRAND_KELSALL ? 6 : 1;
-  extern __shared__ double sRows[];  // kAdjWaves rows of n_params + 1 (not used by JAC)
-  __shared__ LineAdjTables tables;
-  const ModelPtr M = as_const(a.f.m);
+// The weighted passes: one wave per tile of 64 / a.split rays, whose lanes are adjacent;
+// see adjoint_body, whose rows, weights and order of additions these are. Every thread of
+// the block must call it, after the tables are built.
+template <class RAY>
+__device__ __forceinline__ void weighted_body(const AdjArgs& a, RAY ray) {
+  extern __shared__ double sRows[];  // kAdjWaves rows of n_params + 1
   const int tid = threadIdx.x;
   const int wave = tid / kWave, lane = tid % kWave;
   const int np1 = a.n_params + 1;
-  if constexpr (!JAC) {
-    for (int i = tid; i < np1 * kAdjWaves; i += kAdjBlock) sRows[i] = 0.0;
-  }
-  LineAdjCtx cx = line_adj_ctx(M, tables);
-  cx.split = a.split;
-  cx.sub = lane & (a.split - 1);
-  cx.share = a.share != 0;
+  for (int i = tid; i < np1 * kAdjWaves; i += kAdjBlock) sRows[i] = 0.0;
+  __syncthreads();
   const int rays = kWave / a.split;
-  double* row = JAC ? nullptr : sRows + wave * np1;
+  double* row = sRows + wave * np1;
   const int64_t stride = (int64_t)gridDim.x * kAdjWaves;
   for (int64_t tile = (int64_t)blockIdx.x * kAdjWaves + wave; tile < a.f.n_tiles;
        tile += stride) {
     Ray y = find_ray(a.f, tile * rays, lane / a.split);
     read_ray(a.f, y);
-    double gscale = 1.0;
-    if constexpr (!JAC) {
-      gscale = 0.0;
-      if (a.mode == ZODI_ADJ_CHI2) {
-        double chi = 0.0;
-        if (y.active) {
-          const double I = a.model_vals[y.r];
-          const double iv = a.inv_var != nullptr ? a.inv_var[y.r] : a.inv_var_scalar;
-          const double res = I - a.target[y.r];
-          chi = cx.sub == 0 ? res * res * iv : 0.0;
-          gscale = 2.0 * res * iv;
-        }
-        chi = wave_sum(chi);
-        if (lane == 0) row[a.n_params] += chi;
-      } else if (a.mode == ZODI_ADJ_VJP_SUM) {
-        gscale = y.active ? a.weights[y.r] : 0.0;
+    double gscale = 0.0;
+    if (a.mode == ZODI_ADJ_CHI2) {
+      double chi = 0.0;
+      if (y.active) {
+        const double I = a.model_vals[y.r];
+        const double iv = a.inv_var != nullptr ? a.inv_var[y.r] : a.inv_var_scalar;
+        const double res = I - a.target[y.r];
+        chi = (lane & (a.split - 1)) == 0 ? res * res * iv : 0.0;
+        gscale = 2.0 * res * iv;
       }
+      chi = wave_sum(chi);
+      if (lane == 0) row[a.n_params] += chi;
+    } else if (a.mode == ZODI_ADJ_VJP_SUM) {
+      gscale = y.active ? a.weights[y.r] : 0.0;
     }
-    double sh[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    double total = 0.0;
-    line_adj_layout<SCAT, JAC>(LAYOUT{}, cx, a, y, gscale, row, lane, sh, total);
-    if constexpr (JAC) {
-      if (y.active && cx.sub == 0) {
-        a.model_vals_out[y.r] = total;
-#pragma unroll
-        for (int q = 0; q < NSH; ++q) a.jac[M->grad_shared[q] * a.ld_jac + y.r] = sh[q];
-      }
-    } else {
-#pragma unroll
-      for (int q = 0; q < NSH; ++q) sh[q] = wave_sum(sh[q]);
-      if (lane == 0) {
-#pragma unroll
-        for (int q = 0; q < NSH; ++q) row[M->grad_shared[q]] += sh[q];
-      }
-    }
+    ray(y, gscale, row, lane);
   }
-  if constexpr (JAC) return;
   __syncthreads();
   for (int p = tid; p < np1; p += kAdjBlock) {
     double s = sRows[p];
 #pragma unroll
     for (int w = 1; w < kAdjWaves; ++w) s += sRows[w * np1 + p];
     a.partials[(int64_t)blockIdx.x * np1 + p] = s;
+  }
+}
+
+// The Jacobian pass (each ray's column and I_r) or the weighted pass of a layout.
+template <class LAYOUT, int SCAT, bool JAC>
+__device__ __forceinline__ void line_adj_body(const AdjArgs& a) {
+  constexpr int NSH = layout_integrand<LAYOUT>() == ZODI_INTEGRAND_KELSALL ? 6 : 1;
+  __shared__ LineAdjTables tables;
+  const ModelPtr M = as_const(a.f.m);
+  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+  LineAdjCtx cx = line_adj_ctx(M, tables);
+  cx.split = a.split;
+  cx.sub = lane & (a.split - 1);
+  cx.share = a.share != 0;
+  if constexpr (JAC) {
+    const int rays = kWave / a.split;
+    const int64_t stride = (int64_t)gridDim.x * kAdjWaves;
+    for (int64_t tile = (int64_t)blockIdx.x * kAdjWaves + wave; tile < a.f.n_tiles;
+         tile += stride) {
+      Ray y = find_ray(a.f, tile * rays, lane / a.split);
+      read_ray(a.f, y);
+      double sh[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+      double total = 0.0;
+      line_adj_layout<SCAT, true>(LAYOUT{}, cx, a, y, 1.0, nullptr, lane, sh, total);
+      if (y.active && cx.sub == 0) {
+        a.model_vals_out[y.r] = total;
+#pragma unroll
+        for (int q = 0; q < NSH; ++q) a.jac[M->grad_shared[q] * a.ld_jac + y.r] = sh[q];
+      }
+    }
+  } else {
+    weighted_body(a, [&](Ray& y, double gscale, double* row, int ln) {
+      double sh[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+      double total = 0.0;
+      line_adj_layout<SCAT, false>(LAYOUT{}, cx, a, y, gscale, row, ln, sh, total);
+#pragma unroll
+      for (int q = 0; q < NSH; ++q) sh[q] = wave_sum(sh[q]);
+      if (ln == 0) {
+#pragma unroll
+        for (int q = 0; q < NSH; ++q) row[M->grad_shared[q]] += sh[q];
+      }
+    });
   }
 }
 

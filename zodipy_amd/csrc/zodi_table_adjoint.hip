@@ -37,7 +37,7 @@
 
 #include <utility>
 
-#include "zodi_adjoint.hpp"
+#include "zodi_line_rrm.hpp"
 
 namespace zodi {
 
@@ -260,11 +260,189 @@ __device__ __forceinline__ void table_ray(const Ctx& cx, const AdjArgs& a, const
   if constexpr (EFF) eff_ray_finish<INTEGRAND>(M, sh, row, lane);
 }
 
-// Registry layouts: the group's kinds (and, with PROPS, the registry forms of the
-// forward kernels) fixed at compile time, the densities inlined. NOSCAT (EFF
-// only): no component scatters and F = 0, so the scattering sums are exact zeros
-// and left out.
-template <int INTEGRAND, int SPLIT, uint32_t PROPS, bool EFF, bool NOSCAT, int... Ks, int... J>
+// One node's share for the table: interval and fraction from the shifted index u1 =
+// (T - T_first)/dT + 1 (planck_shifted).
+struct TableShare {
+  int jt;
+  double f, B;
+};
+
+__device__ __forceinline__ TableShare table_share(double u1, const double2* tab) {
+  uint32_t i = (uint32_t)u1;
+  i = i < (uint32_t)ZODI_N_TEMPS ? i : (uint32_t)ZODI_N_TEMPS;
+  const double2 e = tab[i];
+  TableShare t;
+  t.f = __builtin_amdgcn_fract(u1);
+  t.B = fma(t.f, e.y, e.x);
+  t.jt = (int)i - 1;
+  if (i == 0) {  // below the table: all of it to the first entry
+    t.jt = 0;
+    t.f = 0.0;
+  }
+  return t;
+}
+
+// A group of a registry layout on the ray's line, with the forward kernels' node and
+// densities. NOSCAT (EFF only): no component scatters and F = 0, so the scattering
+// sums are exact zeros and left out. Lane `sub` of the a.split lanes sharing the ray
+// takes nodes sub, sub + split, ...
+template <int INTEGRAND, uint32_t PROPS, bool EFF, bool NOSCAT, class CTX, int... Ks, int... J>
+__device__ __forceinline__ void line_table_group(Grp<Ks...>, std::integer_sequence<int, J...>,
+                                                 const CTX& cx, const AdjArgs& a, const Ray& y,
+                                                 const Line& l, int g, int first, double gscale,
+                                                 double* row, int lane, const PhaseUse& pu,
+                                                 double (&sh)[6]) {
+  constexpr int C = sizeof...(Ks);
+  constexpr int kinds[C] = {Ks...};
+  constexpr bool kKelsall = INTEGRAND == ZODI_INTEGRAND_KELSALL;
+  constexpr bool kScat = EFF && kKelsall && !NOSCAT;
+  const ModelPtr M = cx.M;
+  const int n_last = M->n_temps - 1;
+  double* trow = EFF ? row + M->n_params : row;
+  double h, mid;
+  group_range(M, g, y, h, mid);
+  const double th = l.n * h, tm = fma(l.n, mid, l.t0);
+  double half_delta = 0.0, us = 0.0, uo1 = 0.0;
+  if constexpr (!kKelsall) {
+    half_delta = to_scalar(0.5 * M->group_delta[g]);
+    us = to_scalar(M->group_T0[g] * M->tab_inv_step);
+    uo1 = to_scalar(M->tab_T[0] * M->tab_inv_step - 1.0);
+  }
+  const double calibration = M->shared[ZODI_S_CALIBRATION], solar = M->shared[ZODI_S_SOLAR];
+  const std::tuple<LineComp<Ks>...> lc{LineComp<Ks>(M->comp[first + J], l, y.ex, y.ey)...};
+  LinePhase lp = {0.0, 0.0};
+  if (kScat && pu.angle) lp = line_phase(l);
+  double cw[C];  // h s_c g_c
+  double ca[C];  // EFF: Kelsall h g_c a_c where c scatters (else 0); RRM h g_c
+  double E[C], S[C];
+  (
+      [&] {
+        const int c = first + J;
+        const double s = kKelsall ? M->comp[c][ZODI_P_SCALE] : calibration;
+        const double w = comp_weight(a, y, c, gscale);
+        cw[J] = (h * s) * w;
+        if constexpr (EFF) {
+          E[J] = 0.0;
+          S[J] = 0.0;
+          const double W = y.active ? h * w : 0.0;
+          ca[J] = kKelsall ? ((M->comp_flags[c] & ZODI_CF_SCATTER) ? W * M->comp[c][ZODI_P_ALBEDO]
+                                                                  : 0.0)
+                           : W;
+        }
+      }(),
+      ...);
+  const int K = y.active ? M->n_nodes : 0;
+  TablePending pend;
+  double xnext = M->gl_x[cx.sub], wnext = M->gl_w[cx.sub];
+  for (int k = cx.sub; k < K; k += a.split) {
+    const ModelPtr Mk = opaque(M);
+    const double wk = wnext;
+    const double t = fma(th, xnext, tm);
+    {
+      const int kn = k + a.split < ZODI_MAX_NODES ? k + a.split : 0;
+      xnext = M->gl_x[kn];
+      wnext = M->gl_w[kn];
+    }
+    GradNode nd;
+    double u1, lR2 = 0.0;
+    if constexpr (kKelsall) {
+      nd.t = t;
+      nd.R2 = fma(t, t, l.d2);
+      norm_and_inverse_node(nd.R2, nd.R, nd.inv_R);
+      u1 = pow_table(cx.tab->temperature, cx.pt, nd.R2) - cx.uo1;
+    } else {
+      const RrmNode o = rrm_node(cx, l, t, half_delta, us, uo1);
+      nd = o.nd;
+      lR2 = o.lR2;
+      u1 = fma(o.Rd, us, -uo1);
+    }
+    const TableShare ts = table_share(u1, cx.tab->planck);
+    const double wB = wk * ts.B;
+    PhaseGrad pg = {0.0, 0.0, 0.0, 0.0};
+    double inv_R2 = 0.0, wsu = 0.0;
+    if constexpr (kScat) {
+      if (pu.phase) {
+        pg.phi = pu.phi_const;
+        if (pu.angle) pg = line_phase_grad(lp, l, cx.ec, t, Mk->shared);
+        inv_R2 = nd.inv_R * nd.inv_R;
+        wsu = wk * ((solar * inv_R2) * pg.phi);
+      }
+    }
+    double Sn = 0.0, Sa = 0.0, cut = 0.0;
+    (
+        [&] {
+          const ParamPtr P = Mk->comp[first + J];
+          double n;
+          if constexpr (kKelsall) {
+            n = line_density<kinds[J], cut_mode<PROPS, J, Ks...>()>(
+                P, std::get<J>(lc), cx, l, LineNode{nd.t, nd.R2, nd.R, nd.inv_R}, cut);
+          } else {
+            n = rrm_density<kinds[J]>(P, std::get<J>(lc), cx, l, nd, lR2);
+          }
+          Sn = fma(cw[J], n, Sn);
+          if constexpr (EFF) {
+            if constexpr (kKelsall) {
+              E[J] = fma(wB, n, E[J]);
+              if constexpr (kScat) {
+                S[J] = fma(wsu, n, S[J]);
+                Sa = fma(ca[J], n, Sa);
+              }
+            } else {
+              Sa = fma(ca[J], n, Sa);
+            }
+          }
+        }(),
+        ...);
+    pend.add(trow, n_last, ts.jt, ts.f, wk * Sn);
+    if constexpr (kScat) {
+      if (pu.phase) {
+        const double was = (wk * Sa) * inv_R2;
+        sh[2] += was * pg.phi;
+        const double wasf = was * solar;
+        sh[3] += wasf * pg.d1;
+        sh[4] += wasf * pg.d2;
+        sh[5] += wasf * pg.d3;
+      }
+    }
+    if constexpr (EFF && !kKelsall) sh[0] += wB * Sa;  // calibration
+  }
+  pend.flush(trow, n_last);
+  if constexpr (EFF && kKelsall) {
+    (eff_comp_finish(M, first + J, comp_weight(a, y, first + J, gscale) * (y.active ? h : 0.0),
+                     E[J], S[J], row, lane),
+     ...);
+  }
+}
+
+template <uint32_t PROPS, bool EFF, bool NOSCAT, class CTX, int INTEGRAND, class... Gs, int... G>
+__device__ __forceinline__ void line_table_groups(Layout<INTEGRAND, Gs...>,
+                                                  std::integer_sequence<int, G...>,
+                                                  const CTX& cx, const AdjArgs& a, const Ray& y,
+                                                  double gscale, double* row, int lane) {
+  double sh[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  PhaseUse pu = {false, false, 0.0};
+  if constexpr (EFF && INTEGRAND == ZODI_INTEGRAND_KELSALL && !NOSCAT)
+    pu = phase_use(cx.M, cx.M->shared[ZODI_S_SOLAR]);
+  const Line l = make_line(y.ux, y.uy, y.uz, y.ox, y.oy, y.oz);
+  (line_table_group<INTEGRAND, props_shift(PROPS, group_first<Gs...>(G)), EFF, NOSCAT>(
+       Gs{}, std::make_integer_sequence<int, Gs::size>{}, cx, a, y, l, G, group_first<Gs...>(G),
+       gscale, row, lane, pu, sh),
+   ...);
+  if constexpr (EFF && (INTEGRAND != ZODI_INTEGRAND_KELSALL || !NOSCAT))
+    eff_ray_finish<INTEGRAND>(cx.M, sh, row, lane);
+}
+
+template <uint32_t PROPS, bool EFF, bool NOSCAT, class CTX, int INTEGRAND, class... Gs>
+__device__ __forceinline__ void run_line_table(Layout<INTEGRAND, Gs...> lay, const CTX& cx,
+                                               const AdjArgs& a, const Ray& y, double gscale,
+                                               double* row, int lane) {
+  line_table_groups<PROPS, EFF, NOSCAT>(lay, std::make_integer_sequence<int, sizeof...(Gs)>{}, cx,
+                                        a, y, gscale, row, lane);
+}
+
+// Registry layouts whose blocks the line kernels do not take: the group's kinds fixed at
+// compile time, the densities inlined.
+template <int INTEGRAND, int SPLIT, bool EFF, int... Ks, int... J>
 __device__ __forceinline__ void table_group(Grp<Ks...>, std::integer_sequence<int, J...>,
                                             const Ctx& cx, const AdjArgs& a, const Ray& y, int g,
                                             int first, double gscale, double* row, int lane,
@@ -272,7 +450,8 @@ __device__ __forceinline__ void table_group(Grp<Ks...>, std::integer_sequence<in
   constexpr int C = sizeof...(Ks);
   constexpr int kinds[C] = {Ks...};
   constexpr bool kKelsall = INTEGRAND == ZODI_INTEGRAND_KELSALL;
-  constexpr bool kScat = EFF && kKelsall && !NOSCAT;
+  constexpr bool kScat = EFF && kKelsall;
+  constexpr uint32_t PROPS = 0u;
   const ModelPtr M = cx.M;
   const int n_last = M->n_temps - 1;
   double* trow = EFF ? row + M->n_params : row;
@@ -383,37 +562,32 @@ __device__ __forceinline__ void table_group(Grp<Ks...>, std::integer_sequence<in
   }
 }
 
-template <int SPLIT, uint32_t PROPS, bool EFF, bool NOSCAT, int INTEGRAND, class... Gs, int... G>
+template <int SPLIT, bool EFF, int INTEGRAND, class... Gs, int... G>
 __device__ __forceinline__ void table_groups(Layout<INTEGRAND, Gs...>,
                                              std::integer_sequence<int, G...>, const Ctx& cx,
                                              const AdjArgs& a, const Ray& y, double gscale,
                                              double* row, int lane, int sub, const PhaseUse& pu,
                                              double (&sh)[6]) {
-  (table_group<INTEGRAND, SPLIT, props_shift(PROPS, group_first<Gs...>(G)), EFF, NOSCAT>(
-       Gs{}, std::make_integer_sequence<int, Gs::size>{}, cx, a, y, G, group_first<Gs...>(G),
-       gscale, row, lane, sub, pu, sh),
+  (table_group<INTEGRAND, SPLIT, EFF>(Gs{}, std::make_integer_sequence<int, Gs::size>{}, cx, a, y,
+                                      G, group_first<Gs...>(G), gscale, row, lane, sub, pu, sh),
    ...);
 }
 
-template <int SPLIT, uint32_t PROPS, bool EFF, bool NOSCAT, int INTEGRAND, class... Gs>
+template <int SPLIT, bool EFF, int INTEGRAND, class... Gs>
 __device__ __forceinline__ void run_table(Layout<INTEGRAND, Gs...> lay, const Ctx& cx,
                                           const AdjArgs& a, const Ray& y, double gscale,
                                           double* row, int lane, int sub) {
   double sh[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
   PhaseUse pu = {false, false, 0.0};
-  if constexpr (EFF && INTEGRAND == ZODI_INTEGRAND_KELSALL && !NOSCAT)
-    pu = phase_use(cx.M, cx.solar);
-  table_groups<SPLIT, PROPS, EFF, NOSCAT>(lay, std::make_integer_sequence<int, sizeof...(Gs)>{},
-                                          cx, a, y, gscale, row, lane, sub, pu, sh);
-  if constexpr (EFF && (INTEGRAND != ZODI_INTEGRAND_KELSALL || !NOSCAT))
-    eff_ray_finish<INTEGRAND>(cx.M, sh, row, lane);
+  if constexpr (EFF && INTEGRAND == ZODI_INTEGRAND_KELSALL) pu = phase_use(cx.M, cx.solar);
+  table_groups<SPLIT, EFF>(lay, std::make_integer_sequence<int, sizeof...(Gs)>{}, cx, a, y, gscale,
+                           row, lane, sub, pu, sh);
+  if constexpr (EFF) eff_ray_finish<INTEGRAND>(cx.M, sh, row, lane);
 }
 
 // Resident waves per SIMD of the registry-layout kernels (their register budget):
 // four, or three for the Kelsall layouts' spectral sums with the scattering terms
-// (at four those spill more and ran 20 % slower). Measured on MI355X, four waves
-// with a small spill beat three without it for the RRM layouts (5 %) and for the
-// DIRBE spectral sums without scattering (3.5 %).
+// (at four those spill more and ran 20 % slower).
 template <class LAYOUT, bool EFF, bool NOSCAT>
 constexpr int table_waves() {
   return layout_integrand<LAYOUT>() == ZODI_INTEGRAND_KELSALL && EFF && !NOSCAT
@@ -421,18 +595,34 @@ constexpr int table_waves() {
              : kTableWavesLayout;
 }
 
-// SPEC: the registry forms (RegistryProps, with the shared band cut-off when the
-// host finds the block allows it: SHARE).
-template <class LAYOUT, int SPLIT, bool SPEC, bool SHARE, bool EFF, bool NOSCAT>
+// The line kernels. SHARE: the bands that share a radial cut-off reuse it (kShareCut).
+template <class LAYOUT, bool SHARE, bool EFF, bool NOSCAT>
 __global__ __launch_bounds__(kAdjBlock) __attribute__((
-    amdgpu_waves_per_eu(table_waves<LAYOUT, EFF, NOSCAT>()))) void table_layout(AdjArgs a) {
-  constexpr uint32_t PROPS =
-      !SPEC ? 0u
-            : (SHARE ? RegistryProps<LAYOUT>::value
-                     : props_without_share(RegistryProps<LAYOUT>::value));
+    amdgpu_waves_per_eu(table_waves<LAYOUT, EFF, NOSCAT>()))) void table_line(AdjArgs a) {
+  constexpr uint32_t PROPS = SHARE ? RegistryProps<LAYOUT>::value
+                                   : props_without_share(RegistryProps<LAYOUT>::value);
+  if constexpr (layout_integrand<LAYOUT>() == ZODI_INTEGRAND_KELSALL) {
+    __shared__ LineTables tables;
+    const LineCtx cx = line_ctx(as_const(a.f.m), tables, threadIdx.x & (a.split - 1));
+    weighted_body(a, [&](const Ray& y, double gscale, double* row, int lane) {
+      run_line_table<PROPS, EFF, NOSCAT>(LAYOUT{}, cx, a, y, gscale, row, lane);
+    });
+  } else {
+    __shared__ LineAdjTables tables;
+    LineAdjCtx cx = line_adj_ctx(as_const(a.f.m), tables);
+    cx.sub = threadIdx.x & (a.split - 1);
+    weighted_body(a, [&](const Ray& y, double gscale, double* row, int lane) {
+      run_line_table<PROPS, EFF, NOSCAT>(LAYOUT{}, cx, a, y, gscale, row, lane);
+    });
+  }
+}
+
+template <class LAYOUT, int SPLIT, bool EFF>
+__global__ __launch_bounds__(kAdjBlock) __attribute__((
+    amdgpu_waves_per_eu(table_waves<LAYOUT, EFF, false>()))) void table_layout(AdjArgs a) {
   adjoint_body<SPLIT, false, 0>(
       a, [&](const Ctx& cx, const Ray& y, double gscale, double* row, int lane, int sub, double*) {
-        run_table<SPLIT, PROPS, EFF, NOSCAT>(LAYOUT{}, cx, a, y, gscale, row, lane, sub);
+        run_table<SPLIT, EFF>(LAYOUT{}, cx, a, y, gscale, row, lane, sub);
       });
 }
 
@@ -459,41 +649,40 @@ AdjKernel pick_table_split(int split) {
   }
 }
 
-template <class LAYOUT, bool SPEC, bool SHARE, bool EFF, bool NOSCAT>
-TableKernel pick_table_layout_split(int split) {
-  constexpr int kWaves = table_waves<LAYOUT, EFF, NOSCAT>();
-  switch (split) {
-    case 1:
-      return {table_layout<LAYOUT, 1, SPEC, SHARE, EFF, NOSCAT>, kWaves};
-    case 2:
-      return {table_layout<LAYOUT, 2, SPEC, SHARE, EFF, NOSCAT>, kWaves};
-    case 4:
-      return {table_layout<LAYOUT, 4, SPEC, SHARE, EFF, NOSCAT>, kWaves};
-    default:
-      return {nullptr, 0};
-  }
-}
-
 // NOSCAT applies to the Kelsall layouts with EFF (the RRM integrand has no
 // scattering term, and without EFF nothing is summed for it).
-template <class LAYOUT, bool SPEC, bool SHARE, bool EFF>
-TableKernel pick_table_noscat(int split, bool noscat) {
+template <class LAYOUT, bool SHARE, bool EFF>
+TableKernel pick_table_line(bool noscat) {
   if constexpr (EFF && layout_integrand<LAYOUT>() == ZODI_INTEGRAND_KELSALL) {
-    if (noscat) return pick_table_layout_split<LAYOUT, SPEC, SHARE, true, true>(split);
+    if (noscat)
+      return {table_line<LAYOUT, SHARE, true, true>, table_waves<LAYOUT, true, true>()};
   }
-  return pick_table_layout_split<LAYOUT, SPEC, SHARE, EFF, false>(split);
+  return {table_line<LAYOUT, SHARE, EFF, false>, table_waves<LAYOUT, EFF, false>()};
 }
 
+// The line kernels under the forward's conditions, else the layout kernels.
 template <class LAYOUT, bool EFF>
 TableKernel pick_table_layout(const zodi_model* m, int split) {
   constexpr uint32_t kProps = RegistryProps<LAYOUT>::value;
-  const bool noscat = block_noscat(m);
-  if constexpr (kProps != props_without_share(kProps)) {
-    if (props_match(m, kProps)) return pick_table_noscat<LAYOUT, true, true, EFF>(split, noscat);
+  constexpr bool kKelsall = layout_integrand<LAYOUT>() == ZODI_INTEGRAND_KELSALL;
+  if (props_match(m, props_without_share(kProps)) && (!kKelsall || line_match(m))) {
+    const bool noscat = block_noscat(m);
+    if constexpr (kProps != props_without_share(kProps)) {
+      if (props_match(m, kProps)) return pick_table_line<LAYOUT, true, EFF>(noscat);
+    }
+    return pick_table_line<LAYOUT, false, EFF>(noscat);
   }
-  if (props_match(m, props_without_share(kProps)))
-    return pick_table_noscat<LAYOUT, true, false, EFF>(split, noscat);
-  return pick_table_noscat<LAYOUT, false, false, EFF>(split, noscat);
+  constexpr int kWaves = table_waves<LAYOUT, EFF, false>();
+  switch (split) {
+    case 1:
+      return {table_layout<LAYOUT, 1, EFF>, kWaves};
+    case 2:
+      return {table_layout<LAYOUT, 2, EFF>, kWaves};
+    case 4:
+      return {table_layout<LAYOUT, 4, EFF>, kWaves};
+    default:
+      return {nullptr, 0};
+  }
 }
 
 template <bool EFF>
