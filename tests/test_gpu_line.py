@@ -134,3 +134,21 @@ def test_ragged_counts(gpu, n, lanes, name):
     want = model.device_model.forward(torch.as_tensor(healpix.pix2vec(16)[:, ::3].copy()), obs,
                                       obs, out_mode=OUT_COMPS).cpu().numpy()[:, :n]
     assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("rays", [1, 7, 17, 3072, 12289, 20011, 49153, 150001])
+@pytest.mark.parametrize("nodes", [1, 9, 50])
+@pytest.mark.parametrize("name,x", [("dirbe", 1.25 * u.micron), ("planck18", 857 * u.GHz),
+                                    ("rrm-experimental", 25 * u.micron)])
+def test_default_split_gives_the_bits_of_one_lane(gpu, name, x, nodes, rays):
+    """The lanes per ray (1 to 32) that the launch picks from the ray count, with a last
+    node step that is full, partial or the only one, against one lane per ray: equal."""
+    model = Model(x, name=name, gauss_quad_degree=nodes)
+    rng = np.random.default_rng(rays + nodes)
+    v = rng.normal(size=(3, rays))
+    v /= np.linalg.norm(v, axis=0)
+    obs = np.array([0.9, 0.4, 0.02])
+    for mode in ({}, {"out_mode": OUT_COMPS}):
+        got = model.device_model.forward(v, obs, obs, **mode)
+        one = model.device_model.forward(v, obs, obs, launch=Launch(256, 1, 0, 1), **mode)
+        assert torch.equal(got, one)

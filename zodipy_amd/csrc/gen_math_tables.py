@@ -3,7 +3,10 @@
 * EXP2_TABLE[j] = 2^(j/256), j = 0..255 (table-driven exp, Tang 1989,
   ACM TOMS 15(2):144-157);
 * LOG_INV[j] = 1/c_j and LOG_C[j] = log(c_j) with c_j = 1/2 + j/512,
-  j = 0..255 (table-driven log, Tang 1990, ACM TOMS 16(4):378-400).
+  j = 0..255 (table-driven log, Tang 1990, ACM TOMS 16(4):378-400);
+* LINE_INV[j] = 1/(1/2 + (j + 1/2)/512) rounded to a multiple of 2^-12 and
+  LINE_LOG[j] = -log(LINE_INV[j]) (zodi_line.hpp: the product of a mantissa and a
+  13-bit LINE_INV is exact inside an FMA).
 
 Values are evaluated with mpmath at 200 bits and rounded to nearest double.
 Run ``python -m zodipy_amd.csrc.gen_math_tables`` to regenerate.
@@ -40,6 +43,14 @@ def main() -> None:
     lines[-1] = lines[-1].rstrip(" \\").rstrip(",")
     lines += ["// log(c_j)", "#define ZODI_LOG_C_TABLE \\"]
     lines += [f"  {_hex(v)}, \\" for v in logc]
+    lines[-1] = lines[-1].rstrip(" \\").rstrip(",")
+    short = [mpmath.nint(4096 / (mpmath.mpf(1) / 2 + (mpmath.mpf(j) + mpmath.mpf(1) / 2) / 512))
+             / 4096 for j in range(256)]
+    lines += ["// 1/(1/2 + (j + 1/2)/512) to 2^-12", "#define ZODI_LINE_INV_TABLE \\"]
+    lines += [f"  {_hex(v)}, \\" for v in short]
+    lines[-1] = lines[-1].rstrip(" \\").rstrip(",")
+    lines += ["// -log of the same", "#define ZODI_LINE_LOG_TABLE \\"]
+    lines += [f"  {_hex(-mpmath.log(v))}, \\" for v in short]
     lines[-1] = lines[-1].rstrip(" \\").rstrip(",")
     OUT.write_text("\n".join(lines) + "\n")
     print(OUT)

@@ -33,7 +33,7 @@ struct FwdArgs {
   const uint32_t* beyond;
   double* out;
   int32_t out_mode;
-  int32_t pad;
+  int32_t lanes;  // split line kernels: lanes per ray
   int64_t n_tiles;
 };
 
@@ -595,13 +595,112 @@ __device__ __forceinline__ double line_density(ParamPtr P, const LineComp<KIND>&
   if constexpr (KIND == ZODI_FEATURE) return line_feature(P, c, cx, l, nd);
 }
 
+// A ray's node sums over a group of C components: the terms are added in node order
+// whatever the lanes per ray, so every split gives the bits of one lane per ray.
+//   SPLIT 1: one lane a ray, one register a sum.
+//   SPLIT 2, 4: the ray's lanes evaluate consecutive nodes at once, and every lane adds
+//     all their terms, which it takes from its neighbours of the quad by DPP moves.
+//   SPLIT 8: `lanes` lanes (8 to 32, a runtime value); every component's terms are added
+//     by one lane (component j by lane j), which reads them from LDS. The
+//     lanes of a ray are in one wave, whose LDS operations complete in order, so a
+//     compiler barrier orders them.
+constexpr int kSplitBlock = 512;               // largest block of the split kernels
+constexpr int kSplitStride = kSplitBlock + 2;  // row of one component's terms
+
+template <int CTRL>
+__device__ __forceinline__ double quad_move(double x) {
+  const int2 v = __builtin_bit_cast(int2, x);
+  return __builtin_bit_cast(double, int2{__builtin_amdgcn_mov_dpp(v.x, CTRL, 0xf, 0xf, true),
+                                         __builtin_amdgcn_mov_dpp(v.y, CTRL, 0xf, 0xf, true)});
+}
+
+// quad_perm control that gives each lane of a group of SPLIT the value of its lane S.
+template <int SPLIT, int S>
+constexpr int kQuadFrom = SPLIT == 4 ? S * 0x55 : S * 0x55 + 0xa0;
+
+template <int SPLIT, int C>
+struct LaneSums {
+  static_assert(C <= 8);
+  double acc[SPLIT == 8 ? 1 : C] = {};
+
+  __device__ __forceinline__ static void order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+
+  template <int S>
+  __device__ __forceinline__ void add_from(const NodeTerm (&t)[C], int n) {
+    if constexpr (S < SPLIT) {
+      if (S < n) {  // uniform over the grid
+#pragma unroll
+        for (int j = 0; j < C; ++j)
+          acc[j] = node_add(acc[j], NodeTerm{quad_move<kQuadFrom<SPLIT, S>>(t[j].a),
+                                             quad_move<kQuadFrom<SPLIT, S>>(t[j].b)});
+      }
+      add_from<S + 1>(t, n);
+    }
+  }
+
+  // The term of this lane's node; `left` nodes from the first lane's on.
+  __device__ __forceinline__ void add(const NodeTerm (&t)[C], double2* terms, int lanes, int sub,
+                                      int left) {
+    if constexpr (SPLIT == 1) {
+#pragma unroll
+      for (int j = 0; j < C; ++j) acc[j] = node_add(acc[j], t[j]);
+    } else if constexpr (SPLIT < 8) {
+      add_from<0>(t, left);
+    } else {
+      const int tid = threadIdx.x, n = left < lanes ? left : lanes;
+#pragma unroll
+      for (int j = 0; j < C; ++j) terms[j * kSplitStride + tid] = double2{t[j].a, t[j].b};
+      order();
+      if (sub < C) {
+        const double2* row = terms + sub * kSplitStride + (tid - sub);
+#pragma unroll 8
+        for (int s = 0; s < n; ++s) acc[0] = node_add(acc[0], NodeTerm{row[s].x, row[s].y});
+      }
+      order();
+    }
+  }
+
+  // Writes the components' values value(c, sum), or adds them to `total` in order (the
+  // first lane of a ray writes that).
+  template <class F>
+  __device__ __forceinline__ void finish(const FwdArgs& a, const Ray& y, int first, int lanes,
+                                         int sub, double& total, F value) const {
+    if constexpr (SPLIT < 8) {
+#pragma unroll
+      for (int j = 0; j < C; ++j) {
+        const double e = value(first + j, acc[j]);
+        if (a.out_mode == ZODI_OUT_COMPS) {
+          if (y.active && sub == 0) a.out[(int64_t)(first + j) * a.n_rays + y.r] = e;
+        } else {
+          total = __dadd_rn(total, e);
+        }
+      }
+    } else {
+      double e = 0.0;
+      if (sub < C) {
+        e = value(first + sub, acc[0]);
+        if (a.out_mode == ZODI_OUT_COMPS && y.active)
+          a.out[(int64_t)(first + sub) * a.n_rays + y.r] = e;
+      }
+      if (a.out_mode != ZODI_OUT_COMPS) {
+#pragma unroll
+        for (int j = 0; j < C; ++j) total = __dadd_rn(total, __shfl(e, j, lanes));
+      }
+    }
+  }
+};
+
 // One group of a Kelsall registry layout for one ray: group_pass on the ray's line.
 // PROPS: only its kShareCut bits are read (every band is centred with p = 4, every other
 // component but the cloud centred; the host checks, props_match and line_match).
-template <int L, uint32_t PROPS, bool NOSCAT, int... Ks, int... J>
+template <int SPLIT, uint32_t PROPS, bool NOSCAT, int... Ks, int... J>
 __device__ __forceinline__ void line_group(Grp<Ks...>, std::integer_sequence<int, J...>,
                                            const LineCtx& cx, const FwdArgs& a, const Ray& y,
-                                           const Line& l, int g, int first, double& total) {
+                                           const Line& l, int g, int first, double2* terms,
+                                           double& total) {
   constexpr int C = sizeof...(Ks);
   constexpr int kinds[C] = {Ks...};
   const ModelPtr M = cx.M;
@@ -615,11 +714,12 @@ __device__ __forceinline__ void line_group(Grp<Ks...>, std::integer_sequence<int
   }
   LinePhase lp = {0.0, 0.0};
   if (scatter) lp = line_phase(l);
-  double acc[C] = {};
-  for (int k0 = 0; k0 < cx.K; k0 += L) {
-    // with L lanes a ray, lane `sub` takes node k0 + sub (past the last node it repeats
-    // that one, and its term is not added)
-    const int k = L == 1 ? k0 : (k0 + cx.sub < cx.K ? k0 + cx.sub : cx.K - 1);
+  const int lanes = SPLIT == 8 ? a.lanes : SPLIT;
+  LaneSums<SPLIT, C> acc;
+  for (int k0 = 0; k0 < cx.K; k0 += lanes) {
+    // with several lanes a ray, lane `sub` takes node k0 + sub (past the last node it
+    // repeats that one, and its term is not added)
+    const int k = SPLIT == 1 ? k0 : (k0 + cx.sub < cx.K ? k0 + cx.sub : cx.K - 1);
     const ModelPtr Mk = opaque(M);
     const double wk = Mk->gl_w[k];
     LineNode nd;
@@ -642,31 +742,18 @@ __device__ __forceinline__ void line_group(Grp<Ks...>, std::integer_sequence<int
                                                               std::get<J>(lc), cx, l, nd, cut),
           Mk->shared[ZODI_S_SOLAR])),
      ...);
-    if constexpr (L == 1) {
-      ((acc[J] = node_add(acc[J], t[J])), ...);
-    } else {
-      add_in_node_order<L>(acc, t, cx.K - k0);
-    }
+    acc.add(t, terms, lanes, cx.sub, cx.K - k0);
   }
-  const bool write = y.active && cx.sub == 0;
-  (
-      [&] {
-        const double e = finish<ZODI_INTEGRAND_KELSALL, NOSCAT>(
-            M->comp[first + J], M->comp_flags[first + J], acc[J], h, 0.0);
-        if (a.out_mode == ZODI_OUT_COMPS) {
-          if (write) a.out[(int64_t)(first + J) * a.n_rays + y.r] = e;
-        } else {
-          total = __dadd_rn(total, e);
-        }
-      }(),
-      ...);
+  acc.finish(a, y, first, lanes, cx.sub, total, [&](int c, double sum) {
+    return finish<ZODI_INTEGRAND_KELSALL, NOSCAT>(M->comp[c], M->comp_flags[c], sum, h, 0.0);
+  });
 }
 
-template <int L, uint32_t PROPS, bool NOSCAT, int INTEGRAND, class... Gs, int... G>
+template <int SPLIT, uint32_t PROPS, bool NOSCAT, int INTEGRAND, class... Gs, int... G>
 __device__ __forceinline__ void run_line_groups(Layout<INTEGRAND, Gs...>,
                                                 std::integer_sequence<int, G...>,
                                                 const LineCtx& cx, const FwdArgs& a, Ray& y,
-                                                double& total) {
+                                                double2* terms, double& total) {
   (
       [&] {
         // The first group's node loop needs the registers: what the later groups take
@@ -677,18 +764,19 @@ __device__ __forceinline__ void run_line_groups(Layout<INTEGRAND, Gs...>,
           read_ray(again, y);
         }
         const Line l = make_line(y.ux, y.uy, y.uz, y.ox, y.oy, y.oz);
-        line_group<L, props_shift(PROPS, group_first<Gs...>(G)), NOSCAT>(
+        line_group<SPLIT, props_shift(PROPS, group_first<Gs...>(G)), NOSCAT>(
             Gs{}, std::make_integer_sequence<int, Gs::size>{}, cx, a, y, l, G,
-            group_first<Gs...>(G), total);
+            group_first<Gs...>(G), terms, total);
       }(),
       ...);
 }
 
-template <int L, uint32_t PROPS, bool NOSCAT, int INTEGRAND, class... Gs>
+template <int SPLIT, uint32_t PROPS, bool NOSCAT, int INTEGRAND, class... Gs>
 __device__ __forceinline__ void run_line(Layout<INTEGRAND, Gs...> lay, const LineCtx& cx,
-                                         const FwdArgs& a, Ray& y, double& total) {
-  run_line_groups<L, PROPS, NOSCAT>(lay, std::make_integer_sequence<int, sizeof...(Gs)>{}, cx, a,
-                                    y, total);
+                                         const FwdArgs& a, Ray& y, double2* terms,
+                                         double& total) {
+  run_line_groups<SPLIT, PROPS, NOSCAT>(lay, std::make_integer_sequence<int, sizeof...(Gs)>{},
+                                        cx, a, y, terms, total);
 }
 
 }  // namespace zodi

@@ -164,20 +164,38 @@ forward_layout(FwdArgs a) {
 // (kShareCut), for blocks whose delta_r values allow it (the registry parameters; a fit
 // that moves them runs without). NOSCAT (with SHARE): no component scatters, so no
 // scattering code is compiled in.
-template <class LAYOUT, int BLOCK, int L, bool SHARE, bool NOSCAT>
+template <class LAYOUT, int BLOCK, bool SHARE, bool NOSCAT>
 __global__ __launch_bounds__(BLOCK)
-__attribute__((amdgpu_waves_per_eu(L == 1 ? ForwardOccupancy<LAYOUT>::value : 2))) void
+__attribute__((amdgpu_waves_per_eu(ForwardOccupancy<LAYOUT>::value))) void
 forward_line(FwdArgs a) {
   __shared__ LineTables tables;
-  const LineCtx cx = line_ctx(as_const(a.m), tables, threadIdx.x % L);
-  constexpr int RAYS = BLOCK / L;
+  const LineCtx cx = line_ctx(as_const(a.m), tables, 0);
   constexpr uint32_t kProps = SHARE ? RegistryProps<LAYOUT>::value
                                     : props_without_share(RegistryProps<LAYOUT>::value);
-  const int local = threadIdx.x / L;
   for (int64_t tile = blockIdx.x; tile < a.n_tiles; tile += gridDim.x) {
-    Ray y = load_ray<RAYS>(a, tile, local);
+    Ray y = load_ray<BLOCK>(a, tile, threadIdx.x);
     double total = 0.0;
-    run_line<L, kProps, NOSCAT>(LAYOUT{}, cx, a, y, total);
+    run_line<1, kProps, NOSCAT>(LAYOUT{}, cx, a, y, nullptr, total);
+    if (a.out_mode == ZODI_OUT_SUM && y.active) a.out[y.r] = total;
+  }
+}
+
+// The same for small launches, a.lanes lanes per ray (2 to 32).
+template <class LAYOUT, int SPLIT, bool SHARE, bool NOSCAT>
+__global__ __launch_bounds__(kSplitBlock) __attribute__((amdgpu_waves_per_eu(2))) void
+forward_line_split(FwdArgs a) {
+  __shared__ LineTables tables;
+  __shared__ double2 terms[SPLIT == 8 ? kMaxSlots * kSplitStride : 1];
+  const int lanes = SPLIT == 8 ? a.lanes : SPLIT;
+  const LineCtx cx = line_ctx(as_const(a.m), tables, threadIdx.x & (lanes - 1));
+  constexpr uint32_t kProps = SHARE ? RegistryProps<LAYOUT>::value
+                                    : props_without_share(RegistryProps<LAYOUT>::value);
+  const int rays = blockDim.x / lanes;
+  for (int64_t tile = blockIdx.x; tile < a.n_tiles; tile += gridDim.x) {
+    Ray y = find_ray(a, tile * rays, threadIdx.x / lanes);
+    read_ray(a, y);
+    double total = 0.0;
+    run_line<SPLIT, kProps, NOSCAT>(LAYOUT{}, cx, a, y, terms, total);
     if (a.out_mode == ZODI_OUT_SUM && y.active && cx.sub == 0) a.out[y.r] = total;
   }
 }
@@ -186,19 +204,34 @@ forward_line(FwdArgs a) {
 // cycles per wave and node over the six groups where the arc sines, sines, cosines and
 // powers of every node took 6750 (and less where a wave skips a branch). Measured: RRM 25
 // um, 196 608 rays with the pixel vectors, 0.524 -> 0.329 ms.
-template <class LAYOUT, int BLOCK, int L>
+template <class LAYOUT, int BLOCK>
 __global__ __launch_bounds__(BLOCK)
-__attribute__((amdgpu_waves_per_eu(L == 1 ? ForwardOccupancy<LAYOUT>::value : 2))) void
+__attribute__((amdgpu_waves_per_eu(ForwardOccupancy<LAYOUT>::value))) void
 forward_rrm(FwdArgs a) {
   __shared__ LineAdjTables tables;
-  LineAdjCtx cx = line_adj_ctx(as_const(a.m), tables);
-  cx.sub = threadIdx.x % L;
-  constexpr int RAYS = BLOCK / L;
-  const int local = threadIdx.x / L;
+  const LineAdjCtx cx = line_adj_ctx(as_const(a.m), tables);
   for (int64_t tile = blockIdx.x; tile < a.n_tiles; tile += gridDim.x) {
-    const Ray y = load_ray<RAYS>(a, tile, local);
+    const Ray y = load_ray<BLOCK>(a, tile, threadIdx.x);
     double total = 0.0;
-    run_rrm<L>(LAYOUT{}, cx, a, y, total);
+    run_rrm<1>(LAYOUT{}, cx, a, y, nullptr, total);
+    if (a.out_mode == ZODI_OUT_SUM && y.active) a.out[y.r] = total;
+  }
+}
+
+template <class LAYOUT, int SPLIT>
+__global__ __launch_bounds__(kSplitBlock) __attribute__((amdgpu_waves_per_eu(2))) void
+forward_rrm_split(FwdArgs a) {
+  __shared__ LineAdjTables tables;
+  __shared__ double2 terms[SPLIT == 8 ? kMaxSlots * kSplitStride : 1];
+  LineAdjCtx cx = line_adj_ctx(as_const(a.m), tables);
+  const int lanes = SPLIT == 8 ? a.lanes : SPLIT;
+  cx.sub = threadIdx.x & (lanes - 1);
+  const int rays = blockDim.x / lanes;
+  for (int64_t tile = blockIdx.x; tile < a.n_tiles; tile += gridDim.x) {
+    Ray y = find_ray(a, tile * rays, threadIdx.x / lanes);
+    read_ray(a, y);
+    double total = 0.0;
+    run_rrm<SPLIT>(LAYOUT{}, cx, a, y, terms, total);
     if (a.out_mode == ZODI_OUT_SUM && y.active && cx.sub == 0) a.out[y.r] = total;
   }
 }
@@ -380,32 +413,13 @@ FwdKernel pick_layout_block(int block, int L) {
   }
 }
 
-template <class LAYOUT, int BLOCK>
-FwdKernel pick_rrm_lanes(int L) {
-  switch (L) {
-    case 1:
-      return forward_rrm<LAYOUT, BLOCK, 1>;
-    case 2:
-      return forward_rrm<LAYOUT, BLOCK, 2>;
-    case 4:
-      return forward_rrm<LAYOUT, BLOCK, 4>;
-    case 8:
-      return forward_rrm<LAYOUT, BLOCK, 8>;
-    default:
-      return nullptr;
-  }
-}
-
 template <class LAYOUT>
 FwdKernel pick_rrm(int block, int L) {
-  switch (block) {
-    case 256:
-      return pick_rrm_lanes<LAYOUT, 256>(L);
-    case 512:
-      return pick_rrm_lanes<LAYOUT, 512>(L);
-    default:
-      return nullptr;
-  }
+  if (block != 256 && block != 512) return nullptr;
+  if (L == 2) return forward_rrm_split<LAYOUT, 2>;
+  if (L == 4) return forward_rrm_split<LAYOUT, 4>;
+  if (L > 4) return forward_rrm_split<LAYOUT, 8>;
+  return block == 256 ? forward_rrm<LAYOUT, 256> : forward_rrm<LAYOUT, 512>;
 }
 
 // Whether no component of the block has its scattering term (ZODI_CF_SCATTER).
@@ -415,46 +429,28 @@ inline bool no_scattering(const zodi_model* m) {
   return true;
 }
 
-template <class LAYOUT, int BLOCK, int L>
-FwdKernel pick_line_terms(bool share, bool noscat) {
-  if (L > 1 || !share) return forward_line<LAYOUT, BLOCK, L, false, false>;
-  if (noscat) return forward_line<LAYOUT, BLOCK, 1, true, true>;
-  return forward_line<LAYOUT, BLOCK, 1, true, false>;
-}
-
-template <class LAYOUT, int BLOCK>
-FwdKernel pick_line_lanes(int L, bool share, bool noscat) {
-  switch (L) {
-    case 1:
-      return pick_line_terms<LAYOUT, BLOCK, 1>(share, noscat);
-    case 2:
-      return pick_line_terms<LAYOUT, BLOCK, 2>(share, noscat);
-    case 4:
-      return pick_line_terms<LAYOUT, BLOCK, 4>(share, noscat);
-    case 8:
-      return pick_line_terms<LAYOUT, BLOCK, 8>(share, noscat);
-    default:
-      return nullptr;
-  }
+template <class LAYOUT, bool SHARE, bool NOSCAT>
+FwdKernel pick_line_block(int block, int L) {
+  if (block != 256 && block != 512) return nullptr;
+  if (L == 2) return forward_line_split<LAYOUT, 2, SHARE, NOSCAT>;
+  if (L == 4) return forward_line_split<LAYOUT, 4, SHARE, NOSCAT>;
+  if (L > 4) return forward_line_split<LAYOUT, 8, SHARE, NOSCAT>;
+  return block == 256 ? forward_line<LAYOUT, 256, SHARE, NOSCAT>
+                      : forward_line<LAYOUT, 512, SHARE, NOSCAT>;
 }
 
 template <class LAYOUT>
 FwdKernel pick_line(const zodi_model* m, int block, int L) {
-  const bool share = props_match(m, RegistryProps<LAYOUT>::value), noscat = no_scattering(m);
-  switch (block) {
-    case 256:
-      return pick_line_lanes<LAYOUT, 256>(L, share, noscat);
-    case 512:
-      return pick_line_lanes<LAYOUT, 512>(L, share, noscat);
-    default:
-      return nullptr;
-  }
+  if (!props_match(m, RegistryProps<LAYOUT>::value))
+    return pick_line_block<LAYOUT, false, false>(block, L);
+  return no_scattering(m) ? pick_line_block<LAYOUT, true, true>(block, L)
+                          : pick_line_block<LAYOUT, true, false>(block, L);
 }
 
 // The line kernels when the block has the layout's registry properties (the Kelsall
-// layouts: with the shared cut-offs for one lane per ray, the launch the tuner picks
-// for large batches, and without scattering code when no component scatters), else the
-// one that tests each component's flags.
+// layouts: with the shared cut-offs where the delta_r values allow it, and then without
+// scattering code when no component scatters), else the one that tests each component's
+// flags.
 template <class LAYOUT>
 bool line_eligible(const zodi_model* m) {
   constexpr bool kKelsall = layout_integrand<LAYOUT>() == ZODI_INTEGRAND_KELSALL;
@@ -520,6 +516,8 @@ FwdKernel pick_generic(int block, int L) {
   }
 }
 
+bool takes_line(const zodi_model* m, LayoutId id);
+
 constexpr int kGenericWaves = 3;
 
 // Resident waves per SIMD of the kernel pick_forward chooses.
@@ -538,15 +536,39 @@ int forward_waves(const zodi_model* m, int variant) {
   }
 }
 
-// Lanes per ray when the caller leaves it open: the node terms are added in node
-// order whatever the split, so it only sets the speed. A small launch whose one
-// lane per ray leaves SIMDs idle, or one wave on a SIMD with nothing to hide its
-// latency, splits each ray's nodes over up to 8 lanes while the waves still fit
-// the resident slots (kernel waves per SIMD x 4 SIMDs x CUs). Measured (DIRBE,
-// one observer): 3072 rays 102 -> 36 us at 8 lanes, 49 152 rays 107 -> 76 us at
-// 4, and 196 608 rays fastest at 1.
+// Lanes per ray when the caller leaves it open: the node terms are added in node order
+// whatever the split, so it only sets the speed.
+//
+// The line kernels: with r waves of L lanes a ray on a SIMD and K nodes a ray, a launch
+// takes (r + 1) (ceil(K / L) + 4) units within some 10 % (4: a wave's work beside its
+// nodes; 1: the latency of its chains, which r waves share; below two waves it shows in
+// full), and the cheapest L is taken. Measured with 50 nodes (us, up to 8 lanes with the
+// sums fetched by ds_bpermute -> this rule; DIRBE, then RRM): 3072 rays 33 -> 14 and
+// 48 -> 21, 12 288 rays 43 -> 22 and 57 -> 38, 49 152 rays 67 -> 43 and 101 -> 92,
+// 150 000 rays 141 -> 108 and 297 -> 244. Past 5 waves a SIMD the Kelsall kernels of one
+// lane a ray, which keep 5, are as fast or faster (196 608 rays: 123 at 1, 126 at 2); the
+// RRM kernels, which keep 4, up to 8 (196 608 rays: 298 at 1, 282 at 2).
+//
+// The general kernel: up to 8 lanes while the waves still fit the resident slots.
 int default_lanes(const zodi_model* m, int variant, int64_t n_rays) {
-  const int64_t slots = (int64_t)forward_waves(m, variant) * 4 * cu_count();
+  const LayoutId id = variant == 0 ? kLayoutGeneric : match_layout(m);
+  const int64_t simds = (int64_t)4 * cu_count();
+  if (takes_line(m, id)) {
+    const int most = id == kLayoutDirbe || id == kLayoutKelsall4 ? 5 : 8;
+    int best = 1;
+    int64_t least = INT64_MAX;
+    for (int L : {1, 2, 4, 8, 16, 32}) {
+      const int64_t waves = (n_rays * L + 63) / 64, r = (waves + simds - 1) / simds;
+      if (L > 1 && r > most) break;
+      const int64_t cost = (std::max<int64_t>(r, 2) + 1) * ((m->n_nodes + L - 1) / L + 4);
+      if (cost <= least) {
+        least = cost;
+        best = L;
+      }
+    }
+    return best;
+  }
+  const int64_t slots = forward_waves(m, variant) * simds;
   for (int L : {8, 4, 2})
     if ((n_rays * L + 63) / 64 <= slots) return L;
   return 1;
@@ -601,7 +623,7 @@ zodi_status fill_args(FwdArgs& a, const zodi_model* model_host, const zodi_model
   a.beyond = beyond;
   a.out = nullptr;
   a.out_mode = 0;
-  a.pad = 0;
+  a.lanes = 1;
   a.n_tiles = 0;
   return ZODI_OK;
 }
@@ -642,9 +664,10 @@ zodi_status zodi_forward(const zodi_model* model_host, const zodi_model* model_d
   }
   if (variant < 0 || variant > 1) return fail(ZODI_ERR_ARG, "unknown variant %d", variant);
   if (L < 0) return fail(ZODI_ERR_ARG, "lanes_per_ray %d < 0", L);
-  if (L == 0) L = default_lanes(model_host, variant, n_rays);
   if (L > block) return fail(ZODI_ERR_ARG, "lanes_per_ray %d > block %d", L, block);
-  FwdKernel k = pick_forward(model_host, block, L, variant);
+  const bool lanes_ok = L <= 8 && (L & (L - 1)) == 0;  // 16 and 32 are the default's own
+  if (L == 0) L = std::min(default_lanes(model_host, variant, n_rays), block);
+  FwdKernel k = lanes_ok ? pick_forward(model_host, block, L, variant) : nullptr;
   if (k == nullptr)
     return fail(ZODI_ERR_ARG, "unsupported launch: block %d, lanes_per_ray %d", block, L);
   if (per_cu < 0 || per_cu > 64)
@@ -657,6 +680,7 @@ zodi_status zodi_forward(const zodi_model* model_host, const zodi_model* model_d
   if (grid > 0x7fffffff) return fail(ZODI_ERR_TOO_LARGE, "grid of %lld blocks", (long long)grid);
   a.out = out;
   a.out_mode = out_mode;
+  a.lanes = L;
   a.n_tiles = n_tiles;
   hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(block), 0, (hipStream_t)stream, a);
   return check_hip(hipGetLastError(), "forward launch");

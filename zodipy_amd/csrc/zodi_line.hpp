@@ -121,12 +121,24 @@ __device__ __forceinline__ ExpConst exp_const() {
   return e;
 }
 
+// 2^(j/256) in LDS (stage_line_tables).
+__shared__ __attribute__((aligned(2048))) double g_exp2[256];
+
+__constant__ double kLineInv[256] = {ZODI_LINE_INV_TABLE};  // inv_j of PowTable
+__constant__ double kLineLog[256] = {ZODI_LINE_LOG_TABLE};  // -log inv_j
+
+// Every thread of the block must call this before exp_neg_node.
+__device__ __forceinline__ void stage_line_tables() {
+  for (int i = threadIdx.x; i < 256; i += blockDim.x) g_exp2[i] = kMathTablesConst[i];
+  __syncthreads();
+}
+
 __device__ __forceinline__ double exp_node_tail(const ExpConst& e, double f, int k) {
   double q = fma(f, e.c4, e.c3);
   q = fma(q, f, e.c2);
   q = fma(q, f, e.c1);
   q = q * f;
-  const double t = *(const double*)((const char*)g_math + ((uint32_t)(k << 3) & 0x7f8u));
+  const double t = *(const double*)((const char*)g_exp2 + ((uint32_t)(k << 3) & 0x7f8u));
   return __builtin_amdgcn_ldexp(fma(t, q, t), k >> 8);
 }
 
@@ -186,40 +198,34 @@ __device__ __forceinline__ PowPoly pow_poly(double p) {
   return {to_scalar(q.b1), to_scalar(q.b2), to_scalar(q.b3), q.b4, to_scalar(q.b5)};
 }
 
-// inv_j: 2/(1 + (j + 1/2)/256) rounded to a multiple of 2^-12 (13 significant bits), so
-// its product with a 53-bit mantissa fits the FMA exactly and only r is rounded.
-__device__ __forceinline__ double pow_inverse(int j) {
-  const double c = 0.5 + ((double)j + 0.5) * (1.0 / 512.0);
-  return __builtin_rint(4096.0 / c) * (1.0 / 4096.0);
-}
+// inv_j (kLineInv): 2/(1 + (j + 1/2)/256) rounded to a multiple of 2^-12 (13 significant
+// bits), so its product with a 53-bit mantissa fits the FMA exactly and only r is rounded.
 
 // 2^z for the exact z = zh + zl, |zl| tiny.
-__device__ __forceinline__ double exp2_table(double zh, double zl) {
+__device__ __forceinline__ double exp2_table(const ExpConst& ec, double zh, double zl) {
   const double k = __builtin_rint(zh);
   const double f = (zh - k) + zl;
   constexpr double kLn2Hi = 0x1.62e42fefa39efp-1, kLn2Lo = 0x1.abc9e3b39803fp-56;
   const double y = f * kLn2Hi;
   const double yl = fma(f, kLn2Hi, -y) + f * kLn2Lo;
-  const double e = exp_fast_bounded(y);
+  const double e = exp_neg_any(ec, -y);
   return __builtin_amdgcn_ldexp(fma(e, yl, e), (int)k);
 }
 
 // Entries i, i + stride, ... of the table of x^p, the whole multiplied by `factor`;
-// exponents from e_first on. stage_math_tables() must have run.
-__device__ __forceinline__ void build_pow_table(PowTable& t, double p, double factor, int e_first,
-                                                int i, int stride) {
-  for (int j = i; j < 384; j += stride) {
-    if (j < 256) {
-      const double inv = pow_inverse(j);
-      // inv^-p; -p log(inv) is below |p| 0.7, so its rounding stays below an ulp
-      t.c[j] = double2{inv, exp_fast_bounded(-p * log_pos(inv))};
-    } else {
-      const int e = e_first + (j - 256);
-      const double zh = p * (double)e;
-      const double zl = fma(p, (double)e, -zh);
-      // frexp's exponent e: x = 2^e m, m in [1/2, 1); its biased exponent is e + 1022
-      t.scale[(e + 1022) & 127] = factor * exp2_table(zh, zl);
-    }
+// exponents from e_first on. stage_line_tables() must have run.
+__device__ __forceinline__ void build_pow_table(PowTable& t, const ExpConst& ec, double p,
+                                                double factor, int e_first, int i, int stride) {
+  for (int j = i; j < 256; j += stride) {
+    // inv^-p; -p log(inv) is below |p| 0.7, so its rounding stays below an ulp
+    t.c[j] = double2{kLineInv[j], exp_neg_any(ec, -(p * kLineLog[j]))};
+  }
+  for (int j = i; j < 128; j += stride) {
+    const int e = e_first + j;
+    const double zh = p * (double)e;
+    const double zl = fma(p, (double)e, -zh);
+    // frexp's exponent e: x = 2^e m, m in [1/2, 1); its biased exponent is e + 1022
+    t.scale[(e + 1022) & 127] = factor * exp2_table(ec, zh, zl);
   }
 }
 
@@ -293,13 +299,14 @@ struct LineCtx {
 
 // Builds the block's tables (every thread of the block must call it).
 __device__ __forceinline__ LineCtx line_ctx(ModelPtr M, LineTables& tab, int sub) {
-  stage_math_tables();
+  stage_line_tables();
+  const ExpConst ec = exp_const();
   const int i = threadIdx.x, n = blockDim.x;
   const ParamPtr P = M->comp[0];  // the cloud (the layouts' first component)
   const double pt = -0.5 * M->group_delta[0], pr = -0.5 * P[7], pv = P[9];
-  build_pow_table(tab.temperature, pt, M->group_T0[0] * M->tab_inv_step, kPowRadiusFirst, i, n);
-  build_pow_table(tab.radial, pr, P[6], kPowRadiusFirst, i, n);
-  build_pow_table(tab.vertical, pv, 1.0, kPowUnitFirst, i, n);
+  build_pow_table(tab.temperature, ec, pt, M->group_T0[0] * M->tab_inv_step, kPowRadiusFirst, i, n);
+  build_pow_table(tab.radial, ec, pr, P[6], kPowRadiusFirst, i, n);
+  build_pow_table(tab.vertical, ec, pv, 1.0, kPowUnitFirst, i, n);
   load_planck(M, tab.planck, i, n);
   __syncthreads();
   LineCtx cx;
@@ -309,7 +316,7 @@ __device__ __forceinline__ LineCtx line_ctx(ModelPtr M, LineTables& tab, int sub
   cx.pr = pow_poly(pr);
   cx.pv = pow_poly(pv);
   cx.uo1 = to_scalar(M->tab_T[0] * M->tab_inv_step - 1.0);
-  cx.ec = exp_const();
+  cx.ec = ec;
   cx.K = M->n_nodes;
   cx.sub = sub;
   return cx;

@@ -25,7 +25,7 @@
 namespace zodi {
 
 // ---------------------------------------------------------------- log
-// log x for positive normal x from a table of (inv_j, -log inv_j) (pow_inverse) and the
+// log x for positive normal x from a table of (inv_j, -log inv_j) (kLineInv) and the
 // Taylor series of log(1 + r) to r^5, |r| < 2^-8.9 (first term left out 1.4e-17).
 struct LogConst {
   double c4;           // vector register: -1/4
@@ -68,11 +68,9 @@ struct LineAdjCtx {
 };
 
 __device__ __forceinline__ LineAdjCtx line_adj_ctx(ModelPtr M, LineAdjTables& tab) {
-  stage_math_tables();
-  for (int j = threadIdx.x; j < 256; j += blockDim.x) {
-    const double inv = pow_inverse(j);
-    tab.log_tab[j] = double2{inv, -log_pos(inv)};
-  }
+  stage_line_tables();
+  for (int j = threadIdx.x; j < 256; j += blockDim.x)
+    tab.log_tab[j] = double2{kLineInv[j], kLineLog[j]};
   load_planck(M, tab.planck, threadIdx.x, blockDim.x);
   __syncthreads();
   LineAdjCtx cx;

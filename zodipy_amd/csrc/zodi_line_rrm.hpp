@@ -101,13 +101,13 @@ template <>
 struct LineComp<ZODI_NARROW_BAND> : PlaneComp {
   double lo2;  // log R_outer^2
   __device__ __forceinline__ LineComp(ParamPtr P, const Line& l, double, double)
-      : PlaneComp(P, l, P[8]), lo2(to_scalar(2.0 * log_pos(P[11]))) {}
+      : PlaneComp(P, l, P[8]), lo2(to_scalar(2.0 * log(P[11]))) {}
 };
 template <>
 struct LineComp<ZODI_BROAD_BAND> : PlaneComp {
   double lo2;
   __device__ __forceinline__ LineComp(ParamPtr P, const Line& l, double, double)
-      : PlaneComp(P, l, P[8]), lo2(to_scalar(2.0 * log_pos(P[11]))) {}
+      : PlaneComp(P, l, P[8]), lo2(to_scalar(2.0 * log(P[11]))) {}
 };
 template <>
 struct LineComp<ZODI_RING_RRM> : LineComp<ZODI_RING> {
@@ -218,10 +218,11 @@ __device__ __forceinline__ RrmNode rrm_node(const LineAdjCtx& cx, const Line& l,
 }
 
 // ---------------------------------------------------------------- forward
-template <int L, int... Ks, int... J>
+template <int SPLIT, int... Ks, int... J>
 __device__ __forceinline__ void rrm_group(Grp<Ks...>, std::integer_sequence<int, J...>,
                                           const LineAdjCtx& cx, const FwdArgs& a, const Ray& y,
-                                          const Line& l, int g, int first, double& total) {
+                                          const Line& l, int g, int first, double2* terms,
+                                          double& total) {
   constexpr int C = sizeof...(Ks);
   constexpr int kinds[C] = {Ks...};
   const ModelPtr M = cx.M;
@@ -232,52 +233,41 @@ __device__ __forceinline__ void rrm_group(Grp<Ks...>, std::integer_sequence<int,
   const double us = to_scalar(M->group_T0[g] * M->tab_inv_step);
   const double uo1 = to_scalar(M->tab_T[0] * M->tab_inv_step - 1.0);
   const std::tuple<LineComp<Ks>...> lc{LineComp<Ks>(M->comp[first + J], l, y.ex, y.ey)...};
-  double acc[C] = {};
-  for (int k0 = 0; k0 < cx.K; k0 += L) {
-    const int k = L == 1 ? k0 : (k0 + cx.sub < cx.K ? k0 + cx.sub : cx.K - 1);
+  const int lanes = SPLIT == 8 ? a.lanes : SPLIT;
+  LaneSums<SPLIT, C> acc;
+  for (int k0 = 0; k0 < cx.K; k0 += lanes) {
+    const int k = SPLIT == 1 ? k0 : (k0 + cx.sub < cx.K ? k0 + cx.sub : cx.K - 1);
     const ModelPtr Mk = opaque(M);
     const double wk = Mk->gl_w[k];
     const RrmNode o = rrm_node(cx, l, fma(th, Mk->gl_x[k], tm), half_delta, us, uo1);
     const double wB = wk * o.B;
     const NodeTerm t[C] = {NodeTerm{
         wB, rrm_density<kinds[J]>(Mk->comp[first + J], std::get<J>(lc), cx, l, o.nd, o.lR2)}...};
-    if constexpr (L == 1) {
-      ((acc[J] = node_add(acc[J], t[J])), ...);
-    } else {
-      add_in_node_order<L>(acc, t, cx.K - k0);
-    }
+    acc.add(t, terms, lanes, cx.sub, cx.K - k0);
   }
   const double cal = M->shared[ZODI_S_CALIBRATION];
-  const bool write = y.active && cx.sub == 0;
-  (
-      [&] {
-        const double e = finish<ZODI_INTEGRAND_RRM>(M->comp[first + J], M->comp_flags[first + J],
-                                                    acc[J], h, cal);
-        if (a.out_mode == ZODI_OUT_COMPS) {
-          if (write) a.out[(int64_t)(first + J) * a.n_rays + y.r] = e;
-        } else {
-          total = __dadd_rn(total, e);
-        }
-      }(),
-      ...);
+  acc.finish(a, y, first, lanes, cx.sub, total, [&](int c, double sum) {
+    return finish<ZODI_INTEGRAND_RRM>(M->comp[c], M->comp_flags[c], sum, h, cal);
+  });
 }
 
-template <int L, class... Gs, int... G>
+template <int SPLIT, class... Gs, int... G>
 __device__ __forceinline__ void rrm_groups(Layout<ZODI_INTEGRAND_RRM, Gs...>,
                                            std::integer_sequence<int, G...>,
                                            const LineAdjCtx& cx, const FwdArgs& a, const Ray& y,
-                                           const Line& l, double& total) {
-  (rrm_group<L>(Gs{}, std::make_integer_sequence<int, Gs::size>{}, cx, a, y, l, G,
-                group_first<Gs...>(G), total),
+                                           const Line& l, double2* terms, double& total) {
+  (rrm_group<SPLIT>(Gs{}, std::make_integer_sequence<int, Gs::size>{}, cx, a, y, l, G,
+                    group_first<Gs...>(G), terms, total),
    ...);
 }
 
-template <int L, class... Gs>
+template <int SPLIT, class... Gs>
 __device__ __forceinline__ void run_rrm(Layout<ZODI_INTEGRAND_RRM, Gs...> lay,
                                         const LineAdjCtx& cx, const FwdArgs& a, const Ray& y,
-                                        double& total) {
+                                        double2* terms, double& total) {
   const Line l = make_line(y.ux, y.uy, y.uz, y.ox, y.oy, y.oz);
-  rrm_groups<L>(lay, std::make_integer_sequence<int, sizeof...(Gs)>{}, cx, a, y, l, total);
+  rrm_groups<SPLIT>(lay, std::make_integer_sequence<int, sizeof...(Gs)>{}, cx, a, y, l, terms,
+                    total);
 }
 
 // ---------------------------------------------------------------- partials
