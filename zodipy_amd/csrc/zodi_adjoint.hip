@@ -84,7 +84,7 @@ __global__ __launch_bounds__(256) void adjoint_reduce(const double* __restrict__
 // parameters [y P, y P + P). Thread t takes the ray pairs (r, r + 1) with
 // r = x R + 2 t + 512 i over the largest multiple of 512 rays of the range, then
 // single rays t, t + 256, ... of the rest, adding r before r + 1. Each wave sums its
-// lanes with the xor butterfly, and the waves' sums are added in wave order into
+// lanes (wave_fold), and the waves' sums are added in wave order into
 // partials[x][p] (entry n_params: chi^2, from the y = 0 blocks). adjoint_reduce
 // then adds the partials of all x in a fixed order.
 //
@@ -163,10 +163,14 @@ __global__ __launch_bounds__(256) void jacobian_chi2(const double* __restrict__ 
       if (q < np) acc[q] += g * col[q * ld];
     }
   }
+  static_assert(kJacParams == 32);
 #pragma unroll
-  for (int q = 0; q < kJacParams; ++q) {
-    const double v = wave_sum(acc[q]);
-    if (lane == 0) red[wave][q] = v;
+  for (int half = 0; half < 2; ++half) {
+    double v[16];
+#pragma unroll
+    for (int q = 0; q < 16; ++q) v[q] = acc[16 * half + q];
+    const double s = wave_fold<32>(v);
+    if ((lane & 3) == 0) red[wave][16 * half + fold_index(lane)] = s;
   }
   chi = wave_sum(chi);
   if (lane == 0) red[wave][kJacParams] = chi;

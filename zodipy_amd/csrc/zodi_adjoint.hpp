@@ -43,6 +43,76 @@ __device__ __forceinline__ double wave_sum(double v) {
   return v;
 }
 
+// Sums over the wave of up to 16 values at once. Each step halves the values held: a
+// lane keeps one value of a pair and gives the other to its partner (v_permlane32_swap
+// and v_permlane16_swap, then DPP moves into half the banks), 15 additions and two more
+// for the quad where 16 butterflies take 96 and 192 ds_bpermute. Lane l returns the sum
+// of value fold_index(l).
+template <int CTRL, int BANKS>
+__device__ __forceinline__ double dpp_into(double old, double x) {
+  const int2 o = __builtin_bit_cast(int2, old), v = __builtin_bit_cast(int2, x);
+  return __builtin_bit_cast(
+      double, int2{__builtin_amdgcn_update_dpp(o.x, v.x, CTRL, 0xf, BANKS, false),
+                   __builtin_amdgcn_update_dpp(o.y, v.y, CTRL, 0xf, BANKS, false)});
+}
+
+__device__ __forceinline__ int fold_index(int lane) {
+  return (lane >> 5 & 1) | (lane >> 3 & 2) | (lane >> 1 & 4) | (lane << 1 & 8);
+}
+
+// a's sum over the lanes l and l ^ BIT where bit BIT of l is 0, b's where it is 1.
+template <int BIT>
+__device__ __forceinline__ double fold_pair(double a, double b) {
+  if constexpr (BIT >= 16) {
+    const uint2 x = __builtin_bit_cast(uint2, a), y = __builtin_bit_cast(uint2, b);
+    typedef unsigned pair __attribute__((ext_vector_type(2)));
+    pair lo, hi;
+    if constexpr (BIT == 32) {
+      lo = __builtin_amdgcn_permlane32_swap(x.x, y.x, false, false);
+      hi = __builtin_amdgcn_permlane32_swap(x.y, y.y, false, false);
+    } else {
+      lo = __builtin_amdgcn_permlane16_swap(x.x, y.x, false, false);
+      hi = __builtin_amdgcn_permlane16_swap(x.y, y.y, false, false);
+    }
+    return __builtin_bit_cast(double, uint2{lo[0], hi[0]}) +
+           __builtin_bit_cast(double, uint2{lo[1], hi[1]});
+  } else if constexpr (BIT == 8) {  // row_ror:8
+    return dpp_into<0x128, 0xc>(a, b) + dpp_into<0x128, 0x3>(b, a);
+  } else {  // row_ror:4 and row_ror:12
+    return dpp_into<0x124, 0xa>(a, b) + dpp_into<0x12c, 0x5>(b, a);
+  }
+}
+
+template <int BIT, int N>
+__device__ __forceinline__ double wave_fold(const double (&v)[N]) {
+  static_assert(N >= 1 && N <= (BIT == 32 ? 16 : BIT == 16 ? 8 : BIT == 8 ? 4 : 2));
+  double w[(N + 1) / 2];
+#pragma unroll
+  for (int i = 0; i < (N + 1) / 2; ++i)
+    w[i] = fold_pair<BIT>(v[2 * i], 2 * i + 1 < N ? v[(2 * i + 1) % N] : 0.0);
+  if constexpr (BIT > 4) {
+    return wave_fold<BIT / 2>(w);
+  } else {
+    const double q = w[0] + dpp_into<0x4e, 0xf>(w[0], w[0]);  // quad_perm 2 3 0 1
+    return q + dpp_into<0xb1, 0xf>(q, q);                     // quad_perm 1 0 3 2
+  }
+}
+
+// Onto a row of the wave's own, whose other additions come in program order.
+__device__ __forceinline__ void lds_add(double* p, double x) {
+  __hip_atomic_fetch_add(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+}
+
+// The wave's sums of one component's derivatives v (geometry and shape parameters at off
+// and on, then the entries ia and ib) onto its row; entries may coincide.
+template <int N>
+__device__ __forceinline__ void add_folded(const double (&v)[N], double* row, int lane, int off,
+                                           int ia, int ib) {
+  const double s = wave_fold<32>(v);
+  const int i = fold_index(lane);
+  if ((lane & 3) == 0 && i < N) lds_add(row + (i < N - 2 ? off + i : (i == N - 2 ? ia : ib)), s);
+}
+
 // B(T) of the Planck table on its index axis, u = (T - T_first)/dT, as
 // planck_lookup_u forms it, and the table slope dB/dT of the interval (0 where
 // the table clamps, u <= 0 or u >= ZODI_N_TEMPS - 1; the LDS entries past the

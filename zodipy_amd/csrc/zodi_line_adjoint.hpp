@@ -539,20 +539,14 @@ __device__ __forceinline__ void line_adj_group(Grp<Ks...>, std::integer_sequence
             col[M->grad_spec_b[c] * ld] = da;
           }
         } else {
+          double v[5 + NP + 2];
 #pragma unroll
-          for (int q = 0; q < 5; ++q) geo[q] = wave_sum(geo[q]);
+          for (int q = 0; q < 5; ++q) v[q] = geo[q];
 #pragma unroll
-          for (int q = 0; q < NP; ++q) dp[q] = wave_sum(dp[q]);
-          const double sde = wave_sum(de), sda = wave_sum(da);
-          if (lane == 0) {
-            const int off = M->grad_comp[c];
-#pragma unroll
-            for (int q = 0; q < 5; ++q) row[off + q] += geo[q];
-#pragma unroll
-            for (int q = 0; q < NP; ++q) row[off + 5 + q] += dp[q];
-            row[M->grad_spec_a[c]] += sde;
-            row[M->grad_spec_b[c]] += sda;
-          }
+          for (int q = 0; q < NP; ++q) v[5 + q] = dp[q];
+          v[5 + NP] = de;
+          v[6 + NP] = da;
+          add_folded(v, row, lane, M->grad_comp[c], M->grad_spec_a[c], M->grad_spec_b[c]);
         }
       }(),
       ...);
@@ -664,12 +658,12 @@ __device__ __forceinline__ void line_adj_body(const AdjArgs& a) {
       double sh[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
       double total = 0.0;
       line_adj_layout<SCAT, false>(LAYOUT{}, cx, a, y, gscale, row, ln, sh, total);
+      double v[NSH];
 #pragma unroll
-      for (int q = 0; q < NSH; ++q) sh[q] = wave_sum(sh[q]);
-      if (ln == 0) {
-#pragma unroll
-        for (int q = 0; q < NSH; ++q) row[M->grad_shared[q]] += sh[q];
-      }
+      for (int q = 0; q < NSH; ++q) v[q] = sh[q];
+      const double s = wave_fold<32>(v);
+      const int i = fold_index(ln);
+      if ((ln & 3) == 0 && i < NSH) lds_add(row + M->grad_shared[i], s);
     });
   }
 }

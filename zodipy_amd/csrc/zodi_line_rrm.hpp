@@ -604,20 +604,14 @@ __device__ __forceinline__ void rrm_adj_group(Grp<Ks...>, std::integer_sequence<
             col[M->grad_spec_b[c] * ld] = dd;
           }
         } else {
+          double v[5 + NP + 2];
 #pragma unroll
-          for (int q = 0; q < 5; ++q) geo[q] = wave_sum(geo[q]);
+          for (int q = 0; q < 5; ++q) v[q] = geo[q];
 #pragma unroll
-          for (int q = 0; q < NP; ++q) dp[q] = wave_sum(dp[q]);
-          const double sT = wave_sum(dT), sD = wave_sum(dd);
-          if (lane == 0) {
-            const int off = M->grad_comp[c];
-#pragma unroll
-            for (int q = 0; q < 5; ++q) row[off + q] += geo[q];
-#pragma unroll
-            for (int q = 0; q < NP; ++q) row[off + 5 + q] += dp[q];
-            row[M->grad_spec_a[c]] += sT;
-            row[M->grad_spec_b[c]] += sD;
-          }
+          for (int q = 0; q < NP; ++q) v[5 + q] = dp[q];
+          v[5 + NP] = dT;
+          v[6 + NP] = dd;
+          add_folded(v, row, lane, M->grad_comp[c], M->grad_spec_a[c], M->grad_spec_b[c]);
         }
       }(),
       ...);

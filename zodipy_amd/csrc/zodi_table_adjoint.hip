@@ -43,10 +43,6 @@ namespace zodi {
 
 namespace {
 
-__device__ __forceinline__ void lds_add(double* p, double x) {
-  __hip_atomic_fetch_add(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-}
-
 // A lane's pending shares of consecutive nodes in one table interval: entry j
 // gets s0, entry j + 1 gets s1 (none past the last entry). Nodes along a ray
 // change temperature slowly, so most of them only add to registers; the LDS
