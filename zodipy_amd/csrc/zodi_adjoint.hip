@@ -265,13 +265,14 @@ AdjKernel pick_adj_layout(int chunk, int split, bool jac) {
   }
 }
 
-AdjKernel pick_adjoint(const zodi_model* m, int chunk, int split, bool jac) {
+AdjKernel pick_adjoint(const zodi_model* m, int chunk, int split, int pass) {
+  const bool jac = pass == kPassJac;
   const LayoutId id = match_layout(m);
   if (takes_line(m)) {
     if (id == kLayoutRRM || id == kLayoutRRMSplit)
       return line_adjoint_rrm(id == kLayoutRRMSplit, jac);
     const int scat = block_noscat(m) ? 0 : ((m->flags & 1) == 0 ? 1 : 2);
-    return id == kLayoutDirbe ? line_adjoint_dirbe(scat, jac) : line_adjoint_kelsall4(scat, jac);
+    return id == kLayoutDirbe ? line_adjoint_dirbe(scat, pass) : line_adjoint_kelsall4(scat, pass);
   }
   switch (id) {
     case kLayoutDirbe:
@@ -444,6 +445,15 @@ zodi_status table_plan(const zodi_model* m, const zodi_launch* launch, int64_t n
 // MI355X's 288 GB of HBM); larger problems recompute the integrand instead.
 constexpr int64_t kJacobianMaxBytes = int64_t(72) << 30;
 
+// The chi^2 mode of the Kelsall line kernels takes one pass that needs neither J nor I of
+// another: I and the derivatives of a ray come from the same sums. Its held derivatives
+// and tables leave room in 64 KB of LDS for the rows of kOnePassParams parameters.
+constexpr int kOnePassParams = 128;
+
+bool chi2_one_pass(const zodi_model* m) {
+  return m->integrand == ZODI_INTEGRAND_KELSALL && m->n_params <= kOnePassParams && takes_line(m);
+}
+
 // Workspace of the recompute path: block partials, then I.
 int64_t recompute_bytes(const AdjPlan& p, int np1, int64_t n_rays) {
   return (p.grid * np1 + n_rays) * (int64_t)sizeof(double);
@@ -511,15 +521,15 @@ zodi_status check_rays(const zodi_model* model_host, const zodi_model* model_dev
   return ZODI_OK;
 }
 
-AdjKernel pick_checked(const zodi_model* model_host, const AdjPlan& plan, bool jac,
+AdjKernel pick_checked(const zodi_model* model_host, const AdjPlan& plan, int pass,
                        zodi_status& st) {
   st = validate_grad_layout(model_host);
   if (st != ZODI_OK) return nullptr;
   // Registry layouts run their layout kernels; any other layout the generic one
   // (one component per pass; the components-per-pass choice does not apply).
   AdjKernel k = match_layout(model_host) == kLayoutGeneric
-                    ? generic_adjoint_kernel(model_host->integrand, plan.split, jac)
-                    : pick_adjoint(model_host, plan.chunk, plan.split, jac);
+                    ? generic_adjoint_kernel(model_host->integrand, plan.split, pass == kPassJac)
+                    : pick_adjoint(model_host, plan.chunk, plan.split, pass);
   if (k == nullptr) {
     st = fail(ZODI_ERR_ARG, "no adjoint kernel for %d components per pass and %d lanes per ray",
               plan.chunk, plan.split);
@@ -540,17 +550,19 @@ struct RayArgs {
   const uint32_t* beyond;
 };
 
-// The recompute path: in chi^2 mode the forward kernel first writes I to vals;
-// the adjoint kernel then writes one partial row per block ([plan.grid][n_params
-// + 1], every entry written) and adjoint_reduce adds them in block order.
+// The recompute path: in chi^2 mode the forward kernel first writes I to vals, unless the
+// kernel is a chi^2 pass (it writes I itself if vals is not null); the adjoint kernel then
+// writes one partial row per block ([plan.grid][n_params + 1], every entry written) and
+// adjoint_reduce adds them in block order.
 zodi_status adjoint_recompute(const zodi_model* model_host, const zodi_model* model_dev,
                               const RayArgs& r, int32_t mode, const double* weights,
                               const double* target, const double* inv_var,
-                              double inv_var_scalar, const AdjPlan& plan, AdjKernel k,
+                              double inv_var_scalar, const AdjPlan& plan, AdjKernel k, int pass,
                               double* partials, double* vals, double* grad, void* stream) {
   const int np = model_host->n_params;
   const int np1 = np + 1;
-  if (mode == ZODI_ADJ_CHI2 && r.n_rays > 0) {
+  const bool one_pass = mode == ZODI_ADJ_CHI2 && pass == kPassChi2;
+  if (mode == ZODI_ADJ_CHI2 && r.n_rays > 0 && !one_pass) {
     const zodi_status st =
         zodi_forward(model_host, model_dev, r.u, r.n_rays, r.seg_offsets, r.n_seg, r.obs,
                      r.earth, r.obs_mode, r.beyond, vals, ZODI_OUT_SUM, nullptr, stream);
@@ -562,7 +574,10 @@ zodi_status adjoint_recompute(const zodi_model* model_host, const zodi_model* mo
   a.target = target;
   a.inv_var = inv_var;
   a.inv_var_scalar = inv_var_scalar;
-  a.model_vals = vals;
+  if (one_pass)
+    a.model_vals_out = vals;
+  else
+    a.model_vals = vals;
   a.partials = partials;
   a.mode = mode;
   const size_t lds = (size_t)np1 * kAdjWaves * sizeof(double);
@@ -615,7 +630,7 @@ zodi_status table_vjp(bool eff, const zodi_model* model_host, const zodi_model* 
   zodi_model shape = *model_host;
   shape.n_params = row - 1;
   return adjoint_recompute(&shape, model_dev, r, mode, weights, target, inv_var, inv_var_scalar,
-                           plan, k, workspace, vals, grad, stream);
+                           plan, k, kPassVjp, workspace, vals, grad, stream);
 }
 
 // Device address of this GPU's copy of `scratch`, looked up once per device with
@@ -679,7 +694,7 @@ zodi_status zodi_jacobian(const zodi_model* model_host, const zodi_model* model_
   AdjPlan plan;
   st = adjoint_plan(model_host, launch, n_rays, true, plan);
   if (st != ZODI_OK) return st;
-  AdjKernel k = pick_checked(model_host, plan, true, st);
+  AdjKernel k = pick_checked(model_host, plan, kPassJac, st);
   if (k == nullptr) return st;
   if (n_rays == 0) return ZODI_OK;
   AdjArgs a = make_args(model_dev, u, n_rays, seg_offsets, n_seg, obs, earth, obs_mode, beyond,
@@ -713,13 +728,28 @@ zodi_status zodi_adjoint(const zodi_model* model_host, const zodi_model* model_d
   const int np = model_host->n_params;
   const int np1 = np + 1;
 
-  // chi^2 with room for the Jacobian: one pass writes J and I, then J^T g.
-  if (mode == ZODI_ADJ_CHI2 && jacobian_eligible(launch, np, n_rays) &&
-      workspace_bytes >= jacobian_bytes(np, n_rays)) {
+  const RayArgs r = {u, n_rays, seg_offsets, n_seg, obs, earth, obs_mode, beyond};
+  const bool jacobian = mode == ZODI_ADJ_CHI2 && jacobian_eligible(launch, np, n_rays) &&
+                        workspace_bytes >= jacobian_bytes(np, n_rays);
+  // chi^2 in one pass: lanes per ray as the Jacobian pass takes them, and the room for J
+  // holds its partials (32 rays or more a block). Measured against J and J^T g: see
+  // Chi2Ray.
+  if (jacobian && n_rays > 0 && chi2_one_pass(model_host)) {
     AdjPlan plan;
     st = adjoint_plan(model_host, launch, n_rays, true, plan);
     if (st != ZODI_OK) return st;
-    AdjKernel k = pick_checked(model_host, plan, true, st);
+    AdjKernel k = pick_checked(model_host, plan, kPassChi2, st);
+    if (k == nullptr) return st;
+    return adjoint_recompute(model_host, model_dev, r, mode, weights, target, inv_var,
+                             inv_var_scalar, plan, k, kPassChi2, workspace, model_out, grad,
+                             stream);
+  }
+  // chi^2 with room for the Jacobian: one pass writes J and I, then J^T g.
+  if (jacobian) {
+    AdjPlan plan;
+    st = adjoint_plan(model_host, launch, n_rays, true, plan);
+    if (st != ZODI_OK) return st;
+    AdjKernel k = pick_checked(model_host, plan, kPassJac, st);
     if (k == nullptr) return st;
     const int64_t chunk_rays = jacobian_chunk_rays(n_rays);
     const int64_t chunks = (n_rays + chunk_rays - 1) / chunk_rays;
@@ -753,16 +783,15 @@ zodi_status zodi_adjoint(const zodi_model* model_host, const zodi_model* model_d
   AdjPlan plan;
   st = adjoint_plan(model_host, launch, n_rays, false, plan);
   if (st != ZODI_OK) return st;
-  AdjKernel k = pick_checked(model_host, plan, false, st);
+  AdjKernel k = pick_checked(model_host, plan, kPassVjp, st);
   if (k == nullptr) return st;
   const int64_t need = recompute_bytes(plan, np1, n_rays);
   if (workspace_bytes < need)
     return fail(ZODI_ERR_ARG, "workspace of %lld bytes needed, %lld given", (long long)need,
                 (long long)workspace_bytes);
   double* vals = model_out != nullptr ? model_out : workspace + plan.grid * np1;
-  const RayArgs r = {u, n_rays, seg_offsets, n_seg, obs, earth, obs_mode, beyond};
   return adjoint_recompute(model_host, model_dev, r, mode, weights, target, inv_var,
-                           inv_var_scalar, plan, k, workspace, vals, grad, stream);
+                           inv_var_scalar, plan, k, kPassVjp, workspace, vals, grad, stream);
 }
 
 int64_t zodi_table_vjp_workspace(const zodi_model* model_host, int64_t n_rays,
@@ -825,7 +854,7 @@ zodi_status zodi_adjoint_noalloc(const zodi_model* model_host, const zodi_model*
   AdjPlan plan;
   st = adjoint_plan(model_host, launch, n_rays, false, plan);
   if (st != ZODI_OK) return st;
-  AdjKernel k = pick_checked(model_host, plan, false, st);
+  AdjKernel k = pick_checked(model_host, plan, kPassVjp, st);
   if (k == nullptr) return st;
   const int64_t need = plan.grid * np1;
   if (need > kScratchDoubles)
@@ -838,7 +867,7 @@ zodi_status zodi_adjoint_noalloc(const zodi_model* model_host, const zodi_model*
   if (st != ZODI_OK) return st;
   const RayArgs r = {u, n_rays, seg_offsets, n_seg, obs, earth, obs_mode, beyond};
   return adjoint_recompute(model_host, model_dev, r, mode, weights, target, inv_var,
-                           inv_var_scalar, plan, k, partials, model_out, grad, stream);
+                           inv_var_scalar, plan, k, kPassVjp, partials, model_out, grad, stream);
 }
 
 }  // extern "C"

@@ -18,6 +18,10 @@ constexpr int kWave = 64;
 constexpr int kAdjWaves = 4;
 constexpr int kAdjBlock = kWave * kAdjWaves;
 
+// What an adjoint kernel leaves of a ray: the wave's weighted gradient row (weights of a.mode), the
+// ray's Jacobian column, or the wave's row of the chi^2 gradient.
+enum Pass { kPassVjp, kPassJac, kPassChi2 };
+
 struct AdjArgs {
   FwdArgs f;
   const double* weights;   // VJP_SUM: [n_rays]; VJP_COMPS: [n_comps][n_rays]
@@ -620,10 +624,10 @@ inline bool block_noscat(const zodi_model* m) {
 using AdjKernel = void (*)(AdjArgs);
 AdjKernel generic_adjoint_kernel(int integrand, int split, bool jac);
 
-// The line kernels of the Kelsall registry layouts (scat: see zodi_line_adjoint.hpp), and
-// whether a block that meets the layout's registry properties may take them.
-AdjKernel line_adjoint_dirbe(int scat, bool jac);
-AdjKernel line_adjoint_kelsall4(int scat, bool jac);
+// The line kernels of the Kelsall registry layouts (scat, pass: see zodi_line_adjoint.hpp),
+// and whether a block that meets the layout's registry properties may take them.
+AdjKernel line_adjoint_dirbe(int scat, int pass);
+AdjKernel line_adjoint_kelsall4(int scat, int pass);
 AdjKernel line_adjoint_rrm(bool split_layout, bool jac);
 
 // Resident blocks per CU (waves per SIMD) that the line adjoint kernels are compiled for.

@@ -367,14 +367,30 @@ __device__ __forceinline__ double split_sum(double v, int split) {
   return v;
 }
 
-// Group g of one ray. JAC: the ray's Jacobian column; else the wave's gradient row, with
-// the weights of a.mode. sh: the ray's sums for the shared parameters (T0, delta, F, C1..C3),
-// at unit weight in JAC, else weighted.
-template <int SCAT, bool JAC, uint32_t PROPS, int... Ks, int... J>
+// The chi^2 pass: a ray's gradient is g = 2 (I - d) / sigma^2 times its derivatives, and I
+// is whole only after the last group. So the groups after the first go before it and leave
+// their derivatives at unit weight in LDS (kHoldRow doubles a component and thread), and
+// group 0, whose sums are still in registers then, forms I and g. Against the Jacobian
+// pass and J^T g (78 columns written and read), in us of both: 196 608 rays of DIRBE 250
+// -> 212, 400 000 rays of planck13 533 -> 481; the VJP pass with I known takes 209 and 479.
+constexpr int kHoldRow = 13;  // most of a later component: the feature's 5 + 6 + 2
+template <int NC, int C0>
+struct Chi2Ray {
+  // first double of component c (not of group 0) in a thread's held derivatives
+  static __device__ __forceinline__ int held(int c) { return (c - C0) * kHoldRow * kAdjBlock; }
+  double e[NC];  // the components' emission
+  double g, chi;
+};
+
+// Group g of one ray. sh: the ray's sums for the shared parameters (T0, delta, F, C1..C3),
+// weighted in kPassVjp, else at unit weight.
+template <int SCAT, int PASS, uint32_t PROPS, int NC, int C0, int... Ks, int... J>
 __device__ __forceinline__ void line_adj_group(Grp<Ks...>, std::integer_sequence<int, J...>,
                                                const LineAdjCtx& cx, const AdjArgs& a, Ray& y,
                                                int g, int first, double gscale, double* row,
-                                               int lane, double (&sh)[6], double& total) {
+                                               int lane, double (&sh)[6], double& total,
+                                               Chi2Ray<NC, C0>& cr, double* hold) {
+  constexpr bool JAC = PASS == kPassJac, CHI2 = PASS == kPassChi2;
   constexpr int C = sizeof...(Ks);
   constexpr int kinds[C] = {Ks...};
   const ModelPtr M = cx.M;
@@ -396,7 +412,7 @@ __device__ __forceinline__ void line_adj_group(Grp<Ks...>, std::integer_sequence
         const ParamPtr P = M->comp[first + J];
         cn[J] = to_scalar(P[ZODI_P_K0] * P[ZODI_P_SCALE]);
         ca[J] = SCAT == 2 ? to_scalar(P[ZODI_P_K0] * P[ZODI_P_ALBEDO]) : 0.0;
-        if (!JAC && a.mode == ZODI_ADJ_VJP_COMPS) {
+        if (PASS == kPassVjp && a.mode == ZODI_ADJ_VJP_COMPS) {
           const double gc = y.active ? a.weights[(int64_t)(first + J) * a.f.n_rays + y.r] : 0.0;
           cn[J] *= gc;
           ca[J] *= gc;
@@ -490,7 +506,37 @@ __device__ __forceinline__ void line_adj_group(Grp<Ks...>, std::integer_sequence
   const Line l = make_line(y.ux, y.uy, y.uz, y.ox, y.oy, y.oz);
   if (!y.active) h = 0.0;
   const auto sum = [&](double v) { return JAC ? split_sum(v, cx.split) : v; };
-  const double wsh = JAC || a.mode == ZODI_ADJ_VJP_COMPS ? h : h * gscale;
+  const double wsh = PASS != kPassVjp || a.mode == ZODI_ADJ_VJP_COMPS ? h : h * gscale;
+  // Component J's emission over h amp: e = (1 - a) eps B + a F Phi/R^2 (with SCAT 2 already
+  // in the sums of the derivatives)
+  const auto value = [&](ParamPtr P, double b, double f) {
+    return SCAT == 2 ? fma(P[ZODI_P_ALBEDO], f, P[ZODI_P_SCALE] * b) : P[ZODI_P_SCALE] * b;
+  };
+  if constexpr (CHI2) {
+    (
+        [&] {
+          const ParamPtr P = M->comp[first + J];
+          const double b = split_sum(s0[J], cx.split);
+          const double f = SCAT == 2 ? split_sum(s1[J], cx.split) : 0.0;
+          cr.e[first + J] = h * (P[ZODI_P_K0] * value(P, b, f));
+        }(),
+        ...);
+    if (g == 0) {
+#pragma unroll
+      for (int c = 0; c < NC; ++c) total = __dadd_rn(total, cr.e[c]);
+      cr.g = 0.0;
+      cr.chi = 0.0;
+      if (y.active) {
+        const double iv = a.inv_var != nullptr ? a.inv_var[y.r] : a.inv_var_scalar;
+        const double res = total - a.target[y.r];
+        if (cx.sub == 0) {
+          cr.chi = res * res * iv;
+          if (a.model_vals_out != nullptr) a.model_vals_out[y.r] = total;
+        }
+        cr.g = 2.0 * res * iv;
+      }
+    }
+  }
   (
       [&] {
         constexpr int KIND = kinds[J];
@@ -503,20 +549,19 @@ __device__ __forceinline__ void line_adj_group(Grp<Ks...>, std::integer_sequence
         for (int q = 0; q < A.kSlots; ++q) A.s[q] = sum(A.s[q]);
         const double b = sum(s0[J]), f = sum(s1[J]);
         const double amp = P[ZODI_P_K0];
-        const double scale = P[ZODI_P_SCALE], alb = P[ZODI_P_ALBEDO];
-        double W = h;
-        if (!JAC) {
+        const double scale = P[ZODI_P_SCALE];
+        double W = CHI2 && g == 0 ? h * cr.g : h;
+        if (PASS == kPassVjp) {
           W = a.mode == ZODI_ADJ_VJP_COMPS
                   ? (y.active ? h * a.weights[(int64_t)c * a.f.n_rays + y.r] : 0.0)
                   : h * gscale;
         }
-        // e = (1 - a) eps B + a F Phi/R^2: with SCAT 2 already in the sums
         const double We = SCAT == 2 ? W * amp : W * amp * scale;
         double m[7], dp[NP], geo[5];
         A.partials(P, m, dp);
         line_geo<FEATURE>(P, l, m, FEATURE ? earth_term(P, y.ex, y.ey) : EarthTerm{0.0, 0.0},
                           geo);
-        const double e0 = SCAT == 2 ? fma(alb, f, scale * b) : scale * b;
+        const double e0 = value(P, b, f);
         dp[0] = (KIND == ZODI_BAND ? 3.0 : 1.0) * (W * e0);
 #pragma unroll
         for (int q = 0; q < 5; ++q) geo[q] *= We;
@@ -546,6 +591,12 @@ __device__ __forceinline__ void line_adj_group(Grp<Ks...>, std::integer_sequence
           for (int q = 0; q < NP; ++q) v[5 + q] = dp[q];
           v[5 + NP] = de;
           v[6 + NP] = da;
+          if (CHI2 && g != 0) {
+            static_assert(KIND == ZODI_CLOUD || 5 + NP + 2 <= kHoldRow);
+#pragma unroll
+            for (int q = 0; q < 5 + NP + 2; ++q) hold[cr.held(c) + q * kAdjBlock] = v[q];
+            return;
+          }
           add_folded(v, row, lane, M->grad_comp[c], M->grad_spec_a[c], M->grad_spec_b[c]);
         }
       }(),
@@ -560,33 +611,80 @@ __device__ __forceinline__ void line_adj_group(Grp<Ks...>, std::integer_sequence
   }
 }
 
-template <int SCAT, bool JAC, uint32_t PROPS, class... Gs, int... G>
+// The held derivatives of a later group's components, weighted onto the wave's row.
+template <int NC, int C0, int... Ks, int... J>
+__device__ __forceinline__ void add_held(Grp<Ks...>, std::integer_sequence<int, J...>,
+                                         ModelPtr M, int first, const Chi2Ray<NC, C0>& cr, double* row, int lane,
+                                         const double* hold) {
+  constexpr int kinds[sizeof...(Ks)] = {Ks...};
+  (
+      [&] {
+        const int c = first + J;
+        double v[5 + kind_nparams<kinds[J]>() + 2];
+#pragma unroll
+        for (int q = 0; q < 5 + kind_nparams<kinds[J]>() + 2; ++q)
+          v[q] = cr.g * hold[cr.held(c) + q * kAdjBlock];
+        add_folded(v, row, lane, M->grad_comp[c], M->grad_spec_a[c], M->grad_spec_b[c]);
+      }(),
+      ...);
+}
+
+// Components of a Kelsall layout, and of its group 0.
+template <class... Gs>
+constexpr int layout_comps(Layout<ZODI_INTEGRAND_KELSALL, Gs...>) {
+  return (Gs::size + ...);
+}
+template <class G0, class... Gs>
+constexpr int layout_group0(Layout<ZODI_INTEGRAND_KELSALL, G0, Gs...>) {
+  return G0::size;
+}
+
+template <int SCAT, int PASS, uint32_t PROPS, class... Gs, int... G>
 __device__ __forceinline__ void line_adj_groups(Layout<ZODI_INTEGRAND_KELSALL, Gs...>,
                                                 std::integer_sequence<int, G...>,
                                                 const LineAdjCtx& cx, const AdjArgs& a, Ray& y,
                                                 double gscale, double* row, int lane,
-                                                double (&sh)[6], double& total) {
-  (line_adj_group<SCAT, JAC, props_shift(PROPS, group_first<Gs...>(G))>(
-       Gs{}, std::make_integer_sequence<int, Gs::size>{}, cx, a, y, G, group_first<Gs...>(G),
-       gscale, row, lane, sh, total),
-   ...);
+                                                double (&sh)[6], double& total, double& chi,
+                                                double* hold) {
+  using L = Layout<ZODI_INTEGRAND_KELSALL, Gs...>;
+  Chi2Ray<layout_comps(L{}), layout_group0(L{})> cr;
+  const auto run = [&](auto grp, auto index) {
+    constexpr int g = decltype(index)::value, first = group_first<Gs...>(g);
+    line_adj_group<SCAT, PASS, props_shift(PROPS, first)>(
+        grp, std::make_integer_sequence<int, decltype(grp)::size>{}, cx, a, y, g, first, gscale,
+        row, lane, sh, total, cr, hold);
+  };
+  if constexpr (PASS == kPassChi2) {
+    ((G != 0 ? run(Gs{}, std::integral_constant<int, G>{}) : void()), ...);
+    ((G == 0 ? run(Gs{}, std::integral_constant<int, G>{}) : void()), ...);
+    ((G != 0 ? add_held(Gs{}, std::make_integer_sequence<int, Gs::size>{}, cx.M,
+                        group_first<Gs...>(G), cr, row, lane, hold)
+             : void()),
+     ...);
+#pragma unroll
+    for (int q = 0; q < 6; ++q) sh[q] *= cr.g;
+    chi = cr.chi;
+  } else {
+    (run(Gs{}, std::integral_constant<int, G>{}), ...);
+  }
 }
 
-template <int SCAT, bool JAC, class... Gs>
+template <int SCAT, int PASS, class... Gs>
 __device__ __forceinline__ void line_adj_layout(Layout<ZODI_INTEGRAND_KELSALL, Gs...> lay,
                                                 const LineAdjCtx& cx, const AdjArgs& a, Ray& y,
                                                 double gscale, double* row, int lane,
-                                                double (&sh)[6], double& total) {
-  line_adj_groups<SCAT, JAC, RegistryProps<Layout<ZODI_INTEGRAND_KELSALL, Gs...>>::value>(
+                                                double (&sh)[6], double& total, double& chi,
+                                                double* hold) {
+  line_adj_groups<SCAT, PASS, RegistryProps<Layout<ZODI_INTEGRAND_KELSALL, Gs...>>::value>(
       lay, std::make_integer_sequence<int, sizeof...(Gs)>{}, cx, a, y, gscale, row, lane, sh,
-      total);
+      total, chi, hold);
 }
 
-// The weighted passes: one wave per tile of 64 / a.split rays, whose lanes are adjacent;
-// see adjoint_body, whose rows, weights and order of additions these are. Every thread of
+// The passes that leave a row: one wave per tile of 64 / a.split rays, whose lanes are
+// adjacent; see adjoint_body, whose rows and order of additions these are. Every thread of
 // the block must call it, after the tables are built.
 template <class RAY>
-__device__ __forceinline__ void weighted_body(const AdjArgs& a, RAY ray) {
+__device__ __forceinline__ void rows_body(const AdjArgs& a, RAY ray) {
   extern __shared__ double sRows[];  // kAdjWaves rows of n_params + 1
   const int tid = threadIdx.x;
   const int wave = tid / kWave, lane = tid % kWave;
@@ -600,6 +698,21 @@ __device__ __forceinline__ void weighted_body(const AdjArgs& a, RAY ray) {
        tile += stride) {
     Ray y = find_ray(a.f, tile * rays, lane / a.split);
     read_ray(a.f, y);
+    ray(y, row, lane);
+  }
+  __syncthreads();
+  for (int p = tid; p < np1; p += kAdjBlock) {
+    double s = sRows[p];
+#pragma unroll
+    for (int w = 1; w < kAdjWaves; ++w) s += sRows[w * np1 + p];
+    a.partials[(int64_t)blockIdx.x * np1 + p] = s;
+  }
+}
+
+// The weighted passes, with the weights of a.mode (chi^2: from the stored I).
+template <class RAY>
+__device__ __forceinline__ void weighted_body(const AdjArgs& a, RAY ray) {
+  rows_body(a, [&](Ray& y, double* row, int lane) {
     double gscale = 0.0;
     if (a.mode == ZODI_ADJ_CHI2) {
       double chi = 0.0;
@@ -616,18 +729,11 @@ __device__ __forceinline__ void weighted_body(const AdjArgs& a, RAY ray) {
       gscale = y.active ? a.weights[y.r] : 0.0;
     }
     ray(y, gscale, row, lane);
-  }
-  __syncthreads();
-  for (int p = tid; p < np1; p += kAdjBlock) {
-    double s = sRows[p];
-#pragma unroll
-    for (int w = 1; w < kAdjWaves; ++w) s += sRows[w * np1 + p];
-    a.partials[(int64_t)blockIdx.x * np1 + p] = s;
-  }
+  });
 }
 
-// The Jacobian pass (each ray's column and I_r) or the weighted pass of a layout.
-template <class LAYOUT, int SCAT, bool JAC>
+// A layout's Jacobian pass (each ray's column and I_r), weighted pass or chi^2 pass.
+template <class LAYOUT, int SCAT, int PASS>
 __device__ __forceinline__ void line_adj_body(const AdjArgs& a) {
   constexpr int NSH = layout_integrand<LAYOUT>() == ZODI_INTEGRAND_KELSALL ? 6 : 1;
   __shared__ LineAdjTables tables;
@@ -637,7 +743,8 @@ __device__ __forceinline__ void line_adj_body(const AdjArgs& a) {
   cx.split = a.split;
   cx.sub = lane & (a.split - 1);
   cx.share = a.share != 0;
-  if constexpr (JAC) {
+  double chi = 0.0;
+  if constexpr (PASS == kPassJac) {
     const int rays = kWave / a.split;
     const int64_t stride = (int64_t)gridDim.x * kAdjWaves;
     for (int64_t tile = (int64_t)blockIdx.x * kAdjWaves + wave; tile < a.f.n_tiles;
@@ -646,18 +753,35 @@ __device__ __forceinline__ void line_adj_body(const AdjArgs& a) {
       read_ray(a.f, y);
       double sh[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
       double total = 0.0;
-      line_adj_layout<SCAT, true>(LAYOUT{}, cx, a, y, 1.0, nullptr, lane, sh, total);
+      line_adj_layout<SCAT, PASS>(LAYOUT{}, cx, a, y, 1.0, nullptr, lane, sh, total, chi,
+                                  nullptr);
       if (y.active && cx.sub == 0) {
         a.model_vals_out[y.r] = total;
 #pragma unroll
         for (int q = 0; q < NSH; ++q) a.jac[M->grad_shared[q] * a.ld_jac + y.r] = sh[q];
       }
     }
+  } else if constexpr (PASS == kPassChi2) {
+    constexpr int kHeld = (layout_comps(LAYOUT{}) - layout_group0(LAYOUT{})) * kHoldRow;
+    __shared__ double held[kHeld > 0 ? kHeld * kAdjBlock : 1];
+    double* hold = held + (kHeld > 0 ? threadIdx.x : 0);
+    rows_body(a, [&](Ray& y, double* row, int ln) {
+      double v[7] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+      double sh[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+      double total = 0.0;
+      line_adj_layout<SCAT, PASS>(LAYOUT{}, cx, a, y, 0.0, row, ln, sh, total, chi, hold);
+#pragma unroll
+      for (int q = 0; q < 6; ++q) v[q] = sh[q];
+      v[6] = chi;
+      const double s = wave_fold<32>(v);
+      const int i = fold_index(ln);
+      if ((ln & 3) == 0 && i < 7) lds_add(row + (i < 6 ? M->grad_shared[i] : a.n_params), s);
+    });
   } else {
     weighted_body(a, [&](Ray& y, double gscale, double* row, int ln) {
       double sh[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
       double total = 0.0;
-      line_adj_layout<SCAT, false>(LAYOUT{}, cx, a, y, gscale, row, ln, sh, total);
+      line_adj_layout<SCAT, PASS>(LAYOUT{}, cx, a, y, gscale, row, ln, sh, total, chi, nullptr);
       double v[NSH];
 #pragma unroll
       for (int q = 0; q < NSH; ++q) v[q] = sh[q];
@@ -668,23 +792,25 @@ __device__ __forceinline__ void line_adj_body(const AdjArgs& a) {
   }
 }
 
-template <class LAYOUT, int SCAT, bool JAC>
+template <class LAYOUT, int SCAT, int PASS>
 __global__ __launch_bounds__(kAdjBlock)
 __attribute__((amdgpu_waves_per_eu(kLineAdjWaves, kLineAdjWaves))) void
 line_adjoint(AdjArgs a) {
-  line_adj_body<LAYOUT, SCAT, JAC>(a);
+  line_adj_body<LAYOUT, SCAT, PASS>(a);
+}
+
+template <class LAYOUT, int SCAT>
+AdjKernel pick_line_pass(int pass) {
+  return pass == kPassVjp   ? line_adjoint<LAYOUT, SCAT, kPassVjp>
+         : pass == kPassJac ? line_adjoint<LAYOUT, SCAT, kPassJac>
+                            : line_adjoint<LAYOUT, SCAT, kPassChi2>;
 }
 
 template <class LAYOUT>
-AdjKernel pick_line_adjoint(int scat, bool jac) {
-  switch (scat) {
-    case 0:
-      return jac ? line_adjoint<LAYOUT, 0, true> : line_adjoint<LAYOUT, 0, false>;
-    case 1:
-      return jac ? line_adjoint<LAYOUT, 1, true> : line_adjoint<LAYOUT, 1, false>;
-    default:
-      return jac ? line_adjoint<LAYOUT, 2, true> : line_adjoint<LAYOUT, 2, false>;
-  }
+AdjKernel pick_line_adjoint(int scat, int pass) {
+  return scat == 0   ? pick_line_pass<LAYOUT, 0>(pass)
+         : scat == 1 ? pick_line_pass<LAYOUT, 1>(pass)
+                     : pick_line_pass<LAYOUT, 2>(pass);
 }
 
 }  // namespace zodi

@@ -6,6 +6,6 @@
 
 namespace zodi {
 
-AdjKernel line_adjoint_dirbe(int scat, bool jac) { return pick_line_adjoint<LayoutDirbe>(scat, jac); }
+AdjKernel line_adjoint_dirbe(int scat, int pass) { return pick_line_adjoint<LayoutDirbe>(scat, pass); }
 
 }  // namespace zodi

@@ -6,6 +6,6 @@
 
 namespace zodi {
 
-AdjKernel line_adjoint_kelsall4(int scat, bool jac) { return pick_line_adjoint<LayoutKelsall4>(scat, jac); }
+AdjKernel line_adjoint_kelsall4(int scat, int pass) { return pick_line_adjoint<LayoutKelsall4>(scat, pass); }
 
 }  // namespace zodi

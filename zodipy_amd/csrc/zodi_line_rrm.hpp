@@ -628,12 +628,13 @@ __device__ __forceinline__ void rrm_adj_groups(Layout<ZODI_INTEGRAND_RRM, Gs...>
    ...);
 }
 
-template <int SCAT, bool JAC, class... Gs>
+template <int SCAT, int PASS, class... Gs>
 __device__ __forceinline__ void line_adj_layout(Layout<ZODI_INTEGRAND_RRM, Gs...> lay,
                                                 const LineAdjCtx& cx, const AdjArgs& a, Ray& y,
                                                 double gscale, double* row, int lane,
-                                                double (&sh)[6], double& total) {
-  rrm_adj_groups<JAC>(lay, std::make_integer_sequence<int, sizeof...(Gs)>{}, cx, a, y, gscale,
+                                                double (&sh)[6], double& total, double&,
+                                                double*) {
+  rrm_adj_groups<PASS == kPassJac>(lay, std::make_integer_sequence<int, sizeof...(Gs)>{}, cx, a, y, gscale,
                       row, lane, sh, total);
 }
 
@@ -641,7 +642,7 @@ template <class LAYOUT, bool JAC>
 __global__ __launch_bounds__(kAdjBlock)
 __attribute__((amdgpu_waves_per_eu(kRrmAdjWaves, kRrmAdjWaves))) void
 rrm_adjoint(AdjArgs a) {
-  line_adj_body<LAYOUT, 0, JAC>(a);
+  line_adj_body<LAYOUT, 0, JAC ? kPassJac : kPassVjp>(a);
 }
 
 }  // namespace zodi
