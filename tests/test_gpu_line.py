@@ -21,6 +21,7 @@ from oracle.zodi_oracle import OracleModel
 from zodipy_amd import Model, healpix
 from zodipy_amd import units as u
 from zodipy_amd._lib import Launch
+from zodipy_amd.fitting import LineOfSightProblem
 from zodipy_amd.runtime import OUT_COMPS
 
 pytestmark = pytest.mark.gpu
@@ -152,3 +153,40 @@ def test_default_split_gives_the_bits_of_one_lane(gpu, name, x, nodes, rays):
         got = model.device_model.forward(v, obs, obs, **mode)
         one = model.device_model.forward(v, obs, obs, launch=Launch(256, 1, 0, 1), **mode)
         assert torch.equal(got, one)
+
+
+@pytest.mark.parametrize("name,x,rays,lanes", [
+    ("dirbe", 25 * u.micron, 393_217, 0), ("dirbe", 25 * u.micron, 200_000, 4),
+    ("planck18", 857 * u.GHz, 420_001, 0), ("rrm-experimental", 25 * u.micron, 800_001, 0),
+    ("dirbe", 1.25 * u.micron, 2_001, 0), ("dirbe", 1.25 * u.micron, 1, 0)])
+def test_block_rows_beyond_the_resident_ones(gpu, name, x, rays, lanes):
+    """The passes that take more blocks than stay resident (three rounds of tiles and more;
+    4 lanes a ray reach it with the smallest workspace) against the resident blocks, and
+    the chi^2 pass against the recompute path, which adds the same terms in another order:
+    n additions of relative error below 2^-53 each on sums of like sign."""
+    model = Model(x, name=name)
+    rng = np.random.default_rng(rays)
+    v = rng.normal(size=(3, rays))
+    v /= np.linalg.norm(v, axis=0)
+    obs = np.array([0.9, 0.4, 0.02])
+    prob = LineOfSightProblem(model, v, obs, obs)
+    theta = prob.space.theta0
+    w = torch.as_tensor(rng.uniform(0.5, 1.5, rays), device="cuda")
+    data = prob.forward(theta) * torch.as_tensor(rng.uniform(0.9, 0.99, rays), device="cuda")
+    per_cu = 4 if name == "rrm-experimental" else 2
+    got = {}
+    for key, blocks in (("more", 0), ("resident", per_cu)):
+        prob.launch = Launch(0, lanes, blocks, 0)
+        got[key] = [prob.vjp(theta, w), torch.cat([g.reshape(-1) for g in
+                                                   prob.chi2_and_grad(theta, data)]),
+                    torch.cat([g.reshape(-1) for g in prob.chi2_spectral_grad(theta, data)])]
+    prob.launch = None
+    prob.store_jacobian = False
+    got["recompute"] = [None, torch.cat([g.reshape(-1) for g in
+                                         prob.chi2_and_grad(theta, data)]), None]
+    for key in ("more", "recompute"):
+        for a, b in zip(got[key], got["resident"]):
+            if a is not None:
+                # entries that cancel are judged against the gradient's largest
+                tol = 1e-10 * b.abs() + 1e-13 * b.abs().max()
+                assert torch.all((a - b).abs() <= tol)

@@ -413,6 +413,37 @@ zodi_status adjoint_plan(const zodi_model* m, const zodi_launch* launch, int64_t
   return ZODI_OK;
 }
 
+// Blocks of a pass when the launch leaves them open: at most `most`, `per_cu` per CU. The
+// plan's blocks stay resident and take their tiles in turn; from three rounds of tiles on,
+// more blocks, which the CUs start as they come free, even out rays of different cost.
+int64_t pass_blocks(const zodi_launch* launch, const AdjPlan& p, int per_cu, int64_t most) {
+  const int64_t resident = (int64_t)p.per_cu * cu_count();
+  if ((launch != nullptr && launch->blocks_per_cu > 0) || p.n_tiles < 3 * resident * kAdjWaves)
+    return p.grid;
+  const int64_t blocks =
+      std::min((p.n_tiles + kAdjWaves - 1) / kAdjWaves, (int64_t)per_cu * cu_count());
+  return std::max(p.grid, std::min(blocks, most));
+}
+
+// Most blocks per CU for pass_blocks. Line kernels, VJP in us at the plan's blocks and at
+// these: DIRBE 196 608 rays 209 and 231, 300 000 348 and 360, 600 000 740 and 689, 4.46 M
+// 5021 and 4556; RRM 300 000 684 and 688, 600 000 1319 and 1252, 4.46 M 9220 and 7880.
+// Table kernels, forward and gradient: planck13 200 000 rays 357 and 385, 1 M 1340 and
+// 1263, 4 M 5098 and 4790; RRM 1 M 3605 and 3415. The other kernels keep the plan's.
+constexpr int kTableBlocksPerCu = 12;
+
+int line_blocks_per_cu(const zodi_model* m) {
+  return !takes_line(m) ? 0 : (m->integrand == ZODI_INTEGRAND_RRM ? 48 : 24);
+}
+
+// Blocks of a VJP pass, the same with and without a workspace: rows for the plan's blocks
+// and the room of I (recompute_bytes), which a VJP does not keep, within the static array.
+int64_t vjp_blocks(const zodi_model* m, const zodi_launch* launch, const AdjPlan& p,
+                   int64_t n_rays, int np1) {
+  return pass_blocks(launch, p, line_blocks_per_cu(m),
+                     std::min(kScratchDoubles, p.grid * np1 + n_rays) / np1);
+}
+
 // Rows of the Planck-table gradient: one entry per table temperature, then chi^2;
 // with the effective spectral parameters (eff), the parameter vector first.
 constexpr int kTableRow = ZODI_N_TEMPS + 1;
@@ -626,7 +657,12 @@ zodi_status table_vjp(bool eff, const zodi_model* model_host, const zodi_model* 
   if (workspace_bytes < need)
     return fail(ZODI_ERR_ARG, "workspace of %lld bytes needed, %lld given", (long long)need,
                 (long long)workspace_bytes);
-  double* vals = model_out != nullptr ? model_out : workspace + plan.grid * row;
+  // I, where it goes to the workspace, takes the last of it; block rows the rest
+  const int64_t room = workspace_bytes / (int64_t)sizeof(double);
+  const bool own_vals = mode == ZODI_ADJ_CHI2 && model_out == nullptr;
+  double* vals = own_vals ? workspace + (room - r.n_rays) : model_out;
+  plan.grid = pass_blocks(launch, plan, kTableBlocksPerCu,
+                          (room - (own_vals ? r.n_rays : 0)) / row);
   zodi_model shape = *model_host;
   shape.n_params = row - 1;
   return adjoint_recompute(&shape, model_dev, r, mode, weights, target, inv_var, inv_var_scalar,
@@ -702,7 +738,8 @@ zodi_status zodi_jacobian(const zodi_model* model_host, const zodi_model* model_
   a.jac = jac;
   a.ld_jac = ld_jac;
   a.model_vals_out = model_out;
-  hipLaunchKernelGGL(k, dim3((unsigned)plan.grid), dim3(kAdjBlock), 0, (hipStream_t)stream, a);
+  const int64_t grid = pass_blocks(launch, plan, line_blocks_per_cu(model_host), INT32_MAX);
+  hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(kAdjBlock), 0, (hipStream_t)stream, a);
   return check_hip(hipGetLastError(), "jacobian launch");
 }
 
@@ -740,6 +777,7 @@ zodi_status zodi_adjoint(const zodi_model* model_host, const zodi_model* model_d
     if (st != ZODI_OK) return st;
     AdjKernel k = pick_checked(model_host, plan, kPassChi2, st);
     if (k == nullptr) return st;
+    plan.grid = pass_blocks(launch, plan, line_blocks_per_cu(model_host), INT32_MAX);
     return adjoint_recompute(model_host, model_dev, r, mode, weights, target, inv_var,
                              inv_var_scalar, plan, k, kPassChi2, workspace, model_out, grad,
                              stream);
@@ -761,8 +799,8 @@ zodi_status zodi_adjoint(const zodi_model* model_host, const zodi_model* model_d
       a.jac = workspace;
       a.ld_jac = n_rays;
       a.model_vals_out = vals;
-      hipLaunchKernelGGL(k, dim3((unsigned)plan.grid), dim3(kAdjBlock), 0, (hipStream_t)stream,
-                         a);
+      const int64_t grid = pass_blocks(launch, plan, line_blocks_per_cu(model_host), INT32_MAX);
+      hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(kAdjBlock), 0, (hipStream_t)stream, a);
       st = check_hip(hipGetLastError(), "jacobian launch");
       if (st != ZODI_OK) return st;
       const dim3 g2((unsigned)chunks, (unsigned)((np + kJacParams - 1) / kJacParams));
@@ -790,6 +828,7 @@ zodi_status zodi_adjoint(const zodi_model* model_host, const zodi_model* model_d
     return fail(ZODI_ERR_ARG, "workspace of %lld bytes needed, %lld given", (long long)need,
                 (long long)workspace_bytes);
   double* vals = model_out != nullptr ? model_out : workspace + plan.grid * np1;
+  if (mode != ZODI_ADJ_CHI2) plan.grid = vjp_blocks(model_host, launch, plan, n_rays, np1);
   return adjoint_recompute(model_host, model_dev, r, mode, weights, target, inv_var,
                            inv_var_scalar, plan, k, kPassVjp, workspace, vals, grad, stream);
 }
@@ -862,6 +901,7 @@ zodi_status zodi_adjoint_noalloc(const zodi_model* model_host, const zodi_model*
                 "the allocation-free adjoint holds %lld block partials, this launch needs %lld "
                 "(%lld blocks x %d entries): use fewer blocks_per_cu or zodi_adjoint",
                 (long long)kScratchDoubles, (long long)need, (long long)plan.grid, np1);
+  if (mode != ZODI_ADJ_CHI2) plan.grid = vjp_blocks(model_host, launch, plan, n_rays, np1);
   double* partials = nullptr;
   st = scratch_address(&partials);
   if (st != ZODI_OK) return st;

@@ -356,6 +356,7 @@ class LineOfSightProblem:
             err = self.lib.zodi_last_error().decode(errors="replace")
             msg = f"{name}_workspace rejected the model or launch: {err}"
             raise RuntimeError(msg)
+        need += 8 * self.n_rays  # room for more block rows (pass_blocks in zodi_adjoint.hip)
         ws = torch.empty(max((need + 7) // 8, 1), dtype=torch.float64, device=self.device)
         n_row = N_TEMPS + 1 + (self.n_params if eff else 0)
         grad = torch.empty(n_row, dtype=torch.float64, device=self.device)
