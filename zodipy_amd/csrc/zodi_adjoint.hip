@@ -52,7 +52,7 @@ adjoint_layout(AdjArgs a) {
   adjoint_body<SPLIT, JAC, kLdsSlots>(
       a, [&](const Ctx& cx, const Ray& y, double gscale, double* row, int lane, int sub,
              double* lane_acc) {
-        run_adjoint<SPLIT, CHUNK, NREG, JAC, 0u, false>(LAYOUT{}, cx, a, y, gscale, row, lane,
+        run_adjoint<SPLIT, CHUNK, NREG, JAC>(LAYOUT{}, cx, a, y, gscale, row, lane,
                                                         sub, lane_acc);
       });
 }

@@ -229,14 +229,7 @@ constexpr int layout_lds_slots(Layout<INTEGRAND, Gs...>) {
 // as a column of the Jacobian, dI_r/dtheta_p -> jac[p][r], instead of reducing
 // them over the wave; `total` receives I_r, each component's node sum finished
 // as the forward kernel finishes it and added in component order.
-//
-// PROPS: 4 bits per component of the group (component J at bits 4J; see
-// density_k): the frame mode and kFast, the registry forms of the band's
-// partials (p = 4, the pre-scaled plane normal, the R^2 cut-off). NOSCAT: the
-// block has no scattering component and no solar irradiance (the host checks),
-// so every scattering sum is an exact zero and is left out.
-template <int INTEGRAND, int SPLIT, bool JAC, int NREG, int S, uint32_t PROPS, bool NOSCAT,
-          int... Ks, int... J>
+template <int INTEGRAND, int SPLIT, bool JAC, int NREG, int S, int... Ks, int... J>
 __device__ __forceinline__ void adjoint_group(Grp<Ks...>, std::integer_sequence<int, J...>,
                                               const Ctx& cx, const AdjArgs& a, const Ray& y,
                                               int g, int first, double gscale, double* row,
@@ -283,7 +276,7 @@ __device__ __forceinline__ void adjoint_group(Grp<Ks...>, std::integer_sequence<
   // Phi enters d/d(albedo) when F != 0, and d/dF, d/dC_i when an albedo is non-zero.
   // With every albedo 0 the C_i partials are multiplied by 0, and with C2 = C3 = 0
   // Phi = N (C1 + 1) does not depend on the scattering angle: skip the angle.
-  const bool need_phase = !NOSCAT && INTEGRAND == ZODI_INTEGRAND_KELSALL &&
+  const bool need_phase = INTEGRAND == ZODI_INTEGRAND_KELSALL &&
                           (solar != 0.0 || (M->flags & 1) != 0);
   const bool need_angle = need_phase && ((M->flags & 1) != 0 || M->shared[ZODI_S_C2] != 0.0 ||
                                          M->shared[ZODI_S_C3] != 0.0);
@@ -328,31 +321,25 @@ __device__ __forceinline__ void adjoint_group(Grp<Ks...>, std::integer_sequence<
     }
     const double inv_R2 = nd.inv_R * nd.inv_R;
     double sw = 0.0;  // Kelsall: sum over the chunk of w n (1 - a) eps, for T_0 and delta
-    CutShare cs = {0.0, 0.0};  // a band's cut-off, for the bands that share it (in order)
     (
         [&] {
           constexpr int KIND = kinds[J];
           constexpr int NP = kind_nparams<KIND>();
           constexpr int G = geo_moments<is_feature(KIND)>();
-          constexpr int CUT = cut_mode<PROPS, J, Ks...>();
-          static_assert(CUT != kCutReuse || first_band<Ks...>() >= S,
-                        "a band that reuses a cut-off needs its publisher in the same pass");
           const ParamPtr P = Mk->comp[first + J];
           const uint32_t flags = Mk->comp_flags[first + J];
-          constexpr uint32_t PC = (PROPS >> (4 * J)) & 15u;
           const CompFrame f =
-              comp_frame<PC & 3>(P, flags, nd.X0, nd.X1, nd.X2, nd.R, nd.inv_R, nd.R2);
-          const DensGrad<NP> dg =
-              density_grad<KIND, (PC & kFast) != 0, CUT>(P, flags, f, fdir[J - S], logR, cs);
+              comp_frame(P, flags, nd.X0, nd.X1, nd.X2, nd.R, nd.inv_R, nd.R2);
+          const DensGrad<NP> dg = density_grad<KIND>(P, flags, f, fdir[J - S], logR);
           auto& A = std::get<J - S>(acc);
           const double wn = wk * W[J - S];
           if constexpr (INTEGRAND == ZODI_INTEGRAND_KELSALL) {
             // f = [(1 - a) eps B + a F Phi / R^2] n   (zodipy/brightness.py:21-56)
             const double alb = P[ZODI_P_ALBEDO], eps = P[ZODI_P_EMISSIVITY];
             const double oma = P[ZODI_P_ONE_MINUS_ALBEDO];
-            const double scat_unit = NOSCAT ? 0.0 : (solar * inv_R2) * pg.phi;  // F Phi / R^2
+            const double scat_unit = (solar * inv_R2) * pg.phi;  // F Phi / R^2
             double e = oma * (eps * nd.B);
-            if (!NOSCAT && (flags & ZODI_CF_SCATTER)) e += alb * scat_unit;
+            if (flags & ZODI_CF_SCATTER) e += alb * scat_unit;
             const double we = wn * e;
             geo_accumulate<is_feature(KIND)>(A, we, f, dg.dR, dg.dZ, dg.dth);
 #pragma unroll
@@ -360,7 +347,7 @@ __device__ __forceinline__ void adjoint_group(Grp<Ks...>, std::integer_sequence<
             const double wnn = wn * dg.n;
             if constexpr (JAC) {
               A.add(G + NP, (wk * nd.B) * dg.n);
-              if constexpr (!NOSCAT) A.add(G + NP + 1, (wk * scat_unit) * dg.n);
+              A.add(G + NP + 1, (wk * scat_unit) * dg.n);
             } else {
               A.add(G + NP, wnn * (oma * nd.B));                  // emissivity
               A.add(G + NP + 1, wnn * (scat_unit - eps * nd.B));  // albedo
@@ -368,7 +355,7 @@ __device__ __forceinline__ void adjoint_group(Grp<Ks...>, std::integer_sequence<
             // (1 - a) eps, packed with the same rounding as oma * eps
             sw += wnn * P[ZODI_P_SCALE];
             // F, C1..C3 enter through a Phi / R^2, which is 0 when a == 0
-            if (!NOSCAT && (flags & ZODI_CF_SCATTER)) {
+            if (flags & ZODI_CF_SCATTER) {
               const double was = wnn * alb * inv_R2;
               sh[2] += was * pg.phi;
               const double wasf = was * solar;
@@ -480,8 +467,7 @@ constexpr std::integer_sequence<int, (S + I)...> shift_seq(std::integer_sequence
 }
 
 // Group g in chunks of at most CHUNK components, from component S of the group.
-template <int INTEGRAND, int SPLIT, int CHUNK, int NREG, bool JAC, int S, uint32_t PROPS,
-          bool NOSCAT, int... Ks>
+template <int INTEGRAND, int SPLIT, int CHUNK, int NREG, bool JAC, int S, int... Ks>
 __device__ __forceinline__ void adjoint_chunks(Grp<Ks...> grp, const Ctx& cx, const AdjArgs& a,
                                                const Ray& y, int g, int first, double gscale,
                                                double* row, int lane, int sub, double (&sh)[6],
@@ -489,24 +475,22 @@ __device__ __forceinline__ void adjoint_chunks(Grp<Ks...> grp, const Ctx& cx, co
   constexpr int C = sizeof...(Ks);
   if constexpr (S < C) {
     constexpr int N = (C - S) < CHUNK ? (C - S) : CHUNK;
-    adjoint_group<INTEGRAND, SPLIT, JAC, NREG, S, PROPS, NOSCAT>(
+    adjoint_group<INTEGRAND, SPLIT, JAC, NREG, S>(
         grp, shift_seq<S>(std::make_integer_sequence<int, N>{}), cx, a, y, g, first, gscale, row,
         lane, sub, sh, total, lane_acc);
-    adjoint_chunks<INTEGRAND, SPLIT, CHUNK, NREG, JAC, S + N, PROPS, NOSCAT>(
+    adjoint_chunks<INTEGRAND, SPLIT, CHUNK, NREG, JAC, S + N>(
         grp, cx, a, y, g, first, gscale, row, lane, sub, sh, total, lane_acc);
   }
 }
 
 // Every group of the layout, with its first component known at compile time.
-template <int SPLIT, int CHUNK, int NREG, bool JAC, uint32_t PROPS, bool NOSCAT, int INTEGRAND,
-          class... Gs, int... G>
+template <int SPLIT, int CHUNK, int NREG, bool JAC, int INTEGRAND, class... Gs, int... G>
 __device__ __forceinline__ void adjoint_groups(Layout<INTEGRAND, Gs...>,
                                                std::integer_sequence<int, G...>, const Ctx& cx,
                                                const AdjArgs& a, const Ray& y, double gscale,
                                                double* row, int lane, int sub, double (&sh)[6],
                                                double& total, double* lane_acc) {
-  (adjoint_chunks<INTEGRAND, SPLIT, CHUNK, NREG, JAC, 0,
-                  props_shift(PROPS, group_first<Gs...>(G)), NOSCAT>(
+  (adjoint_chunks<INTEGRAND, SPLIT, CHUNK, NREG, JAC, 0>(
        Gs{}, cx, a, y, G, group_first<Gs...>(G), gscale, row, lane, sub, sh, total, lane_acc),
    ...);
 }
@@ -537,14 +521,13 @@ __device__ __forceinline__ void adjoint_ray_tail(const Ctx& cx, const AdjArgs& a
 }
 
 // Every group of the layout for one ray, then adjoint_ray_tail.
-template <int SPLIT, int CHUNK, int NREG, bool JAC, uint32_t PROPS, bool NOSCAT, int INTEGRAND,
-          class... Gs>
+template <int SPLIT, int CHUNK, int NREG, bool JAC, int INTEGRAND, class... Gs>
 __device__ __forceinline__ void run_adjoint(Layout<INTEGRAND, Gs...> lay, const Ctx& cx,
                                             const AdjArgs& a, const Ray& y, double gscale,
                                             double* row, int lane, int sub, double* lane_acc) {
   double sh[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
   double total = 0.0;
-  adjoint_groups<SPLIT, CHUNK, NREG, JAC, PROPS, NOSCAT>(
+  adjoint_groups<SPLIT, CHUNK, NREG, JAC>(
       lay, std::make_integer_sequence<int, sizeof...(Gs)>{}, cx, a, y, gscale, row, lane, sub, sh,
       total, lane_acc);
   adjoint_ray_tail<INTEGRAND, JAC>(cx, a, y, sh, total, row, lane);

@@ -23,10 +23,8 @@ __device__ __forceinline__ void generic_component(const Ctx& cx, const AdjArgs& 
                                                   int g, int c, double gscale, double* row,
                                                   int lane, int sub, double (&sh)[6],
                                                   double& total) {
-  adjoint_group<INTEGRAND, SPLIT, JAC, 1, 0, 0u, false>(Grp<KIND>{},
-                                                        std::integer_sequence<int, 0>{}, cx, a, y,
-                                                        g, c, gscale, row, lane, sub, sh, total,
-                                                        nullptr);
+  adjoint_group<INTEGRAND, SPLIT, JAC, 1, 0>(Grp<KIND>{}, std::integer_sequence<int, 0>{}, cx, a,
+                                             y, g, c, gscale, row, lane, sub, sh, total, nullptr);
 }
 
 // Every component of every group for one ray, in model order, then the

@@ -299,39 +299,29 @@ inline LayoutId match_layout(const zodi_model* m) {
 }
 
 // ---------------------------------------------------------- per-ray forward evaluation
-// Static properties of a layout kernel's component, 4 bits each: the frame mode
-// (FrameMode, bits 0-1), kFast (bit 2): a Kelsall kind evaluated with its
-// registry-only shortcuts (the band's p = 4, the cloud's floored g; see their
-// density functions), and kShareCut (bit 3, a band of the forward kernels): its
-// radial cut-off 1 - exp(-(R/delta_r)^20) is that of the first band of its group
-// (both centred and fast, the same 1/delta_r^2 bit for bit, so the same R^2 and the
-// same x), which the band reuses instead of forming it again. The DIRBE bands 1
-// and 3 share delta_r = 1.5.
+// What the line kernels take for granted of a registry layout's component, 4 bits each
+// (the host checks it: props_match): the frame (bits 0-1), kFast (bit 2): a band with
+// p = 4, a cloud with gamma >= 1/2, and kShareCut (bit 3): a band whose radial cut-off
+// 1 - exp(-(R/delta_r)^20) is that of the first band of its group (both centred and fast,
+// the same 1/delta_r^2 bit for bit, so the same x), which it reuses instead of forming it
+// again. The DIRBE bands 1 and 3 share delta_r = 1.5.
+enum FrameMode { kFrameCentred = 1, kFrameOffset = 2 };
 constexpr uint32_t kFast = 4u;
 constexpr uint32_t kShareCut = 8u;
 
-// The property word without the kShareCut bits (the adjoint kernels form every
-// band's cut-off and its partials themselves).
+// The property word without the kShareCut bits, for blocks whose delta_r differ.
 constexpr uint32_t props_without_share(uint32_t props) { return props & 0x77777777u; }
 
-template <int PROPS>
-constexpr bool fast_of() {
-  return (PROPS & kFast) != 0;
-}
-
-// Density of a component whose kind and properties are known at compile time.
-// CUT (bands): see band_density; `cut` carries the shared cut-off within a node.
-template <int KIND, int PROPS, int CUT = kCutOwn>
+// Density of a component whose kind is known at compile time.
+template <int KIND>
 __device__ __forceinline__ double density_k(ParamPtr P, uint32_t flags, const Node& nd,
-                                            const FeatureDir& fd, double& cut) {
+                                            const FeatureDir& fd) {
   if constexpr (KIND == ZODI_INTERSTELLAR) {
     return P[6];
   } else {
-    constexpr bool FAST = fast_of<PROPS>();
-    const CompFrame f =
-        comp_frame<PROPS & 3>(P, flags, nd.X0, nd.X1, nd.X2, nd.R, nd.inv_R, nd.R2);
-    if constexpr (KIND == ZODI_CLOUD) return cloud_density<FAST>(P, f);
-    if constexpr (KIND == ZODI_BAND) return band_density<FAST, CUT>(P, flags, f, cut);
+    const CompFrame f = comp_frame(P, flags, nd.X0, nd.X1, nd.X2, nd.R, nd.inv_R, nd.R2);
+    if constexpr (KIND == ZODI_CLOUD) return cloud_density(P, f);
+    if constexpr (KIND == ZODI_BAND) return band_density(P, flags, f);
     if constexpr (KIND == ZODI_RING) return ring_density(P, f);
     if constexpr (KIND == ZODI_FEATURE) return feature_density(P, f, fd);
     if constexpr (KIND == ZODI_FAN) return fan_density(P, f);
@@ -371,8 +361,8 @@ constexpr int cut_mode() {
   return shared && J == first_band<Ks...>() ? kCutPublish : kCutOwn;
 }
 
-// PROPS: 4 bits per component of the group (see density_k), component J at bits 4J.
-template <int INTEGRAND, int L, uint32_t PROPS, bool NOSCAT, int... Ks, int... J>
+// One group of any layout for one ray.
+template <int INTEGRAND, int L, int... Ks, int... J>
 __device__ __forceinline__ void group_pass(Grp<Ks...>, std::integer_sequence<int, J...>,
                                            const Ctx& cx, const FwdArgs& a, const Ray& y, int g,
                                            int first, double& total) {
@@ -392,7 +382,7 @@ __device__ __forceinline__ void group_pass(Grp<Ks...>, std::integer_sequence<int
                                    : FeatureDir{1.0, 0.0}),
    ...);
   bool scatter = false;
-  if constexpr (INTEGRAND == ZODI_INTEGRAND_KELSALL && !NOSCAT) {
+  if constexpr (INTEGRAND == ZODI_INTEGRAND_KELSALL) {
     ((scatter = scatter || (M->comp_flags[first + J] & ZODI_CF_SCATTER)), ...);
   }
 
@@ -415,12 +405,11 @@ __device__ __forceinline__ void group_pass(Grp<Ks...>, std::integer_sequence<int
         }
       }
       const double wB = wk * nd.B;
-      double cut = 0.0;  // a band's cut-off, for the bands that share it (in order)
       ((acc[J] = node_add(
-            acc[J], node_term<INTEGRAND, NOSCAT>(
+            acc[J], node_term<INTEGRAND>(
                         Mk->comp[first + J], Mk->comp_flags[first + J], nd, wk, wB,
-                        density_k<kinds[J], (PROPS >> (4 * J)) & 15, cut_mode<PROPS, J, Ks...>()>(
-                            Mk->comp[first + J], Mk->comp_flags[first + J], nd, fdir[J], cut),
+                        density_k<kinds[J]>(Mk->comp[first + J],
+                                            Mk->comp_flags[first + J], nd, fdir[J]),
                         Mk->shared[ZODI_S_SOLAR]))),
        ...);
     }
@@ -441,12 +430,10 @@ __device__ __forceinline__ void group_pass(Grp<Ks...>, std::integer_sequence<int
         }
       }
       const double wB = wk * nd.B;
-      double cut = 0.0;
       NodeTerm t[C];
-      ((t[J] = node_term<INTEGRAND, NOSCAT>(
+      ((t[J] = node_term<INTEGRAND>(
             Mk->comp[first + J], Mk->comp_flags[first + J], nd, wk, wB,
-            density_k<kinds[J], (PROPS >> (4 * J)) & 15, cut_mode<PROPS, J, Ks...>()>(
-                Mk->comp[first + J], Mk->comp_flags[first + J], nd, fdir[J], cut),
+            density_k<kinds[J]>(Mk->comp[first + J], Mk->comp_flags[first + J], nd, fdir[J]),
             Mk->shared[ZODI_S_SOLAR])),
        ...);
       add_in_node_order<L>(acc, t, cx.K - k0);
@@ -455,9 +442,8 @@ __device__ __forceinline__ void group_pass(Grp<Ks...>, std::integer_sequence<int
   const bool write = y.active && cx.sub == 0;
   (
       [&] {
-        const double e = finish<INTEGRAND, NOSCAT>(M->comp[first + J],
-                                                   M->comp_flags[first + J], acc[J], h,
-                                                   cx.calibration);
+        const double e = finish<INTEGRAND>(M->comp[first + J], M->comp_flags[first + J], acc[J],
+                                           h, cx.calibration);
         if (a.out_mode == ZODI_OUT_COMPS) {
           if (write) a.out[(int64_t)(first + J) * a.n_rays + y.r] = e;
         } else {
@@ -492,28 +478,24 @@ constexpr int layout_integrand() {
   return LayoutIntegrand<LAYOUT>::value;
 }
 
-// PROPS: 4 bits per component of the layout (see density_k), component c at bits 4c.
-template <int L, uint32_t PROPS, bool NOSCAT, int INTEGRAND, class... Gs, int... G>
+template <int L, int INTEGRAND, class... Gs, int... G>
 __device__ __forceinline__ void run_layout_groups(Layout<INTEGRAND, Gs...>,
                                                   std::integer_sequence<int, G...>, const Ctx& cx,
                                                   const FwdArgs& a, const Ray& y, double& total) {
-  (group_pass<INTEGRAND, L, props_shift(PROPS, group_first<Gs...>(G)), NOSCAT>(
-       Gs{}, std::make_integer_sequence<int, Gs::size>{}, cx, a, y, G, group_first<Gs...>(G),
-       total),
+  (group_pass<INTEGRAND, L>(Gs{}, std::make_integer_sequence<int, Gs::size>{}, cx, a, y, G,
+                            group_first<Gs...>(G), total),
    ...);
 }
 
-template <int L, uint32_t PROPS, bool NOSCAT, int INTEGRAND, class... Gs>
+template <int L, int INTEGRAND, class... Gs>
 __device__ __forceinline__ void run_layout(Layout<INTEGRAND, Gs...> lay, const Ctx& cx,
                                            const FwdArgs& a, const Ray& y, double& total) {
-  run_layout_groups<L, PROPS, NOSCAT>(lay, std::make_integer_sequence<int, sizeof...(Gs)>{}, cx,
-                                      a, y, total);
+  run_layout_groups<L>(lay, std::make_integer_sequence<int, sizeof...(Gs)>{}, cx, a, y, total);
 }
 
-// Component properties of a layout kernel's registry variant: every component is
-// centred on the Sun except the Kelsall cloud (the first component of the DIRBE
-// and Kelsall4 layouts), and the Kelsall components take their fast forms. At most
-// 8 components (4 bits each).
+// A layout's properties in the registry: every component is centred on the Sun except
+// the Kelsall cloud (the first component of the DIRBE and Kelsall4 layouts), and the
+// Kelsall components are fast. At most 8 components (4 bits each).
 template <class LAYOUT>
 struct RegistryProps;
 template <int INTEGRAND, class... Gs>
@@ -535,12 +517,10 @@ struct RegistryProps<LayoutKelsall4> {  // cloud offset, 3 centred, all fast; ba
   static constexpr uint32_t value = (0x555u << 4 | kFrameOffset | 0x4444u) | kShareCut << 12;
 };
 
-// Whether a model block meets the preconditions of a layout kernel with these
-// properties: every component fixed as centred carries ZODI_CF_CENTERED (the
-// offset path is exact for any component); a fast band has p = 4
-// (ZODI_CF_P_IS_4) and a fast cloud gamma >= 1/2; a band with kShareCut and the
-// first band of its group are both centred and fast and hold the same
-// 1/delta_r^2.
+// Whether a model block has these properties: every component given as centred carries
+// ZODI_CF_CENTERED; a fast band has p = 4 (ZODI_CF_P_IS_4) and a fast cloud gamma >= 1/2; a
+// band with kShareCut and the first band of its group are both centred and fast and hold
+// the same 1/delta_r^2.
 inline bool props_match(const zodi_model* m, uint32_t props) {
   for (int c = 0; c < m->n_comps && c < 8; ++c) {
     const uint32_t pc = (props >> (4 * c)) & 15u;

@@ -149,7 +149,7 @@ forward_layout(FwdArgs a) {
   for (int64_t tile = blockIdx.x; tile < a.n_tiles; tile += gridDim.x) {
     const Ray y = load_ray<RAYS>(a, tile, local);
     double total = 0.0;
-    run_layout<L, 0u, false>(LAYOUT{}, cx, a, y, total);
+    run_layout<L>(LAYOUT{}, cx, a, y, total);
     if (a.out_mode == ZODI_OUT_SUM && y.active && cx.sub == 0) a.out[y.r] = total;
   }
 }

@@ -400,6 +400,10 @@ __device__ __forceinline__ double line_cloud(ParamPtr P, const LineComp<ZODI_CLO
   return pow_table(cx.tab->radial, cx.pr, r2) * exp_neg_node(cx.ec, P[8] * gg);
 }
 
+// What a band of the line kernels does with its cut-off term: forms it for itself, forms
+// it for the bands of its group that share it too, or takes the published one.
+enum BandCut { kCutOwn = 0, kCutPublish = 1, kCutReuse = 2 };
+
 // exp(-zeta_d^6) is 0 from 746 on: those nodes add nothing and are left out for the waves
 // whose lanes all lie there (a map's rings at higher latitudes). NaN takes the branch.
 template <int CUT>

@@ -153,6 +153,12 @@ struct LineGrad<ZODI_CLOUD> {
   }
 };
 
+// A band's radial cut-off argument x = (R/delta_r)^20 and exp(-x) (0 where
+// 1 - exp(-x) rounds to 1), shared within a node by bands with the same cut-off.
+struct CutShare {
+  double x, ex;
+};
+
 template <>
 struct LineGrad<ZODI_BAND> {
   static constexpr int kSlots = 8;

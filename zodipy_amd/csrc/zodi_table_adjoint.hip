@@ -447,7 +447,6 @@ __device__ __forceinline__ void table_group(Grp<Ks...>, std::integer_sequence<in
   constexpr int kinds[C] = {Ks...};
   constexpr bool kKelsall = INTEGRAND == ZODI_INTEGRAND_KELSALL;
   constexpr bool kScat = EFF && kKelsall;
-  constexpr uint32_t PROPS = 0u;
   const ModelPtr M = cx.M;
   const int n_last = M->n_temps - 1;
   double* trow = EFF ? row + M->n_params : row;
@@ -498,11 +497,10 @@ __device__ __forceinline__ void table_group(Grp<Ks...>, std::integer_sequence<in
     const double uc = fmin(fmax(u, 0.0), (double)(ZODI_N_TEMPS - 1));
     const int jt = (int)uc;
     const double f = __builtin_amdgcn_fract(uc);
-    double cut = 0.0;
     if constexpr (!EFF) {
       double Sn = 0.0;
-      ((Sn += cw[J] * density_k<kinds[J], (PROPS >> (4 * J)) & 15, cut_mode<PROPS, J, Ks...>()>(
-                Mk->comp[first + J], Mk->comp_flags[first + J], nd, fdir[J], cut)),
+      ((Sn += cw[J] * density_k<kinds[J]>(Mk->comp[first + J], Mk->comp_flags[first + J], nd,
+                                            fdir[J])),
        ...);
       pend.add(trow, n_last, jt, f, wk * Sn);
     } else {
@@ -521,9 +519,8 @@ __device__ __forceinline__ void table_group(Grp<Ks...>, std::integer_sequence<in
       double Sn = 0.0, Sa = 0.0;
       (
           [&] {
-            const double n =
-                density_k<kinds[J], (PROPS >> (4 * J)) & 15, cut_mode<PROPS, J, Ks...>()>(
-                    Mk->comp[first + J], Mk->comp_flags[first + J], nd, fdir[J], cut);
+            const double n = density_k<kinds[J]>(Mk->comp[first + J],
+                                                 Mk->comp_flags[first + J], nd, fdir[J]);
             Sn += cw[J] * n;
             if constexpr (kKelsall) {
               E[J] = fma(wB, n, E[J]);
