@@ -667,7 +667,7 @@ def main() -> int:
         "traffic_source": "profiles/forward_batched_dirbe12_traffic.json: rocprofv3 --pmc "
                           "FETCH_SIZE and WRITE_SIZE of this kernel on this workload, scaled by "
                           "a 1 GiB copy (not measured in this run)",
-        "kernel": "forward_layout (DIRBE layout)",
+        "kernel": "forward_line (DIRBE layout)",
         "flop_per_launch": flops,
         "algorithmic_bytes_per_launch": n_rays * (24 + 8),
         "output_write_GBs": round(n_rays * 8 / (ms_per_step / 1e3) / 1e9, 3),

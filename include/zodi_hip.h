@@ -185,10 +185,12 @@ enum {
 
 /* Launch configuration (0 in any field selects the built-in default). */
 typedef struct zodi_launch {
-  int32_t block;          /* threads per block: 64, 128, 256, 512 */
+  int32_t block;          /* threads per block: 64, 128, 256, 512 (the registry models' */
+                          /* kernels run 64 and 128 as 256) */
   int32_t lanes_per_ray;  /* 1, 2, 4, 8: Gauss-Legendre nodes split over this many lanes */
                           /* (zodi_forward adds the node terms in node order, so its */
-                          /* results do not depend on it; 0: chosen from n_rays)     */
+                          /* results do not depend on it; 0: chosen from n_rays, up */
+                          /* to 32)                                                  */
   int32_t blocks_per_cu;  /* > 0: grid-stride launch of this many blocks per CU; 0 = one block per tile */
   int32_t variant;        /* 0 generic, 1 specialised layout if available */
 } zodi_launch;
@@ -319,15 +321,16 @@ enum {
  * same n_rays, mode and launch. In ZODI_ADJ_CHI2 mode that size includes the
  * per-ray Jacobian when it fits in 72 GiB and launch allows one lane per ray:
  * one pass then writes the Jacobian and I (zodi_jacobian) and a second forms
- * chi2 and J^T g from them; with less workspace, or a larger problem, the
- * forward kernel writes I and the adjoint kernel recomputes the integrand with
- * the weights g. The two paths agree to rounding. launch may be NULL; otherwise
- * block must be 0 or 256, lanes_per_ray 0 (chosen from n_rays), 1, 2 or 4 (lanes
- * sharing one ray's nodes), blocks_per_cu 0..64 (0 = 2), and variant the
- * components evaluated per pass over a group's nodes: 0 (default: 4 in the
- * Jacobian pass, 2 otherwise), 1, 2 or 4 (four in the Jacobian pass, the sums of
- * up to two of them in LDS where registers do not hold all four; two in the
- * weighted pass).
+ * chi2 and J^T g from them (the Kelsall registry models form I, chi2 and the
+ * gradient in one pass instead, and use the workspace for its partial rows); with
+ * less workspace, or a larger problem, the forward kernel writes I and the adjoint
+ * kernel recomputes the integrand with the weights g. The paths agree to rounding.
+ * launch may be NULL; otherwise block must be 0 or 256, lanes_per_ray 0 (chosen from
+ * n_rays), 1, 2 or 4 (lanes sharing one ray's nodes), blocks_per_cu 0..64 (0: chosen
+ * from n_rays), and variant the components evaluated per pass over a group's nodes:
+ * 0 (default: 4 in the Jacobian pass, 2 otherwise), 1, 2 or 4 (four in the Jacobian
+ * pass, the sums of up to two of them in LDS; two in the weighted pass). The registry
+ * models' own kernels take every component of a group in one pass whatever variant is.
  * Every component layout the block can describe is supported: the registry
  * layouts (the Kelsall cloud and three bands, optionally followed by the ring
  * and the feature; the RRM model in its registry grouping or one component per
@@ -361,11 +364,12 @@ zodi_status zodi_adjoint(const zodi_model* model_host, const zodi_model* model_d
  * chi^2 (ZODI_ADJ_CHI2; else 0). A node between entries j and j + 1 at fraction f
  * contributes (1 - f) and f; a node at or past the last entry, or clamped below
  * the first, all of it to that entry. workspace: zodi_table_vjp_workspace bytes
- * (block partials, then I unless model_out is given). launch: block,
- * lanes_per_ray and blocks_per_cu as in zodi_adjoint (blocks_per_cu 0: as many
- * as the kernel keeps resident); variant is ignored. Any component layout. The
- * reduction order is fixed by the launch shape; within a wave, lanes that meet
- * in one entry add in hardware order.
+ * (block partials, and I unless model_out is given) or more: many rays take more
+ * blocks as far as workspace_bytes has rows for them. launch: block, lanes_per_ray
+ * and blocks_per_cu as in zodi_adjoint; variant is ignored. Any component layout.
+ * The reduction order is fixed by the launch shape (n_rays, launch and
+ * workspace_bytes); within a wave, lanes that meet in one entry add in hardware
+ * order.
  */
 int64_t zodi_table_vjp_workspace(const zodi_model* model_host, int64_t n_rays,
                                  const zodi_launch* launch);

@@ -1,7 +1,7 @@
 // Fused FP64 line-of-sight kernels for MI355X (gfx950) and their C ABI.
 //
-// One ray per lane (or per `L` adjacent lanes, which then split the
-// Gauss-Legendre nodes and combine with cross-lane shuffles). For each ray the
+// One ray per lane (or per group of adjacent lanes, which then split the
+// Gauss-Legendre nodes and add their terms in node order). For each ray the
 // per-ray sphere-intersection setup runs once; then, per group of components
 // sharing a line-of-sight range and temperature law, the node loop evaluates
 // position, 1/R, temperature and the Planck lookup once and every component
