@@ -7,6 +7,8 @@
 * LINE_INV[j] = 1/(1/2 + (j + 1/2)/512) rounded to a multiple of 2^-12 and
   LINE_LOG[j] = -log(LINE_INV[j]) (zodi_line.hpp: the product of a mantissa and a
   13-bit LINE_INV is exact inside an FMA).
+* LINE_ANGLE[2 j], LINE_ANGLE[2 j + 1] = cos, sin of the double j * (pi/128), j = 0..128
+  (zodi_line.hpp: unit_angle).
 
 Values are evaluated with mpmath at 200 bits and rounded to nearest double.
 Run ``python -m zodipy_amd.csrc.gen_math_tables`` to regenerate.
@@ -14,6 +16,7 @@ Run ``python -m zodipy_amd.csrc.gen_math_tables`` to regenerate.
 
 from __future__ import annotations
 
+import math
 from pathlib import Path
 
 import mpmath
@@ -51,6 +54,11 @@ def main() -> None:
     lines[-1] = lines[-1].rstrip(" \\").rstrip(",")
     lines += ["// -log of the same", "#define ZODI_LINE_LOG_TABLE \\"]
     lines += [f"  {_hex(-mpmath.log(v))}, \\" for v in short]
+    lines[-1] = lines[-1].rstrip(" \\").rstrip(",")
+    angle = [f(mpmath.mpf(j * (math.pi / 128))) for j in range(129)
+             for f in (mpmath.cos, mpmath.sin)]
+    lines += ["// cos and sin of j pi/128", "#define ZODI_LINE_ANGLE_TABLE \\"]
+    lines += [f"  {_hex(v)}, \\" for v in angle]
     lines[-1] = lines[-1].rstrip(" \\").rstrip(",")
     OUT.write_text("\n".join(lines) + "\n")
     print(OUT)

@@ -7,6 +7,7 @@
 
 #include <cstdint>
 #include <tuple>
+#include <type_traits>
 #include <utility>
 
 #include "zodi_common.hpp"

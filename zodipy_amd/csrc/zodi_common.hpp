@@ -175,16 +175,15 @@ __device__ __forceinline__ Node node_geometry(const Ray& y, double h, double mid
 // Kelsall (zodipy/brightness.py:21-56): (1 - a) eps B n, plus a F/R^2 Phi n with
 // scattering; without scattering the constant (1 - a) eps is applied once to the
 // node sum (finish). RRM (zodipy/brightness.py:59-83): B n, calibration applied
-// in finish. NOSCAT: no component of the block scatters (no ZODI_CF_SCATTER flag,
-// which the host checks), so the flag is not tested.
+// in finish.
 struct NodeTerm {
   double a, b;
 };
 
-template <int INTEGRAND, bool NOSCAT = false>
+template <int INTEGRAND>
 __device__ __forceinline__ NodeTerm node_term(ParamPtr P, uint32_t flags, const Node& nd,
                                               double wk, double wB, double dens, double solar) {
-  if constexpr (INTEGRAND == ZODI_INTEGRAND_KELSALL && !NOSCAT) {
+  if constexpr (INTEGRAND == ZODI_INTEGRAND_KELSALL) {
     if (flags & ZODI_CF_SCATTER) {
       double em = P[ZODI_P_ONE_MINUS_ALBEDO] * (P[ZODI_P_EMISSIVITY] * nd.B);
       em += (P[ZODI_P_ALBEDO] * (solar * (nd.inv_R * nd.inv_R))) * nd.phi;
@@ -213,11 +212,11 @@ __device__ __forceinline__ void add_in_node_order(double (&acc)[C], const NodeTe
 }
 
 // Integrated value of one component from its node sum; h = (stop - start)/2.
-template <int INTEGRAND, bool NOSCAT = false>
+template <int INTEGRAND>
 __device__ __forceinline__ double finish(ParamPtr P, uint32_t flags, double acc, double h,
                                          double calibration) {
   if constexpr (INTEGRAND == ZODI_INTEGRAND_KELSALL) {
-    if (!NOSCAT && (flags & ZODI_CF_SCATTER)) return __dmul_rn(acc, h);
+    if (flags & ZODI_CF_SCATTER) return __dmul_rn(acc, h);
     return __dmul_rn(__dmul_rn(acc, P[ZODI_P_SCALE]), h);
   } else {
     return __dmul_rn(__dmul_rn(acc, calibration), h);
@@ -706,26 +705,35 @@ __device__ __forceinline__ void line_group(Grp<Ks...>, std::integer_sequence<int
     nd.t = fma(th, Mk->gl_x[k], tm);
     nd.R2 = fma(nd.t, nd.t, l.d2);
     norm_and_inverse_node(nd.R2, nd.R, nd.inv_R);
-    Node tn;  // what node_term reads
-    tn.inv_R = nd.inv_R;
-    tn.B = planck_shifted(pow_table(cx.tab->temperature, cx.pt, nd.R2) - cx.uo1, cx.tab->planck);
-    tn.phi = 0.0;
+    const double B = planck_shifted(pow_table(cx.tab->temperature, cx.pt, nd.R2) - cx.uo1,
+                                    cx.tab->planck);
+    const double wB = wk * B;
+    double ws = 0.0;  // w F Phi / R^2
     if constexpr (!NOSCAT) {
-      if (scatter) tn.phi = line_phase_function(lp, l, cx.ec, nd.t, Mk->shared);
+      if (scatter) {
+        const ParamPtr S = Mk->shared;
+        ws = wk * ((S[ZODI_S_SOLAR] * (nd.inv_R * nd.inv_R)) *
+                   line_phase_function(lp, l, cx.tab->angles, cx.ec, nd.t, nd.inv_R, S));
+      }
     }
-    const double wB = wk * tn.B;
     double cut = 0.0;  // a band's cut-off, for the bands that share it (in order)
     NodeTerm t[C];
-    ((t[J] = node_term<ZODI_INTEGRAND_KELSALL, NOSCAT>(
-          Mk->comp[first + J], Mk->comp_flags[first + J], tn, wk, wB,
-          line_density<kinds[J], cut_mode<PROPS, J, Ks...>()>(Mk->comp[first + J],
-                                                              std::get<J>(lc), cx, l, nd, cut),
-          Mk->shared[ZODI_S_SOLAR])),
-     ...);
+    (
+        [&] {
+          const ParamPtr P = Mk->comp[first + J];
+          double u = wB;
+          if (!NOSCAT && scatter) {
+            u = P[ZODI_P_SCALE] * wB;
+            if (Mk->comp_flags[first + J] & ZODI_CF_SCATTER) u = fma(P[ZODI_P_ALBEDO], ws, u);
+          }
+          t[J] = {u, line_density<kinds[J], cut_mode<PROPS, J, Ks...>()>(P, std::get<J>(lc), cx,
+                                                                         l, nd, cut)};
+        }(),
+        ...);
     acc.add(t, terms, lanes, cx.sub, cx.K - k0);
   }
   acc.finish(a, y, first, lanes, cx.sub, total, [&](int c, double sum) {
-    return finish<ZODI_INTEGRAND_KELSALL, NOSCAT>(M->comp[c], M->comp_flags[c], sum, h, 0.0);
+    return __dmul_rn(scatter ? sum : __dmul_rn(sum, M->comp[c][ZODI_P_SCALE]), h);
   });
 }
 

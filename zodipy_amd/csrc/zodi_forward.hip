@@ -166,7 +166,7 @@ forward_layout(FwdArgs a) {
 // scattering code is compiled in.
 template <class LAYOUT, int BLOCK, bool SHARE, bool NOSCAT>
 __global__ __launch_bounds__(BLOCK)
-__attribute__((amdgpu_waves_per_eu(ForwardOccupancy<LAYOUT>::value))) void
+__attribute__((amdgpu_waves_per_eu(NOSCAT ? ForwardOccupancy<LAYOUT>::value : 4))) void
 forward_line(FwdArgs a) {
   __shared__ LineTables tables;
   const LineCtx cx = line_ctx(as_const(a.m), tables, 0);
@@ -209,7 +209,8 @@ __global__ __launch_bounds__(BLOCK)
 __attribute__((amdgpu_waves_per_eu(ForwardOccupancy<LAYOUT>::value))) void
 forward_rrm(FwdArgs a) {
   __shared__ LineAdjTables tables;
-  const LineAdjCtx cx = line_adj_ctx(as_const(a.m), tables);
+  __shared__ AngleTable angles;
+  const LineAdjCtx cx = line_adj_ctx(as_const(a.m), tables, &angles);
   for (int64_t tile = blockIdx.x; tile < a.n_tiles; tile += gridDim.x) {
     const Ray y = load_ray<BLOCK>(a, tile, threadIdx.x);
     double total = 0.0;
@@ -223,7 +224,8 @@ __global__ __launch_bounds__(kSplitBlock) __attribute__((amdgpu_waves_per_eu(2))
 forward_rrm_split(FwdArgs a) {
   __shared__ LineAdjTables tables;
   __shared__ double2 terms[SPLIT == 8 ? kMaxSlots * kSplitStride : 1];
-  LineAdjCtx cx = line_adj_ctx(as_const(a.m), tables);
+  __shared__ AngleTable angles;
+  LineAdjCtx cx = line_adj_ctx(as_const(a.m), tables, &angles);
   const int lanes = SPLIT == 8 ? a.lanes : SPLIT;
   cx.sub = threadIdx.x & (lanes - 1);
   const int rays = blockDim.x / lanes;

@@ -279,12 +279,48 @@ __device__ __forceinline__ double planck_shifted(double u1, const double2* tab) 
   return fma(__builtin_amdgcn_fract(u1), e.y, e.x);
 }
 
+// ---------------------------------------------------------------- angles
+// Angle of the unit vector (c, s), s >= 0, from the x axis: turned by the nearest of 129
+// tabulated directions j pi/128, found from the arc cosine in single precision (within
+// 4e-4, Abramowitz and Stegun 4.4.45), its sine is below 0.0127 and the arc sine's series
+// ends at the seventh power (next term 1e-18): 11 FP64 operations and no quotient where
+// axis_angle takes some 35. An error that c and s share (of 1/|X|) only scales the small
+// turn. Near 0 the direction is (1, 0), so the angle keeps the digits of s.
+struct AngleTable {
+  double2 e[129];
+};
+
+__constant__ double kLineAngle[258] = {ZODI_LINE_ANGLE_TABLE};
+
+__device__ __forceinline__ void load_angles(AngleTable& t) {
+  for (int i = threadIdx.x; i < 129; i += blockDim.x)
+    t.e[i] = double2{kLineAngle[2 * i], kLineAngle[2 * i + 1]};
+}
+
+__device__ __forceinline__ double unit_angle(const AngleTable& t, double c, double s) {
+  constexpr float kPerRad = 40.743665f;  // 128 / pi
+  const float x = (float)c, a = fminf(fabsf(x), 1.0f);
+  float q = fmaf(a, -0.0187293f * kPerRad, 0.0742610f * kPerRad);
+  q = fmaf(q, a, -0.2121144f * kPerRad);
+  q = fmaf(q, a, 1.5707288f * kPerRad);
+  q *= __builtin_amdgcn_sqrtf(1.0f - a);
+  q = x < 0.0f ? 128.0f - q : q;
+  const uint32_t j = (uint32_t)rintf(q) & 0xffu;
+  const uint32_t jc = j < 128u ? j : 128u;  // NaN converts to 0
+  const double2 e = t.e[jc];
+  const double d = fma(s, e.x, -(c * e.y)), z = d * d;
+  double w = fma(z, 15.0 / 336.0, 3.0 / 40.0);
+  w = fma(w, z, 1.0 / 6.0);
+  return fma((double)jc, 0x1.921fb54442d18p-6, fma(d * z, w, d));
+}
+
 // ---------------------------------------------------------------- per-launch tables
 struct LineTables {
   PowTable temperature;  // T0/dT (|X|^2)^(-delta/2)
   PowTable radial;       // the cloud's n_0 (r^2)^(-alpha/2)
   PowTable vertical;     // the cloud's g^gamma
   double2 planck[ZODI_N_TEMPS + 1];
+  AngleTable angles;
 };
 
 // Everything the node loops read besides the model block.
@@ -308,6 +344,7 @@ __device__ __forceinline__ LineCtx line_ctx(ModelPtr M, LineTables& tab, int sub
   build_pow_table(tab.radial, ec, pr, P[6], kPowRadiusFirst, i, n);
   build_pow_table(tab.vertical, ec, pv, 1.0, kPowUnitFirst, i, n);
   load_planck(M, tab.planck, i, n);
+  load_angles(tab.angles);
   __syncthreads();
   LineCtx cx;
   cx.M = M;
@@ -471,28 +508,59 @@ __device__ __forceinline__ LinePhase line_phase(const Line& l) {
 // arccos(-u . X / |X|), whose cosine is -n t / |X|. As the angle of (-n t, sqrt(|X|^2 -
 // n^2 t^2)) it needs no quotient by |X| and keeps its digits near 0 and pi, where the
 // arc cosine loses half of them; for a unit pointing the second is the ray's d.
-__device__ __forceinline__ double line_phase_function(const LinePhase& p, const Line& l,
-                                                      const ExpConst& e, double t, ParamPtr S) {
+__device__ __forceinline__ double scattering_angle(const LinePhase& p, const Line& l, double t) {
   double y = p.d;
   if (p.k != 0.0) y = sqrt(fmax(fma(t * t, p.k, l.d2), 0.0));  // clipped like the cosine
-  const double theta = axis_angle(-l.n * t, y);
+  return axis_angle(-l.n * t, y);
+}
+
+__device__ __forceinline__ double scattering_angle(const LinePhase& p, const Line& l, double t,
+                                                   const AngleTable& tab, double inv_R) {
+  if (p.k != 0.0) return scattering_angle(p, l, t);
+  return unit_angle(tab, (-l.n * t) * inv_R, p.d * inv_R);
+}
+
+__device__ __forceinline__ double line_phase_function(const LinePhase& p, const Line& l,
+                                                      const AngleTable& tab, const ExpConst& e,
+                                                      double t, double inv_R, ParamPtr S) {
+  const double theta = scattering_angle(p, l, t, tab, inv_R);
   return S[ZODI_S_PHASE_NORM] *
          (S[ZODI_S_C1] + S[ZODI_S_C2] * theta + exp_neg_any(e, -(S[ZODI_S_C3] * theta)));
+}
+
+// |theta| of the feature at the node: the angle of the rotated point from the centre line,
+// by the table, with its y, rho^2 and 1/rho (of a point scaled up where rho^2 would leave
+// the normal range).
+__device__ __forceinline__ double feature_angle(const LineComp<ZODI_FEATURE>& c, const Line& l,
+                                                const AngleTable& tab, double t, double& y,
+                                                double& rho2, double& inv_rho) {
+  double x = c.x.at(t);
+  y = c.y.at(t);
+  rho2 = fma(x, x, y * y);
+  double r2 = rho2, rho;
+  if (r2 < 0x1p-900) {
+    if (x == 0.0 && y == 0.0) {  // on the axis: see feature_dtheta
+      const double sg = __builtin_signbit(fma(l.vx, t, l.px)) ? -1.0 : 1.0;
+      x = sg * c.d.c;
+      y = -sg * c.d.s;
+    } else {
+      x *= 0x1p600;
+      y *= 0x1p600;
+    }
+    r2 = fma(x, x, y * y);
+  }
+  norm_and_inverse_node(r2, rho, inv_rho);
+  return unit_angle(tab, x * inv_rho, fabs(y) * inv_rho);
 }
 
 __device__ __forceinline__ double line_feature(ParamPtr P, const LineComp<ZODI_FEATURE>& c,
                                                const LineCtx& cx, const Line& l,
                                                const LineNode& nd) {
-  double x = c.x.at(nd.t), y = c.y.at(nd.t);
-  if (x == 0.0 && y == 0.0) {  // on the axis: see feature_dtheta
-    const double sg = __builtin_signbit(fma(l.vx, nd.t, l.px)) ? -1.0 : 1.0;
-    x = sg * c.d.c;
-    y = -sg * c.d.s;
-  }
   const double d = nd.R - P[7];
   double e = (d * d) * P[13];
   e = fma(fabs(c.z.at(nd.t)), P[14], e);
-  const double theta = axis_angle(x, y);
+  double y, rho2, inv_rho;
+  const double theta = feature_angle(c, l, cx.tab->angles, nd.t, y, rho2, inv_rho);
   e = fma(theta * theta, P[15], e);
   return P[6] * exp_neg_any(cx.ec, e);
 }

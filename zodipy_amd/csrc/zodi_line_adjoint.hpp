@@ -65,13 +65,29 @@ struct LineAdjCtx {
   LogConst lc;
   int K, sub, split;
   bool share;  // band 3 takes band 1's cut-off (props_match with kShareCut)
+  const AngleTable* angles;
+  static constexpr bool kAngles = false;
 };
 
-__device__ __forceinline__ LineAdjCtx line_adj_ctx(ModelPtr M, LineAdjTables& tab) {
+// For the passes that take angles from the table: with scattering (SCAT 2), chi^2 of 196 608
+// rays of DIRBE at 1.25 um takes 296 us for 314, of 400 000 672 for 741. The passes without,
+// whose only angle is the feature's, spill more registers for it than it saves (VJP of
+// 150 000 rays 210 us for 205, RRM chi^2 of 49 152 168 for 165) and keep axis_angle.
+struct LineAdjCtxAngles : LineAdjCtx {
+  static constexpr bool kAngles = true;
+};
+
+template <int SCAT>
+using AdjCtx = std::conditional_t<SCAT == 2, LineAdjCtxAngles, LineAdjCtx>;
+
+// Builds the block's tables, `angles` too if given (every thread of the block must call it).
+__device__ __forceinline__ LineAdjCtx line_adj_ctx(ModelPtr M, LineAdjTables& tab,
+                                                   AngleTable* angles = nullptr) {
   stage_line_tables();
   for (int j = threadIdx.x; j < 256; j += blockDim.x)
     tab.log_tab[j] = double2{kLineInv[j], kLineLog[j]};
   load_planck(M, tab.planck, threadIdx.x, blockDim.x);
+  if (angles != nullptr) load_angles(*angles);
   __syncthreads();
   LineAdjCtx cx;
   cx.M = M;
@@ -82,6 +98,7 @@ __device__ __forceinline__ LineAdjCtx line_adj_ctx(ModelPtr M, LineAdjTables& ta
   cx.sub = 0;
   cx.split = 1;
   cx.share = false;
+  cx.angles = angles;
   return cx;
 }
 
@@ -272,16 +289,28 @@ struct LineGrad<ZODI_FEATURE> {
   __device__ __forceinline__ LineGrad(ParamPtr P, const Line& l, double ex, double ey)
       : c(P, l, ex, ey), s{} {}
 
-  __device__ __forceinline__ double add(ParamPtr P, const LineAdjCtx& cx, const Line& l,
+  template <class CTX>
+  __device__ __forceinline__ double add(ParamPtr P, const CTX& cx, const Line& l,
                                         const GradNode& nd, double u) {
-    double x = c.x.at(nd.t), y = c.y.at(nd.t);
-    const double rho2 = fma(x, x, y * y);
-    if (x == 0.0 && y == 0.0) {  // on the axis: see feature_dtheta
-      const double sg = __builtin_signbit(fma(l.vx, nd.t, l.px)) ? -1.0 : 1.0;
-      x = sg * c.d.c;
-      y = -sg * c.d.s;
+    double y, inv_rho2, angle;
+    if constexpr (CTX::kAngles) {
+      double rho2, inv_rho;
+      angle = feature_angle(c, l, *cx.angles, nd.t, y, rho2, inv_rho);
+      inv_rho2 = inv_rho * inv_rho;
+      inv_rho2 = fma(inv_rho2, fma(-rho2, inv_rho2, 1.0), inv_rho2);
+      if (rho2 < 0x1p-900) inv_rho2 = rcp_fast(rho2);  // inv_rho is that of a scaled point
+    } else {
+      double x = c.x.at(nd.t);
+      y = c.y.at(nd.t);
+      inv_rho2 = rcp_fast(fma(x, x, y * y));
+      if (x == 0.0 && y == 0.0) {  // on the axis: see feature_dtheta
+        const double sg = __builtin_signbit(fma(l.vx, nd.t, l.px)) ? -1.0 : 1.0;
+        x = sg * c.d.c;
+        y = -sg * c.d.s;
+      }
+      angle = axis_angle(x, y);
     }
-    const double th = __builtin_copysign(axis_angle(x, y), y);
+    const double th = __builtin_copysign(angle, y);
     const double d = nd.R - P[7];
     const double zc = c.z.at(nd.t);
     double e = (d * d) * P[13];
@@ -302,7 +331,7 @@ struct LineGrad<ZODI_FEATURE> {
     const double qt = q * th;
     s[7] += qt;
     s[8] = fma(qt, th, s[8]);
-    const double qr = qt * rcp_fast(rho2);
+    const double qr = qt * inv_rho2;
     s[9] += qr;
     s[10] = fma(qr, nd.t, s[10]);
     return nu;
@@ -350,11 +379,8 @@ __device__ __forceinline__ void line_geo(ParamPtr P, const Line& l, const double
 
 // ---------------------------------------------------------------- one group
 // Kelsall phase function at the node with its partials (phase_grad) on the line.
-__device__ __forceinline__ PhaseGrad line_phase_grad(const LinePhase& p, const Line& l,
-                                                     const ExpConst& e, double t, ParamPtr S) {
-  double y = p.d;
-  if (p.k != 0.0) y = sqrt(fmax(fma(t * t, p.k, l.d2), 0.0));
-  const double theta = axis_angle(-l.n * t, y);
+__device__ __forceinline__ PhaseGrad line_phase_grad(double theta, const ExpConst& e,
+                                                     ParamPtr S) {
   const double C1 = S[ZODI_S_C1], C2 = S[ZODI_S_C2], C3 = S[ZODI_S_C3];
   const double N = S[ZODI_S_PHASE_NORM];
   const double e3 = exp_neg_any(e, -(C3 * theta));
@@ -466,7 +492,14 @@ __device__ __forceinline__ void line_adj_group(Grp<Ks...>, std::integer_sequence
       PhaseGrad pg = {phi_const, 0.0, 0.0, 0.0};
       double ws = 0.0;  // w F Phi / R^2
       if constexpr (SCAT != 0) {
-        if (need_angle) pg = line_phase_grad(lp, l, cx.ec, nd.t, M->shared);
+        if (need_angle) {
+          double theta;
+          if constexpr (SCAT == 2)
+            theta = scattering_angle(lp, l, nd.t, *cx.angles, nd.inv_R);
+          else
+            theta = scattering_angle(lp, l, nd.t);
+          pg = line_phase_grad(theta, cx.ec, M->shared);
+        }
         ws = wk * ((solar * nd.iR2) * pg.phi);
       }
       double sn = 0.0;  // sum of (1 - a) eps n over the components
@@ -484,7 +517,7 @@ __device__ __forceinline__ void line_adj_group(Grp<Ks...>, std::integer_sequence
               CutShare own = {0.0, 0.0};
               nu = A.add(P, cx, nd, CUT == kCutOwn ? own : cs, CUT == kCutReuse && cx.share, u);
             } else {
-              nu = A.add(P, cx, l, nd, u);
+              nu = A.add(P, static_cast<const AdjCtx<SCAT>&>(cx), l, nd, u);
             }
             s0[J] = fma(wB, nu, s0[J]);
             if constexpr (SCAT != 0) s1[J] = fma(ws, nu, s1[J]);
@@ -745,7 +778,8 @@ __device__ __forceinline__ void line_adj_body(const AdjArgs& a) {
   __shared__ LineAdjTables tables;
   const ModelPtr M = as_const(a.f.m);
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  LineAdjCtx cx = line_adj_ctx(M, tables);
+  __shared__ AngleTable angles;
+  AdjCtx<SCAT> cx{line_adj_ctx(M, tables, SCAT == 2 ? &angles : nullptr)};
   cx.split = a.split;
   cx.sub = lane & (a.split - 1);
   cx.share = a.share != 0;

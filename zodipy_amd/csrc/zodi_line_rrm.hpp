@@ -176,13 +176,8 @@ __device__ __forceinline__ double rrm_density(ParamPtr P, const LineComp<KIND>& 
            exp_neg_any(cx.ec, fma(d * d, P[13], fabs(c.z.at(nd.t)) * P[14]));
   } else {
     static_assert(KIND == ZODI_FEATURE_RRM, "an RRM component");
-    double x = c.x.at(nd.t), y = c.y.at(nd.t);
-    if (x == 0.0 && y == 0.0) {
-      const double sg = __builtin_signbit(fma(l.vx, nd.t, l.px)) ? -1.0 : 1.0;
-      x = sg * c.d.c;
-      y = -sg * c.d.s;
-    }
-    const double th = axis_angle(x, y);
+    double y, rho2, inv_rho;
+    const double th = feature_angle(c, l, *cx.angles, nd.t, y, rho2, inv_rho);
     const double d = nd.R - P[7];
     double e = (d * d) * P[13];
     e = fma(fabs(c.z.at(nd.t)), P[14], e);

@@ -359,7 +359,9 @@ __device__ __forceinline__ void line_table_group(Grp<Ks...>, std::integer_sequen
     if constexpr (kScat) {
       if (pu.phase) {
         pg.phi = pu.phi_const;
-        if (pu.angle) pg = line_phase_grad(lp, l, cx.ec, t, Mk->shared);
+        if (pu.angle)
+          pg = line_phase_grad(scattering_angle(lp, l, t, cx.tab->angles, nd.inv_R), cx.ec,
+                               Mk->shared);
         inv_R2 = nd.inv_R * nd.inv_R;
         wsu = wk * ((solar * inv_R2) * pg.phi);
       }
@@ -602,7 +604,8 @@ __global__ __launch_bounds__(kAdjBlock) __attribute__((
     });
   } else {
     __shared__ LineAdjTables tables;
-    LineAdjCtx cx = line_adj_ctx(as_const(a.f.m), tables);
+    __shared__ AngleTable angles;
+    LineAdjCtx cx = line_adj_ctx(as_const(a.f.m), tables, &angles);
     cx.sub = threadIdx.x & (a.split - 1);
     weighted_body(a, [&](const Ray& y, double gscale, double* row, int lane) {
       run_line_table<PROPS, EFF, NOSCAT>(LAYOUT{}, cx, a, y, gscale, row, lane);
