@@ -190,3 +190,32 @@ def test_block_rows_beyond_the_resident_ones(gpu, name, x, rays, lanes):
                 # entries that cancel are judged against the gradient's largest
                 tol = 1e-10 * b.abs() + 1e-13 * b.abs().max()
                 assert torch.all((a - b).abs() <= tol)
+
+
+@pytest.mark.parametrize("rays", [1, 5_000, 40_001, 98_305, 131_072, 150_001])
+@pytest.mark.parametrize("x", [25 * u.micron, 1.25 * u.micron])
+def test_gradient_splits_against_one_lane(gpu, x, rays):
+    """The lanes per ray that the gradient passes pick from the ray count against one lane
+    and the recompute path: the same terms in another order (tolerance as above)."""
+    rng = np.random.default_rng(rays)
+    v = rng.normal(size=(3, rays))
+    v /= np.linalg.norm(v, axis=0)
+    obs = np.array([0.9, 0.4, 0.02])
+    prob = LineOfSightProblem(Model(x), v, obs, obs)
+    theta = prob.space.theta0
+    w = torch.as_tensor(rng.uniform(0.5, 1.5, rays), device="cuda")
+    data = prob.forward(theta) * torch.as_tensor(rng.uniform(0.9, 0.99, rays), device="cuda")
+
+    def both():
+        c, g, model = prob.chi2_and_grad(theta, data, return_model=True)
+        return torch.cat([c.reshape(1), g]), prob.vjp(theta, w), model
+
+    got = both()
+    prob.launch = Launch(0, 1, 0, 0)
+    one = both()
+    prob.store_jacobian = False
+    again = both()
+    for a, b, c in zip(got, one, again):
+        for other in (a, c):
+            tol = 1e-10 * b.abs() + 1e-13 * b.abs().max()
+            assert torch.all((other - b).abs() <= tol)

@@ -355,18 +355,27 @@ struct AdjPlan {
   int64_t grid;
 };
 
-// Launch plan. With lanes_per_ray = 0 one lane owns a ray unless the rays do not
-// fill every resident wave once; then the smallest split (2 or 4 lanes per ray)
-// that does. Each extra lane per ray repeats the per-ray set-up and the wave
-// reductions, which costs more than a partly idle last round (VJP of 196 608 rays of
-// DIRBE, 1.5 rounds: 209 us at one lane, 242 at two). The Jacobian and chi^2 passes (jac)
-// use one lane per ray, the line kernels' up to 8 where rays are few.
+// Launch plan. Lanes per ray when the caller leaves them open:
+//
+// Kelsall line kernels: with r waves of s lanes a ray on a SIMD and K nodes a ray a pass
+// takes (r + 1) (ceil(K / s) + 13) units (13: the ray's set-up and reductions beside its
+// nodes; 1: latency, which r waves share; below two waves it shows in full), and the
+// cheapest of 1, 2, 4 lanes (8 where I comes with the pass) is taken. Measured against the
+// largest split whose waves are all resident, chi^2 of DIRBE in us: 49 152 rays 88 -> 74,
+// 98 304 157 -> 118, 150 000 210 -> 192, and 131 072 rays keep one lane (157; 167 at two).
+//
+// RRM line kernels: the Jacobian pass the largest split, up to 8, whose waves are all
+// resident; the VJP, and the other kernels' passes, one lane unless the rays do not fill
+// every resident wave once, then the smallest split (2 or 4) that does (VJP of 196 608
+// rays of DIRBE, 1.5 rounds: 209 us at one lane, 242 at two). The other kernels' Jacobian
+// pass uses one lane.
 zodi_status adjoint_plan(const zodi_model* m, const zodi_launch* launch, int64_t n_rays, bool jac,
-                         AdjPlan& p) {
+                         AdjPlan& p, bool table = false) {
+  const bool line = !table && takes_line(m);
   p.chunk = jac ? kDefaultJacChunk : kDefaultChunk;
   p.split = 0;
   p.per_cu = kDefaultBlocksPerCu;
-  if (m->integrand == ZODI_INTEGRAND_RRM && takes_line(m)) p.per_cu = kRrmAdjWaves;
+  if (m->integrand == ZODI_INTEGRAND_RRM && line) p.per_cu = kRrmAdjWaves;
   if (launch != nullptr) {
     if (launch->block != 0 && launch->block != kAdjBlock)
       return fail(ZODI_ERR_ARG, "adjoint block must be %d, got %d", kAdjBlock, launch->block);
@@ -386,21 +395,28 @@ zodi_status adjoint_plan(const zodi_model* m, const zodi_launch* launch, int64_t
     p.split = launch->lanes_per_ray;
     if (launch->blocks_per_cu > 0) p.per_cu = launch->blocks_per_cu;
   }
-  if (jac) {
-    if (p.split > 1)
-      return fail(ZODI_ERR_ARG, "the Jacobian pass uses one lane per ray, got lanes_per_ray %d",
-                  p.split);
-    // Small ray counts leave the line kernels' resident waves idle: up to 8 lanes a ray.
-    if (p.split == 0 && takes_line(m)) {
-      const int64_t slots = (int64_t)p.per_cu * cu_count() * kAdjWaves;
-      p.split = 8;
-      while (p.split > 1 && (n_rays * p.split + kWave - 1) / kWave > slots) p.split /= 2;
-    } else {
-      p.split = 1;
-    }
-  }
   const int64_t waves = (int64_t)p.per_cu * cu_count() * kAdjWaves;
-  if (p.split == 0) {
+  if (jac && p.split > 1)
+    return fail(ZODI_ERR_ARG, "the Jacobian pass uses one lane per ray, got lanes_per_ray %d",
+                p.split);
+  if (p.split == 0 && line && m->integrand == ZODI_INTEGRAND_KELSALL) {
+    const int64_t simds = (int64_t)4 * cu_count();
+    int64_t least = INT64_MAX;
+    for (int s : {1, 2, 4, 8}) {
+      if (s == 8 && !jac) break;
+      const int64_t w = (n_rays * s + kWave - 1) / kWave, r = (w + simds - 1) / simds;
+      const int64_t cost = (std::max<int64_t>(r, 2) + 1) * ((m->n_nodes + s - 1) / s + 13);
+      if (cost < least) {
+        least = cost;
+        p.split = s;
+      }
+    }
+  } else if (jac && p.split == 0 && line) {
+    p.split = 8;
+    while (p.split > 1 && (n_rays * p.split + kWave - 1) / kWave > waves) p.split /= 2;
+  } else if (jac) {
+    p.split = 1;
+  } else if (p.split == 0) {
     p.split = 4;
     for (int s : {1, 2}) {
       if ((n_rays * s + kWave - 1) / kWave >= waves) {
@@ -466,7 +482,7 @@ zodi_status table_plan(const zodi_model* m, const zodi_launch* launch, int64_t n
   zodi_launch l = launch != nullptr ? *launch : zodi_launch{0, 0, 0, 0};
   if (l.blocks_per_cu == 0) l.blocks_per_cu = any.waves;
   l.variant = 0;
-  const zodi_status st = adjoint_plan(m, &l, n_rays, false, p);
+  const zodi_status st = adjoint_plan(m, &l, n_rays, false, p, true);
   if (st != ZODI_OK) return st;
   k = table_adjoint_kernel(m, p.split, eff).k;
   if (k == nullptr)
