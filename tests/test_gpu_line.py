@@ -219,3 +219,15 @@ def test_gradient_splits_against_one_lane(gpu, x, rays):
         for other in (a, c):
             tol = 1e-10 * b.abs() + 1e-13 * b.abs().max()
             assert torch.all((other - b).abs() <= tol)
+
+
+@pytest.mark.parametrize("name", ["dirbe", "rrm-experimental"])
+def test_feature_angle_next_to_the_axis(gpu, name):
+    """Points whose squared distance from the z axis leaves the normal range (the feature's
+    angle is then that of a scaled point) against the kind switch, which takes atan2."""
+    v = np.array([[1e-170, -3e-200, 0.0, 2e-155], [2e-170, 1e-180, 1e-160, -1e-156],
+                  [1.0, 1.0, 1.0, 1.0]])
+    obs = np.array([0.0, 0.0, 1.1])
+    same(*both(Model(25 * u.micron, name=name), v, obs))
+    if name == "dirbe":
+        same(*both(Model(1.25 * u.micron), v, obs))

@@ -155,12 +155,12 @@ forward_layout(FwdArgs a) {
 }
 
 // The Kelsall layouts' registry blocks (props_match without the shared cut-off, and
-// line_match) on the ray's line (zodi_line.hpp): bound by FP64 vector issue, the three node
-// loops of the DIRBE layout take 1346 issue cycles per wave and node where forming every
-// node's position and its powers by exp(p log x) took 1968. Measured: DIRBE 12 um, 50.7 M
-// rays, 34.4 -> 25.2 ms (7.4e10 -> 1.01e11 ray-nodes/s);
-// planck18 857 GHz, 22.5 M rays, 8.29 -> 6.12 ms; DIRBE 1.25 um with scattering, 196 608
-// rays, 0.317 -> 0.26 ms. SHARE: the bands that share a radial cut-off reuse it
+// line_match) on the ray's line (zodi_line.hpp): bound by FP64 vector issue, 335 vector
+// instructions a ray and node of the DIRBE layout where forming every node's position and
+// its powers by exp(p log x) took 487. Measured: DIRBE 12 um, 50.7 M rays, 38.3 -> 26.6 ms
+// (6.6e10 -> 9.5e10 ray-nodes/s); planck18 857 GHz, 22.5 M rays, 9.14 -> 6.71 ms; DIRBE
+// 1.25 um with scattering, 196 608 rays, 0.316 -> 0.219 ms (compiled for 4 waves a SIMD,
+// without spills: 214 -> 200 us of kernel against 5). SHARE: the bands that share a radial cut-off reuse it
 // (kShareCut), for blocks whose delta_r values allow it (the registry parameters; a fit
 // that moves them runs without). NOSCAT (with SHARE): no component scatters, so no
 // scattering code is compiled in.
@@ -203,7 +203,7 @@ forward_line_split(FwdArgs a) {
 // The RRM layouts' registry blocks (every component centred) on the ray's line: 3580 issue
 // cycles per wave and node over the six groups where the arc sines, sines, cosines and
 // powers of every node took 6750 (and less where a wave skips a branch). Measured: RRM 25
-// um, 196 608 rays with the pixel vectors, 0.524 -> 0.329 ms.
+// um, 196 608 rays with the pixel vectors, 0.524 -> 0.300 ms (two lanes a ray).
 template <class LAYOUT, int BLOCK>
 __global__ __launch_bounds__(BLOCK)
 __attribute__((amdgpu_waves_per_eu(ForwardOccupancy<LAYOUT>::value))) void
