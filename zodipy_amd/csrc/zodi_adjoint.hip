@@ -10,8 +10,8 @@
 // store the Jacobian with I, or let the forward kernel write I first.
 //
 // The kernels of this file, for what the line kernels (zodi_line_adjoint.hpp,
-// zodi_line_rrm.hpp) do not take: one wave owns a tile of 64 rays, one ray per lane. Per chunk of components
-// of a group (components sharing a range; the chunk size is a compile-time
+// zodi_line_rrm.hpp) do not take: one wave owns a tile of 64 rays, one ray per lane. Per
+// chunk of components of a group (components sharing a range; the chunk size is a compile-time
 // choice that trades recomputed node geometry for register pressure), each
 // node's geometry, B(T), dB/dT and the phase function with its C1..C3 partials
 // are formed once; every component of the chunk then adds its contributions to

@@ -160,8 +160,8 @@ forward_layout(FwdArgs a) {
 // its powers by exp(p log x) took 487. Measured: DIRBE 12 um, 50.7 M rays, 38.3 -> 26.6 ms
 // (6.6e10 -> 9.5e10 ray-nodes/s); planck18 857 GHz, 22.5 M rays, 9.14 -> 6.71 ms; DIRBE
 // 1.25 um with scattering, 196 608 rays, 0.316 -> 0.219 ms (compiled for 4 waves a SIMD,
-// without spills: 214 -> 200 us of kernel against 5). SHARE: the bands that share a radial cut-off reuse it
-// (kShareCut), for blocks whose delta_r values allow it (the registry parameters; a fit
+// without spills: 214 -> 200 us of kernel against 5). SHARE: the bands that share a radial
+// cut-off reuse it (kShareCut), for blocks whose delta_r values allow it (the registry parameters; a fit
 // that moves them runs without). NOSCAT (with SHARE): no component scatters, so no
 // scattering code is compiled in.
 template <class LAYOUT, int BLOCK, bool SHARE, bool NOSCAT>
