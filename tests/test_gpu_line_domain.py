@@ -1,0 +1,111 @@
+"""Parameters and pointings at the edges of what the line kernels' tables hold.
+
+The registry models' forward (line kernels, or the general layout kernels where a block is
+outside their ranges) against the kind switch (variant 0), which forms every position and
+every power by itself, and the gradients against the general kernels, which run for a block
+whose centred components carry no ZODI_CF_CENTERED flag (the values are the same).
+
+Tolerance: 1e-10 relative (see test_gpu_line.py); gradient entries that cancel are judged
+against the largest one.
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from zodipy_amd import Model, healpix
+from zodipy_amd import units as u
+from zodipy_amd._lib import ADJ_CHI2, Launch
+from zodipy_amd.fitting import LineOfSightProblem
+from zodipy_amd.packing import CF_CENTERED
+from zodipy_amd.runtime import OUT_COMPS
+
+pytestmark = pytest.mark.gpu
+
+OBS = np.array([0.98, 0.17, 0.004])
+RTOL = 1e-10
+
+
+def changed(name, values, x=25 * u.micron):
+    """A model with parameters replaced: {"delta": v} or {"comp": {"field": v}}."""
+    model = Model(x, name=name)
+    p = model.get_parameters()
+    for k, v in values.items():
+        if isinstance(v, dict):
+            p["comps"][k].update(v)
+        else:
+            p[k] = v
+    with np.errstate(all="ignore"):
+        model.update_parameters(p)
+    return model
+
+
+def same(got, want, scale=None, rtol=RTOL):
+    """NaN and infinities in the same places, the rest within rtol (of `scale` if given)."""
+    got, want = np.asarray(got), np.asarray(want)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    inf = np.isinf(want)
+    assert np.array_equal(got[inf], want[inf]) and not np.isinf(got[~inf]).any()
+    ok = np.isfinite(want)
+    # below the normal range a value is a rounding of the smallest double
+    floor = np.finfo(float).tiny if scale is None else scale
+    assert np.all(np.abs(got - want)[ok] <= rtol * np.maximum(np.abs(want[ok]), floor) + 5e-324)
+
+
+def forward_agrees(model, v, rtol=RTOL):
+    dm = model.device_model
+    got = dm.forward(v, OBS, OBS, out_mode=OUT_COMPS).cpu().numpy()
+    want = dm.forward(v, OBS, OBS, out_mode=OUT_COMPS, launch=Launch(variant=0)).cpu().numpy()
+    same(got, want, rtol=rtol)
+    return got
+
+
+def general_block(model):
+    """The model's block with every component taken through its offset frame."""
+    host = np.ascontiguousarray(model._packed.block).copy()
+    host["comp_flags"] &= ~np.uint32(CF_CENTERED)
+    return host, torch.from_numpy(host.view(np.uint8).copy()).cuda()
+
+
+def gradients_agree(model, v):
+    """chi^2 and its gradients of the registry route against the general kernels'."""
+    prob = LineOfSightProblem(model, v, OBS, OBS)
+    data = torch.full((v.shape[1],), 0.7, dtype=torch.float64, device="cuda")
+    host = np.ascontiguousarray(model._packed.block)
+    line = (host, torch.from_numpy(host.view(np.uint8).copy()).cuda())
+    res = []
+    for blocks in (line, general_block(model)):
+        g = prob._adjoint(None, ADJ_CHI2, target=data, blocks=blocks)
+        t = prob._table_adjoint(None, ADJ_CHI2, target=data, blocks=blocks, eff=True)
+        res.append((g.cpu().numpy(), t.cpu().numpy()))
+    for got, want in zip(*res):
+        with np.errstate(all="ignore"):
+            top = np.abs(want[np.isfinite(want)]).max(initial=0.0)
+        same(got, want, scale=1e-3 * top)
+    return res[0][0]
+
+
+@pytest.mark.parametrize("cloud", [{"mu": -1.9}, {"mu": -2.0}, {"mu": -3.0}, {"mu": -4.5},
+                                   {"mu": -3.0, "beta": 1e6, "gamma": 6.0}, {"x_0": 2e4},
+                                   {"y_0": -1e9}, {"z_0": 1e17}, {"x_0": 1e19}])
+@pytest.mark.parametrize("x", [25 * u.micron, 1.25 * u.micron])
+def test_power_table_range(gpu, cloud, x):
+    """g of the cloud at 2 and more, its centre beyond 10 000 AU."""
+    model = changed("dirbe", {"cloud": cloud}, x)
+    v = healpix.pix2vec(4)
+    forward_agrees(model, v)
+    gradients_agree(model, v)
+
+
+@pytest.mark.parametrize("length", [0.5, 3.0, 1e5, 1e8])
+@pytest.mark.parametrize("name,x", [("dirbe", 25 * u.micron), ("dirbe", 1.25 * u.micron),
+                                    ("rrm-experimental", 25 * u.micron)])
+def test_pointing_lengths(gpu, name, x, length):
+    """Pointings whose x and y are not those of a unit vector: positions s u + o out to
+    5e8 AU. A node's distance h x + mid carries a rounding of its largest value, which the
+    length multiplies: 3e-16 AU of |X| per unit of length, and the ring's exponent changes by
+    up to 2.2e3 per AU where its density is not yet 0."""
+    v = healpix.pix2vec(4) * np.array([[length], [length], [1.0]])
+    forward_agrees(Model(x, name=name), v, rtol=RTOL + 7e-13 * length)

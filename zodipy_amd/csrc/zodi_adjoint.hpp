@@ -622,14 +622,6 @@ AdjKernel line_adjoint_rrm(bool split_layout, bool jac);
 constexpr int kLineAdjWaves = 2;
 constexpr int kRrmAdjWaves = 4;
 
-inline bool line_adjoint_match(const zodi_model* m) {
-  if (m->integrand == ZODI_INTEGRAND_RRM) return true;
-  const auto in = [](double v, double most) { return v >= -most && v <= most; };
-  for (int g = 0; g < m->n_groups; ++g)
-    if (!in(m->group_delta[g], 1e3)) return false;
-  return in(m->comp[0][7], 1e3) && in(m->comp[0][8], 1e6) && in(m->comp[0][9], 1e3);
-}
-
 // Resident waves per SIMD the table kernels are compiled for (their register
 // budgets): the registry layouts; the Kelsall ones with the spectral sums of
 // scattering components; the kind switch (at three rather than its

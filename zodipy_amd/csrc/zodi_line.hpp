@@ -26,6 +26,7 @@
 #pragma once
 
 #include "zodi_device.hpp"
+#include "zodi_line_domain.hpp"
 
 namespace zodi {
 
@@ -160,12 +161,12 @@ __device__ __forceinline__ double exp_neg_any(const ExpConst& e, double x) {
 
 // ---------------------------------------------------------------- x^p, p fixed
 // In LDS: entry j is (inv_j, inv_j^-p) for mantissas in [1/2 + j/512, 1/2 + (j+1)/512);
-// scale[i] = factor 2^(p e) for the exponents e whose biased value is i modulo 128 and
-// that lie in [e_first, e_first + 128). An argument outside [2^(e_first - 1),
-// 2^(e_first + 127)) is the caller's to exclude (NaN passes).
+// scale[i] = factor 2^(p e) for the exponents e whose biased value is i modulo 256 and
+// that lie in [e_first, e_first + 256). An argument outside [2^(e_first - 1),
+// 2^(e_first + 255)) is the caller's to exclude (NaN passes).
 struct PowTable {
   double2 c[256];
-  double scale[128];
+  double scale[256];
 };
 
 // Binomial coefficients of (1 + r)^p, r^1..r^5, in scalar registers but the fourth: |r| < 2^-8.9, the
@@ -220,12 +221,12 @@ __device__ __forceinline__ void build_pow_table(PowTable& t, const ExpConst& ec,
     // inv^-p; -p log(inv) is below |p| 0.7, so its rounding stays below an ulp
     t.c[j] = double2{kLineInv[j], exp_neg_any(ec, -(p * kLineLog[j]))};
   }
-  for (int j = i; j < 128; j += stride) {
+  for (int j = i; j < 256; j += stride) {
     const int e = e_first + j;
     const double zh = p * (double)e;
     const double zl = fma(p, (double)e, -zh);
     // frexp's exponent e: x = 2^e m, m in [1/2, 1); its biased exponent is e + 1022
-    t.scale[(e + 1022) & 127] = factor * exp2_table(ec, zh, zl);
+    t.scale[(e + 1022) & 255] = factor * exp2_table(ec, zh, zl);
   }
 }
 
@@ -233,10 +234,10 @@ __device__ __forceinline__ void build_pow_table(PowTable& t, const ExpConst& ec,
 __device__ __forceinline__ double pow_table(const PowTable& t, const PowPoly& q, double x) {
   const uint32_t hi = (uint32_t)(__builtin_bit_cast(uint64_t, x) >> 32);
   const double m = __builtin_amdgcn_frexp_mant(x);
-  // byte offsets: 16 (hi >> 12 & 255) and 8 (hi >> 20 & 127), a shift right and an and
+  // byte offsets: 16 (hi >> 12 & 255) and 8 (hi >> 20 & 255), a shift right and an and
   // each (2 cycles apiece; a shift left takes 4)
   const double2 c = *(const double2*)((const char*)t.c + ((hi >> 8) & 0xff0u));
-  const double s = *(const double*)((const char*)t.scale + ((hi >> 17) & 0x3f8u));
+  const double s = *(const double*)((const char*)t.scale + ((hi >> 17) & 0x7f8u));
   const double r = fma(m, c.x, -1.0);
   double y = fma(r, q.b5, q.b4);
   y = fma(y, r, q.b3);
@@ -248,11 +249,10 @@ __device__ __forceinline__ double pow_table(const PowTable& t, const PowPoly& q,
 }
 
 // Exponent ranges: squared radii from 2^-101 (below which a position's own rounding,
-// 1e-16 AU, leaves nothing of it) to 2^27 (radii to 11 000 AU; the host sends blocks with
-// larger cut-off spheres to the general kernel), and the cloud's g from 2^-128 to 1.
+// 1e-16 AU, leaves nothing of it) to 2^155, and the cloud's g from 2^-254 to 2^2; the host
+// sends blocks that can leave them to the general kernel (zodi_line_domain.hpp).
 constexpr int kPowRadiusFirst = -100;
-constexpr int kPowUnitFirst = -126;
-constexpr double kPowMaxRadius = 2048.0;
+constexpr int kPowUnitFirst = -253;
 
 // ---------------------------------------------------------------- Planck table
 // In LDS, shifted by one entry: entry 0 is (B_0, 0), entry i (T_{i-1}'s interval) is
@@ -359,22 +359,6 @@ __device__ __forceinline__ LineCtx line_ctx(ModelPtr M, LineTables& tab, int sub
   return cx;
 }
 
-// Whether a block that meets a layout's registry properties (props_match) may take the
-// line kernels: one temperature law for all groups, the three exponents and the cut-off
-// radii inside the power tables' ranges, and the cloud's exponent inside exp_node's.
-// NaN parameters fail every test and take the general kernel.
-inline bool line_match(const zodi_model* m) {
-  const auto in = [](double v, double lo, double hi) { return v >= lo && v <= hi; };
-  for (int g = 0; g < m->n_groups; ++g) {
-    if (m->group_T0[g] != m->group_T0[0] || m->group_delta[g] != m->group_delta[0]) return false;
-    if (!in(m->group_r_in[g], 0.0, kPowMaxRadius) || !in(m->group_r_out[g], 0.0, kPowMaxRadius))
-      return false;
-  }
-  const double* P = m->comp[0];
-  return in(m->group_delta[0], -12.0, 2.0) && in(P[7], -12.0, 2.0) && in(P[9], 0.5, 6.0) &&
-         in(P[8], -1e6, 1e6);
-}
-
 // ---------------------------------------------------------------- densities
 // The reference's densities (see zodi_device.hpp for each expression's source) on the
 // line's linear forms; LineComp<KIND> holds a component's constants for one ray.
@@ -432,8 +416,8 @@ __device__ __forceinline__ double line_cloud(ParamPtr P, const LineComp<ZODI_CLO
   // selection (two vcc-masked moves in a row stall the SIMD for about 20 cycles)
   const double m = fmin(zeta, mu);
   const double g = fma(m * m, inv_2mu, zeta - m);
-  // the floor changes nothing: with gamma >= 1/2 both powers are below 2^-63
-  const double gg = pow_table(cx.tab->vertical, cx.pv, fmax(g, 0x1p-127));
+  // the floor changes nothing: with gamma >= 1/2 both powers are below 2^-126
+  const double gg = pow_table(cx.tab->vertical, cx.pv, fmax(g, 0x1p-253));
   return pow_table(cx.tab->radial, cx.pr, r2) * exp_neg_node(cx.ec, P[8] * gg);
 }
 
