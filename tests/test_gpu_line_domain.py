@@ -109,3 +109,17 @@ def test_pointing_lengths(gpu, name, x, length):
     up to 2.2e3 per AU where its density is not yet 0."""
     v = healpix.pix2vec(4) * np.array([[length], [length], [1.0]])
     forward_agrees(Model(x, name=name), v, rtol=RTOL + 7e-13 * length)
+
+
+@pytest.mark.parametrize("mu", [0.0, 5e-324, 1e-300, 1e-14])
+@pytest.mark.parametrize("x", [25 * u.micron, 1.25 * u.micron])
+def test_cloud_without_a_rounded_middle(gpu, mu, x):
+    """mu = 0 (and 1/(2 mu) infinite): g is zeta itself, the reference's second case."""
+    model = changed("dirbe", {"cloud": {"mu": np.float64(mu)}}, x)
+    v = healpix.pix2vec(4)
+    got = forward_agrees(model, v)
+    gradients_agree(model, v)
+    # next to mu = 0 the emission is that of a small mu to about beta mu/2
+    near = changed("dirbe", {"cloud": {"mu": 1e-9}}, x)
+    want = near.device_model.forward(v, OBS, OBS, out_mode=OUT_COMPS).cpu().numpy()
+    same(got, want, rtol=1e-8)

@@ -81,6 +81,9 @@ def test_registry_models_take_the_line(takes, name):
     ({"mu": 3.0, "beta": 1e6, "gamma": 6.0}, True, True), ({"beta": 1.1e6}, False, False),
     ({"x_0": 2.0**60}, True, True), ({"z_0": -(2.0**60)}, True, True),
     ({"x_0": 2.0**60 * 1.01}, False, False), ({"y_0": -(2.0**61)}, False, False),
+    ({"mu": np.float64(0)}, False, False), ({"mu": np.float64(-0.0)}, False, False),
+    ({"mu": np.float64(5e-324)}, False, False), ({"mu": 1e-300}, False, False),
+    ({"mu": 1e-12}, True, True), ({"mu": -1e-12}, True, True),
     ({"alpha": 2.0}, True, True), ({"alpha": 2.1}, False, True),
 ])
 def test_cloud_ranges(takes, cloud, forward, adjoint):

@@ -19,13 +19,18 @@ constexpr double kLineMaxRadius = 0x1p60;
 constexpr double kLineMinMu = -4.0;
 constexpr double kLineMaxExponent = 5e6;  // beta g^gamma (exp_neg_node)
 
+// Of 1/(2 mu): g is formed as m^2/(2 mu) + (zeta - m), m = min(zeta, mu), which is NaN where
+// 1/(2 mu) is infinite (mu = 0), and the partial with respect to mu squares it.
+constexpr double kLineMaxInverse = 1e15;
+
 // The cloud's centre and fall-off (component 0 of the Kelsall layouts).
 inline bool line_cloud_match(const zodi_model* m) {
   const double* P = m->comp[0];
   for (int q = ZODI_P_X0; q <= ZODI_P_Z0; ++q)
     if (!within(P[q], -kLineMaxRadius, kLineMaxRadius)) return false;
   const double beta = P[8], gamma = P[9], mu = P[10];
-  return mu >= kLineMinMu && within(beta, -1e6, 1e6) &&
+  return mu >= kLineMinMu && within(P[13], -kLineMaxInverse, kLineMaxInverse) &&
+         within(beta, -1e6, 1e6) &&
          (mu > 0.0 || std::fabs(beta) * std::pow(1.0 - 0.5 * mu, gamma) <= kLineMaxExponent);
 }
 
