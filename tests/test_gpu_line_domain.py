@@ -123,3 +123,50 @@ def test_cloud_without_a_rounded_middle(gpu, mu, x):
     near = changed("dirbe", {"cloud": {"mu": 1e-9}}, x)
     want = near.device_model.forward(v, OBS, OBS, out_mode=OUT_COMPS).cpu().numpy()
     same(got, want, rtol=1e-8)
+
+
+BAD = [("dirbe", "cloud", f, v) for f, v in
+       [("i", np.nan), ("Omega", np.nan), ("mu", np.nan), ("n_0", np.nan), ("beta", np.nan)]]
+BAD += [("dirbe", "band1", f, v) for f, v in
+        [("i", np.nan), ("delta_r", np.nan), ("v", np.nan), ("n_0", np.nan), ("n_0", np.inf),
+         ("delta_zeta", np.nan), ("delta_r", np.inf)]]
+BAD += [("dirbe", "ring", "i", np.nan), ("dirbe", "ring", "sigma_z", 1e-100),
+        ("dirbe", "feature", "theta", np.nan), ("dirbe", "feature", "sigma_theta", 1e-60)]
+BAD += [("rrm-experimental", c, f, np.nan) for c, f in
+        [("fan", "i"), ("fan", "Omega"), ("fan", "P"), ("fan", "Z_0"), ("fan", "Q"),
+         ("fan", "gamma"), ("comet", "i"), ("comet", "amp"), ("inner_narrow_band", "i"),
+         ("inner_narrow_band", "G"), ("broad_band", "i"), ("broad_band", "Omega"),
+         ("interstellar", "amp"), ("ring_rrm", "i")]]
+BAD += [("rrm-experimental", "broad_band", "sigma_bb", 1e-100),
+        ("rrm-experimental", "broad_band", "R_outer", np.inf),
+        ("rrm-experimental", "fan", "R_outer", np.inf)]
+
+
+@pytest.mark.parametrize("name,comp,field,value", BAD)
+def test_non_finite_parameters(gpu, name, comp, field, value):
+    """NaN, infinite and extreme parameters: NaN where the kind switch gives it, and a chi^2
+    and gradients that are NaN wherever the emission is."""
+    v = healpix.pix2vec(4)
+    model = changed(name, {comp: {field: value}})
+    got = forward_agrees(model, v)
+    chi2_grad = gradients_agree(model, v)
+    if np.isnan(got).any():
+        assert np.isnan(chi2_grad[-1])
+
+
+@pytest.mark.parametrize("name,law", [("dirbe", "delta"), ("dirbe", "T_0"),
+                                      ("planck18", "delta"), ("planck18", "T_0")])
+def test_nan_temperature_law(gpu, name, law):
+    x = 857 * u.GHz if name == "planck18" else 25 * u.micron
+    v = healpix.pix2vec(4)
+    model = changed(name, {law: np.nan}, x)
+    dm = model.device_model
+    assert np.isnan(dm.forward(v, OBS, OBS, out_mode=OUT_COMPS).cpu().numpy()).all()
+    prob = LineOfSightProblem(model, v, OBS, OBS)
+    data = torch.full((v.shape[1],), 0.7, dtype=torch.float64, device="cuda")
+    assert np.isnan(float(prob.chi2_and_grad(prob.space.theta0, data)[0]))
+
+
+def test_infinite_temperature(gpu):
+    """Past the Planck table its last value is taken."""
+    forward_agrees(changed("dirbe", {"T_0": np.inf}), healpix.pix2vec(4))

@@ -90,3 +90,32 @@ def test_cloud_ranges(takes, cloud, forward, adjoint):
     assert takes(changed("dirbe", {"cloud": cloud})) == (forward, adjoint)
     x = 857 * u.GHz
     assert takes(changed("planck18", {"cloud": cloud}, x)) == (forward, adjoint)
+
+
+NOT_FINITE = [np.nan, np.inf, -np.inf, 1e18]  # (angles are packed in radians)
+
+
+@pytest.mark.parametrize("value", NOT_FINITE)
+@pytest.mark.parametrize("name", ["dirbe", "planck18", "rrm-experimental"])
+def test_non_finite_parameters(takes, name, value):
+    """Every parameter of every component, one at a time (derived constants follow them)."""
+    x = 857 * u.GHz if name == "planck18" else 25 * u.micron
+    model = Model(x, name=name)
+    for label, comp in model.get_parameters()["comps"].items():
+        for field in comp:
+            if field in ("i", "Omega", "theta") and abs(value) == 1e18:
+                continue  # an angle: its sine and cosine are finite
+            if field in ("x_0", "y_0", "z_0") and abs(value) == 1e18:
+                continue  # offsets: test_cloud_ranges
+            if np.isinf(value) and field in ("i", "Omega", "theta"):
+                continue  # the angle is refused before it is packed, or its sine is NaN
+            got = takes(changed(name, {label: {field: np.float64(value)}}, x))
+            assert got == (False, False), (label, field)
+
+
+@pytest.mark.parametrize("value,ok", [(np.nan, True), (np.inf, False), (-np.inf, False),
+                                      (12.1, False), (-12.1, False)])
+def test_temperature_law(takes, value, ok):
+    """A NaN exponent makes every temperature NaN by itself; larger ones overflow."""
+    assert takes(changed("dirbe", {"delta": value})) == (ok, ok)
+    assert takes(changed("planck18", {"delta": value}, 857 * u.GHz)) == (ok, ok)

@@ -455,9 +455,7 @@ FwdKernel pick_line(const zodi_model* m, int block, int L) {
 // flags.
 template <class LAYOUT>
 bool line_eligible(const zodi_model* m) {
-  constexpr bool kKelsall = layout_integrand<LAYOUT>() == ZODI_INTEGRAND_KELSALL;
-  return props_match(m, props_without_share(RegistryProps<LAYOUT>::value)) &&
-         (!kKelsall || line_match(m));
+  return props_match(m, props_without_share(RegistryProps<LAYOUT>::value)) && line_match(m);
 }
 
 bool takes_line(const zodi_model* m, LayoutId id) {

@@ -660,8 +660,7 @@ TableKernel pick_table_line(bool noscat) {
 template <class LAYOUT, bool EFF>
 TableKernel pick_table_layout(const zodi_model* m, int split) {
   constexpr uint32_t kProps = RegistryProps<LAYOUT>::value;
-  constexpr bool kKelsall = layout_integrand<LAYOUT>() == ZODI_INTEGRAND_KELSALL;
-  if (props_match(m, props_without_share(kProps)) && (!kKelsall || line_match(m))) {
+  if (props_match(m, props_without_share(kProps)) && line_match(m)) {
     const bool noscat = block_noscat(m);
     if constexpr (kProps != props_without_share(kProps)) {
       if (props_match(m, kProps)) return pick_table_line<LAYOUT, true, EFF>(noscat);
