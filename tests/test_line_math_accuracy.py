@@ -1,0 +1,122 @@
+"""Accuracy of the line kernels' elementary functions (zodipy_amd/csrc/zodi_line_math.hpp).
+
+The header compiles for the host with g++: the same operation sequences and the same tables
+(-ffp-contract=off keeps the host from fusing more than the device source asks for).
+Errors are measured against mpmath, relative ones of the exact value in units of 2^-53 of
+it (an ulp is one to two such units).
+"""
+
+from __future__ import annotations
+
+import ctypes as ct
+import shutil
+import subprocess
+from pathlib import Path
+
+import mpmath
+import numpy as np
+import pytest
+
+CSRC = Path(__file__).resolve().parents[1] / "zodipy_amd" / "csrc"
+
+HARNESS = r"""
+#include "zodi_line_math.hpp"
+using namespace zodi;
+extern "C" void eval(int which, const double* x, double* out, long n) {
+  const ExpConst e = exp_const();
+  for (long i = 0; i < n; ++i) {
+    switch (which) {
+      case 0: out[i] = exp_neg_node(e, x[i]); break;
+      case 2: out[i] = exp_neg_cut(e, x[i]); break;
+      default: out[i] = exp_neg_any(e, x[i]); break;
+    }
+  }
+}
+"""
+
+P = ct.POINTER(ct.c_double)
+EPS = 2.0**-53
+
+
+@pytest.fixture(scope="module")
+def lib(tmp_path_factory):
+    cxx = shutil.which("g++")
+    if cxx is None:
+        pytest.skip("g++ not available")
+    d = tmp_path_factory.mktemp("line_math")
+    (d / "harness.cpp").write_text(HARNESS)
+    subprocess.run([cxx, "-O2", "-ffp-contract=off", "-std=c++17", "-shared", "-fPIC",
+                    f"-I{CSRC}", str(d / "harness.cpp"), "-o", str(d / "lib.so")], check=True)
+    return ct.CDLL(str(d / "lib.so"))
+
+
+def rows(*arrays):
+    return [np.ascontiguousarray(a, dtype=np.float64) for a in np.broadcast_arrays(*arrays)]
+
+
+def ptr(a):
+    return a.ctypes.data_as(P)
+
+
+@pytest.fixture(scope="module")
+def fn(lib):
+    def f(which, x):
+        (x,) = rows(x)
+        out = np.empty_like(x)
+        lib.eval(which, ptr(x), ptr(out), ct.c_long(x.size))
+        return out
+
+    return f
+
+
+def relative(got, exact):
+    """|got - exact| / (2^-53 |exact|) for mpmath values, above the subnormal range."""
+    return np.array([float(abs((mpmath.mpf(g) - e) / e)) for g, e in zip(got, exact)]) / EPS
+
+
+@pytest.fixture(autouse=True)
+def precision():
+    mpmath.mp.prec = 160
+
+
+@pytest.mark.parametrize("which", [0, 1])
+@pytest.mark.parametrize("lo,hi", [(-5.0, 0.0), (0.0, 1.0), (1.0, 10.0), (10.0, 40.0),
+                                   (40.0, 200.0), (200.0, 700.0)])
+def test_exp(fn, which, lo, hi):
+    """Within 2^-53 (1 + 1.3) of the exact value: the table entry and the result are
+    rounded (half an ulp, at most 2^-53 each) and the series leaves out 3.8e-17 (0.34);
+    the argument's reduction adds nothing that grows with it."""
+    x = np.random.default_rng(int(lo + 10) + which).uniform(lo, hi, 4000)
+    err = relative(fn(which, x), [mpmath.exp(-mpmath.mpf(v)) for v in x])
+    assert err.max() <= 2.4, err.max()
+    assert err.mean() <= 0.8, err.mean()
+
+
+def test_exp_small_arguments(fn):
+    """1 - exp(-x), the bands' radial cut-off, keeps its digits: exp is correctly rounded
+    next to 1."""
+    s = np.concatenate([10.0 ** np.linspace(-12, -3.2, 50), [1e-300, 5e-324, 0.0]])
+    for sign in (-1.0, 1.0):
+        exact = np.array([float(mpmath.exp(-mpmath.mpf(sign * v))) for v in s])
+        np.testing.assert_array_equal(fn(0, sign * s), exact)
+        np.testing.assert_array_equal(fn(1, sign * s), exact)
+        np.testing.assert_array_equal(fn(2, sign * s), exact)
+
+
+def test_exp_of_the_cut_off(fn):
+    """1 - exp(-x) and x exp(-x) to a rounding of 1 and of the largest x exp(-x)."""
+    x = np.random.default_rng(5).uniform(0.0, 38.0, 6000)
+    got = fn(2, x)
+    exact = [mpmath.exp(-mpmath.mpf(v)) for v in x]
+    err = np.array([float(abs(mpmath.mpf(g) - e)) for g, e in zip(got, exact)])
+    own = np.array([float(e) for e in exact]) * 2.4 * EPS  # exp's own (test_exp)
+    assert np.all(err <= own + 6e-18) and np.all(x * err <= x * own + 8e-18)
+
+
+def test_exp_ends(fn):
+    x = np.array([746.0, 800.0, 5e6, np.nan, -710.0])
+    for which in (0, 1):
+        got = fn(which, x)
+        assert np.all(got[:3] == 0.0) and np.isnan(got[3]) and np.isinf(got[4])
+    # the exponent's integer saturates on the device; below 2^31 it does on the host too
+    assert fn(1, np.array([5.7e6]))[0] == 0.0

@@ -31,6 +31,7 @@ HEADERS = [
     CSRC / "zodi_line.hpp",
     CSRC / "zodi_line_adjoint.hpp",
     CSRC / "zodi_line_domain.hpp",
+    CSRC / "zodi_line_math.hpp",
     CSRC / "zodi_line_rrm.hpp",
     CSRC / "zodi_math.hpp",
     CSRC / "zodi_trig.hpp",

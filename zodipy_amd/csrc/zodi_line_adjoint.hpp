@@ -24,34 +24,6 @@
 
 namespace zodi {
 
-// ---------------------------------------------------------------- log
-// log x for positive normal x from a table of (inv_j, -log inv_j) (kLineInv) and the
-// Taylor series of log(1 + r) to r^5, |r| < 2^-8.9 (first term left out 1.4e-17).
-struct LogConst {
-  double c4;           // vector register: -1/4
-  double c5, c3, ln2;  // scalar registers
-};
-
-__device__ __forceinline__ LogConst log_const() {
-  LogConst l = {-0.25, 0.2, 1.0 / 3.0, 0x1.62e42fefa39efp-1};
-  asm volatile("" : "+v"(l.c4));
-  asm volatile("" : "+s"(l.c5), "+s"(l.c3), "+s"(l.ln2));
-  return l;
-}
-
-__device__ __forceinline__ double log_node(const double2* tab, const LogConst& l, double x) {
-  const uint32_t hi = (uint32_t)(__builtin_bit_cast(uint64_t, x) >> 32);
-  const double m = __builtin_amdgcn_frexp_mant(x);
-  const double de = (double)__builtin_amdgcn_frexp_exp(x);
-  const double2 c = *(const double2*)((const char*)tab + ((hi >> 8) & 0xff0u));
-  const double r = fma(m, c.x, -1.0);
-  double p = fma(r, l.c5, l.c4);
-  p = fma(p, r, l.c3);
-  p = fma(p, r, -0.5);
-  const double l1p = fma(p * r, r, r);
-  return fma(de, l.ln2, c.y + l1p);
-}
-
 // ---------------------------------------------------------------- per-block tables
 struct LineAdjTables {
   double2 log_tab[256];
@@ -87,7 +59,7 @@ __device__ __forceinline__ LineAdjCtx line_adj_ctx(ModelPtr M, LineAdjTables& ta
   for (int j = threadIdx.x; j < 256; j += blockDim.x)
     tab.log_tab[j] = double2{kLineInv[j], kLineLog[j]};
   load_planck(M, tab.planck, threadIdx.x, blockDim.x);
-  if (angles != nullptr) load_angles(*angles);
+  if (angles != nullptr) load_angles(*angles, threadIdx.x, blockDim.x);
   __syncthreads();
   LineAdjCtx cx;
   cx.M = M;
@@ -195,7 +167,7 @@ struct LineGrad<ZODI_BAND> {
       const double y4 = y2 * y2;
       cs.x = (y4 * y4) * y2;
       cs.ex = 0.0;
-      if (cs.x < 38.0) cs.ex = exp_neg_node(cx.ec, cs.x);
+      if (cs.x < 38.0) cs.ex = exp_neg_cut(cx.ec, cs.x);
     }
     const double zq = c.z.at(nd.t) * nd.inv_R;  // signed
     const double zd2 = zq * zq;

@@ -17,23 +17,6 @@
 
 namespace zodi {
 
-// asin(s) for 0 <= s <= 1 (the reduction of acos_fast). The half above 1/2 costs a
-// square root and is entered only by the waves that have such a point.
-__device__ __forceinline__ double asin_unit(double s) {
-  constexpr double kQ[] = {ZODI_ASIN_POLY};
-  double w = s, z = s * s, up = 0.0;
-  if (s > 0.5) {
-    z = fma(-0.5, s, 0.5);
-    double inv;
-    norm_and_inverse(z, w, inv);
-    w = z == 0.0 ? 0.0 : w;
-    up = 1.0;
-  }
-  const double v = fma(w * z, zodi_trig::horner(kQ, z), w);
-  // pi/2 - 2 asin(sqrt((1 - s)/2)) above 1/2
-  return fma(up, zodi_trig::kPiHalfHi, fma(up, -3.0 * v, v));
-}
-
 // sin(beta) of a point, its size capped at 1 (1/R carries an error of 5e-15).
 __device__ __forceinline__ double line_sin_beta(const Linear& z, const GradNode& nd, double& zc) {
   zc = z.at(nd.t);
