@@ -24,10 +24,14 @@ HARNESS = r"""
 using namespace zodi;
 extern "C" void eval(int which, const double* x, double* out, long n) {
   const ExpConst e = exp_const();
+  const LogConst l = log_const();
+  static double2 log_tab[256];
+  for (int j = 0; j < 256; ++j) log_tab[j] = double2{kLineInv[j], kLineLog[j]};
   for (long i = 0; i < n; ++i) {
     switch (which) {
       case 0: out[i] = exp_neg_node(e, x[i]); break;
       case 2: out[i] = exp_neg_cut(e, x[i]); break;
+      case 3: out[i] = log_node(log_tab, l, x[i]); break;
       default: out[i] = exp_neg_any(e, x[i]); break;
     }
   }
@@ -120,3 +124,21 @@ def test_exp_ends(fn):
         assert np.all(got[:3] == 0.0) and np.isnan(got[3]) and np.isinf(got[4])
     # the exponent's integer saturates on the device; below 2^31 it does on the host too
     assert fn(1, np.array([5.7e6]))[0] == 0.0
+
+
+@pytest.mark.parametrize("lo,hi", [(-1.0, 1.0), (-20.0, 10.0), (-100.0, 155.0), (-900.0, 900.0)])
+def test_log(fn, lo, hi):
+    """Half an ulp of the result, two roundings of values below 1 (the table entry and the
+    sum of it and log(1 + r), 2^-54 each) and 1.4e-17 left out of the series."""
+    rng = np.random.default_rng(int(hi))
+    x = 2.0 ** rng.uniform(lo, hi, 6000)
+    got = fn(3, x)
+    err = np.array([float(abs(mpmath.mpf(g) - mpmath.log(mpmath.mpf(v)))) for g, v in zip(got, x)])
+    bound = 0.5 * np.spacing(np.abs(got)) + 2 * 2.0**-54 + 2e-17
+    assert np.all(err <= bound), (err - bound).max()
+
+
+def test_log_special_values(fn):
+    got = fn(3, np.array([np.nan, 2.0, 2.0**-1000]))
+    assert np.isnan(got[0]) and abs(got[1] - np.log(2.0)) <= 2.0**-53
+    assert abs(got[2] + 1000 * np.log(2.0)) <= np.spacing(1000 * np.log(2.0))

@@ -245,17 +245,18 @@ ZODI_MATH_FN double pow_table(const PowTable& t, const PowPoly& q, double x) {
 
 // ---------------------------------------------------------------- log
 // log x for positive normal x from a table of (inv_j, -log inv_j) (kLineInv) and the
-// Taylor series of log(1 + r) to r^5, |r| < 2^-8.9 (first term left out 1.4e-17).
+// Taylor series of log(1 + r) to r^5, |r| < 2^-8.9 (first term left out 1.4e-17); e ln2 with
+// both words of ln2 (with one the error is 2.3e-17 |e| more).
 struct LogConst {
-  double c4;           // vector register: -1/4
-  double c5, c3, ln2;  // scalar registers
+  double c4;                   // vector register: -1/4
+  double c5, c3, ln2, ln2_lo;  // scalar registers
 };
 
 ZODI_MATH_FN LogConst log_const() {
-  LogConst l = {-0.25, 0.2, 1.0 / 3.0, 0x1.62e42fefa39efp-1};
+  LogConst l = {-0.25, 0.2, 1.0 / 3.0, 0x1.62e42fefa39efp-1, 0x1.abc9e3b39803fp-56};
 #if defined(__HIP_DEVICE_COMPILE__)
   asm volatile("" : "+v"(l.c4));
-  asm volatile("" : "+s"(l.c5), "+s"(l.c3), "+s"(l.ln2));
+  asm volatile("" : "+s"(l.c5), "+s"(l.c3), "+s"(l.ln2), "+s"(l.ln2_lo));
 #endif
   return l;
 }
@@ -270,7 +271,7 @@ ZODI_MATH_FN double log_node(const double2* tab, const LogConst& l, double x) {
   p = fma(p, r, l.c3);
   p = fma(p, r, -0.5);
   const double l1p = fma(p * r, r, r);
-  return fma(de, l.ln2, c.y + l1p);
+  return fma(de, l.ln2, c.y + fma(de, l.ln2_lo, l1p));
 }
 
 // ---------------------------------------------------------------- angles
