@@ -32,9 +32,16 @@ extern "C" void eval(int which, const double* x, double* out, long n) {
       case 0: out[i] = exp_neg_node(e, x[i]); break;
       case 2: out[i] = exp_neg_cut(e, x[i]); break;
       case 3: out[i] = log_node(log_tab, l, x[i]); break;
+      case 4: out[i] = asin_unit(x[i]); break;
       default: out[i] = exp_neg_any(e, x[i]); break;
     }
   }
+}
+extern "C" void angle(int which, const double* x, const double* y, double* out, long n) {
+  static AngleTable tab;
+  load_angles(tab, 0, 1);
+  for (long i = 0; i < n; ++i)
+    out[i] = which == 0 ? unit_angle(tab, x[i], y[i]) : axis_angle(x[i], y[i]);
 }
 """
 
@@ -68,6 +75,17 @@ def fn(lib):
         (x,) = rows(x)
         out = np.empty_like(x)
         lib.eval(which, ptr(x), ptr(out), ct.c_long(x.size))
+        return out
+
+    return f
+
+
+@pytest.fixture(scope="module")
+def angle(lib):
+    def f(which, x, y):
+        x, y = rows(x, y)
+        out = np.empty_like(x)
+        lib.angle(which, ptr(x), ptr(y), ptr(out), ct.c_long(x.size))
         return out
 
     return f
@@ -142,3 +160,68 @@ def test_log_special_values(fn):
     got = fn(3, np.array([np.nan, 2.0, 2.0**-1000]))
     assert np.isnan(got[0]) and abs(got[1] - np.log(2.0)) <= 2.0**-53
     assert abs(got[2] + 1000 * np.log(2.0)) <= np.spacing(1000 * np.log(2.0))
+
+
+def exact_angle(x, y):
+    return [mpmath.atan2(mpmath.mpf(b), mpmath.mpf(a)) for a, b in zip(x, y)]
+
+
+def directions(seed):
+    """Angles over [0, pi], next to both ends, to pi/2 and to the middles between entries."""
+    rng = np.random.default_rng(seed)
+    th = np.concatenate([rng.uniform(0, np.pi, 4000), 10.0 ** rng.uniform(-12, 0, 500),
+                         np.pi - 10.0 ** rng.uniform(-12, 0, 500),
+                         np.arange(1, 256) * (np.pi / 256), [0.0, np.pi / 2]])
+    return np.cos(th), np.sin(th)
+
+
+def test_unit_angle(angle):
+    """Half an ulp of the angle and the turn's: the direction's two roundings (2^-54 each,
+    times c and s), that of the product c sin (2^-54) and of the difference (below 2^-60);
+    next to 0 the relative error of s."""
+    c, s = directions(1)
+    got = angle(0, c, s)
+    exact = exact_angle(c, s)
+    err = np.array([float(abs(mpmath.mpf(g) - e)) for g, e in zip(got, exact)])
+    bound = 0.5 * np.spacing(got) + (np.sqrt(2.0) + 1.0) * 2.0**-54 + 2.0**-59
+    assert np.all(err <= bound), (err - bound).max()
+    small = got < 0.012
+    assert small.sum() > 300
+    assert relative(got[small & (s > 0)], [e for e, k in zip(exact, small & (s > 0)) if k]
+                    ).max() <= 4.0
+
+
+def test_unit_angle_ends(angle):
+    got = angle(0, np.array([1.0, 0.0, -1.0, np.nan, 0.5]), np.array([0.0, 1.0, 0.0, 0.5, np.nan]))
+    assert got[0] == 0.0 and abs(got[1] - np.pi / 2) <= 2.3e-16 and abs(got[2] - np.pi) <= 4.5e-16
+    assert np.isnan(got[3:]).all()
+
+
+def test_axis_angle(angle):
+    """As atan2_fast (2 ulp) over vectors of any length."""
+    rng = np.random.default_rng(2)
+    c, s = directions(3)
+    r = 10.0 ** rng.uniform(-6, 3, c.size)
+    x, y = c * r, s * r
+    got = angle(1, x, y)
+    exact = exact_angle(x, y)
+    nonzero = np.array([e != 0 for e in exact])
+    ulp = np.spacing(np.abs(got))
+    err = np.array([float(abs(mpmath.mpf(g) - e)) for g, e in zip(got, exact)])
+    assert np.all(err[nonzero] <= 2.0 * ulp[nonzero]), (err / ulp)[nonzero].max()
+    assert np.all(got[~nonzero] == 0.0)
+    # the reflections round to the double nearest pi/2 and pi
+    np.testing.assert_array_equal(angle(1, [0.0, -1.0, 1.0], [1.0, 0.0, 1.0]),
+                                  [np.pi / 2, np.pi, np.pi / 4])
+
+
+def test_asin(fn):
+    rng = np.random.default_rng(4)
+    x = np.concatenate([rng.uniform(0, 1, 3000), 10.0 ** rng.uniform(-15, 0, 500),
+                        1 - 10.0 ** rng.uniform(-16, 0, 500), [0.5, np.nextafter(0.5, 1), 1.0]])
+    got = fn(4, x)
+    exact = [mpmath.asin(mpmath.mpf(v)) for v in x]
+    ulp = np.array([float(abs(mpmath.mpf(g) - e)) for g, e in zip(got, exact)]) / np.spacing(got)
+    assert ulp.max() <= 2.0, ulp.max()
+    assert fn(4, np.array([0.0]))[0] == 0.0 and fn(4, np.array([1.0]))[0] == np.pi / 2
+    assert np.isnan(fn(4, np.array([np.nan]))[0])

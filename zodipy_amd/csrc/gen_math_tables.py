@@ -5,10 +5,10 @@
 * LOG_INV[j] = 1/c_j and LOG_C[j] = log(c_j) with c_j = 1/2 + j/512,
   j = 0..255 (table-driven log, Tang 1990, ACM TOMS 16(4):378-400);
 * LINE_INV[j] = 1/(1/2 + (j + 1/2)/512) rounded to a multiple of 2^-12 and
-  LINE_LOG[j] = -log(LINE_INV[j]) (zodi_line.hpp: the product of a mantissa and a
+  LINE_LOG[j] = -log(LINE_INV[j]) (zodi_line_math.hpp: the product of a mantissa and a
   13-bit LINE_INV is exact inside an FMA).
-* LINE_ANGLE[2 j], LINE_ANGLE[2 j + 1] = cos, sin of the double j * (pi/128), j = 0..128
-  (zodi_line.hpp: unit_angle).
+* LINE_ANGLE[2 j], LINE_ANGLE[2 j + 1] = cos, sin of the exact product of j and the double
+  pi/128, j = 0..128 (zodi_line_math.hpp: unit_angle).
 
 Values are evaluated with mpmath at 200 bits and rounded to nearest double.
 Run ``python -m zodipy_amd.csrc.gen_math_tables`` to regenerate.
@@ -55,7 +55,7 @@ def main() -> None:
     lines += ["// -log of the same", "#define ZODI_LINE_LOG_TABLE \\"]
     lines += [f"  {_hex(-mpmath.log(v))}, \\" for v in short]
     lines[-1] = lines[-1].rstrip(" \\").rstrip(",")
-    angle = [f(mpmath.mpf(j * (math.pi / 128))) for j in range(129)
+    angle = [f(j * mpmath.mpf(math.pi / 128)) for j in range(129)
              for f in (mpmath.cos, mpmath.sin)]
     lines += ["// cos and sin of j pi/128", "#define ZODI_LINE_ANGLE_TABLE \\"]
     lines += [f"  {_hex(v)}, \\" for v in angle]

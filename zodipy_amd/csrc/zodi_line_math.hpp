@@ -276,11 +276,13 @@ ZODI_MATH_FN double log_node(const double2* tab, const LogConst& l, double x) {
 
 // ---------------------------------------------------------------- angles
 // Angle of the unit vector (c, s), s >= 0, from the x axis: turned by the nearest of 129
-// tabulated directions j pi/128, found from the arc cosine in single precision (within
-// 4e-4, Abramowitz and Stegun 4.4.45), its sine is below 0.0127 and the arc sine's series
-// ends at the seventh power (next term 1e-18): 11 FP64 operations and no quotient where
-// axis_angle takes some 35. An error that c and s share (of 1/|X|) only scales the small
-// turn. Near 0 the direction is (1, 0), so the angle keeps the digits of s.
+// tabulated directions j C, C the double nearest pi/128, found from the arc cosine in single
+// precision (within 4e-4, Abramowitz and Stegun 4.4.45), its sine is below 0.0127 and the arc
+// sine's series ends at the seventh power (next term 1e-18): 11 FP64 operations and no
+// quotient where axis_angle takes some 37. The table holds the directions of the exact
+// products j C, so that the last FMA is the angle's only rounding. An error that c and s
+// share (of 1/|X|) only scales the small turn. Near 0 the direction is (1, 0), so the angle
+// keeps the digits of s.
 struct AngleTable {
   double2 e[129];
 };
@@ -312,19 +314,21 @@ ZODI_MATH_FN double unit_angle(const AngleTable& t, double c, double s) {
 }
 
 // Angle of (x, y) from the x axis, in [0, pi]; the octant, half-angle and quadrant steps of
-// atan2_fast as multiplications by 0, 1 and -1 instead of selections.
+// atan2_fast as multiplications by 0, 1 and -1 instead of selections: the angle is
+// +-atan(t) + k pi/4 for an integer k, with both words of pi/4.
 ZODI_MATH_FN double axis_angle(double x, double y) {
   constexpr double kP[] = {ZODI_ATAN_POLY};
   const double m = fmax(fabs(x), fabs(y)), n = fmin(fabs(x), fabs(y));
   const double up = n > zodi_trig::kTanPi8 * m ? 1.0 : 0.0;
   const double t = zodi_trig::quotient(fma(-up, m, n), fma(up, n, m));
   const double s = t * t;
-  double a = fma(t * s, zodi_trig::horner(kP, s), t);
-  a = fma(up, zodi_trig::kPiQuarterHi, a);
+  const double a = fma(t * s, zodi_trig::horner(kP, s), t);
   const double sw = fabs(y) > fabs(x) ? -1.0 : 1.0;
-  a = fma(sw, a, fma(-sw, zodi_trig::kPiQuarterHi, zodi_trig::kPiQuarterHi));
   const double sx = __builtin_copysign(1.0, x);
-  return fma(sx, a, fma(-sx, zodi_trig::kPiHalfHi, zodi_trig::kPiHalfHi));
+  // sx (sw (a + up pi/4) + (1 - sw) pi/4) + (1 - sx) pi/2
+  const double k = fma(sx, fma(sw, up - 1.0, -1.0), 2.0);
+  const double r = fma(k, zodi_trig::kPiQuarterHi, (sx * sw) * a);
+  return fma(k, zodi_trig::kPiQuarterLo, r);
 }
 
 // asin(s) for 0 <= s <= 1 (the reduction of acos_fast). The half above 1/2 costs a
@@ -345,7 +349,8 @@ ZODI_MATH_FN double asin_unit(double s) {
   }
   const double v = fma(w * z, zodi_trig::horner(kQ, z), w);
   // pi/2 - 2 asin(sqrt((1 - s)/2)) above 1/2
-  return fma(up, zodi_trig::kPiHalfHi, fma(up, -3.0 * v, v));
+  const double r = fma(up, zodi_trig::kPiHalfHi, fma(-3.0 * up, v, v));
+  return fma(up, zodi_trig::kPiHalfLo, r);
 }
 
 }  // namespace zodi
