@@ -7,6 +7,8 @@
 * LINE_INV[j] = 1/(1/2 + (j + 1/2)/512) rounded to a multiple of 2^-12 and
   LINE_LOG[j] = -log(LINE_INV[j]) (zodi_line_math.hpp: the product of a mantissa and a
   13-bit LINE_INV is exact inside an FMA).
+* EXP2_LO[j] and LINE_LOG2[2 j], LINE_LOG2[2 j + 1]: what EXP2_TABLE[j] leaves out of
+  2^(j/256), and -log2(LINE_INV[j]) in two words (zodi_line_math.hpp: build_pow_table).
 * LINE_ANGLE[2 j], LINE_ANGLE[2 j + 1] = cos, sin of the exact product of j and the double
   pi/128, j = 0..128 (zodi_line_math.hpp: unit_angle).
 
@@ -54,6 +56,16 @@ def main() -> None:
     lines[-1] = lines[-1].rstrip(" \\").rstrip(",")
     lines += ["// -log of the same", "#define ZODI_LINE_LOG_TABLE \\"]
     lines += [f"  {_hex(-mpmath.log(v))}, \\" for v in short]
+    lines[-1] = lines[-1].rstrip(" \\").rstrip(",")
+    low = [v - mpmath.mpf(float(v)) for v in exp2]
+    lines += ["// 2^(j/256) less its entry above", "#define ZODI_EXP2_LO_TABLE \\"]
+    lines += [f"  {_hex(v)}, \\" for v in low]
+    lines[-1] = lines[-1].rstrip(" \\").rstrip(",")
+    log2 = [-mpmath.log(v, 2) for v in short]
+    pairs = [w for v in log2 for w in (float(v), float(v - mpmath.mpf(float(v))))]
+    lines += ["// -log2 of the 1/(1/2 + (j + 1/2)/512), two words each",
+              "#define ZODI_LINE_LOG2_TABLE \\"]
+    lines += [f"  {_hex(v)}, \\" for v in pairs]
     lines[-1] = lines[-1].rstrip(" \\").rstrip(",")
     angle = [f(j * mpmath.mpf(math.pi / 128)) for j in range(129)
              for f in (mpmath.cos, mpmath.sin)]

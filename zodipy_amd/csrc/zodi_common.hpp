@@ -705,7 +705,7 @@ __device__ __forceinline__ void line_group(Grp<Ks...>, std::integer_sequence<int
     nd.t = fma(th, Mk->gl_x[k], tm);
     nd.R2 = fma(nd.t, nd.t, l.d2);
     norm_and_inverse_node(nd.R2, nd.R, nd.inv_R);
-    const double B = planck_shifted(pow_table(cx.tab->temperature, cx.pt, nd.R2) - cx.uo1,
+    const double B = planck_shifted(pow_table_less(cx.tab->temperature, cx.pt, nd.R2, cx.uo1),
                                     cx.tab->planck);
     const double wB = wk * B;
     double ws = 0.0;  // w F Phi / R^2

@@ -36,6 +36,8 @@ __shared__ __attribute__((aligned(2048))) double g_exp2[256];
 __constant__ double kLineInv[256] = {ZODI_LINE_INV_TABLE};  // inv_j of PowTable
 __constant__ double kLineLog[256] = {ZODI_LINE_LOG_TABLE};  // -log inv_j
 __constant__ double kLineAngle[258] = {ZODI_LINE_ANGLE_TABLE};
+__constant__ double kExp2Lo[256] = {ZODI_EXP2_LO_TABLE};        // 2^(j/256) - g_exp2[j]
+__constant__ double kLineLog2[512] = {ZODI_LINE_LOG2_TABLE};    // -log2 inv_j, two words
 
 // Every thread of the block must call this before exp_neg_node.
 __device__ __forceinline__ void stage_line_tables() {
@@ -46,6 +48,8 @@ __device__ __forceinline__ void stage_line_tables() {
 inline constexpr double kLineInv[256] = {ZODI_LINE_INV_TABLE};
 inline constexpr double kLineLog[256] = {ZODI_LINE_LOG_TABLE};
 inline constexpr double kLineAngle[258] = {ZODI_LINE_ANGLE_TABLE};
+inline constexpr double kExp2Lo[256] = {ZODI_EXP2_LO_TABLE};
+inline constexpr double kLineLog2[512] = {ZODI_LINE_LOG2_TABLE};
 #endif
 
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -158,8 +162,9 @@ struct PowTable {
   double scale[256];
 };
 
-// Binomial coefficients of (1 + r)^p, r^1..r^5, in scalar registers but the fourth: |r| < 2^-8.9, the
-// first term left out is below 2^-53.4 |binom(p, 6)| < 5e-17 for -1 <= p <= 6.
+// Binomial coefficients of (1 + r)^p, r^1..r^5, in scalar registers but the fourth:
+// |r| < 2^-8.9, the first term left out is below 8.4e-17 |binom(p, 6)|, for -1 <= p <= 6 at
+// most 8.4e-17 (p = -1 and 6), 5e-18 for the temperature law of the registry.
 struct PowPoly {
   double b1, b2, b3, b4, b5;
 };
@@ -197,36 +202,48 @@ ZODI_MATH_FN PowPoly pow_poly(double p) {
 // inv_j (kLineInv): 2/(1 + (j + 1/2)/256) rounded to a multiple of 2^-12 (13 significant
 // bits), so its product with a 53-bit mantissa fits the FMA exactly and only r is rounded.
 
-// 2^z for the exact z = zh + zl, |zl| tiny.
-ZODI_MATH_FN double exp2_table(const ExpConst& ec, double zh, double zl) {
-  const double k = __builtin_rint(zh);
-  const double f = (zh - k) + zl;
-  constexpr double kLn2Hi = 0x1.62e42fefa39efp-1, kLn2Lo = 0x1.abc9e3b39803fp-56;
-  const double y = f * kLn2Hi;
-  const double yl = fma(f, kLn2Hi, -y) + f * kLn2Lo;
-  const double e = exp_neg_any(ec, -y);
-  return math_ldexp(fma(e, yl, e), (int)k);
+// factor 2^(zh + zl), |zl| tiny, rounded once: 2^(j/256) in two words, the series of
+// 2^(f/256) - 1 to f^5 (first term left out 9e-21), and the product with `factor` exact.
+ZODI_MATH_FN double exp2_scaled(const ExpConst& ec, double zh, double zl, double factor) {
+  const double kd = __builtin_rint(zh * 256.0);
+  const double f = fma(zh, 256.0, -kd) + zl * 256.0;
+  double q = fma(f, 0x1.5d87fe78a6731p-50, ec.c4);  // (ln2/256)^5/120
+  q = fma(q, f, ec.c3);
+  q = fma(q, f, ec.c2);
+  q = fma(q, f, ec.c1);
+  const int k = (int)kd, j = k & 255;
+  const double t = ZODI_LINE_EXP2[j];
+  const double low = fma(t, q * f, kExp2Lo[j]);
+  const double p = factor * t;
+  return math_ldexp(p + fma(factor, low, fma(factor, t, -p)), k >> 8);
 }
 
 // Entries i, i + stride, ... of the table of x^p, the whole multiplied by `factor`;
-// exponents from e_first on. stage_line_tables() must have run.
+// exponents from e_first on. Every entry is the exact value rounded once. Mean relative
+// errors of x^p, 1e-16, with entries of exp's accuracy -> these, and of exp(p log x):
+// temperature law (p = -0.233) 0.94 -> 0.81 and 0.64, cloud's radius (-0.67) 0.93 -> 0.77 and
+// 1.1, its g (0.942) 0.91 -> 0.81 and 1.7; of T/dT on the table's axis (pow_table_less, where
+// the last product is not rounded) the mean is 6.1e-15 and the largest 3.5e-14, where
+// exp(p log x) gives 5.7e-15 and 6.3e-14. stage_line_tables() must have run.
 ZODI_MATH_FN void build_pow_table(PowTable& t, const ExpConst& ec, double p, double factor,
                                   int e_first, int i, int stride) {
   for (int j = i; j < 256; j += stride) {
-    // inv^-p; -p log(inv) is below |p| 0.7, so its rounding stays below an ulp
-    t.c[j] = double2{kLineInv[j], exp_neg_any(ec, -(p * kLineLog[j]))};
+    const double lh = kLineLog2[2 * j], zh = p * lh;
+    const double zl = fma(p, lh, -zh) + p * kLineLog2[2 * j + 1];
+    t.c[j] = double2{kLineInv[j], exp2_scaled(ec, zh, zl, 1.0)};
   }
   for (int j = i; j < 256; j += stride) {
     const int e = e_first + j;
     const double zh = p * (double)e;
     const double zl = fma(p, (double)e, -zh);
     // frexp's exponent e: x = 2^e m, m in [1/2, 1); its biased exponent is e + 1022
-    t.scale[(e + 1022) & 255] = factor * exp2_table(ec, zh, zl);
+    t.scale[(e + 1022) & 255] = exp2_scaled(ec, zh, zl, factor);
   }
 }
 
-// factor x^p from the table, for x in the table's range (NaN passes).
-ZODI_MATH_FN double pow_table(const PowTable& t, const PowPoly& q, double x) {
+// inv_j^-p and factor 2^(p e) (1 + r)^p, whose product is factor x^p, for x in the table's
+// range (NaN passes).
+ZODI_MATH_FN double2 pow_factors(const PowTable& t, const PowPoly& q, double x) {
   const uint32_t hi = (uint32_t)(__builtin_bit_cast(uint64_t, x) >> 32);
   const double m = frexp_mant(x);
   // byte offsets: 16 (hi >> 12 & 255) and 8 (hi >> 20 & 255), a shift right and an and
@@ -239,8 +256,19 @@ ZODI_MATH_FN double pow_table(const PowTable& t, const PowPoly& q, double x) {
   y = fma(y, r, q.b2);
   y = fma(y, r, q.b1);
   y = y * r;
-  const double w = c.y * s;
-  return fma(w, y, w);
+  return double2{c.y, fma(s, y, s)};
+}
+
+// factor x^p
+ZODI_MATH_FN double pow_table(const PowTable& t, const PowPoly& q, double x) {
+  const double2 w = pow_factors(t, q, x);
+  return w.x * w.y;
+}
+
+// factor x^p - u, the product unrounded (the temperature on the Planck table's axis)
+ZODI_MATH_FN double pow_table_less(const PowTable& t, const PowPoly& q, double x, double u) {
+  const double2 w = pow_factors(t, q, x);
+  return fma(w.x, w.y, -u);
 }
 
 // ---------------------------------------------------------------- log

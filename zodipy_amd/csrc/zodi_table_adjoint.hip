@@ -345,7 +345,7 @@ __device__ __forceinline__ void line_table_group(Grp<Ks...>, std::integer_sequen
       nd.t = t;
       nd.R2 = fma(t, t, l.d2);
       norm_and_inverse_node(nd.R2, nd.R, nd.inv_R);
-      u1 = pow_table(cx.tab->temperature, cx.pt, nd.R2) - cx.uo1;
+      u1 = pow_table_less(cx.tab->temperature, cx.pt, nd.R2, cx.uo1);
     } else {
       const RrmNode o = rrm_node(cx, l, t, half_delta, us, uo1);
       nd = o.nd;
