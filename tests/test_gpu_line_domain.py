@@ -170,3 +170,31 @@ def test_nan_temperature_law(gpu, name, law):
 def test_infinite_temperature(gpu):
     """Past the Planck table its last value is taken."""
     forward_agrees(changed("dirbe", {"T_0": np.inf}), healpix.pix2vec(4))
+
+
+@pytest.mark.parametrize("values", [{"cloud": {"alpha": 2.5}}, {"cloud": {"alpha": -20.0}},
+                                    {"cloud": {"gamma": 9.0}}, {"delta": 5.0}, {"delta": -11.0},
+                                    {"cloud": {"alpha": 3.0}, "band1": {"delta_r": 1.4}}])
+@pytest.mark.parametrize("name,x", [("dirbe", 25 * u.micron), ("dirbe", 1.25 * u.micron),
+                                    ("planck18", 857 * u.GHz)])
+def test_exponents_outside_the_power_tables(gpu, name, x, values):
+    """Powers by logarithms, with and without the bands' shared cut-off."""
+    model = changed(name, values, x)
+    v = healpix.pix2vec(8)
+    forward_agrees(model, v)
+    gradients_agree(model, v)
+
+
+@pytest.mark.parametrize("rays", [1, 17, 3072, 49_153, 150_001, 250_007])
+@pytest.mark.parametrize("x", [25 * u.micron, 1.25 * u.micron])
+def test_split_outside_the_power_tables(gpu, x, rays):
+    """The same bits for every number of lanes per ray."""
+    model = changed("dirbe", {"cloud": {"alpha": 2.5}}, x)
+    rng = np.random.default_rng(rays)
+    v = rng.normal(size=(3, rays))
+    v /= np.linalg.norm(v, axis=0)
+    dm = model.device_model
+    one = dm.forward(v, OBS, OBS, out_mode=OUT_COMPS, launch=Launch(256, 1, 0, 1))
+    for launch in (None, Launch(256, 2, 0, 1), Launch(512, 4, 0, 1), Launch(512, 8, 0, 1),
+                   Launch(512, 1, 0, 1)):
+        assert torch.equal(dm.forward(v, OBS, OBS, out_mode=OUT_COMPS, launch=launch), one)

@@ -25,7 +25,7 @@ HARNESS = r"""
 #include "zodi_line_domain.hpp"
 extern "C" int takes(int which, const void* block) {
   const zodi_model* m = (const zodi_model*)block;
-  return which == 0 ? zodi::line_match(m) : zodi::line_adjoint_match(m);
+  return which == 0 ? zodi::line_match(m) : zodi::line_log_match(m);
 }
 """
 

@@ -222,7 +222,7 @@ AdjKernel pick_adj_split(int split, bool jac) {
 template <class LAYOUT>
 bool line_eligible(const zodi_model* m) {
   return props_match(m, props_without_share(RegistryProps<LAYOUT>::value)) &&
-         line_adjoint_match(m);
+         line_log_match(m);
 }
 
 bool takes_line(const zodi_model* m) {

@@ -564,9 +564,9 @@ __device__ __forceinline__ Ctx make_ctx(ModelPtr M, const double* sTab, int sub)
 
 
 // ---------------------------------------------------------- line kernels (Kelsall)
-template <int KIND, int CUT>
+template <int KIND, int CUT, class CTX>
 __device__ __forceinline__ double line_density(ParamPtr P, const LineComp<KIND>& c,
-                                               const LineCtx& cx, const Line& l,
+                                               const CTX& cx, const Line& l,
                                                const LineNode& nd, double& cut) {
   if constexpr (KIND == ZODI_CLOUD) return line_cloud(P, c, cx, nd);
   if constexpr (KIND == ZODI_BAND) return line_band<CUT>(P, c, cx, nd, cut);
@@ -675,9 +675,9 @@ struct LaneSums {
 // One group of a Kelsall registry layout for one ray: group_pass on the ray's line.
 // PROPS: only its kShareCut bits are read (every band is centred with p = 4, every other
 // component but the cloud centred; the host checks, props_match and line_match).
-template <int SPLIT, uint32_t PROPS, bool NOSCAT, int... Ks, int... J>
+template <int SPLIT, uint32_t PROPS, bool NOSCAT, class CTX, int... Ks, int... J>
 __device__ __forceinline__ void line_group(Grp<Ks...>, std::integer_sequence<int, J...>,
-                                           const LineCtx& cx, const FwdArgs& a, const Ray& y,
+                                           const CTX& cx, const FwdArgs& a, const Ray& y,
                                            const Line& l, int g, int first, double2* terms,
                                            double& total) {
   constexpr int C = sizeof...(Ks);
@@ -693,6 +693,7 @@ __device__ __forceinline__ void line_group(Grp<Ks...>, std::integer_sequence<int
   }
   LinePhase lp = {0.0, 0.0};
   if (scatter) lp = line_phase(l);
+  const LineLaw law = line_law(cx, g);
   const int lanes = SPLIT == 8 ? a.lanes : SPLIT;
   LaneSums<SPLIT, C> acc;
   for (int k0 = 0; k0 < cx.K; k0 += lanes) {
@@ -705,15 +706,14 @@ __device__ __forceinline__ void line_group(Grp<Ks...>, std::integer_sequence<int
     nd.t = fma(th, Mk->gl_x[k], tm);
     nd.R2 = fma(nd.t, nd.t, l.d2);
     norm_and_inverse_node(nd.R2, nd.R, nd.inv_R);
-    const double B = planck_shifted(pow_table_less(cx.tab->temperature, cx.pt, nd.R2, cx.uo1),
-                                    cx.tab->planck);
+    const double B = planck_shifted(line_axis(cx, law, nd.R2), cx.tab->planck);
     const double wB = wk * B;
     double ws = 0.0;  // w F Phi / R^2
     if constexpr (!NOSCAT) {
       if (scatter) {
         const ParamPtr S = Mk->shared;
         ws = wk * ((S[ZODI_S_SOLAR] * (nd.inv_R * nd.inv_R)) *
-                   line_phase_function(lp, l, cx.tab->angles, cx.ec, nd.t, nd.inv_R, S));
+                   line_phase_function(lp, l, line_angles(cx), cx.ec, nd.t, nd.inv_R, S));
       }
     }
     double cut = 0.0;  // a band's cut-off, for the bands that share it (in order)
@@ -737,10 +737,10 @@ __device__ __forceinline__ void line_group(Grp<Ks...>, std::integer_sequence<int
   });
 }
 
-template <int SPLIT, uint32_t PROPS, bool NOSCAT, int INTEGRAND, class... Gs, int... G>
+template <int SPLIT, uint32_t PROPS, bool NOSCAT, class CTX, int INTEGRAND, class... Gs, int... G>
 __device__ __forceinline__ void run_line_groups(Layout<INTEGRAND, Gs...>,
                                                 std::integer_sequence<int, G...>,
-                                                const LineCtx& cx, const FwdArgs& a, Ray& y,
+                                                const CTX& cx, const FwdArgs& a, Ray& y,
                                                 double2* terms, double& total) {
   (
       [&] {
@@ -759,8 +759,8 @@ __device__ __forceinline__ void run_line_groups(Layout<INTEGRAND, Gs...>,
       ...);
 }
 
-template <int SPLIT, uint32_t PROPS, bool NOSCAT, int INTEGRAND, class... Gs>
-__device__ __forceinline__ void run_line(Layout<INTEGRAND, Gs...> lay, const LineCtx& cx,
+template <int SPLIT, uint32_t PROPS, bool NOSCAT, class CTX, int INTEGRAND, class... Gs>
+__device__ __forceinline__ void run_line(Layout<INTEGRAND, Gs...> lay, const CTX& cx,
                                          const FwdArgs& a, Ray& y, double2* terms,
                                          double& total) {
   run_line_groups<SPLIT, PROPS, NOSCAT>(lay, std::make_integer_sequence<int, sizeof...(Gs)>{},

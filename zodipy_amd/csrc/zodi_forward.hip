@@ -154,6 +154,21 @@ forward_layout(FwdArgs a) {
   }
 }
 
+// The context of a forward line kernel and its tables in LDS (every thread must call it).
+template <bool LOGS>
+__device__ __forceinline__ auto line_tables(ModelPtr M, int sub) {
+  if constexpr (LOGS) {
+    __shared__ LineLogTables tables;
+    __shared__ AngleTable angles;
+    LineLogCtx cx = line_log_ctx(M, tables, &angles);
+    cx.sub = sub;
+    return cx;
+  } else {
+    __shared__ LineTables tables;
+    return line_ctx(M, tables, sub);
+  }
+}
+
 // The Kelsall layouts' registry blocks (props_match without the shared cut-off, and
 // line_match) on the ray's line (zodi_line.hpp): bound by FP64 vector issue, 335 vector
 // instructions a ray and node of the DIRBE layout where forming every node's position and
@@ -163,13 +178,13 @@ forward_layout(FwdArgs a) {
 // without spills: 214 -> 200 us of kernel against 5). SHARE: the bands that share a radial
 // cut-off reuse it (kShareCut), for blocks whose delta_r values allow it (the registry parameters; a fit
 // that moves them runs without). NOSCAT (with SHARE): no component scatters, so no
-// scattering code is compiled in.
-template <class LAYOUT, int BLOCK, bool SHARE, bool NOSCAT>
+// scattering code is compiled in. LOGS (without NOSCAT): powers by logarithms, for
+// exponents that the tables do not hold (line_match).
+template <class LAYOUT, int BLOCK, bool SHARE, bool NOSCAT, bool LOGS = false>
 __global__ __launch_bounds__(BLOCK)
 __attribute__((amdgpu_waves_per_eu(NOSCAT ? ForwardOccupancy<LAYOUT>::value : 4))) void
 forward_line(FwdArgs a) {
-  __shared__ LineTables tables;
-  const LineCtx cx = line_ctx(as_const(a.m), tables, 0);
+  const auto cx = line_tables<LOGS>(as_const(a.m), 0);
   constexpr uint32_t kProps = SHARE ? RegistryProps<LAYOUT>::value
                                     : props_without_share(RegistryProps<LAYOUT>::value);
   for (int64_t tile = blockIdx.x; tile < a.n_tiles; tile += gridDim.x) {
@@ -181,13 +196,12 @@ forward_line(FwdArgs a) {
 }
 
 // The same for small launches, a.lanes lanes per ray (2 to 32).
-template <class LAYOUT, int SPLIT, bool SHARE, bool NOSCAT>
+template <class LAYOUT, int SPLIT, bool SHARE, bool NOSCAT, bool LOGS = false>
 __global__ __launch_bounds__(kSplitBlock) __attribute__((amdgpu_waves_per_eu(2))) void
 forward_line_split(FwdArgs a) {
-  __shared__ LineTables tables;
   __shared__ double2 terms[SPLIT == 8 ? kMaxSlots * kSplitStride : 1];
   const int lanes = SPLIT == 8 ? a.lanes : SPLIT;
-  const LineCtx cx = line_ctx(as_const(a.m), tables, threadIdx.x & (lanes - 1));
+  const auto cx = line_tables<LOGS>(as_const(a.m), threadIdx.x & (lanes - 1));
   constexpr uint32_t kProps = SHARE ? RegistryProps<LAYOUT>::value
                                     : props_without_share(RegistryProps<LAYOUT>::value);
   const int rays = blockDim.x / lanes;
@@ -208,9 +222,9 @@ template <class LAYOUT, int BLOCK>
 __global__ __launch_bounds__(BLOCK)
 __attribute__((amdgpu_waves_per_eu(ForwardOccupancy<LAYOUT>::value))) void
 forward_rrm(FwdArgs a) {
-  __shared__ LineAdjTables tables;
+  __shared__ LineLogTables tables;
   __shared__ AngleTable angles;
-  const LineAdjCtx cx = line_adj_ctx(as_const(a.m), tables, &angles);
+  const LineLogCtx cx = line_log_ctx(as_const(a.m), tables, &angles);
   for (int64_t tile = blockIdx.x; tile < a.n_tiles; tile += gridDim.x) {
     const Ray y = load_ray<BLOCK>(a, tile, threadIdx.x);
     double total = 0.0;
@@ -222,10 +236,10 @@ forward_rrm(FwdArgs a) {
 template <class LAYOUT, int SPLIT>
 __global__ __launch_bounds__(kSplitBlock) __attribute__((amdgpu_waves_per_eu(2))) void
 forward_rrm_split(FwdArgs a) {
-  __shared__ LineAdjTables tables;
+  __shared__ LineLogTables tables;
   __shared__ double2 terms[SPLIT == 8 ? kMaxSlots * kSplitStride : 1];
   __shared__ AngleTable angles;
-  LineAdjCtx cx = line_adj_ctx(as_const(a.m), tables, &angles);
+  LineLogCtx cx = line_log_ctx(as_const(a.m), tables, &angles);
   const int lanes = SPLIT == 8 ? a.lanes : SPLIT;
   cx.sub = threadIdx.x & (lanes - 1);
   const int rays = blockDim.x / lanes;
@@ -431,20 +445,23 @@ inline bool no_scattering(const zodi_model* m) {
   return true;
 }
 
-template <class LAYOUT, bool SHARE, bool NOSCAT>
+template <class LAYOUT, bool SHARE, bool NOSCAT, bool LOGS = false>
 FwdKernel pick_line_block(int block, int L) {
   if (block != 256 && block != 512) return nullptr;
-  if (L == 2) return forward_line_split<LAYOUT, 2, SHARE, NOSCAT>;
-  if (L == 4) return forward_line_split<LAYOUT, 4, SHARE, NOSCAT>;
-  if (L > 4) return forward_line_split<LAYOUT, 8, SHARE, NOSCAT>;
-  return block == 256 ? forward_line<LAYOUT, 256, SHARE, NOSCAT>
-                      : forward_line<LAYOUT, 512, SHARE, NOSCAT>;
+  if (L == 2) return forward_line_split<LAYOUT, 2, SHARE, NOSCAT, LOGS>;
+  if (L == 4) return forward_line_split<LAYOUT, 4, SHARE, NOSCAT, LOGS>;
+  if (L > 4) return forward_line_split<LAYOUT, 8, SHARE, NOSCAT, LOGS>;
+  return block == 256 ? forward_line<LAYOUT, 256, SHARE, NOSCAT, LOGS>
+                      : forward_line<LAYOUT, 512, SHARE, NOSCAT, LOGS>;
 }
 
 template <class LAYOUT>
 FwdKernel pick_line(const zodi_model* m, int block, int L) {
-  if (!props_match(m, RegistryProps<LAYOUT>::value))
-    return pick_line_block<LAYOUT, false, false>(block, L);
+  const bool share = props_match(m, RegistryProps<LAYOUT>::value);
+  if (!line_match(m))
+    return share ? pick_line_block<LAYOUT, true, false, true>(block, L)
+                 : pick_line_block<LAYOUT, false, false, true>(block, L);
+  if (!share) return pick_line_block<LAYOUT, false, false>(block, L);
   return no_scattering(m) ? pick_line_block<LAYOUT, true, true>(block, L)
                           : pick_line_block<LAYOUT, true, false>(block, L);
 }
@@ -455,7 +472,7 @@ FwdKernel pick_line(const zodi_model* m, int block, int L) {
 // flags.
 template <class LAYOUT>
 bool line_eligible(const zodi_model* m) {
-  return props_match(m, props_without_share(RegistryProps<LAYOUT>::value)) && line_match(m);
+  return props_match(m, props_without_share(RegistryProps<LAYOUT>::value)) && line_log_match(m);
 }
 
 bool takes_line(const zodi_model* m, LayoutId id) {

@@ -165,6 +165,91 @@ __device__ __forceinline__ LineCtx line_ctx(ModelPtr M, LineTables& tab, int sub
   return cx;
 }
 
+// The same with powers as exp(p log x), for the passes that need the logarithms anyway (the
+// gradients, RRM) and for exponents that the power tables do not hold (line_match).
+struct LineLogTables {
+  double2 log_tab[256];
+  double2 planck[ZODI_N_TEMPS + 1];
+};
+
+struct LineLogCtx {
+  ModelPtr M;
+  const LineLogTables* tab;
+  ExpConst ec;
+  LogConst lc;
+  int K, sub, split;
+  bool share;  // gradients: band 3 takes band 1's cut-off (props_match with kShareCut)
+  const AngleTable* angles;
+  static constexpr bool kAngles = false;
+};
+
+// Builds the block's tables, `angles` too if given (every thread of the block must call it).
+__device__ __forceinline__ LineLogCtx line_log_ctx(ModelPtr M, LineLogTables& tab,
+                                                   AngleTable* angles = nullptr) {
+  stage_line_tables();
+  for (int j = threadIdx.x; j < 256; j += blockDim.x)
+    tab.log_tab[j] = double2{kLineInv[j], kLineLog[j]};
+  load_planck(M, tab.planck, threadIdx.x, blockDim.x);
+  if (angles != nullptr) load_angles(*angles, threadIdx.x, blockDim.x);
+  __syncthreads();
+  LineLogCtx cx;
+  cx.M = M;
+  cx.tab = &tab;
+  cx.ec = exp_const();
+  cx.lc = log_const();
+  cx.K = M->n_nodes;
+  cx.sub = 0;
+  cx.split = 1;
+  cx.share = false;
+  cx.angles = angles;
+  return cx;
+}
+
+// A group's temperature law as the node loop takes it: T/dT - T_first/dT + 1.
+struct LineLaw {
+  double half_delta, us, uo1;
+};
+
+__device__ __forceinline__ LineLaw line_law(const LineCtx& cx, int) { return {0.0, 0.0, cx.uo1}; }
+
+__device__ __forceinline__ LineLaw line_law(const LineLogCtx& cx, int g) {
+  const ModelPtr M = cx.M;
+  return {to_scalar(0.5 * M->group_delta[g]), to_scalar(M->group_T0[g] * M->tab_inv_step),
+          to_scalar(M->tab_T[0] * M->tab_inv_step - 1.0)};
+}
+
+__device__ __forceinline__ double line_axis(const LineCtx& cx, const LineLaw& law, double R2) {
+  return pow_table_less(cx.tab->temperature, cx.pt, R2, law.uo1);
+}
+
+__device__ __forceinline__ double line_axis(const LineLogCtx& cx, const LineLaw& law, double R2) {
+  const double Rd = exp_neg_any(cx.ec, law.half_delta * log_node(cx.tab->log_tab, cx.lc, R2));
+  return fma(Rd, law.us, -law.uo1);
+}
+
+// The cloud's density from r^2 and g. The floor under g changes nothing: with gamma >= 1/2
+// both powers are below 2^-126.
+__device__ __forceinline__ double cloud_profile(ParamPtr P, const LineCtx& cx, double r2,
+                                                double g) {
+  const double gg = pow_table(cx.tab->vertical, cx.pv, fmax(g, 0x1p-253));
+  return pow_table(cx.tab->radial, cx.pr, r2) * exp_neg_node(cx.ec, P[8] * gg);
+}
+
+__device__ __forceinline__ double cloud_profile(ParamPtr P, const LineLogCtx& cx, double r2,
+                                                double g) {
+  const double lg = log_node(cx.tab->log_tab, cx.lc, fmax(g, 0x1p-253));
+  const double gg = exp_neg_any(cx.ec, -(P[9] * lg));
+  const double lr = log_node(cx.tab->log_tab, cx.lc, r2);
+  return P[6] * exp_neg_any(cx.ec, fma(0.5 * P[7], lr, P[8] * gg));
+}
+
+__device__ __forceinline__ const AngleTable& line_angles(const LineCtx& cx) {
+  return cx.tab->angles;
+}
+__device__ __forceinline__ const AngleTable& line_angles(const LineLogCtx& cx) {
+  return *cx.angles;
+}
+
 // ---------------------------------------------------------------- densities
 // The reference's densities (see zodi_device.hpp for each expression's source) on the
 // line's linear forms; LineComp<KIND> holds a component's constants for one ray.
@@ -211,8 +296,9 @@ struct LineNode {
   double t, R2, R, inv_R;
 };
 
+template <class CTX>
 __device__ __forceinline__ double line_cloud(ParamPtr P, const LineComp<ZODI_CLOUD>& c,
-                                             const LineCtx& cx, const LineNode& nd) {
+                                             const CTX& cx, const LineNode& nd) {
   const double mu = P[10], inv_2mu = P[13];
   const double r2 = c.o.r2(nd.t);
   double r, inv_r;
@@ -222,9 +308,7 @@ __device__ __forceinline__ double line_cloud(ParamPtr P, const LineComp<ZODI_CLO
   // selection (two vcc-masked moves in a row stall the SIMD for about 20 cycles)
   const double m = fmin(zeta, mu);
   const double g = fma(m * m, inv_2mu, zeta - m);
-  // the floor changes nothing: with gamma >= 1/2 both powers are below 2^-126
-  const double gg = pow_table(cx.tab->vertical, cx.pv, fmax(g, 0x1p-253));
-  return pow_table(cx.tab->radial, cx.pr, r2) * exp_neg_node(cx.ec, P[8] * gg);
+  return cloud_profile(P, cx, r2, g);
 }
 
 // What a band of the line kernels does with its cut-off term: forms it for itself, forms
@@ -233,9 +317,9 @@ enum BandCut { kCutOwn = 0, kCutPublish = 1, kCutReuse = 2 };
 
 // exp(-zeta_d^6) is 0 from 746 on: those nodes add nothing and are left out for the waves
 // whose lanes all lie there (a map's rings at higher latitudes). NaN takes the branch.
-template <int CUT>
+template <int CUT, class CTX>
 __device__ __forceinline__ double line_band(ParamPtr P, const LineComp<ZODI_BAND>& c,
-                                            const LineCtx& cx, const LineNode& nd, double& cut) {
+                                            const CTX& cx, const LineNode& nd, double& cut) {
   double term4;
   if constexpr (CUT == kCutReuse) {
     term4 = cut;
@@ -261,8 +345,9 @@ __device__ __forceinline__ double line_band(ParamPtr P, const LineComp<ZODI_BAND
   return n;
 }
 
+template <class CTX>
 __device__ __forceinline__ double line_ring(ParamPtr P, const LineComp<ZODI_RING>& c,
-                                            const LineCtx& cx, const LineNode& nd) {
+                                            const CTX& cx, const LineNode& nd) {
   const double d = nd.R - P[7];
   return P[6] * exp_neg_any(cx.ec, fma(d * d, P[13], fabs(c.z.at(nd.t)) * P[14]));
 }
@@ -327,14 +412,15 @@ __device__ __forceinline__ double feature_angle(const LineComp<ZODI_FEATURE>& c,
   return unit_angle(tab, x * inv_rho, fabs(y) * inv_rho);
 }
 
+template <class CTX>
 __device__ __forceinline__ double line_feature(ParamPtr P, const LineComp<ZODI_FEATURE>& c,
-                                               const LineCtx& cx, const Line& l,
+                                               const CTX& cx, const Line& l,
                                                const LineNode& nd) {
   const double d = nd.R - P[7];
   double e = (d * d) * P[13];
   e = fma(fabs(c.z.at(nd.t)), P[14], e);
   double y, rho2, inv_rho;
-  const double theta = feature_angle(c, l, cx.tab->angles, nd.t, y, rho2, inv_rho);
+  const double theta = feature_angle(c, l, line_angles(cx), nd.t, y, rho2, inv_rho);
   e = fma(theta * theta, P[15], e);
   return P[6] * exp_neg_any(cx.ec, e);
 }

@@ -24,55 +24,17 @@
 
 namespace zodi {
 
-// ---------------------------------------------------------------- per-block tables
-struct LineAdjTables {
-  double2 log_tab[256];
-  double2 planck[ZODI_N_TEMPS + 1];
-};
-
-struct LineAdjCtx {
-  ModelPtr M;
-  const LineAdjTables* tab;
-  ExpConst ec;
-  LogConst lc;
-  int K, sub, split;
-  bool share;  // band 3 takes band 1's cut-off (props_match with kShareCut)
-  const AngleTable* angles;
-  static constexpr bool kAngles = false;
-};
-
+// ---------------------------------------------------------------- angles
 // For the passes that take angles from the table: with scattering (SCAT 2), chi^2 of 196 608
 // rays of DIRBE at 1.25 um takes 296 us for 314, of 400 000 672 for 741. The passes without,
 // whose only angle is the feature's, spill more registers for it than it saves (VJP of
 // 150 000 rays 210 us for 205, RRM chi^2 of 49 152 168 for 165) and keep axis_angle.
-struct LineAdjCtxAngles : LineAdjCtx {
+struct LineLogCtxAngles : LineLogCtx {
   static constexpr bool kAngles = true;
 };
 
 template <int SCAT>
-using AdjCtx = std::conditional_t<SCAT == 2, LineAdjCtxAngles, LineAdjCtx>;
-
-// Builds the block's tables, `angles` too if given (every thread of the block must call it).
-__device__ __forceinline__ LineAdjCtx line_adj_ctx(ModelPtr M, LineAdjTables& tab,
-                                                   AngleTable* angles = nullptr) {
-  stage_line_tables();
-  for (int j = threadIdx.x; j < 256; j += blockDim.x)
-    tab.log_tab[j] = double2{kLineInv[j], kLineLog[j]};
-  load_planck(M, tab.planck, threadIdx.x, blockDim.x);
-  if (angles != nullptr) load_angles(*angles, threadIdx.x, blockDim.x);
-  __syncthreads();
-  LineAdjCtx cx;
-  cx.M = M;
-  cx.tab = &tab;
-  cx.ec = exp_const();
-  cx.lc = log_const();
-  cx.K = M->n_nodes;
-  cx.sub = 0;
-  cx.split = 1;
-  cx.share = false;
-  cx.angles = angles;
-  return cx;
-}
+using AdjCtx = std::conditional_t<SCAT == 2, LineLogCtxAngles, LineLogCtx>;
 
 // One node as the components see it.
 struct GradNode {
@@ -98,7 +60,7 @@ struct LineGrad<ZODI_CLOUD> {
       : c(P, l, ex, ey), s{}, kz(to_scalar(P[8] * P[9] * (2.0 * P[13]))),
         ha(to_scalar(0.5 * P[7])), og(to_scalar(1.0 - P[9])) {}
 
-  __device__ __forceinline__ double add(ParamPtr P, const LineAdjCtx& cx, const Line&,
+  __device__ __forceinline__ double add(ParamPtr P, const LineLogCtx& cx, const Line&,
                                         const GradNode& nd, double u) {
     const double alpha = P[7], beta = P[8], mu = P[10], inv_2mu = P[13];
     const double r2 = c.o.r2(nd.t);
@@ -159,7 +121,7 @@ struct LineGrad<ZODI_BAND> {
 
   // cs: the radial cut-off's x and exp(-x), formed here unless `have`. Past zeta_d^6 =
   // 746 the density and every partial are exact zeros (line_band).
-  __device__ __forceinline__ double add(ParamPtr P, const LineAdjCtx& cx, const GradNode& nd,
+  __device__ __forceinline__ double add(ParamPtr P, const LineLogCtx& cx, const GradNode& nd,
                                         CutShare& cs, bool have, double u) {
     if (!have) {
       const double y = nd.R2 * P[ZODI_P_D0 + 6];
@@ -222,7 +184,7 @@ struct LineGrad<ZODI_RING> {
   __device__ __forceinline__ LineGrad(ParamPtr P, const Line& l, double ex, double ey)
       : c(P, l, ex, ey), s{} {}
 
-  __device__ __forceinline__ double add(ParamPtr P, const LineAdjCtx& cx, const Line&,
+  __device__ __forceinline__ double add(ParamPtr P, const LineLogCtx& cx, const Line&,
                                         const GradNode& nd, double u) {
     const double d = nd.R - P[7];
     const double zc = c.z.at(nd.t);
@@ -390,7 +352,7 @@ struct Chi2Ray {
 // weighted in kPassVjp, else at unit weight.
 template <int SCAT, int PASS, uint32_t PROPS, int NC, int C0, int... Ks, int... J>
 __device__ __forceinline__ void line_adj_group(Grp<Ks...>, std::integer_sequence<int, J...>,
-                                               const LineAdjCtx& cx, const AdjArgs& a, Ray& y,
+                                               const LineLogCtx& cx, const AdjArgs& a, Ray& y,
                                                int g, int first, double gscale, double* row,
                                                int lane, double (&sh)[6], double& total,
                                                Chi2Ray<NC, C0>& cr, double* hold) {
@@ -653,7 +615,7 @@ constexpr int layout_group0(Layout<ZODI_INTEGRAND_KELSALL, G0, Gs...>) {
 template <int SCAT, int PASS, uint32_t PROPS, class... Gs, int... G>
 __device__ __forceinline__ void line_adj_groups(Layout<ZODI_INTEGRAND_KELSALL, Gs...>,
                                                 std::integer_sequence<int, G...>,
-                                                const LineAdjCtx& cx, const AdjArgs& a, Ray& y,
+                                                const LineLogCtx& cx, const AdjArgs& a, Ray& y,
                                                 double gscale, double* row, int lane,
                                                 double (&sh)[6], double& total, double& chi,
                                                 double* hold) {
@@ -682,7 +644,7 @@ __device__ __forceinline__ void line_adj_groups(Layout<ZODI_INTEGRAND_KELSALL, G
 
 template <int SCAT, int PASS, class... Gs>
 __device__ __forceinline__ void line_adj_layout(Layout<ZODI_INTEGRAND_KELSALL, Gs...> lay,
-                                                const LineAdjCtx& cx, const AdjArgs& a, Ray& y,
+                                                const LineLogCtx& cx, const AdjArgs& a, Ray& y,
                                                 double gscale, double* row, int lane,
                                                 double (&sh)[6], double& total, double& chi,
                                                 double* hold) {
@@ -747,11 +709,11 @@ __device__ __forceinline__ void weighted_body(const AdjArgs& a, RAY ray) {
 template <class LAYOUT, int SCAT, int PASS>
 __device__ __forceinline__ void line_adj_body(const AdjArgs& a) {
   constexpr int NSH = layout_integrand<LAYOUT>() == ZODI_INTEGRAND_KELSALL ? 6 : 1;
-  __shared__ LineAdjTables tables;
+  __shared__ LineLogTables tables;
   const ModelPtr M = as_const(a.f.m);
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
   __shared__ AngleTable angles;
-  AdjCtx<SCAT> cx{line_adj_ctx(M, tables, SCAT == 2 ? &angles : nullptr)};
+  AdjCtx<SCAT> cx{line_log_ctx(M, tables, SCAT == 2 ? &angles : nullptr)};
   cx.split = a.split;
   cx.sub = lane & (a.split - 1);
   cx.share = a.share != 0;

@@ -54,11 +54,21 @@ inline bool line_cloud_match(const zodi_model* m) {
          (mu > 0.0 || std::fabs(beta) * std::pow(1.0 - 0.5 * mu, gamma) <= kLineMaxExponent);
 }
 
-// Whether a block that meets a layout's registry properties (props_match) may take the
-// forward and table line kernels. The Kelsall ones: one temperature law for all groups, the
-// three exponents and the radii inside the power tables' ranges.
-inline bool line_match(const zodi_model* m) {
+// Whether a block that meets a layout's registry properties (props_match) may take the line
+// kernels that form powers as exp(p log x): the gradients, and the forward and table kernels
+// where line_match fails.
+inline bool line_log_match(const zodi_model* m) {
   if (!line_bounded(m)) return false;
+  if (m->integrand == ZODI_INTEGRAND_RRM) return true;
+  const double* P = m->comp[0];
+  return line_cloud_match(m) && within(P[7], -1e3, 1e3) && within(P[9], -1e3, 1e3);
+}
+
+// Whether the Kelsall forward and table kernels may take their powers from tables: one
+// temperature law for all groups, the three exponents inside the ranges in which the
+// tables' series holds (PowPoly), the radii inside those of the exponents.
+inline bool line_match(const zodi_model* m) {
+  if (!line_log_match(m)) return false;
   if (m->integrand == ZODI_INTEGRAND_RRM) return true;
   const auto same = [](double a, double b) { return a == b || (a != a && b != b); };
   const double delta = m->group_delta[0];
@@ -69,16 +79,7 @@ inline bool line_match(const zodi_model* m) {
       return false;
   }
   const double* P = m->comp[0];
-  return line_cloud_match(m) && !(delta > 2.0) && within(P[7], -12.0, 2.0) &&
-         within(P[9], 0.5, 6.0);
-}
-
-// The same for the adjoint and Jacobian kernels, which take logarithms instead of tables.
-inline bool line_adjoint_match(const zodi_model* m) {
-  if (!line_bounded(m)) return false;
-  if (m->integrand == ZODI_INTEGRAND_RRM) return true;
-  const double* P = m->comp[0];
-  return line_cloud_match(m) && within(P[7], -1e3, 1e3) && within(P[9], -1e3, 1e3);
+  return !(delta > 2.0) && within(P[7], -12.0, 2.0) && within(P[9], 0.5, 6.0);
 }
 
 }  // namespace zodi

@@ -32,7 +32,7 @@ struct LatSine {
 };
 
 template <bool GRAD>
-__device__ __forceinline__ LatSine lat_sine(const LineAdjCtx& cx, ParamPtr P, double Z0,
+__device__ __forceinline__ LatSine lat_sine(const LineLogCtx& cx, ParamPtr P, double Z0,
                                             double inv_Z0, double za, double s, double cb) {
   LatSine o;
   o.su = s;
@@ -108,7 +108,7 @@ struct LineComp<ZODI_INTERSTELLAR> {
 // Density of an RRM component at a node; lR2 = log |X|^2.
 template <int KIND>
 __device__ __forceinline__ double rrm_density(ParamPtr P, const LineComp<KIND>& c,
-                                              const LineAdjCtx& cx, const Line& l,
+                                              const LineLogCtx& cx, const Line& l,
                                               const GradNode& nd, double lR2) {
   if constexpr (KIND == ZODI_INTERSTELLAR) {
     return P[6];
@@ -175,7 +175,7 @@ struct RrmNode {
   double lR2, Rd, B, dB;
 };
 
-__device__ __forceinline__ RrmNode rrm_node(const LineAdjCtx& cx, const Line& l, double t,
+__device__ __forceinline__ RrmNode rrm_node(const LineLogCtx& cx, const Line& l, double t,
                                             double half_delta, double us, double uo1) {
   RrmNode o;
   o.nd.t = t;
@@ -198,7 +198,7 @@ __device__ __forceinline__ RrmNode rrm_node(const LineAdjCtx& cx, const Line& l,
 // ---------------------------------------------------------------- forward
 template <int SPLIT, int... Ks, int... J>
 __device__ __forceinline__ void rrm_group(Grp<Ks...>, std::integer_sequence<int, J...>,
-                                          const LineAdjCtx& cx, const FwdArgs& a, const Ray& y,
+                                          const LineLogCtx& cx, const FwdArgs& a, const Ray& y,
                                           const Line& l, int g, int first, double2* terms,
                                           double& total) {
   constexpr int C = sizeof...(Ks);
@@ -232,7 +232,7 @@ __device__ __forceinline__ void rrm_group(Grp<Ks...>, std::integer_sequence<int,
 template <int SPLIT, class... Gs, int... G>
 __device__ __forceinline__ void rrm_groups(Layout<ZODI_INTEGRAND_RRM, Gs...>,
                                            std::integer_sequence<int, G...>,
-                                           const LineAdjCtx& cx, const FwdArgs& a, const Ray& y,
+                                           const LineLogCtx& cx, const FwdArgs& a, const Ray& y,
                                            const Line& l, double2* terms, double& total) {
   (rrm_group<SPLIT>(Gs{}, std::make_integer_sequence<int, Gs::size>{}, cx, a, y, l, G,
                     group_first<Gs...>(G), terms, total),
@@ -241,7 +241,7 @@ __device__ __forceinline__ void rrm_groups(Layout<ZODI_INTEGRAND_RRM, Gs...>,
 
 template <int SPLIT, class... Gs>
 __device__ __forceinline__ void run_rrm(Layout<ZODI_INTEGRAND_RRM, Gs...> lay,
-                                        const LineAdjCtx& cx, const FwdArgs& a, const Ray& y,
+                                        const LineLogCtx& cx, const FwdArgs& a, const Ray& y,
                                         double2* terms, double& total) {
   const Line l = make_line(y.ux, y.uy, y.uz, y.ox, y.oy, y.oz);
   rrm_groups<SPLIT>(lay, std::make_integer_sequence<int, sizeof...(Gs)>{}, cx, a, y, l, terms,
@@ -281,7 +281,7 @@ struct LineGrad<ZODI_FAN> : RrmSums {
   __device__ __forceinline__ LineGrad(ParamPtr P, const Line& l, double ex, double ey)
       : c(P, l, ex, ey), s{} {}
   __device__ __forceinline__ static double amplitude(ParamPtr) { return 1.0; }
-  __device__ __forceinline__ double add(ParamPtr P, const LineAdjCtx& cx, const Line&,
+  __device__ __forceinline__ double add(ParamPtr P, const LineLogCtx& cx, const Line&,
                                         const GradNode& nd, double lR2, double u) {
     double nu = 0.0;
     if (nd.R <= P[10]) {
@@ -323,7 +323,7 @@ struct LineGrad<ZODI_COMET> : RrmSums {
   __device__ __forceinline__ LineGrad(ParamPtr P, const Line& l, double ex, double ey)
       : c(P, l, ex, ey), s{} {}
   __device__ __forceinline__ static double amplitude(ParamPtr P) { return P[9]; }
-  __device__ __forceinline__ double add(ParamPtr P, const LineAdjCtx& cx, const Line&,
+  __device__ __forceinline__ double add(ParamPtr P, const LineLogCtx& cx, const Line&,
                                         const GradNode& nd, double lR2, double u) {
     double nu = 0.0;
     if (nd.R >= P[10] && nd.R <= P[11]) {
@@ -363,7 +363,7 @@ struct LineGrad<ZODI_NARROW_BAND> : RrmSums {
   __device__ __forceinline__ LineGrad(ParamPtr P, const Line& l, double ex, double ey)
       : c(P, l, ex, ey), s{} {}
   __device__ __forceinline__ static double amplitude(ParamPtr P) { return P[9]; }
-  __device__ __forceinline__ double add(ParamPtr P, const LineAdjCtx& cx, const Line&,
+  __device__ __forceinline__ double add(ParamPtr P, const LineLogCtx& cx, const Line&,
                                         const GradNode& nd, double lR2, double u) {
     double nu = 0.0;
     if (nd.R >= P[10] && nd.R <= P[11]) {
@@ -403,7 +403,7 @@ struct LineGrad<ZODI_BROAD_BAND> : RrmSums {
   __device__ __forceinline__ LineGrad(ParamPtr P, const Line& l, double ex, double ey)
       : c(P, l, ex, ey), s{} {}
   __device__ __forceinline__ static double amplitude(ParamPtr P) { return P[9]; }
-  __device__ __forceinline__ double add(ParamPtr P, const LineAdjCtx& cx, const Line&,
+  __device__ __forceinline__ double add(ParamPtr P, const LineLogCtx& cx, const Line&,
                                         const GradNode& nd, double lR2, double u) {
     double nu = 0.0;
     if (nd.R >= P[10] && nd.R <= P[11]) {
@@ -443,7 +443,7 @@ struct LineGrad<ZODI_INTERSTELLAR> : RrmSums {
   double s[kSlots];
   __device__ __forceinline__ LineGrad(ParamPtr, const Line&, double, double) : s{} {}
   __device__ __forceinline__ static double amplitude(ParamPtr P) { return P[6]; }
-  __device__ __forceinline__ double add(ParamPtr, const LineAdjCtx&, const Line&, const GradNode&,
+  __device__ __forceinline__ double add(ParamPtr, const LineLogCtx&, const Line&, const GradNode&,
                                         double, double) {
     return 1.0;
   }
@@ -458,7 +458,7 @@ template <>
 struct LineGrad<ZODI_RING_RRM> : LineGrad<ZODI_RING> {
   using LineGrad<ZODI_RING>::LineGrad;
   __device__ __forceinline__ static double amplitude(ParamPtr P) { return P[10] * P[6]; }
-  __device__ __forceinline__ double add(ParamPtr P, const LineAdjCtx& cx, const Line& l,
+  __device__ __forceinline__ double add(ParamPtr P, const LineLogCtx& cx, const Line& l,
                                         const GradNode& nd, double, double u) {
     return LineGrad<ZODI_RING>::add(P, cx, l, nd, u);
   }
@@ -476,7 +476,7 @@ template <>
 struct LineGrad<ZODI_FEATURE_RRM> : LineGrad<ZODI_FEATURE> {
   using LineGrad<ZODI_FEATURE>::LineGrad;
   __device__ __forceinline__ static double amplitude(ParamPtr P) { return P[12] * P[6]; }
-  __device__ __forceinline__ double add(ParamPtr P, const LineAdjCtx& cx, const Line& l,
+  __device__ __forceinline__ double add(ParamPtr P, const LineLogCtx& cx, const Line& l,
                                         const GradNode& nd, double, double u) {
     return LineGrad<ZODI_FEATURE>::add(P, cx, l, nd, u);
   }
@@ -494,7 +494,7 @@ struct LineGrad<ZODI_FEATURE_RRM> : LineGrad<ZODI_FEATURE> {
 // component has a temperature law of its own in the parameter vector.
 template <bool JAC, int... Ks, int... J>
 __device__ __forceinline__ void rrm_adj_group(Grp<Ks...>, std::integer_sequence<int, J...>,
-                                              const LineAdjCtx& cx, const AdjArgs& a, Ray& y,
+                                              const LineLogCtx& cx, const AdjArgs& a, Ray& y,
                                               int g, int first, double gscale, double* row,
                                               int lane, double (&sh)[6], double& total) {
   constexpr int C = sizeof...(Ks);
@@ -598,7 +598,7 @@ __device__ __forceinline__ void rrm_adj_group(Grp<Ks...>, std::integer_sequence<
 template <bool JAC, class... Gs, int... G>
 __device__ __forceinline__ void rrm_adj_groups(Layout<ZODI_INTEGRAND_RRM, Gs...>,
                                                std::integer_sequence<int, G...>,
-                                               const LineAdjCtx& cx, const AdjArgs& a, Ray& y,
+                                               const LineLogCtx& cx, const AdjArgs& a, Ray& y,
                                                double gscale, double* row, int lane,
                                                double (&sh)[6], double& total) {
   (rrm_adj_group<JAC>(Gs{}, std::make_integer_sequence<int, Gs::size>{}, cx, a, y, G,
@@ -608,7 +608,7 @@ __device__ __forceinline__ void rrm_adj_groups(Layout<ZODI_INTEGRAND_RRM, Gs...>
 
 template <int SCAT, int PASS, class... Gs>
 __device__ __forceinline__ void line_adj_layout(Layout<ZODI_INTEGRAND_RRM, Gs...> lay,
-                                                const LineAdjCtx& cx, const AdjArgs& a, Ray& y,
+                                                const LineLogCtx& cx, const AdjArgs& a, Ray& y,
                                                 double gscale, double* row, int lane,
                                                 double (&sh)[6], double& total, double&,
                                                 double*) {

@@ -298,12 +298,7 @@ __device__ __forceinline__ void line_table_group(Grp<Ks...>, std::integer_sequen
   double h, mid;
   group_range(M, g, y, h, mid);
   const double th = l.n * h, tm = fma(l.n, mid, l.t0);
-  double half_delta = 0.0, us = 0.0, uo1 = 0.0;
-  if constexpr (!kKelsall) {
-    half_delta = to_scalar(0.5 * M->group_delta[g]);
-    us = to_scalar(M->group_T0[g] * M->tab_inv_step);
-    uo1 = to_scalar(M->tab_T[0] * M->tab_inv_step - 1.0);
-  }
+  const LineLaw law = line_law(cx, g);
   const double calibration = M->shared[ZODI_S_CALIBRATION], solar = M->shared[ZODI_S_SOLAR];
   const std::tuple<LineComp<Ks>...> lc{LineComp<Ks>(M->comp[first + J], l, y.ex, y.ey)...};
   LinePhase lp = {0.0, 0.0};
@@ -345,12 +340,12 @@ __device__ __forceinline__ void line_table_group(Grp<Ks...>, std::integer_sequen
       nd.t = t;
       nd.R2 = fma(t, t, l.d2);
       norm_and_inverse_node(nd.R2, nd.R, nd.inv_R);
-      u1 = pow_table_less(cx.tab->temperature, cx.pt, nd.R2, cx.uo1);
+      u1 = line_axis(cx, law, nd.R2);
     } else {
-      const RrmNode o = rrm_node(cx, l, t, half_delta, us, uo1);
+      const RrmNode o = rrm_node(cx, l, t, law.half_delta, law.us, law.uo1);
       nd = o.nd;
       lR2 = o.lR2;
-      u1 = fma(o.Rd, us, -uo1);
+      u1 = fma(o.Rd, law.us, -law.uo1);
     }
     const TableShare ts = table_share(u1, cx.tab->planck);
     const double wB = wk * ts.B;
@@ -360,7 +355,7 @@ __device__ __forceinline__ void line_table_group(Grp<Ks...>, std::integer_sequen
       if (pu.phase) {
         pg.phi = pu.phi_const;
         if (pu.angle)
-          pg = line_phase_grad(scattering_angle(lp, l, t, cx.tab->angles, nd.inv_R), cx.ec,
+          pg = line_phase_grad(scattering_angle(lp, l, t, line_angles(cx), nd.inv_R), cx.ec,
                                Mk->shared);
         inv_R2 = nd.inv_R * nd.inv_R;
         wsu = wk * ((solar * inv_R2) * pg.phi);
@@ -590,22 +585,23 @@ constexpr int table_waves() {
              : kTableWavesLayout;
 }
 
-// The line kernels. SHARE: the bands that share a radial cut-off reuse it (kShareCut).
-template <class LAYOUT, bool SHARE, bool EFF, bool NOSCAT>
+// The line kernels. SHARE: the bands that share a radial cut-off reuse it (kShareCut). LOGS:
+// powers by logarithms (LineLogCtx), for the exponents that the power tables do not hold.
+template <class LAYOUT, bool SHARE, bool EFF, bool NOSCAT, bool LOGS = false>
 __global__ __launch_bounds__(kAdjBlock) __attribute__((
     amdgpu_waves_per_eu(table_waves<LAYOUT, EFF, NOSCAT>()))) void table_line(AdjArgs a) {
   constexpr uint32_t PROPS = SHARE ? RegistryProps<LAYOUT>::value
                                    : props_without_share(RegistryProps<LAYOUT>::value);
-  if constexpr (layout_integrand<LAYOUT>() == ZODI_INTEGRAND_KELSALL) {
+  if constexpr (layout_integrand<LAYOUT>() == ZODI_INTEGRAND_KELSALL && !LOGS) {
     __shared__ LineTables tables;
     const LineCtx cx = line_ctx(as_const(a.f.m), tables, threadIdx.x & (a.split - 1));
     weighted_body(a, [&](const Ray& y, double gscale, double* row, int lane) {
       run_line_table<PROPS, EFF, NOSCAT>(LAYOUT{}, cx, a, y, gscale, row, lane);
     });
   } else {
-    __shared__ LineAdjTables tables;
+    __shared__ LineLogTables tables;
     __shared__ AngleTable angles;
-    LineAdjCtx cx = line_adj_ctx(as_const(a.f.m), tables, &angles);
+    LineLogCtx cx = line_log_ctx(as_const(a.f.m), tables, &angles);
     cx.sub = threadIdx.x & (a.split - 1);
     weighted_body(a, [&](const Ray& y, double gscale, double* row, int lane) {
       run_line_table<PROPS, EFF, NOSCAT>(LAYOUT{}, cx, a, y, gscale, row, lane);
@@ -647,21 +643,26 @@ AdjKernel pick_table_split(int split) {
 
 // NOSCAT applies to the Kelsall layouts with EFF (the RRM integrand has no
 // scattering term, and without EFF nothing is summed for it).
-template <class LAYOUT, bool SHARE, bool EFF>
+template <class LAYOUT, bool SHARE, bool EFF, bool LOGS = false>
 TableKernel pick_table_line(bool noscat) {
   if constexpr (EFF && layout_integrand<LAYOUT>() == ZODI_INTEGRAND_KELSALL) {
     if (noscat)
-      return {table_line<LAYOUT, SHARE, true, true>, table_waves<LAYOUT, true, true>()};
+      return {table_line<LAYOUT, SHARE, true, true, LOGS>, table_waves<LAYOUT, true, true>()};
   }
-  return {table_line<LAYOUT, SHARE, EFF, false>, table_waves<LAYOUT, EFF, false>()};
+  return {table_line<LAYOUT, SHARE, EFF, false, LOGS>, table_waves<LAYOUT, EFF, false>()};
 }
 
 // The line kernels under the forward's conditions, else the layout kernels.
 template <class LAYOUT, bool EFF>
 TableKernel pick_table_layout(const zodi_model* m, int split) {
   constexpr uint32_t kProps = RegistryProps<LAYOUT>::value;
-  if (props_match(m, props_without_share(kProps)) && line_match(m)) {
+  if (props_match(m, props_without_share(kProps)) && line_log_match(m)) {
     const bool noscat = block_noscat(m);
+    if constexpr (layout_integrand<LAYOUT>() == ZODI_INTEGRAND_KELSALL) {
+      if (!line_match(m))
+        return props_match(m, kProps) ? pick_table_line<LAYOUT, true, EFF, true>(noscat)
+                                      : pick_table_line<LAYOUT, false, EFF, true>(noscat);
+    }
     if constexpr (kProps != props_without_share(kProps)) {
       if (props_match(m, kProps)) return pick_table_line<LAYOUT, true, EFF>(noscat);
     }
