@@ -434,8 +434,10 @@ __device__ __forceinline__ void run_line_table(Layout<INTEGRAND, Gs...> lay, con
 }
 
 // Registry layouts whose blocks the line kernels do not take: the group's kinds fixed at
-// compile time, the densities inlined.
-template <int INTEGRAND, int SPLIT, bool EFF, int... Ks, int... J>
+// compile time, the densities inlined. NOSCAT as in line_table_group: the spectral gradient
+// of 196 608 planck18 rays with an offset band takes 238 us without the scattering code, 257
+// with it.
+template <int INTEGRAND, int SPLIT, bool EFF, bool NOSCAT, int... Ks, int... J>
 __device__ __forceinline__ void table_group(Grp<Ks...>, std::integer_sequence<int, J...>,
                                             const Ctx& cx, const AdjArgs& a, const Ray& y, int g,
                                             int first, double gscale, double* row, int lane,
@@ -443,7 +445,7 @@ __device__ __forceinline__ void table_group(Grp<Ks...>, std::integer_sequence<in
   constexpr int C = sizeof...(Ks);
   constexpr int kinds[C] = {Ks...};
   constexpr bool kKelsall = INTEGRAND == ZODI_INTEGRAND_KELSALL;
-  constexpr bool kScat = EFF && kKelsall;
+  constexpr bool kScat = EFF && kKelsall && !NOSCAT;
   const ModelPtr M = cx.M;
   const int n_last = M->n_temps - 1;
   double* trow = EFF ? row + M->n_params : row;
@@ -552,27 +554,30 @@ __device__ __forceinline__ void table_group(Grp<Ks...>, std::integer_sequence<in
   }
 }
 
-template <int SPLIT, bool EFF, int INTEGRAND, class... Gs, int... G>
+template <int SPLIT, bool EFF, bool NOSCAT, int INTEGRAND, class... Gs, int... G>
 __device__ __forceinline__ void table_groups(Layout<INTEGRAND, Gs...>,
                                              std::integer_sequence<int, G...>, const Ctx& cx,
                                              const AdjArgs& a, const Ray& y, double gscale,
                                              double* row, int lane, int sub, const PhaseUse& pu,
                                              double (&sh)[6]) {
-  (table_group<INTEGRAND, SPLIT, EFF>(Gs{}, std::make_integer_sequence<int, Gs::size>{}, cx, a, y,
-                                      G, group_first<Gs...>(G), gscale, row, lane, sub, pu, sh),
+  (table_group<INTEGRAND, SPLIT, EFF, NOSCAT>(
+       Gs{}, std::make_integer_sequence<int, Gs::size>{}, cx, a, y, G, group_first<Gs...>(G),
+       gscale, row, lane, sub, pu, sh),
    ...);
 }
 
-template <int SPLIT, bool EFF, int INTEGRAND, class... Gs>
+template <int SPLIT, bool EFF, bool NOSCAT, int INTEGRAND, class... Gs>
 __device__ __forceinline__ void run_table(Layout<INTEGRAND, Gs...> lay, const Ctx& cx,
                                           const AdjArgs& a, const Ray& y, double gscale,
                                           double* row, int lane, int sub) {
   double sh[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
   PhaseUse pu = {false, false, 0.0};
-  if constexpr (EFF && INTEGRAND == ZODI_INTEGRAND_KELSALL) pu = phase_use(cx.M, cx.solar);
-  table_groups<SPLIT, EFF>(lay, std::make_integer_sequence<int, sizeof...(Gs)>{}, cx, a, y, gscale,
-                           row, lane, sub, pu, sh);
-  if constexpr (EFF) eff_ray_finish<INTEGRAND>(cx.M, sh, row, lane);
+  if constexpr (EFF && INTEGRAND == ZODI_INTEGRAND_KELSALL && !NOSCAT)
+    pu = phase_use(cx.M, cx.solar);
+  table_groups<SPLIT, EFF, NOSCAT>(lay, std::make_integer_sequence<int, sizeof...(Gs)>{}, cx, a, y,
+                                   gscale, row, lane, sub, pu, sh);
+  if constexpr (EFF && (INTEGRAND != ZODI_INTEGRAND_KELSALL || !NOSCAT))
+    eff_ray_finish<INTEGRAND>(cx.M, sh, row, lane);
 }
 
 // Resident waves per SIMD of the registry-layout kernels (their register budget):
@@ -609,12 +614,12 @@ __global__ __launch_bounds__(kAdjBlock) __attribute__((
   }
 }
 
-template <class LAYOUT, int SPLIT, bool EFF>
+template <class LAYOUT, int SPLIT, bool EFF, bool NOSCAT>
 __global__ __launch_bounds__(kAdjBlock) __attribute__((
-    amdgpu_waves_per_eu(table_waves<LAYOUT, EFF, false>()))) void table_layout(AdjArgs a) {
+    amdgpu_waves_per_eu(table_waves<LAYOUT, EFF, NOSCAT>()))) void table_layout(AdjArgs a) {
   adjoint_body<SPLIT, false, 0>(
       a, [&](const Ctx& cx, const Ray& y, double gscale, double* row, int lane, int sub, double*) {
-        run_table<SPLIT, EFF>(LAYOUT{}, cx, a, y, gscale, row, lane, sub);
+        run_table<SPLIT, EFF, NOSCAT>(LAYOUT{}, cx, a, y, gscale, row, lane, sub);
       });
 }
 
@@ -652,13 +657,29 @@ TableKernel pick_table_line(bool noscat) {
   return {table_line<LAYOUT, SHARE, EFF, false, LOGS>, table_waves<LAYOUT, EFF, false>()};
 }
 
+template <class LAYOUT, bool EFF, bool NOSCAT>
+TableKernel pick_table_general(int split) {
+  constexpr int kWaves = table_waves<LAYOUT, EFF, NOSCAT>();
+  switch (split) {
+    case 1:
+      return {table_layout<LAYOUT, 1, EFF, NOSCAT>, kWaves};
+    case 2:
+      return {table_layout<LAYOUT, 2, EFF, NOSCAT>, kWaves};
+    case 4:
+      return {table_layout<LAYOUT, 4, EFF, NOSCAT>, kWaves};
+    default:
+      return {nullptr, 0};
+  }
+}
+
 // The line kernels under the forward's conditions, else the layout kernels.
 template <class LAYOUT, bool EFF>
 TableKernel pick_table_layout(const zodi_model* m, int split) {
   constexpr uint32_t kProps = RegistryProps<LAYOUT>::value;
+  constexpr bool kKelsall = layout_integrand<LAYOUT>() == ZODI_INTEGRAND_KELSALL;
+  const bool noscat = block_noscat(m);
   if (props_match(m, props_without_share(kProps)) && line_log_match(m)) {
-    const bool noscat = block_noscat(m);
-    if constexpr (layout_integrand<LAYOUT>() == ZODI_INTEGRAND_KELSALL) {
+    if constexpr (kKelsall) {
       if (!line_match(m))
         return props_match(m, kProps) ? pick_table_line<LAYOUT, true, EFF, true>(noscat)
                                       : pick_table_line<LAYOUT, false, EFF, true>(noscat);
@@ -668,17 +689,10 @@ TableKernel pick_table_layout(const zodi_model* m, int split) {
     }
     return pick_table_line<LAYOUT, false, EFF>(noscat);
   }
-  constexpr int kWaves = table_waves<LAYOUT, EFF, false>();
-  switch (split) {
-    case 1:
-      return {table_layout<LAYOUT, 1, EFF>, kWaves};
-    case 2:
-      return {table_layout<LAYOUT, 2, EFF>, kWaves};
-    case 4:
-      return {table_layout<LAYOUT, 4, EFF>, kWaves};
-    default:
-      return {nullptr, 0};
+  if constexpr (EFF && kKelsall) {
+    if (noscat) return pick_table_general<LAYOUT, true, true>(split);
   }
+  return pick_table_general<LAYOUT, EFF, false>(split);
 }
 
 template <bool EFF>
