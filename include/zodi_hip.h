@@ -226,6 +226,22 @@ zodi_status zodi_forward(const zodi_model* model_host, const zodi_model* model_d
                          void* stream);
 
 /*
+ * zodi_forward_route — which of the forward kernels a block takes with this variant
+ * (-1: no valid block), for callers that keep launch shapes: the same route, layout and node
+ * count run the same kernels. The low two bits are one of the first four; registry blocks
+ * on the line kernels have the flags.
+ */
+enum {
+  ZODI_ROUTE_GENERIC = 0,       /* kind switch */
+  ZODI_ROUTE_LAYOUT = 1,        /* layout kernel that tests every component's frame */
+  ZODI_ROUTE_LINE_LOGS = 2,     /* line kernel, powers as exp(p log x) */
+  ZODI_ROUTE_LINE = 3,          /* line kernel (Kelsall: powers from tables) */
+  ZODI_ROUTE_NO_SCATTERING = 4, /* no component scatters */
+  ZODI_ROUTE_SHARED_CUT = 8     /* bands 1 and 3 have the same radial cut-off */
+};
+int32_t zodi_forward_route(const zodi_model* model_host, int32_t variant);
+
+/*
  * zodi_line_of_sight — per-group start and stop distances [AU]: start/stop are
  * [n_groups][n_rays]. Same addressing as zodi_forward.
  */

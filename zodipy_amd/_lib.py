@@ -25,6 +25,7 @@ EXPORTED_SYMBOLS = (
     "zodi_model_size",
     "zodi_last_error",
     "zodi_forward",
+    "zodi_forward_route",
     "zodi_line_of_sight",
     "zodi_number_density",
     "zodi_pix2vec",
@@ -72,6 +73,8 @@ def _bind(lib: ct.CDLL) -> None:
     lib.zodi_forward.restype = ct.c_int32
     lib.zodi_forward.argtypes = [_p, _p, _p, _i64, _p, _i32, _p, _p, _i32, _p, _p, _i32,
                                  ct.POINTER(Launch), _p]
+    lib.zodi_forward_route.restype = ct.c_int32
+    lib.zodi_forward_route.argtypes = [_p, _i32]
     lib.zodi_line_of_sight.restype = ct.c_int32
     lib.zodi_line_of_sight.argtypes = [_p, _p, _p, _i64, _p, _i32, _p, _i32, _p, _p, _p, _p]
     lib.zodi_number_density.restype = ct.c_int32

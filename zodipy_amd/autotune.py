@@ -4,14 +4,18 @@ Candidates are (threads per block, lanes per ray), each launched with one block
 per tile of rays (blocks_per_cu = 0): the hardware dispatcher hands a CU a new
 block whenever one retires, which is dynamic scheduling at tile granularity
 already, so a persistent launch could only save the per-block prologue (staging
-about 9 KB of tables into LDS, ~0.1 % of a block's work) and never shortens the
-tail (one tile). Static grid-stride launches (blocks_per_cu > 0) measured 10 %
-slower, because equal tile counts per block are not equal work. Every candidate
-gives the same bits (lanes sharing a ray add its node terms in node order), so
-the choice only sets the speed. Each candidate is timed with HIP events on a
-representative slice of the real batch and the fastest is kept. Results are cached as JSON keyed by device name, model layout
-(integrand, component kinds, groups), node count and a power-of-two size
-bucket, in ``$ZODI_TUNE_CACHE`` or ``~/.cache/zodipy_amd/tuning.json``.
+the block's tables into LDS) and never shortens the tail (one tile). Static
+grid-stride launches (blocks_per_cu > 0) measured 10 % slower, because equal
+tile counts per block are not equal work. The line kernels of the registry
+models run blocks of 64 and 128 threads as 256, so those are candidates for the
+other kernels only; lanes 0 is the library's own choice (up to 32). Every
+candidate gives the same bits (lanes sharing a ray add its node terms in node
+order), so the choice only sets the speed. Each candidate is timed with HIP
+events on a representative slice of the real batch and the fastest is kept.
+Results are cached as JSON keyed by device name, kernel revision, the kernels the
+block runs (its layout: integrand, component kinds, flags and groups; its
+``zodi_forward_route``), node count and a power-of-two size bucket, in
+``$ZODI_TUNE_CACHE`` or ``~/.cache/zodipy_amd/tuning.json``.
 """
 
 from __future__ import annotations
@@ -30,13 +34,29 @@ from zodipy_amd.runtime import OUT_SUM, DeviceModel
 
 # Kernel variant: 1 = layout-specialised kernel when the model layout has one, else generic.
 VARIANT_AUTO = 1
+# Revision of the forward kernels: shapes tuned for other kernels are not used again.
+KERNEL_REVISION = 2
 
 CANDIDATES = [
     (b, lanes, 0)
     for b in (64, 128, 256, 512)
     for lanes in (1, 2, 4, 8)
     if b // lanes >= 8
-]
+] + [(256, 0, 0)]
+# zodi_forward_route: line kernels, whose smallest block has 256 threads.
+_ROUTE_MASK, _ROUTE_LINE_FIRST, _LINE_MIN_BLOCK = 3, 2, 256
+
+
+def route(dm: DeviceModel) -> int:
+    """The forward kernels the block runs (``zodi_forward_route``)."""
+    return int(dm.lib.zodi_forward_route(_lib.host_ptr(dm.host_block), VARIANT_AUTO))
+
+
+def candidates_for(dm: DeviceModel) -> list[tuple[int, int, int]]:
+    """The launch shapes that run different kernels for this block."""
+    if route(dm) & _ROUTE_MASK >= _ROUTE_LINE_FIRST:
+        return [c for c in CANDIDATES if c[0] >= _LINE_MIN_BLOCK]
+    return CANDIDATES
 
 
 def cache_path() -> Path:
@@ -50,10 +70,11 @@ def layout_key(dm: DeviceModel, n_rays: int) -> str:
     b = dm.host_block[0]
     kinds = ",".join(str(int(k)) for k in b["comp_kind"][: int(b["n_comps"])])
     groups = ",".join(str(int(c)) for c in b["group_count"][: int(b["n_groups"])])
+    flags = ",".join(str(int(f)) for f in b["comp_flags"][: int(b["n_comps"])])
     name = torch.cuda.get_device_name(dm.device).replace(" ", "_")
     bucket = int(np.ceil(np.log2(max(n_rays, 1))))
-    return (f"{name}|v{VARIANT_AUTO}|i{int(b['integrand'])}|k{kinds}|g{groups}"
-            f"|n{int(b['n_nodes'])}|b{bucket}")
+    return (f"{name}|v{VARIANT_AUTO}|r{KERNEL_REVISION}|i{int(b['integrand'])}|k{kinds}|f{flags}"
+            f"|g{groups}|p{route(dm)}|n{int(b['n_nodes'])}|b{bucket}")
 
 
 def _load() -> dict:
@@ -121,7 +142,7 @@ def tune(dm: DeviceModel, u: torch.Tensor, seg, n_seg: int, obs, earth, beyond, 
         n_sub = n_rays
     out = torch.empty((n_sub,), dtype=torch.float64, device=u.device)
     times = {}
-    for b, lanes, per_cu in candidates or CANDIDATES:
+    for b, lanes, per_cu in candidates or candidates_for(dm):
         launch = Launch(b, lanes, per_cu, VARIANT_AUTO)
 
         def fn(launch=launch):

@@ -533,8 +533,6 @@ FwdKernel pick_generic(int block, int L) {
   }
 }
 
-bool takes_line(const zodi_model* m, LayoutId id);
-
 constexpr int kGenericWaves = 3;
 
 // Resident waves per SIMD of the kernel pick_forward chooses.
@@ -612,6 +610,19 @@ FwdKernel pick_forward(const zodi_model* m, int& block, int L, int variant) {
   }
 }
 
+// See zodi_forward_route.
+int forward_route(const zodi_model* m, int variant) {
+  const LayoutId id = variant == 0 ? kLayoutGeneric : match_layout(m);
+  if (id == kLayoutGeneric) return ZODI_ROUTE_GENERIC;
+  if (!takes_line(m, id)) return ZODI_ROUTE_LAYOUT;
+  int route = line_match(m) ? ZODI_ROUTE_LINE : ZODI_ROUTE_LINE_LOGS;
+  if (no_scattering(m)) route |= ZODI_ROUTE_NO_SCATTERING;
+  const bool share =
+      id == kLayoutDirbe ? props_match(m, RegistryProps<LayoutDirbe>::value)
+                         : id == kLayoutKelsall4 && props_match(m, RegistryProps<LayoutKelsall4>::value);
+  return share ? route | ZODI_ROUTE_SHARED_CUT : route;
+}
+
 zodi_status fill_args(FwdArgs& a, const zodi_model* model_host, const zodi_model* model_dev,
                       const double* u, int64_t n_rays, const int64_t* seg_offsets, int32_t n_seg,
                       const double* obs, const double* earth, int32_t obs_mode,
@@ -657,6 +668,11 @@ int32_t zodi_abi_version(void) { return ZODI_ABI_VERSION; }
 int64_t zodi_model_size(void) { return (int64_t)sizeof(zodi_model); }
 
 const char* zodi_last_error(void) { return g_last_error.c_str(); }
+
+int32_t zodi_forward_route(const zodi_model* model_host, int32_t variant) {
+  if (model_host == nullptr || validate_model(model_host) != ZODI_OK) return -1;
+  return forward_route(model_host, variant);
+}
 
 zodi_status zodi_forward(const zodi_model* model_host, const zodi_model* model_dev,
                          const double* u, int64_t n_rays, const int64_t* seg_offsets,
