@@ -495,10 +495,8 @@ zodi_status table_plan(const zodi_model* m, const zodi_launch* launch, int64_t n
 constexpr int64_t kJacobianMaxBytes = int64_t(72) << 30;
 
 // The chi^2 mode of the Kelsall line kernels takes one pass that needs neither J nor I of
-// another: I and the derivatives of a ray come from the same sums. Its held derivatives
-// and tables leave room in 64 KB of LDS for the rows of kOnePassParams parameters.
-constexpr int kOnePassParams = 128;
-
+// another: I and the derivatives of a ray come from the same sums. Its LDS holds the rows of
+// up to kOnePassParams parameters.
 bool chi2_one_pass(const zodi_model* m) {
   return m->integrand == ZODI_INTEGRAND_KELSALL && m->n_params <= kOnePassParams && takes_line(m);
 }

@@ -622,6 +622,12 @@ AdjKernel line_adjoint_rrm(bool split_layout, bool jac);
 constexpr int kLineAdjWaves = 2;
 constexpr int kRrmAdjWaves = 4;
 
+// The one-pass chi^2 keeps a later group's derivatives, its tables and the waves' rows in LDS:
+// 63 KB for DIRBE with scattering and 4 KB of rows at this many parameters (the registry has
+// 78), inside a resident block's share of the CU's 160 KB (checked in line_adj_body).
+constexpr int kOnePassParams = 128;
+constexpr int kLineAdjLds = 160 * 1024 / kLineAdjWaves;
+
 // Resident waves per SIMD the table kernels are compiled for (their register
 // budgets): the registry layouts; the Kelsall ones with the spectral sums of
 // scattering components; the kind switch (at three rather than its

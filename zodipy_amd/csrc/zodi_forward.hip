@@ -589,8 +589,9 @@ int default_lanes(const zodi_model* m, int variant, int64_t n_rays) {
   return 1;
 }
 
-// The line kernels' tables take 12 to 23 KB of LDS a block, so that blocks of 64 and 128
-// threads would leave a CU with few waves: smaller requests run as 256.
+// The line kernels' tables take 10 KB of LDS a block (logarithms, RRM) or 24 KB (power tables),
+// the terms of 8 lanes a ray and more 33 KB besides, so that blocks of 64 and 128 threads would
+// leave a CU with few waves: smaller requests run as 256.
 constexpr int kLineMinBlock = 256;
 
 FwdKernel pick_forward(const zodi_model* m, int& block, int L, int variant) {

@@ -738,6 +738,9 @@ __device__ __forceinline__ void line_adj_body(const AdjArgs& a) {
   } else if constexpr (PASS == kPassChi2) {
     constexpr int kHeld = (layout_comps(LAYOUT{}) - layout_group0(LAYOUT{})) * kHoldRow;
     __shared__ double held[kHeld > 0 ? kHeld * kAdjBlock : 1];
+    static_assert(sizeof(g_exp2) + sizeof(tables) + sizeof(angles) + sizeof(held) +
+                      (kOnePassParams + 1) * kAdjWaves * sizeof(double) <=
+                  kLineAdjLds);
     double* hold = held + (kHeld > 0 ? threadIdx.x : 0);
     rows_body(a, [&](Ray& y, double* row, int ln) {
       double v[7] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
