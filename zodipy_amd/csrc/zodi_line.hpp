@@ -114,7 +114,7 @@ __device__ __forceinline__ void load_planck(ModelPtr M, double2* tab, int i, int
 }
 
 __device__ __forceinline__ double planck_shifted(double u1, const double2* tab) {
-  uint32_t j = (uint32_t)u1;  // saturating: 0 below 0 and for NaN
+  uint32_t j = saturate_u32(u1);  // saturating: 0 below 0 and for NaN
   j = j < (uint32_t)ZODI_N_TEMPS ? j : (uint32_t)ZODI_N_TEMPS;
   const double2 e = tab[j];
   return fma(__builtin_amdgcn_fract(u1), e.y, e.x);

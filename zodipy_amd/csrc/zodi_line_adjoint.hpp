@@ -418,7 +418,7 @@ __device__ __forceinline__ void line_adj_group(Grp<Ks...>, std::integer_sequence
       const double Rd = exp_neg_node(cx.ec, half_delta * lR2);  // R^-delta = dT/dT0
       // B and its step over the table interval (0 outside the table): planck_shifted
       const double u1 = fma(Rd, us, -uo1);
-      uint32_t j = (uint32_t)u1;
+      uint32_t j = saturate_u32(u1);
       j = j < (uint32_t)ZODI_N_TEMPS ? j : (uint32_t)ZODI_N_TEMPS;
       const double2 pl = cx.tab->planck[j];
       const double B = fma(__builtin_amdgcn_fract(u1), pl.y, pl.x);

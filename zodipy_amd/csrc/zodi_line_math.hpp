@@ -84,6 +84,41 @@ ZODI_MATH_FN int frexp_exponent(double x) {
 #endif
 }
 
+// Conversions to 32-bit integers that saturate (NaN: 0), as the hardware's do; a C++ cast of a
+// value out of range is undefined. The sources here are results of plain arithmetic, never of
+// the reciprocal or root instructions, after which a reader needs a wait state that the
+// compiler does not add before an asm.
+ZODI_MATH_FN uint32_t saturate_u32(double x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  uint32_t r;
+  asm("v_cvt_u32_f64 %0, %1" : "=v"(r) : "v"(x));
+  return r;
+#else
+  return x > 0.0 ? (x < 4294967296.0 ? (uint32_t)x : 0xffffffffu) : 0u;
+#endif
+}
+
+ZODI_MATH_FN uint32_t saturate_u32(float x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  uint32_t r;
+  asm("v_cvt_u32_f32 %0, %1" : "=v"(r) : "v"(x));
+  return r;
+#else
+  return saturate_u32((double)x);
+#endif
+}
+
+ZODI_MATH_FN int saturate_i32(double x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  int r;
+  asm("v_cvt_i32_f64 %0, %1" : "=v"(r) : "v"(x));
+  return r;
+#else
+  if (x != x) return 0;
+  return x < -2147483648.0 ? INT32_MIN : (x > 2147483647.0 ? INT32_MAX : (int)x);
+#endif
+}
+
 // ---------------------------------------------------------------- exp
 // exp_neg_node: exp(-x) for |x| < 5.8e6 (NaN passes), within 1.2 ulp. With
 // |x 256/ln2| < 2^31 the integer k = rint(x 256/ln2) is the low word of
@@ -149,7 +184,7 @@ ZODI_MATH_FN double exp_neg_any(const ExpConst& e, double x) {
   const double kd = __builtin_rint(-x * e.inv_l);
   double f = fma(-x, e.inv_l, -kd);
   f = fma(-x, e.inv_lo, f);
-  return exp_node_tail(e, f, (int)kd);
+  return exp_node_tail(e, f, saturate_i32(kd));
 }
 
 // ---------------------------------------------------------------- x^p, p fixed
@@ -211,7 +246,7 @@ ZODI_MATH_FN double exp2_scaled(const ExpConst& ec, double zh, double zl, double
   q = fma(q, f, ec.c3);
   q = fma(q, f, ec.c2);
   q = fma(q, f, ec.c1);
-  const int k = (int)kd, j = k & 255;
+  const int k = saturate_i32(kd), j = k & 255;
   const double t = ZODI_LINE_EXP2[j];
   const double low = fma(t, q * f, kExp2Lo[j]);
   const double p = factor * t;
@@ -332,7 +367,7 @@ ZODI_MATH_FN double unit_angle(const AngleTable& t, double c, double s) {
   q *= sqrtf(1.0f - a);
 #endif
   q = x < 0.0f ? 128.0f - q : q;
-  const uint32_t j = (uint32_t)rintf(q) & 0xffu;
+  const uint32_t j = saturate_u32(rintf(q)) & 0xffu;
   const uint32_t jc = j < 128u ? j : 128u;  // NaN converts to 0
   const double2 e = t.e[jc];
   const double d = fma(s, e.x, -(c * e.y)), z = d * d;

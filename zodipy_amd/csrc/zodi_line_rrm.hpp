@@ -187,7 +187,7 @@ __device__ __forceinline__ RrmNode rrm_node(const LineLogCtx& cx, const Line& l,
   if (o.nd.R2 == 0.0) o.lR2 = __builtin_nan("");
   o.Rd = exp_neg_any(cx.ec, half_delta * o.lR2);
   const double u1 = fma(o.Rd, us, -uo1);
-  uint32_t j = (uint32_t)u1;
+  uint32_t j = saturate_u32(u1);
   j = j < (uint32_t)ZODI_N_TEMPS ? j : (uint32_t)ZODI_N_TEMPS;
   const double2 pl = cx.tab->planck[j];
   o.B = fma(__builtin_amdgcn_fract(u1), pl.y, pl.x);

@@ -264,7 +264,7 @@ struct TableShare {
 };
 
 __device__ __forceinline__ TableShare table_share(double u1, const double2* tab) {
-  uint32_t i = (uint32_t)u1;
+  uint32_t i = saturate_u32(u1);
   i = i < (uint32_t)ZODI_N_TEMPS ? i : (uint32_t)ZODI_N_TEMPS;
   const double2 e = tab[i];
   TableShare t;
