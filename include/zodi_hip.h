@@ -338,7 +338,8 @@ enum {
  * per-ray Jacobian when it fits in 72 GiB and launch allows one lane per ray:
  * one pass then writes the Jacobian and I (zodi_jacobian) and a second forms
  * chi2 and J^T g from them (the Kelsall registry models form I, chi2 and the
- * gradient in one pass instead, and use the workspace for its partial rows); with
+ * gradient in one pass instead, which the same size selects although its partial
+ * rows take a small part of it); with
  * less workspace, or a larger problem, the forward kernel writes I and the adjoint
  * kernel recomputes the integrand with the weights g. The paths agree to rounding.
  * launch may be NULL; otherwise block must be 0 or 256, lanes_per_ray 0 (chosen from

@@ -617,8 +617,9 @@ AdjKernel line_adjoint_rrm(bool split_layout, bool jac);
 
 // Resident blocks per CU (waves per SIMD) that the line adjoint kernels are compiled for.
 // Kelsall at 2: at 3 (168 VGPRs) 42 spilled registers make chi^2 8 % slower on 4.5 M rays.
-// RRM at 4 (128 VGPRs, 33 spilled outside the node loops): the Jacobian of 1 M rays takes
-// 2.46, 2.20 and 2.18 ms at 2, 3 and 4, of 100 000 rays 325, 326 and 294 us.
+// RRM at 4 (128 VGPRs, 43 of the Jacobian's and 65 of the VJP's spilled outside the node
+// loops): the Jacobian of 1 M rays takes 2.03 ms at 3 and 1.99 at 4, of 100 000 rays 335 and
+// 300 us, of 49 152 149 and 155.
 constexpr int kLineAdjWaves = 2;
 constexpr int kRrmAdjWaves = 4;
 

@@ -108,10 +108,11 @@ zodi_status validate_model(const zodi_model* m) {
 
 
 // Minimum waves per SIMD the register allocator must leave room for, per layout
-// (1 = no constraint): the Kelsall layouts at 5 (96 VGPRs; 0.5-1 % faster than at 4), RRM
-// at 4 (105 VGPRs, no spill; at 5 it is 1 % slower). The kind switch (forward_generic)
-// runs at 3. The split-lane variants (L > 1) run only where the launch is small, so
-// they ask for 2 and keep their registers.
+// (1 = no constraint): the Kelsall layouts at 5 (96 VGPRs; at 4, without the 6-component
+// kernel's 10 spilled registers, the batches take the same time within 0.5 %: DIRBE 24.62 and
+// 24.55 ms, planck18 6.19 and 6.22), RRM at 4 (110 VGPRs, no spill; at 5 it is 1 % slower).
+// The kind switch (forward_generic) runs at 3. The split-lane variants (L > 1) run only where
+// the launch is small, so they ask for 2 and keep their registers.
 template <class LAYOUT>
 struct ForwardOccupancy {
   static constexpr int value = 1;
@@ -170,16 +171,17 @@ __device__ __forceinline__ auto line_tables(ModelPtr M, int sub) {
 }
 
 // The Kelsall layouts' registry blocks (props_match without the shared cut-off, and
-// line_match) on the ray's line (zodi_line.hpp): bound by FP64 vector issue, 335 vector
+// line_log_match) on the ray's line (zodi_line.hpp): bound by FP64 vector issue, 339 vector
 // instructions a ray and node of the DIRBE layout where forming every node's position and
-// its powers by exp(p log x) took 487. Measured: DIRBE 12 um, 50.7 M rays, 38.3 -> 26.6 ms
-// (6.6e10 -> 9.5e10 ray-nodes/s); planck18 857 GHz, 22.5 M rays, 9.14 -> 6.71 ms; DIRBE
-// 1.25 um with scattering, 196 608 rays, 0.316 -> 0.219 ms (compiled for 4 waves a SIMD,
+// its powers by exp(p log x) took 487. Measured: DIRBE 12 um, 50.7 M rays, 35.0 -> 24.8 ms
+// (7.2e10 -> 1.02e11 ray-nodes/s); planck18 857 GHz, 22.5 M rays, 8.38 -> 6.22 ms; DIRBE
+// 1.25 um with scattering, 196 608 rays, 0.321 -> 0.223 ms (compiled for 4 waves a SIMD,
 // without spills: 214 -> 200 us of kernel against 5). SHARE: the bands that share a radial
-// cut-off reuse it (kShareCut), for blocks whose delta_r values allow it (the registry parameters; a fit
-// that moves them runs without). NOSCAT (with SHARE): no component scatters, so no
-// scattering code is compiled in. LOGS (without NOSCAT): powers by logarithms, for
-// exponents that the tables do not hold (line_match).
+// cut-off reuse it (kShareCut), for blocks whose delta_r values allow it (the registry
+// parameters; a fit that moves them runs without). NOSCAT (with SHARE): no component
+// scatters, so no scattering code is compiled in. LOGS (without NOSCAT): powers by
+// logarithms, for exponents that the tables do not hold (line_match): 1 M rays at alpha =
+// 2.5 623 us, with tables at 1.34 510.
 template <class LAYOUT, int BLOCK, bool SHARE, bool NOSCAT, bool LOGS = false>
 __global__ __launch_bounds__(BLOCK)
 __attribute__((amdgpu_waves_per_eu(NOSCAT ? ForwardOccupancy<LAYOUT>::value : 4))) void
@@ -217,7 +219,7 @@ forward_line_split(FwdArgs a) {
 // The RRM layouts' registry blocks (every component centred) on the ray's line: 3580 issue
 // cycles per wave and node over the six groups where the arc sines, sines, cosines and
 // powers of every node took 6750 (and less where a wave skips a branch). Measured: RRM 25
-// um, 196 608 rays with the pixel vectors, 0.524 -> 0.300 ms (two lanes a ray).
+// um, 196 608 rays with the pixel vectors, 0.532 -> 0.309 ms (two lanes a ray).
 template <class LAYOUT, int BLOCK>
 __global__ __launch_bounds__(BLOCK)
 __attribute__((amdgpu_waves_per_eu(ForwardOccupancy<LAYOUT>::value))) void
@@ -619,8 +621,8 @@ int forward_route(const zodi_model* m, int variant) {
   int route = line_match(m) ? ZODI_ROUTE_LINE : ZODI_ROUTE_LINE_LOGS;
   if (no_scattering(m)) route |= ZODI_ROUTE_NO_SCATTERING;
   const bool share =
-      id == kLayoutDirbe ? props_match(m, RegistryProps<LayoutDirbe>::value)
-                         : id == kLayoutKelsall4 && props_match(m, RegistryProps<LayoutKelsall4>::value);
+      (id == kLayoutDirbe && props_match(m, RegistryProps<LayoutDirbe>::value)) ||
+      (id == kLayoutKelsall4 && props_match(m, RegistryProps<LayoutKelsall4>::value));
   return share ? route | ZODI_ROUTE_SHARED_CUT : route;
 }
 

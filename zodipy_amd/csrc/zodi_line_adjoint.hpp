@@ -587,8 +587,8 @@ __device__ __forceinline__ void line_adj_group(Grp<Ks...>, std::integer_sequence
 // The held derivatives of a later group's components, weighted onto the wave's row.
 template <int NC, int C0, int... Ks, int... J>
 __device__ __forceinline__ void add_held(Grp<Ks...>, std::integer_sequence<int, J...>,
-                                         ModelPtr M, int first, const Chi2Ray<NC, C0>& cr, double* row, int lane,
-                                         const double* hold) {
+                                         ModelPtr M, int first, const Chi2Ray<NC, C0>& cr,
+                                         double* row, int lane, const double* hold) {
   constexpr int kinds[sizeof...(Ks)] = {Ks...};
   (
       [&] {

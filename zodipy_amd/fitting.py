@@ -17,11 +17,12 @@ recomputes the integrand instead of storing node values:
 * ``emission(theta, problem)`` -- a ``torch.autograd.Function``: forward is the
   line-of-sight integral, backward is one adjoint launch with the incoming
   gradient as weights;
-* ``chi2(theta, problem, data, inv_var)`` -- one library call: one pass writes
-  the model values and the per-ray Jacobian into the workspace and a second
-  forms chi^2 and J^T g (or, with ``store_jacobian=False`` or a Jacobian over
-  72 GiB, the forward kernel writes the model values and one adjoint launch
-  forms chi^2 and d(chi^2)/d(theta)); backward scales the stored gradient;
+* ``chi2(theta, problem, data, inv_var)`` -- one library call: the Kelsall
+  registry models form the model values, chi^2 and its gradient in one pass; the
+  others write the model values and the per-ray Jacobian into the workspace, and
+  a second pass forms chi^2 and J^T g. With ``store_jacobian=False`` or a Jacobian
+  over 72 GiB the forward kernel writes the model values and one adjoint launch
+  forms chi^2 and d(chi^2)/d(theta). Backward scales the stored gradient;
 * ``LineOfSightProblem.jacobian(theta)`` -- the model values and the per-ray
   Jacobian dI_r/dtheta_p themselves, for Gauss-Newton or Fisher-matrix work.
 
@@ -146,8 +147,9 @@ class LineOfSightProblem:
     heliocentric ecliptic positions [AU], (3,) for one observer, (3, n_seg) with
     ``seg_offsets`` (n_seg + 1,) for observers owning consecutive ray ranges, or
     (3, n) with ``per_ray=True`` (one reference call over time-ordered data).
-    ``store_jacobian``: let chi^2 keep the per-ray Jacobian (n_params x n doubles)
-    in its workspace, which saves the separate forward pass.
+    ``store_jacobian``: let chi^2 have a workspace of the per-ray Jacobian's size
+    (n_params x n doubles), which saves the separate forward pass; the Kelsall registry
+    models' one pass is chosen by that size too, though it uses a small part of it.
     """
 
     def __init__(self, model, unit_vectors, obspos, earthpos, seg_offsets=None,
